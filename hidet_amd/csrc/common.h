@@ -188,13 +188,8 @@ inline Workspace split_workspace(void *workspace, int64_t bytes) {
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
-// float32 -> bfloat16 bits, round to nearest even (NaN kept quiet)
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-}
+// float32 -> bfloat16 bits, round to nearest even (NaN kept quiet): v_cvt_pk_bf16_f32
+__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
     _Float16 h = static_cast<_Float16>(f);  // v_cvt_f16_f32: round to nearest even

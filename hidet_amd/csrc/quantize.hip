@@ -15,62 +15,228 @@ __global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
-// amax over the middle axis of [outer, R, inner] when inner > 1 (strided reduction).
-// grid (ceil(inner/64), outer, row_splits); 256 threads = 4 row lanes x 64 columns.
-template <int DT>
-__global__ __launch_bounds__(256) void amax_strided_kernel(const void *__restrict__ w, uint32_t *__restrict__ amax_bits,
-                                                           int64_t R, int64_t inner, int64_t rows_per_split,
-                                                           int use_atomic) {
-    __shared__ float red[4][64];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t col = int64_t(blockIdx.x) * 64 + tx;
-    const int64_t o = blockIdx.y;
-    const int64_t r0 = int64_t(blockIdx.z) * rows_per_split;
-    const int64_t r1 = min(R, r0 + rows_per_split);
-    float m = 0.0f;
-    if (col < inner) {
-        const int64_t base = o * R * inner + col;
-        int64_t r = r0 + ty;
-        for (; r + 28 < r1; r += 32) {
-            float v[8];
+// Nearest integer (ties to even) of v, |v| < 2^21, in the low bits of the returned word.
+__device__ __forceinline__ uint32_t nearest_bits(float v) { return __float_as_uint(v + 12582912.0f); }  // 1.5 * 2^23
+
+// code[e] = round_half_away(fl(x[e] / s[e])) as integers in the low bits, clamped to +-bound: the value IEEE division
+// followed by roundf gives, with the division left out where it cannot matter. x * rcp(s) is within 2^-22 of the quotient
+// (rcp is good to one unit in the last place, then two roundings), so its nearest integer is the answer unless it lies within bound * 2^-21 of a tie. |x| is at most the
+// maximum the scale was made from, so that answer needs no clamp. `fast` is false for a scale whose reciprocal may be
+// imprecise (zero, tiny, huge, NaN); a NaN among x fails the comparison and takes the division. 5 issue slots per element
+// instead of 20: dividing every element kept the quantizers at the VALU's rate.
+__device__ __forceinline__ void round_quotients_f32(const float (&x)[4], const float (&s)[4], const float (&inv)[4], bool fast, float low,
+                                                    float high, uint32_t (&code)[4]) {
+    const float limit = 0.5f - (high + 1.0f) * 0x1p-21f;
+    bool sure = fast;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = load_as_f32<DT>(w, base + (r + 4 * i) * inner);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));
-        }
-        for (; r < r1; r += 4) m = fmaxf(m, fabsf(load_as_f32<DT>(w, base + r * inner)));
+    for (int e = 0; e < 4; ++e) {
+        const float t = __builtin_fmaf(x[e], inv[e], 12582912.0f);
+        code[e] = __float_as_uint(t);
+        sure = sure && fabsf(__builtin_fmaf(x[e], inv[e], 12582912.0f - t)) < limit;
     }
-    red[ty][tx] = m;
+    if (__builtin_expect(!sure, 0)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) code[e] = s[e] != 0.0f ? uint32_t(int(fminf(fmaxf(roundf(x[e] / s[e]), low), high))) : 0u;
+    }
+}
+__device__ __forceinline__ bool reciprocal_is_precise(float s) {
+    const float a = fabsf(s);
+    return a >= 0x1p-100f && a <= 0x1p100f;
+}
+
+// The 16-bit types: rint(rnd(fl(x[e] / s[e]))), rnd = round to the type (ties to even, as the reference's GPU lowering),
+// without the division. q = x * rcp(s) is within 2^-22 of the quotient, its remainder x - q s is exact (s has at most 11
+// significant bits), and one correction leaves q within 2^-24 (1 + 2^-19). A quotient of two 11-bit numbers that is not
+// itself a midpoint between two numbers of the type (12 bits) is at least 2^-23 away from one, and one that is comes out
+// exactly: q rounds as the quotient does. (NaN gives the lowest code, as the clamp of the division's result does.)
+template <int DT>
+__device__ __forceinline__ void round_quotients_16(const float (&x)[4], const float (&s)[4], const float (&inv)[4], bool fast, float low,
+                                                   float high, uint32_t (&code)[4]) {
+    if (__builtin_expect(fast, 1)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float q = x[e] * inv[e];
+            q = __builtin_fmaf(__builtin_fmaf(-q, s[e], x[e]), inv[e], q);
+            code[e] = nearest_bits(__builtin_amdgcn_fmed3f(round_to<DT>(q), low, high));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) code[e] = s[e] != 0.0f ? uint32_t(int(fminf(fmaxf(rintf(round_to<DT>(x[e] / s[e])), low), high))) : 0u;
+    }
+}
+
+// Codes of four elements, in the low bits: saturating_cast(round(rnd(w / scale))), zero where the scale is.
+template <int DT, int QT>
+__device__ __forceinline__ void codes4(const float (&x)[4], const float (&s)[4], const float (&inv)[4], bool fast, uint32_t (&code)[4]) {
+    constexpr float low = QT == HIDET_QMM_I8 ? -128.0f : -32768.0f, high = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
+    if constexpr (DT == HIDET_QMM_F32) round_quotients_f32(x, s, inv, fast, low, high, code);
+    else round_quotients_16<DT>(x, s, inv, fast, low, high, code);
+}
+
+// Scales of four columns from their maxima, and what codes4 wants to know about them.
+template <int DT, int QT>
+__device__ __forceinline__ bool scales4(const float (&amax)[4], float (&s)[4], float (&inv)[4]) {
+    const float qmax = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
+    bool fast = true;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        s[e] = round_to<DT>(amax[e] / qmax);
+        inv[e] = __builtin_amdgcn_rcpf(s[e]);
+        fast = fast && reciprocal_is_precise(s[e]);
+    }
+    return fast;
+}
+
+// Four elements at the alignment of one: rows of an odd length start anywhere (the hardware takes such accesses whole).
+typedef float float4_at4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t half4_at2_t __attribute__((ext_vector_type(4), aligned(2)));
+
+// Elements i .. i + 3, the ones from `count` on left out (read as zero, not stored).
+template <int DT>
+__device__ __forceinline__ void load_upto4(const void *p, int64_t i, int64_t count, float (&x)[4]) {
+    if (count >= 4) {
+        if constexpr (DT == HIDET_QMM_F32) {
+            const float4_at4_t v = *reinterpret_cast<const float4_at4_t *>(static_cast<const float *>(p) + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = v[e];
+        } else {
+            const half4_at2_t v = *reinterpret_cast<const half4_at2_t *>(static_cast<const uint16_t *>(p) + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = DT == HIDET_QMM_F16 ? f16_bits_to_f32(v[e]) : bf16_bits_to_f32(v[e]);
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        x[e] = 0.0f;
+        if (e < count) x[e] = load_as_f32<DT>(p, i + e);
+    }
+}
+template <int DT>
+__device__ __forceinline__ void store_upto4(void *p, int64_t i, int64_t count, const float (&x)[4]) {  // values of the type
+    if (count >= 4) {
+        if constexpr (DT == HIDET_QMM_F32) {
+            *reinterpret_cast<float4_at4_t *>(static_cast<float *>(p) + i) = float4_at4_t{x[0], x[1], x[2], x[3]};
+        } else {
+            half4_at2_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = DT == HIDET_QMM_F16 ? f32_to_f16_bits(x[e]) : f32_to_bf16_bits(x[e]);
+            *reinterpret_cast<half4_at2_t *>(static_cast<uint16_t *>(p) + i) = v;
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (e < count) store_from_f32<DT>(p, i + e, x[e]);
+}
+template <int QT>
+__device__ __forceinline__ void store_codes_upto4(void *p, int64_t i, int64_t count, const uint32_t (&code)[4]) {  // low bits of each
+    if constexpr (QT == HIDET_QMM_I8) {
+        const uint32_t lo = __builtin_amdgcn_perm(code[1], code[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(code[3], code[2], 0x0c0c0400u);
+        const uint32_t packed = lo | (hi << 16);
+        int8_t *o = static_cast<int8_t *>(p) + i;
+        if (count >= 4) {
+            __builtin_memcpy(o, &packed, 4);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < count) o[e] = int8_t(packed >> (8 * e));
+        }
+    } else {
+        int16_t *o = static_cast<int16_t *>(p) + i;
+        if (count >= 4) {
+            *reinterpret_cast<half4_at2_t *>(o) = half4_at2_t{uint16_t(code[0]), uint16_t(code[1]), uint16_t(code[2]), uint16_t(code[3])};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < count) o[e] = int16_t(code[e]);
+        }
+    }
+}
+template <int QT>
+__device__ __forceinline__ void load_codes_upto4(const void *p, int64_t i, int64_t count, float (&code)[4]) {
+    if constexpr (QT == HIDET_QMM_I8) {
+        uint32_t v = 0;
+        const int8_t *q = static_cast<const int8_t *>(p) + i;
+        if (count >= 4) {
+            __builtin_memcpy(&v, q, 4);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < count) v |= uint32_t(uint8_t(q[e])) << (8 * e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) code[e] = float(int8_t(v >> (8 * e)));
+    } else {
+        const int16_t *q = static_cast<const int16_t *>(p) + i;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) code[e] = e < count ? float(q[e]) : 0.0f;
+    }
+}
+
+// Maxima over the middle axis of [outer, R, inner], inner > 1 (strided reduction): kAmaxLanes row lanes x 64 column quads,
+// 4 rows of 16 bytes (float32) in flight per thread. Block x = column block, y = row range, z = outer: the ranges of one
+// column leave their maxima in rows of their own of `amax` [ranges, outer * inner], which the quantizing kernel takes
+// together (one atomic per range and column instead wants the array cleared by a launch of its own). Bound by memory: K = 4096,
+// N = 11008, float32 in 37 - 38 us = 4.8 TB/s, what a copy reaches (4-byte loads, 64 columns per workgroup, and the
+// clearing launch in front: 40.6 us and 2 - 5 us).
+constexpr int kAmaxLanes = 16, kAmaxRows = 4;
+template <int DT>
+__global__ __launch_bounds__(64 * kAmaxLanes) void amax_strided_kernel(const void *__restrict__ w, float *__restrict__ amax, int64_t R,
+                                                                       int64_t inner, int64_t rows_per_range, int64_t nscale) {
+    __shared__ float4_t red[kAmaxLanes][64];
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // a wave's row is a scalar
+    const int64_t col = int64_t(blockIdx.x) * 256 + 4 * tx;
+    const int64_t o = blockIdx.z, count = inner - col;
+    const int64_t r1 = min(R, (int64_t(blockIdx.y) + 1) * rows_per_range);
+    float m[4] = {0.f, 0.f, 0.f, 0.f};
+    if (count > 0) {
+        const int64_t base = o * R * inner;
+        int64_t r = int64_t(blockIdx.y) * rows_per_range + ty;
+        for (; r + kAmaxLanes * (kAmaxRows - 1) < r1; r += kAmaxLanes * kAmaxRows) {
+            float v[kAmaxRows][4];
+#pragma unroll
+            for (int i = 0; i < kAmaxRows; ++i) load_upto4<DT>(w, base + (r + kAmaxLanes * i) * inner + col, count, v[i]);
+#pragma unroll
+            for (int i = 0; i < kAmaxRows; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[i][e]));
+        }
+        for (; r < r1; r += kAmaxLanes) {
+            float v[4];
+            load_upto4<DT>(w, base + r * inner + col, count, v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[e]));
+        }
+    }
+    red[ty][tx] = float4_t{m[0], m[1], m[2], m[3]};
     __syncthreads();
-    if (ty == 0 && col < inner) {
-        m = fmaxf(fmaxf(red[0][tx], red[1][tx]), fmaxf(red[2][tx], red[3][tx]));
-        // |x| >= 0: the unsigned order of the bit patterns is the order of the values
-        if (use_atomic) atomicMax(&amax_bits[o * inner + col], __float_as_uint(m));
-        else amax_bits[o * inner + col] = __float_as_uint(m);
+    if (ty == 0 && count > 0) {
+#pragma unroll 4
+        for (int t = 1; t < kAmaxLanes; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t][tx][e]);
+        store_upto4<HIDET_QMM_F32>(amax, int64_t(blockIdx.y) * nscale + o * inner + col, count, m);
     }
 }
 
 // amax over the last axis of [outer, R] (inner == 1): one wave per row, 4 rows per block.
 template <int DT>
-__global__ __launch_bounds__(256) void amax_contig_kernel(const void *__restrict__ w, uint32_t *__restrict__ amax_bits,
+__global__ __launch_bounds__(256) void amax_contig_kernel(const void *__restrict__ w, float *__restrict__ amax,
                                                           int64_t outer, int64_t R) {
     const int lane = threadIdx.x & 63;
     const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (row >= outer) return;
     float m = 0.0f;
-    for (int64_t r = lane; r < R; r += 64) m = fmaxf(m, fabsf(load_as_f32<DT>(w, row * R + r)));
+    for (int64_t r = lane * 4; r < R; r += 256) {
+        float v[4];
+        load_upto4<DT>(w, row * R + r, R - r, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[e]));
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    if (lane == 0) amax_bits[row] = __float_as_uint(m);
-}
-
-template <int QT>
-__device__ __forceinline__ void store_code(void *q, int64_t i, float r) {
-    if (QT == HIDET_QMM_I8) {
-        static_cast<int8_t *>(q)[i] = static_cast<int8_t>(fminf(fmaxf(r, -128.0f), 127.0f));
-    } else {
-        static_cast<int16_t *>(q)[i] = static_cast<int16_t>(fminf(fmaxf(r, -32768.0f), 32767.0f));
-    }
+    if (lane == 0) amax[row] = m;
 }
 
 // Four-element forms (numel a multiple of 4, 16-byte aligned input, 4-byte aligned codes).
@@ -93,131 +259,76 @@ __device__ __forceinline__ void load4_as_f32(const void *p, int64_t i4, float (&
 // bfloat16 (hrint, cuda/math/bfloat16.py:29; the reference has no HIP bfloat16 math set). Its CPU half types round ties
 // away instead (include/hidet/runtime/cpu/float16.h:747-750): a float16 quotient of exactly n + 0.5 - common, since
 // float16 has a spacing of 1/16 between 64 and 128 - differs by one code between the two targets.
-template <int DT>
-__device__ __forceinline__ float round_code(float q) {
-    return DT == HIDET_QMM_F32 ? roundf(q) : rintf(q);
-}
+// (codes4 and scales4 above.)
 
+// Columns of [outer, R, inner] quantized from their maxima (`ranges` <= kMaxRanges rows of them, amax_strided_kernel):
+// kQuantLanes row lanes x 64 column quads. The workgroup puts its columns' maxima together, a thread works out the scales
+// of its four columns once and takes 8 rows, four 16-byte loads in flight together. Block x counts column blocks, then row
+// blocks of kQuantRows; z = outer. 64 rows per workgroup pay for the maxima and scales (16: 51 us); all eight loads of a
+// thread at once cost the occupancy that hides them (16-bit types: 44 instead of 28 us). K = 4096, N = 11008: float32 35 - 36 us
+// (the second read comes from the last-level cache: 6.3 TB/s), bfloat16 36 -> 28 us (the divisions).
+constexpr int kQuantLanes = 8, kQuantTrip = 4, kQuantRows = 2 * kQuantLanes * kQuantTrip, kMaxRanges = 32;
 template <int DT, int QT>
-__global__ __launch_bounds__(256) void quantize_kernel(const void *__restrict__ w, const uint32_t *__restrict__ amax_bits,
-                                                       void *__restrict__ q, void *__restrict__ scale, int64_t R,
-                                                       int64_t inner, int64_t total) {
-    const float qmax = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int64_t o = i / (R * inner);
-    const int64_t rem = i - o * R * inner;
-    const int64_t r = rem / inner, c = rem - r * inner;
-    const float amax = __uint_as_float(amax_bits[o * inner + c]);
-    const float s = round_to<DT>(amax / qmax);
-    if (r == 0) store_from_f32<DT>(scale, o * inner + c, s);
-    float code = 0.0f;
-    if (s != 0.0f) code = round_code<DT>(round_to<DT>(load_as_f32<DT>(w, i) / s));
-    store_code<QT>(q, i, code);
-}
-
-// Same arithmetic, four consecutive elements of the innermost axis per thread (inner a multiple of 4, tensors aligned
-// for the 4-element accesses): one index division per four elements, 16- or 8-byte loads, 4- or 8-byte code stores.
-// ALONG_REDUCE (inner == 1, reduce a multiple of 4): the four elements lie along the reduced axis and share one scale;
-// R is then reduce / 4 and inner4 is unused.
-template <int DT, int QT, bool ALONG_REDUCE>
-__global__ __launch_bounds__(256) void quantize4_kernel(const void *__restrict__ w, const uint32_t *__restrict__ amax_bits,
-                                                        void *__restrict__ q, void *__restrict__ scale, int64_t R,
-                                                        int64_t inner4, int64_t total4) {
-    const float qmax = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
-    const int64_t i4 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i4 >= total4) return;
-    int64_t r, sidx;
-    uint32_t abits[4];
-    if (ALONG_REDUCE) {
-        sidx = i4 / R;
-        r = i4 - sidx * R;
-        abits[0] = abits[1] = abits[2] = abits[3] = amax_bits[sidx];
-    } else {
-        const int64_t row = i4 / inner4;  // o * R + r
-        const int64_t c4 = i4 - row * inner4;
-        const int64_t o = row / R;
-        r = row - o * R;
-        sidx = (o * inner4 + c4) * 4;
-        const uint4 ab = *reinterpret_cast<const uint4 *>(amax_bits + sidx);
-        abits[0] = ab.x; abits[1] = ab.y; abits[2] = ab.z; abits[3] = ab.w;
-    }
-    float x[4];
-    if (DT == HIDET_QMM_F32) {
-        const float4 v = *reinterpret_cast<const float4 *>(static_cast<const float *>(w) + i4 * 4);
-        x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-    } else {
-        const uint2 v = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(w) + i4 * 4);
-        const uint16_t h[4] = {uint16_t(v.x), uint16_t(v.x >> 16), uint16_t(v.y), uint16_t(v.y >> 16)};
+__global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const void *__restrict__ w, const float *__restrict__ amax, int ranges,
+                                                                         int64_t nscale, void *__restrict__ q, void *__restrict__ scale,
+                                                                         int64_t R, int64_t inner, uint32_t col_blocks) {
+    __shared__ float4_t red[kQuantLanes][64];
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // a wave's row is a scalar
+    const int64_t col = int64_t(blockIdx.x % col_blocks) * 256 + 4 * tx, row0 = int64_t(blockIdx.x / col_blocks) * kQuantRows;
+    const int64_t o = blockIdx.z, count = inner - col;
+    float m[4] = {0.f, 0.f, 0.f, 0.f};
+    if (count > 0) {
+        for (int i = ty; i < ranges; i += kQuantLanes) {
+            float v[4];
+            load_upto4<HIDET_QMM_F32>(amax, i * nscale + o * inner + col, count, v);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = DT == HIDET_QMM_F16 ? f16_bits_to_f32(h[e]) : bf16_bits_to_f32(h[e]);
-    }
-    float code[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float s = round_to<DT>(__uint_as_float(abits[e]) / qmax);
-        if (r == 0 && (!ALONG_REDUCE || e == 0)) store_from_f32<DT>(scale, sidx + (ALONG_REDUCE ? 0 : e), s);
-        code[e] = s != 0.0f ? round_code<DT>(round_to<DT>(x[e] / s)) : 0.0f;
-    }
-    if (QT == HIDET_QMM_I8) {
-        uint32_t packed = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) packed |= uint32_t(uint8_t(int8_t(fminf(fmaxf(code[e], -128.0f), 127.0f)))) << (8 * e);
-        static_cast<uint32_t *>(q)[i4] = packed;
-    } else {
-        uint2 packed;
-        uint32_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = uint32_t(uint16_t(int16_t(fminf(fmaxf(code[e], -32768.0f), 32767.0f))));
-        packed.x = h[0] | (h[1] << 16);
-        packed.y = h[2] | (h[3] << 16);
-        static_cast<uint2 *>(q)[i4] = packed;
-    }
-}
-
-// Same arithmetic for [outer, R, inner] with inner a multiple of 4, laid out so that nothing is recomputed per element:
-// grid (ceil(inner / 256), ceil(R / kQuantRows), outer), 256 threads = 4 row lanes x 64 column quads. A thread keeps its
-// four columns, works out their four scales once (the element-per-thread kernels divide amax / qmax again for every
-// element and pay two 64-bit index divisions per thread) and walks kQuantRows / 4 rows with 16-byte loads.
-constexpr int kQuantRows = 32;
-template <int DT, int QT>
-__global__ __launch_bounds__(256) void quantize_rows_kernel(const void *__restrict__ w, const uint32_t *__restrict__ amax_bits,
-                                                            void *__restrict__ q, void *__restrict__ scale, int64_t R,
-                                                            int64_t inner4) {
-    const float qmax = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t c4 = int64_t(blockIdx.x) * 64 + tx;
-    if (c4 >= inner4) return;
-    const int64_t o = blockIdx.z;
-    const int64_t sidx = (o * inner4 + c4) * 4;
-    const uint4 ab = *reinterpret_cast<const uint4 *>(amax_bits + sidx);
-    const uint32_t abits[4] = {ab.x, ab.y, ab.z, ab.w};
-    float s[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = round_to<DT>(__uint_as_float(abits[e]) / qmax);
-    if (blockIdx.y == 0 && ty == 0) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) store_from_f32<DT>(scale, sidx + e, s[e]);
-    }
-    const int64_t r_end = min(R, (int64_t(blockIdx.y) + 1) * kQuantRows);
-    for (int64_t r = int64_t(blockIdx.y) * kQuantRows + ty; r < r_end; r += 4) {
-        const int64_t i4 = (o * R + r) * inner4 + c4;
-        float x[4], code[4];
-        load4_as_f32<DT>(w, i4, x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) code[e] = s[e] != 0.0f ? round_code<DT>(round_to<DT>(x[e] / s[e])) : 0.0f;
-        if (QT == HIDET_QMM_I8) {
-            uint32_t packed = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) packed |= uint32_t(uint8_t(int8_t(fminf(fmaxf(code[e], -128.0f), 127.0f)))) << (8 * e);
-            static_cast<uint32_t *>(q)[i4] = packed;
-        } else {
-            uint32_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = uint32_t(uint16_t(int16_t(fminf(fmaxf(code[e], -32768.0f), 32767.0f))));
-            static_cast<uint2 *>(q)[i4] = uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], v[e]);
         }
     }
+    red[ty][tx] = float4_t{m[0], m[1], m[2], m[3]};
+    __syncthreads();
+#pragma unroll 4
+    for (int t = 0; t < kQuantLanes; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t][tx][e]);
+    if (count <= 0) return;
+    float s[4], inv[4];
+    const bool fast = scales4<DT, QT>(m, s, inv);
+    if (row0 == 0 && ty == 0) store_upto4<DT>(scale, o * inner + col, count, s);
+    const int64_t r_end = min(R, row0 + kQuantRows);
+    for (int64_t r = row0 + ty; r < r_end; r += kQuantLanes * kQuantTrip) {
+        const int64_t base = (o * R + r) * inner;
+        float x[kQuantTrip][4];
+#pragma unroll
+        for (int j = 0; j < kQuantTrip; ++j)
+            if (r + kQuantLanes * j < r_end) load_upto4<DT>(w, base + kQuantLanes * j * inner + col, count, x[j]);
+#pragma unroll
+        for (int j = 0; j < kQuantTrip; ++j) {
+            if (r + kQuantLanes * j >= r_end) break;
+            uint32_t code[4];
+            codes4<DT, QT>(x[j], s, inv, fast, code);
+            store_codes_upto4<QT>(q, base + kQuantLanes * j * inner + col, count, code);
+        }
+    }
+}
+
+// inner == 1, rows too long for a workgroup's registers: four (or fewer, at a row's end) elements per thread from the
+// row's maximum. Block x counts blocks of 1024 elements within a row, y = row.
+template <int DT, int QT>
+__global__ __launch_bounds__(256) void quantize_long_row_kernel(const void *__restrict__ w, const float *__restrict__ amax, void *__restrict__ q,
+                                                                void *__restrict__ scale, int64_t R, uint32_t blocks_per_row) {
+    const int64_t row = blockIdx.x / blocks_per_row;
+    const int64_t c = (int64_t(blockIdx.x % blocks_per_row) * 256 + threadIdx.x) * 4, count = R - c;
+    if (count <= 0) return;
+    const float a = amax[row];
+    const float m[4] = {a, a, a, a};
+    float s[4], inv[4], x[4];
+    uint32_t code[4];
+    const bool fast = scales4<DT, QT>(m, s, inv);
+    if (c == 0) store_from_f32<DT>(scale, row, s[0]);
+    load_upto4<DT>(w, row * R + c, count, x);
+    codes4<DT, QT>(x, s, inv, fast, code);
+    store_codes_upto4<QT>(q, row * R + c, count, code);
 }
 
 // inner == 1 (one scale per row, e.g. an embedding table): one workgroup per row keeps the whole row in registers
@@ -227,7 +338,6 @@ template <int DT, int QT, int NV>
 __global__ __launch_bounds__(256) void quantize_row_fused_kernel(const void *__restrict__ w, void *__restrict__ q,
                                                                  void *__restrict__ scale, int64_t R4) {
     __shared__ float red[4];
-    const float qmax = QT == HIDET_QMM_I8 ? 127.0f : 32767.0f;
     const int tid = threadIdx.x;
     const int64_t base4 = int64_t(blockIdx.x) * R4;
     float x[NV][4];
@@ -245,202 +355,233 @@ __global__ __launch_bounds__(256) void quantize_row_fused_kernel(const void *__r
     if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float s = round_to<DT>(m / qmax);
-    if (tid == 0) store_from_f32<DT>(scale, blockIdx.x, s);
+    const float mm[4] = {m, m, m, m};
+    float s[4], inv[4];
+    const bool fast = scales4<DT, QT>(mm, s, inv);
+    if (tid == 0) store_from_f32<DT>(scale, blockIdx.x, s[0]);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int64_t j = int64_t(v) * 256 + tid;
         if (j >= R4) continue;
-        float code[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) code[e] = s != 0.0f ? round_code<DT>(round_to<DT>(x[v][e] / s)) : 0.0f;
-        if (QT == HIDET_QMM_I8) {
-            uint32_t packed = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) packed |= uint32_t(uint8_t(int8_t(fminf(fmaxf(code[e], -128.0f), 127.0f)))) << (8 * e);
-            static_cast<uint32_t *>(q)[base4 + j] = packed;
-        } else {
-            uint32_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = uint32_t(uint16_t(int16_t(fminf(fmaxf(code[e], -32768.0f), 32767.0f))));
-            static_cast<uint2 *>(q)[base4 + j] = uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-        }
+        uint32_t code[4];
+        codes4<DT, QT>(x[v], s, inv, fast, code);
+        store_codes_upto4<QT>(q, (base4 + j) * 4, 4, code);
     }
 }
 
+constexpr int kDequantRows = 32;
+// Codes times scales. inner > 1: 256 threads = 4 row lanes x 64 column quads, a thread keeps its four columns' scales over
+// kDequantRows / 4 rows (one index division per workgroup, where a thread per four elements pays two of 64 bits:
+// bfloat16 4096 x 11008
+// 35 -> 22 us, a row length that is no multiple of four 75 -> 31 us). Block x counts column blocks, then row blocks; z = outer.
 template <int QT, int ST>
-__global__ __launch_bounds__(256) void dequantize_kernel(const void *__restrict__ q, const void *__restrict__ scale,
-                                                         void *__restrict__ w, int64_t R, int64_t inner, int64_t total) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int64_t o = i / (R * inner);
-    const int64_t c = (i - o * R * inner) % inner;
-    const float code = QT == HIDET_QMM_I8 ? float(static_cast<const int8_t *>(q)[i]) : float(static_cast<const int16_t *>(q)[i]);
-    store_from_f32<ST>(w, i, round_to<ST>(code * load_as_f32<ST>(scale, o * inner + c)));
-}
-
-// Four consecutive elements per thread: along the innermost axis (inner4 = inner / 4, one scale each) or, with
-// ALONG_REDUCE (inner == 1, R = reduce / 4), along the reduced axis (one scale for all four).
-template <int QT, int ST, bool ALONG_REDUCE>
-__global__ __launch_bounds__(256) void dequantize4_kernel(const void *__restrict__ q, const void *__restrict__ scale,
-                                                          void *__restrict__ w, int64_t R, int64_t inner4, int64_t total4) {
-    const int64_t i4 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i4 >= total4) return;
-    float code[4], sc[4];
-    if (QT == HIDET_QMM_I8) {
-        const uint32_t v = static_cast<const uint32_t *>(q)[i4];
+__global__ __launch_bounds__(256) void dequantize_rows_kernel(const void *__restrict__ q, const void *__restrict__ scale, void *__restrict__ w,
+                                                              int64_t R, int64_t inner, uint32_t col_blocks) {
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int64_t col = int64_t(blockIdx.x % col_blocks) * 256 + 4 * tx, row0 = int64_t(blockIdx.x / col_blocks) * kDequantRows;
+    const int64_t o = blockIdx.z, count = inner - col;
+    if (count <= 0) return;
+    float s[4];
+    load_upto4<ST>(scale, o * inner + col, count, s);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) code[e] = float(int8_t(v >> (8 * e)));
-    } else {
-        const uint2 v = static_cast<const uint2 *>(q)[i4];
-        code[0] = float(int16_t(v.x)); code[1] = float(int16_t(v.x >> 16));
-        code[2] = float(int16_t(v.y)); code[3] = float(int16_t(v.y >> 16));
-    }
-    if (ALONG_REDUCE) {
-        sc[0] = sc[1] = sc[2] = sc[3] = load_as_f32<ST>(scale, i4 / R);
-    } else {
-        const int64_t row = i4 / inner4;
-        const int64_t sidx = ((row / R) * inner4 + (i4 - row * inner4)) * 4;
-        load4_as_f32<ST>(scale, sidx / 4, sc);
-    }
-    float out[4];
+    for (int j = 0; j < kDequantRows / 4; ++j) {
+        const int64_t r = row0 + 4 * j + ty;
+        if (r >= R) break;
+        const int64_t i = (o * R + r) * inner + col;
+        float code[4], out[4];
+        load_codes_upto4<QT>(q, i, count, code);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * sc[e]);
-    if (ST == HIDET_QMM_F32) {
-        static_cast<float4 *>(w)[i4] = float4{out[0], out[1], out[2], out[3]};
-    } else {
-        uint32_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = ST == HIDET_QMM_F16 ? f32_to_f16_bits(out[e]) : f32_to_bf16_bits(out[e]);
-        static_cast<uint2 *>(w)[i4] = uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+        for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * s[e]);
+        store_upto4<ST>(w, i, count, out);
     }
 }
 
-// Group-wise int4: grid (ceil(n/128), k/group); 256 threads = 4 row lanes x 64 column pairs.
+// inner == 1: one scale per row. Block x counts blocks of 4096 elements within a row, then rows.
+template <int QT, int ST>
+__global__ __launch_bounds__(256) void dequantize_long_row_kernel(const void *__restrict__ q, const void *__restrict__ scale, void *__restrict__ w,
+                                                                  int64_t R, uint32_t blocks_per_row) {
+    const int64_t row = blockIdx.x / blocks_per_row;
+    const float s = load_as_f32<ST>(scale, row);
+    const int64_t c0 = int64_t(blockIdx.x % blocks_per_row) * 4096 + threadIdx.x * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int64_t c = c0 + j * 1024, count = R - c;
+        if (count <= 0) break;
+        float code[4], out[4];
+        load_codes_upto4<QT>(q, row * R + c, count, code);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * s);
+        store_upto4<ST>(w, row * R + c, count, out);
+    }
+}
+
+// Group-wise int4: grid (ceil(n / (4 CL)), k / group); 512 threads = 512 / CL row lanes x CL column quads.
 // scale32 = amax / 7 and code = clamp(round_half_away(w / scale32), -7, 7) in float32; two codes per
 // byte along n, low nibble first; the stored scale is scale32 rounded to the scale dtype.
-template <int ST>
-__global__ __launch_bounds__(256) void group_quantize_int4_kernel(const float *__restrict__ w, uint8_t *__restrict__ packed,
-                                                                  void *__restrict__ scales, int64_t n, int group) {
-    __shared__ float red[4][128];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t c0 = int64_t(blockIdx.x) * 128 + 2 * tx;
+//
+// Bound by memory: 4 bytes read and half a byte written per weight. ROWS > 0 (a group of up to ROWS * 512 / CL rows): the
+// workgroup keeps its columns of the group in registers between the maximum and the codes, so the weight is read once.
+// Longer groups take narrower column blocks instead of more rows per thread: with 8 rows per thread (76 registers) three
+// workgroups share a CU and one's loads run under another's codes (16 rows, two workgroups: 42.8 us).
+// ROWS = 0, groups beyond that: the rows are read twice. K = 4096, N = 11008, groups of 128: 82 - 87 us with the group
+// read twice in 8-byte loads, a division per weight and one-byte stores -> 38.3 us = 5.3 TB/s.
+template <int ST, int CL, int ROWS>
+__global__ __launch_bounds__(512, 6) void group_quantize_int4_kernel(const float *__restrict__ w, uint8_t *__restrict__ packed,
+                                                                     void *__restrict__ scales, int64_t n, int group) {
+    constexpr int LANES = 512 / CL;
+    __shared__ float4_t red[LANES][CL];
+    // a row's address is a scalar base (the wave's first row) and one per-lane offset for all rows
+    const int tx = threadIdx.x % CL, ty = threadIdx.x / CL;
+    const int sub = (threadIdx.x & 63) / CL, ty0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (64 / CL);
+    const int64_t b0 = int64_t(blockIdx.x) * (4 * CL), c0 = b0 + 4 * tx;
     const int64_t g = blockIdx.y;
-    const int64_t rbase = g * group;
-    const bool ok = c0 < n;  // n is even: the pair is in or out together
-    float m0 = 0.0f, m1 = 0.0f;
-    if (ok) {
-        for (int r = ty; r < group; r += 4) {
-            float2 v = *reinterpret_cast<const float2 *>(w + (rbase + r) * n + c0);
-            m0 = fmaxf(m0, fabsf(v.x));
-            m1 = fmaxf(m1, fabsf(v.y));
+    const int cols = c0 >= n ? 0 : (n - c0 >= 4 ? 4 : 2);  // n is even
+    const float *base = w + g * group * n + b0;
+    const int64_t lane_off = sub * n + 4 * tx;
+    auto load = [&](int i) {  // row i * LANES + ty of the group
+        float4_t v = {0.f, 0.f, 0.f, 0.f};
+        const float *row = base + int64_t(i * LANES + ty0) * n;
+        if (i * LANES + ty < group) {
+            if (cols == 4) {
+                v = *reinterpret_cast<const float4_at4_t *>(row + lane_off);
+            } else if (cols == 2) {
+                v[0] = row[lane_off];
+                v[1] = row[lane_off + 1];
+            }
         }
+        return v;
+    };
+    const int trips = (group + LANES - 1) / LANES;
+    float4_t x[ROWS > 0 ? ROWS : 1];
+    float4_t m = {0.f, 0.f, 0.f, 0.f};
+    auto larger = [&](const float4_t &v) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[e]));
+    };
+    if constexpr (ROWS > 0) {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) x[i] = load(i);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) larger(x[i]);
+    } else {
+        for (int i = 0; i < trips; ++i) larger(load(i));
     }
-    red[ty][2 * tx] = m0;
-    red[ty][2 * tx + 1] = m1;
+    red[ty][tx] = m;
     __syncthreads();
-    if (!ok) return;
-    m0 = fmaxf(fmaxf(red[0][2 * tx], red[1][2 * tx]), fmaxf(red[2][2 * tx], red[3][2 * tx]));
-    m1 = fmaxf(fmaxf(red[0][2 * tx + 1], red[1][2 * tx + 1]), fmaxf(red[2][2 * tx + 1], red[3][2 * tx + 1]));
-    const float s0 = m0 / 7.0f, s1 = m1 / 7.0f;
-    if (ty == 0) {
-        store_from_f32<ST>(scales, g * n + c0, round_to<ST>(s0));
-        store_from_f32<ST>(scales, g * n + c0 + 1, round_to<ST>(s1));
+#pragma unroll 2  // (the weights are in registers: no room for all of these at once)
+    for (int t = 0; t < LANES; ++t) larger(red[t][tx]);
+    if (cols == 0) return;
+    float s[4], inv[4];
+    bool fast = true;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        s[e] = m[e] / 7.0f;
+        inv[e] = __builtin_amdgcn_rcpf(s[e]);
+        fast = fast && reciprocal_is_precise(s[e]);
     }
-    for (int r = ty; r < group; r += 4) {
-        float2 v = *reinterpret_cast<const float2 *>(w + (rbase + r) * n + c0);
-        float q0 = s0 == 0.0f ? 0.0f : fminf(fmaxf(roundf(v.x / s0), -7.0f), 7.0f);
-        float q1 = s1 == 0.0f ? 0.0f : fminf(fmaxf(roundf(v.y / s1), -7.0f), 7.0f);
-        packed[((rbase + r) * n + c0) >> 1] = uint8_t((int(q0) & 0xF) | ((int(q1) & 0xF) << 4));
+    if (ty == 0) {
+        for (int e = 0; e < cols; ++e) store_from_f32<ST>(scales, g * n + c0 + e, round_to<ST>(s[e]));
+    }
+    uint8_t *out = packed + ((g * group * n + b0) >> 1);  // n is even: every row starts on a byte
+    auto emit = [&](int i, const float4_t &v) {
+        if (i * LANES + ty >= group) return;
+        const float x4[4] = {v[0], v[1], v[2], v[3]};
+        uint32_t n4[4], code = 0;
+        round_quotients_f32(x4, s, inv, fast, -7.0f, 7.0f, n4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) code |= (n4[e] & 0xFu) << (4 * e);
+        uint8_t *o = out + ((int64_t(i * LANES + ty0) * n) >> 1) + (lane_off >> 1);
+        if (cols == 4) __builtin_memcpy(o, &code, 2);
+        else *o = uint8_t(code);
+    };
+    if constexpr (ROWS > 0) {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) emit(i, x[i]);
+    } else {
+        for (int i = 0; i < trips; ++i) emit(i, load(i));
     }
 }
 
 // ---- per-tensor float8 e4m3 -------------------------------------------------------------------
 
+// Elements i .. i + V - 1 (V = 16 bytes of the type) as they lie in memory, zero from `numel` on, at the alignment of one.
+typedef uint32_t uint4_at4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint4_at2_t __attribute__((ext_vector_type(4), aligned(2)));
 template <int DT>
-__global__ __launch_bounds__(256) void amax_all_kernel(const void *__restrict__ x, uint32_t *__restrict__ amax_bits, int64_t numel) {
-    __shared__ float red[4];
-    float m = 0.0f;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < numel; i += int64_t(gridDim.x) * 256)
-        m = fmaxf(m, fabsf(load_as_f32<DT>(x, i)));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        atomicMax(amax_bits, __float_as_uint(m));
-    }
-}
-
-template <int DT>
-__global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restrict__ x, const uint32_t *__restrict__ amax_bits,
-                                                           uint8_t *__restrict__ codes, float *__restrict__ scale, int64_t numel) {
-    const float s = __uint_as_float(*amax_bits) / 448.0f;
-    int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i == 0) *scale = s;
-    if (i >= numel) return;
-    codes[i] = s == 0.0f ? uint8_t(0) : f32_to_e4m3(load_as_f32<DT>(x, i) / s);
-}
-
-template <int DT>
-__global__ __launch_bounds__(256) void amax_all4_kernel(const void *__restrict__ x, uint32_t *__restrict__ amax_bits, int64_t numel4) {
-    __shared__ float red[4];
-    float m = 0.0f;
-    // chunks of 256 threads x 8 independent vector loads, contiguous per workgroup: with one load in flight per thread
-    // this pass ran at 1.9 TB/s
-    constexpr int kLoads = 8;
-    if (DT != HIDET_QMM_F32 && (numel4 & 1) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-        // 16-bit input: 16 bytes = 8 values per load; |x| as an integer compare on the 15 value bits (same order as the
-        // floats for finite values; the reduction below continues in float)
-        const int64_t numel8 = numel4 >> 1;
-        constexpr uint32_t kInfBits = DT == HIDET_QMM_F16 ? 0x7C00u : 0x7F80u;
-        uint32_t mb = 0;
-        for (int64_t base = int64_t(blockIdx.x) * (256 * kLoads); base < numel8; base += int64_t(gridDim.x) * (256 * kLoads)) {
-            uint4 v[kLoads];
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j) {
-                const int64_t i = base + j * 256 + threadIdx.x;
-                v[j] = uint4{0u, 0u, 0u, 0u};
-                if (i < numel8) v[j] = static_cast<const uint4 *>(x)[i];
-            }
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j) {
-                const uint32_t w4[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t lo = w4[e] & 0x7FFFu, hi = (w4[e] >> 16) & 0x7FFFu;
-                    mb = max(mb, max(lo > kInfBits ? 0u : lo, hi > kInfBits ? 0u : hi));  // a NaN is skipped, as fmaxf skips it
-                }
-            }
-        }
-        m = DT == HIDET_QMM_F16 ? f16_bits_to_f32(uint16_t(mb)) : bf16_bits_to_f32(uint16_t(mb));
+__device__ __forceinline__ uint4v_t load_vector(const void *p, int64_t i, int64_t numel) {
+    constexpr int V = DT == HIDET_QMM_F32 ? 4 : 8;
+    uint4v_t v = {0u, 0u, 0u, 0u};
+    if (i + V <= numel) {
+        if constexpr (DT == HIDET_QMM_F32) v = *reinterpret_cast<const uint4_at4_t *>(static_cast<const uint32_t *>(p) + i);
+        else v = *reinterpret_cast<const uint4_at2_t *>(static_cast<const uint16_t *>(p) + i);
     } else {
-        for (int64_t base = int64_t(blockIdx.x) * (256 * kLoads); base < numel4; base += int64_t(gridDim.x) * (256 * kLoads)) {
-            float v[kLoads][4];
 #pragma unroll
-            for (int j = 0; j < kLoads; ++j) {
-                const int64_t i = base + j * 256 + threadIdx.x;
-                v[j][0] = v[j][1] = v[j][2] = v[j][3] = 0.0f;
-                if (i < numel4) load4_as_f32<DT>(x, i, v[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j)
-                m = fmaxf(fmaxf(m, fmaxf(fabsf(v[j][0]), fabsf(v[j][1]))), fmaxf(fabsf(v[j][2]), fabsf(v[j][3])));
+        for (int e = 0; e < V; ++e) {
+            if (i + e >= numel) continue;
+            if constexpr (DT == HIDET_QMM_F32) v[e] = static_cast<const uint32_t *>(p)[i + e];
+            else v[e >> 1] |= uint32_t(static_cast<const uint16_t *>(p)[i + e]) << (16 * (e & 1));
         }
+    }
+    return v;
+}
+template <int DT>
+__device__ __forceinline__ float vector_element(const uint4v_t &v, int e) {
+    if constexpr (DT == HIDET_QMM_F32) return __uint_as_float(v[e]);
+    const uint16_t h = uint16_t(v[e >> 1] >> (16 * (e & 1)));
+    return DT == HIDET_QMM_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+}
+constexpr int kChunkLoads = 4, kChunkVectors = 256 * kChunkLoads;  // 16 KiB of 16-byte vectors: one trip of a workgroup
+
+// Largest magnitude of each workgroup's share of a tensor, one float per workgroup (an atomic on a single word takes
+// longer than the reads, and the word has to be cleared by a launch of its own).
+template <int DT>
+__global__ __launch_bounds__(256) void amax_all_kernel(const void *__restrict__ x, float *__restrict__ amax, int64_t numel, int64_t chunks) {
+    constexpr int V = DT == HIDET_QMM_F32 ? 4 : 8;
+    __shared__ float red[4];
+    float m = 0.0f;
+    for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        uint4v_t v[kChunkLoads];
+#pragma unroll
+        for (int j = 0; j < kChunkLoads; ++j) v[j] = load_vector<DT>(x, (c * kChunkVectors + j * 256 + threadIdx.x) * V, numel);
+#pragma unroll
+        for (int j = 0; j < kChunkLoads; ++j)
+#pragma unroll
+            for (int e = 0; e < V; ++e) m = fmaxf(m, fabsf(vector_element<DT>(v[j], e)));
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        atomicMax(amax_bits, __float_as_uint(m));
+    if (threadIdx.x == 0) amax[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// e4m3 codes of four values: the quotient by the scale, clamped to +-448 (what saturation means for a format whose largest
+// finite value is 448), converted by the hardware's round-to-nearest-even OCP conversion. The product with the reciprocal,
+// within 2^-22 of the quotient, converts alike unless a rounding boundary of the format lies between them; those have at
+// most four significant bits, so a product whose low 19 bits are not within 8 of zero (or that is too small for any code
+// but zero) needs no division.
+__device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, float inv, bool fast) {
+    if (s == 0.0f) return 0u;
+    float q[4];
+    uint32_t nearest = 0xFFFFFFFFu;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        q[e] = x[e] * inv;
+        nearest = min(nearest, (__float_as_uint(fmaxf(fabsf(q[e]), 0x1.1p-12f + 0x1p-20f)) + 8u) & 0x7FFFFu);
     }
+    if (__builtin_expect(!fast || nearest <= 16u, 0)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = x[e] / s;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = __builtin_amdgcn_fmed3f(q[e], -448.0f, 448.0f);
+    int p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+    p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], p, true);
+    return uint32_t(p);
 }
 
 // Small tensors (the activations of a decode step): one workgroup of 1024 threads keeps up to 65536 elements in registers
-// between the amax and the conversion - one launch instead of three. Same arithmetic as fp8_quantize4_kernel.
+// between the amax and the conversion - one launch instead of three. Same arithmetic as fp8_quantize_kernel.
 template <int DT>
 __global__ __launch_bounds__(1024) void fp8_quantize_small_kernel(const void *__restrict__ x, uint32_t *__restrict__ codes,
                                                                   float *__restrict__ scale, int numel4) {
@@ -463,51 +604,58 @@ __global__ __launch_bounds__(1024) void fp8_quantize_small_kernel(const void *__
     m = red[0];
 #pragma unroll
     for (int wv = 1; wv < 16; ++wv) m = fmaxf(m, red[wv]);
-    const float s = m / 448.0f;
+    const float s = m / 448.0f, inv = __builtin_amdgcn_rcpf(s);
+    const bool fast = reciprocal_is_precise(s);
     if (tid == 0) *scale = s;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int i = j * 1024 + tid;
-        if (i >= numel4) continue;
-        uint32_t packed = 0;
-        if (s != 0.0f) {
-            float q[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) q[e] = fminf(fmaxf(v[j][e] / s, -448.0f), 448.0f);
-            int p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
-            p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], p, true);
-            packed = uint32_t(p);
-        }
-        codes[i] = packed;
+        if (i < numel4) codes[i] = e4m3_codes4(v[j], s, inv, fast);
     }
 }
 
-// The quotient is clamped to +-448 (what saturation means for a format whose largest finite value is 448) and converted
-// by the hardware's round-to-nearest-even OCP e4m3 conversion, two values per instruction.
+// One chunk (16 KiB) per workgroup. The loads go out first; the workgroups' maxima (amax_all_kernel) are put together
+// while they are under way. Chunks are taken from the end of the tensor, where the maximum pass read last, each on the
+// XCD that read it then: what is still in that L2 does not come from memory again. 4096 x 8192
+// bfloat16: maxima 11 us (15.4 with atomics, + a clearing launch), codes 22 us (23.7; 27.5 with 32 KiB per workgroup).
 template <int DT>
-__global__ __launch_bounds__(256) void fp8_quantize4_kernel(const void *__restrict__ x, const uint32_t *__restrict__ amax_bits,
-                                                            uint32_t *__restrict__ codes, float *__restrict__ scale, int64_t numel4) {
-    const float s = __uint_as_float(*amax_bits) / 448.0f;
+__global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restrict__ x, const float *__restrict__ amax, int partials,
+                                                           uint8_t *__restrict__ codes, float *__restrict__ scale, int64_t numel, int64_t chunks8) {
+    constexpr int V = DT == HIDET_QMM_F32 ? 4 : 8;
+    __shared__ float red[4];
+    const int64_t c = (chunks8 - 1 - int64_t(blockIdx.x >> 3)) * 8 + (blockIdx.x & 7);
+    uint4v_t v[kChunkLoads];
+#pragma unroll
+    for (int j = 0; j < kChunkLoads; ++j) v[j] = load_vector<DT>(x, (c * kChunkVectors + j * 256 + threadIdx.x) * V, numel);
+    float m = 0.0f;
+    for (int i = threadIdx.x; i < partials; i += 256) m = fmaxf(m, amax[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float s = m / 448.0f, inv = __builtin_amdgcn_rcpf(s);
+    const bool fast = reciprocal_is_precise(s);
     if (blockIdx.x == 0 && threadIdx.x == 0) *scale = s;
-    // four independent vector loads per thread (a workgroup converts 1024 consecutive groups of four values)
-    float v[4][4];
-    const int64_t base = int64_t(blockIdx.x) * 1024 + threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (base + j * 256 < numel4) load4_as_f32<DT>(x, base + j * 256, v[j]);
+    for (int j = 0; j < kChunkLoads; ++j) {
+        const int64_t i = (c * kChunkVectors + j * 256 + threadIdx.x) * V;
+        if (i >= numel) continue;
+        uint32_t out[V / 4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int64_t i = base + j * 256;
-        if (i >= numel4) continue;
-        uint32_t packed = 0;
-        if (s != 0.0f) {
+        for (int h = 0; h < V / 4; ++h) {
+            float t[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[j][e] = fminf(fmaxf(v[j][e] / s, -448.0f), 448.0f);
-            int p = __builtin_amdgcn_cvt_pk_fp8_f32(v[j][0], v[j][1], 0, false);
-            p = __builtin_amdgcn_cvt_pk_fp8_f32(v[j][2], v[j][3], p, true);
-            packed = uint32_t(p);
+            for (int e = 0; e < 4; ++e) t[e] = vector_element<DT>(v[j], 4 * h + e);
+            out[h] = e4m3_codes4(t, s, inv, fast);
         }
-        codes[i] = packed;
+        if (i + V <= numel) {
+            __builtin_memcpy(codes + i, out, V);
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (i + e < numel) codes[i + e] = uint8_t(out[e >> 2] >> (8 * (e & 3)));
+        }
     }
 }
 
@@ -541,73 +689,42 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
     QMM_CHECK(ws.scratch_bytes >= nscale * 4, "workspace too small: its scratch part (three quarters of what follows the first 64 KiB) must hold "
                                                   << nscale * 4 << " bytes, got a workspace of " << workspace_bytes);
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    uint32_t *amax_bits = reinterpret_cast<uint32_t *>(ws.scratch);
+    float *amax = reinterpret_cast<float *>(ws.scratch);
     dispatch_float(w_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        {
-            // rows that fit a workgroup's registers: one pass
-            const int esize0 = DT == HIDET_QMM_F32 ? 4 : 2, qsize0 = q_dtype == HIDET_QMM_I8 ? 1 : 2;
-            if (inner == 1 && reduce > 0 && reduce % 4 == 0 && reduce <= 256 * 4 * 16 && outer < (int64_t(1) << 31) &&
-                aligned(w, 4 * esize0) && aligned(wq, 4 * qsize0) && aligned(scale, esize0)) {
-                auto go = [&](auto kern) { launch(kern, dim3(uint32_t(outer)), dim3(256), 0, stream, w, wq, scale, reduce / 4); };
-                const bool small = reduce <= 256 * 4 * 4;
-                if (q_dtype == HIDET_QMM_I8) small ? go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 4>) : go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 16>);
-                else small ? go(quantize_row_fused_kernel<DT, HIDET_QMM_I16, 4>) : go(quantize_row_fused_kernel<DT, HIDET_QMM_I16, 16>);
-                return;
-            }
-        }
-        if (reduce == 0) {
-            launch_aux(fill_u32_kernel, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, amax_bits, nscale, 0u);
-        } else if (inner == 1) {
-            launch(amax_contig_kernel<DT>, dim3(cdiv(outer, 4)), dim3(256), 0, stream, w, amax_bits, outer, reduce);
-        } else {
-            QMM_CHECK(outer <= 65535, "outer extent " << outer << " exceeds the grid limit");
-            const int64_t col_blocks = cdiv(inner, 64);
-            int64_t splits = 1;
-            if (col_blocks * outer < 1024) splits = std::min<int64_t>(cdiv(1024, col_blocks * outer), cdiv(reduce, 64));
-            splits = std::max<int64_t>(1, std::min<int64_t>(splits, 65535));
-            const int64_t rows_per_split = cdiv(cdiv(reduce, splits), 4) * 4;
-            splits = cdiv(reduce, rows_per_split);
-            if (splits > 1) launch_aux(fill_u32_kernel, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, amax_bits, nscale, 0u);
-            launch(amax_strided_kernel<DT>, dim3(col_blocks, outer, splits), dim3(256), 0, stream, w, amax_bits, reduce,
-                   inner, rows_per_split, int(splits > 1));
-        }
         if (total == 0) return;
         const int esize = DT == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
-        const bool vec_ok = aligned(w, 4 * esize) && aligned(wq, 4 * qsize) && aligned(scale, esize);
-        if (vec_ok && inner % 4 == 0) {
-            const int64_t row_blocks = cdiv(reduce, kQuantRows);
-            if (row_blocks <= 65535 && outer <= 65535) {
-                const dim3 grid(uint32_t(cdiv(inner / 4, 64)), uint32_t(row_blocks), uint32_t(outer));
-                if (q_dtype == HIDET_QMM_I8)
-                    launch(quantize_rows_kernel<DT, HIDET_QMM_I8>, grid, dim3(256), 0, stream, w, amax_bits, wq, scale, reduce, inner / 4);
-                else
-                    launch(quantize_rows_kernel<DT, HIDET_QMM_I16>, grid, dim3(256), 0, stream, w, amax_bits, wq, scale, reduce, inner / 4);
+        QMM_CHECK(aligned(w, esize) && aligned(wq, qsize) && aligned(scale, esize), "a tensor is not aligned to its element type");
+        auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) {
+            if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), 0, stream, args...);
+            else launch(i16, grid, dim3(threads), 0, stream, args...);
+        };
+        if (inner == 1) {
+            // rows that fit a workgroup's registers: one pass
+            if (reduce % 4 == 0 && reduce <= 256 * 4 * 16 && outer < (int64_t(1) << 31) && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
+                const dim3 grid{uint32_t(outer)};
+                if (reduce <= 256 * 4 * 4) go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 4>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 4>, grid, 256, w, wq, scale, reduce / 4);
+                else go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 16>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 16>, grid, 256, w, wq, scale, reduce / 4);
                 return;
             }
-            if (q_dtype == HIDET_QMM_I8)
-                launch(quantize4_kernel<DT, HIDET_QMM_I8, false>, dim3(cdiv(total / 4, 256)), dim3(256), 0, stream, w, amax_bits,
-                       wq, scale, reduce, inner / 4, total / 4);
-            else
-                launch(quantize4_kernel<DT, HIDET_QMM_I16, false>, dim3(cdiv(total / 4, 256)), dim3(256), 0, stream, w, amax_bits,
-                       wq, scale, reduce, inner / 4, total / 4);
+            launch(amax_contig_kernel<DT>, dim3(cdiv(outer, 4)), dim3(256), 0, stream, w, amax, outer, reduce);
+            const int64_t blocks = cdiv(reduce, 1024);
+            QMM_CHECK(blocks * outer < (int64_t(1) << 31), "tensor too large for one launch");
+            go(quantize_long_row_kernel<DT, HIDET_QMM_I8>, quantize_long_row_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(blocks * outer)), 256, w, amax, wq, scale,
+               reduce, uint32_t(blocks));
             return;
         }
-        if (vec_ok && inner == 1 && reduce % 4 == 0) {
-            if (q_dtype == HIDET_QMM_I8)
-                launch(quantize4_kernel<DT, HIDET_QMM_I8, true>, dim3(cdiv(total / 4, 256)), dim3(256), 0, stream, w, amax_bits,
-                       wq, scale, reduce / 4, int64_t(0), total / 4);
-            else
-                launch(quantize4_kernel<DT, HIDET_QMM_I16, true>, dim3(cdiv(total / 4, 256)), dim3(256), 0, stream, w, amax_bits,
-                       wq, scale, reduce / 4, int64_t(0), total / 4);
-            return;
-        }
-        if (q_dtype == HIDET_QMM_I8)
-            launch(quantize_kernel<DT, HIDET_QMM_I8>, dim3(cdiv(total, 256)), dim3(256), 0, stream, w, amax_bits, wq, scale,
-                   reduce, inner, total);
-        else
-            launch(quantize_kernel<DT, HIDET_QMM_I16>, dim3(cdiv(total, 256)), dim3(256), 0, stream, w, amax_bits, wq, scale,
-                   reduce, inner, total);
+        QMM_CHECK(outer <= 65535, "outer extent " << outer << " exceeds the grid limit");
+        const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kQuantRows);
+        QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
+        // enough row ranges for two workgroups per CU, of 64 rows at least, and as many as the scratch memory holds maxima of
+        int64_t ranges = std::min(512 / std::min<int64_t>(512, col_blocks * outer), cdiv(reduce, 64));
+        ranges = std::max<int64_t>(1, std::min<int64_t>({ranges, kMaxRanges, ws.scratch_bytes / (nscale * 4)}));
+        const int64_t rows_per_range = cdiv(reduce, ranges);
+        launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
+               rows_per_range, nscale);
+        go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
+           dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
     });
     if (reduce == 0) {
         // no elements: scale = 0 still has to be written
@@ -631,24 +748,21 @@ HIDET_API void hidet_symmetric_dequantize(const void *wq, const void *scale, voi
     dispatch_float(s_dtype, [&](auto dt) {
         constexpr int ST = decltype(dt)::value;
         const int esize = ST == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
-        const bool vec_ok = aligned(w, 4 * esize) && aligned(wq, 4 * qsize) && aligned(scale, 4 * esize);
-        auto go4 = [&](auto kern, int64_t r4, int64_t in4) {
-            launch(kern, dim3(cdiv(total / 4, 256)), dim3(256), 0, stream, wq, scale, w, r4, in4, total / 4);
-        };
-        if (vec_ok && inner % 4 == 0) {
-            if (q_dtype == HIDET_QMM_I8) go4(dequantize4_kernel<HIDET_QMM_I8, ST, false>, reduce, inner / 4);
-            else go4(dequantize4_kernel<HIDET_QMM_I16, ST, false>, reduce, inner / 4);
+        QMM_CHECK(aligned(w, esize) && aligned(wq, qsize) && aligned(scale, esize), "a tensor is not aligned to its element type");
+        if (inner == 1) {
+            const int64_t blocks = cdiv(reduce, 4096);
+            QMM_CHECK(blocks * outer < (int64_t(1) << 31), "tensor too large for one launch");
+            const dim3 grid{uint32_t(blocks * outer)};
+            if (q_dtype == HIDET_QMM_I8) launch(dequantize_long_row_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, uint32_t(blocks));
+            else launch(dequantize_long_row_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, uint32_t(blocks));
             return;
         }
-        if (vec_ok && inner == 1 && reduce % 4 == 0) {
-            if (q_dtype == HIDET_QMM_I8) go4(dequantize4_kernel<HIDET_QMM_I8, ST, true>, reduce / 4, int64_t(0));
-            else go4(dequantize4_kernel<HIDET_QMM_I16, ST, true>, reduce / 4, int64_t(0));
-            return;
-        }
-        if (q_dtype == HIDET_QMM_I8)
-            launch(dequantize_kernel<HIDET_QMM_I8, ST>, dim3(cdiv(total, 256)), dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
-        else
-            launch(dequantize_kernel<HIDET_QMM_I16, ST>, dim3(cdiv(total, 256)), dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
+        QMM_CHECK(outer <= 65535, "outer extent " << outer << " exceeds the grid limit");
+        const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kDequantRows);
+        QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
+        const dim3 grid(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer));
+        if (q_dtype == HIDET_QMM_I8) launch(dequantize_rows_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, uint32_t(col_blocks));
+        else launch(dequantize_rows_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, uint32_t(col_blocks));
     });
     QMM_ENTRY_END
 }
@@ -666,8 +780,15 @@ HIDET_API void hidet_group_quantize_int4(const void *w, void *packed, void *scal
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     dispatch_float(s_dtype, [&](auto dt) {
         constexpr int ST = decltype(dt)::value;
-        launch(group_quantize_int4_kernel<ST>, dim3(cdiv(n, 128), k / group_size), dim3(256), 0, stream,
-               static_cast<const float *>(w), static_cast<uint8_t *>(packed), scales, n, group_size);
+        auto go = [&](auto kern, int cl) {
+            launch(kern, dim3(cdiv(n, 4 * cl), k / group_size), dim3(512), 0, stream, static_cast<const float *>(w),
+                   static_cast<uint8_t *>(packed), scales, n, group_size);
+        };
+        if (group_size <= 32) go(group_quantize_int4_kernel<ST, 64, 4>, 64);
+        else if (group_size <= 64) go(group_quantize_int4_kernel<ST, 64, 8>, 64);
+        else if (group_size <= 128) go(group_quantize_int4_kernel<ST, 32, 8>, 32);
+        else if (group_size <= 256) go(group_quantize_int4_kernel<ST, 16, 8>, 16);
+        else go(group_quantize_int4_kernel<ST, 64, 0>, 64);
     });
     QMM_ENTRY_END
 }
@@ -680,30 +801,24 @@ HIDET_API void hidet_fp8_quantize_per_tensor(const void *x, void *codes, void *s
     QMM_CHECK(ws.scratch_bytes >= 4, "workspace too small");
     QMM_CHECK(numel == 0 || (x && codes), "null tensor pointer");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    uint32_t *amax_bits = reinterpret_cast<uint32_t *>(ws.scratch);
+    float *amax = reinterpret_cast<float *>(ws.scratch);
     dispatch_float(x_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
         const int esize = DT == HIDET_QMM_F32 ? 4 : 2;
-        if (numel > 0 && numel <= 65536 && numel % 4 == 0 && aligned(x, 4 * esize) && aligned(codes, 4)) {
+        QMM_CHECK(aligned(x, esize), "the tensor is not aligned to its element type");
+        if (numel <= 65536 && numel % 4 == 0 && aligned(x, 4 * esize) && aligned(codes, 4)) {
             launch(fp8_quantize_small_kernel<DT>, dim3(1), dim3(1024), 0, stream, x, static_cast<uint32_t *>(codes),
                    static_cast<float *>(scale), int(numel / 4));
             return;
         }
-        launch_aux(fill_u32_kernel, dim3(1), dim3(64), 0, stream, amax_bits, int64_t(1), 0u);
-        if (numel > 0 && numel % 4 == 0 && aligned(x, 4 * esize) && aligned(codes, 4)) {
-            const int64_t n4 = numel / 4;
-            // at most 512 workgroups: each ends with one atomic on the same word, and 4096 of them took longer than the reads
-            launch(amax_all4_kernel<DT>, dim3(std::min<int64_t>(cdiv(n4, 2048), 512)), dim3(256), 0, stream, x, amax_bits, n4);
-            launch(fp8_quantize4_kernel<DT>, dim3(cdiv(n4, 1024)), dim3(256), 0, stream, x, amax_bits,
-                   static_cast<uint32_t *>(codes), static_cast<float *>(scale), n4);
-            return;
-        }
-        if (numel > 0) {
-            const int64_t blocks = std::min<int64_t>(cdiv(numel, 256 * 8), 512);  // one atomic on one word per workgroup
-            launch(amax_all_kernel<DT>, dim3(blocks), dim3(256), 0, stream, x, amax_bits, numel);
-        }
-        launch(fp8_quantize_kernel<DT>, dim3(std::max<int64_t>(1, cdiv(numel, 256))), dim3(256), 0, stream, x, amax_bits,
-               static_cast<uint8_t *>(codes), static_cast<float *>(scale), numel);
+        const int64_t chunks = cdiv(numel, int64_t(kChunkVectors) * (16 / esize)), chunks8 = cdiv(chunks, 8);
+        QMM_CHECK(chunks8 * 8 < (int64_t(1) << 31), "tensor too large for one launch");
+        // four workgroups per CU, a multiple of the XCDs (a chunk is then converted on the XCD that looked at it); fewer where the
+        // scratch memory holds fewer maxima
+        const int64_t partials = std::min<int64_t>({chunks, 1024, ws.scratch_bytes / 4});
+        launch(amax_all_kernel<DT>, dim3(uint32_t(partials)), dim3(256), 0, stream, x, amax, numel, chunks);
+        launch(fp8_quantize_kernel<DT>, dim3(uint32_t(chunks8 * 8)), dim3(256), 0, stream, x, amax, int(partials), static_cast<uint8_t *>(codes),
+               static_cast<float *>(scale), numel, chunks8);
     });
     QMM_ENTRY_END
 }

@@ -1,0 +1,67 @@
+"""The quantizers at the edges of their kernels' tiles, on values at and next to the rounding ties of a scale that is no
+power of two (where a product with the scale's reciprocal and the quotient could round apart): bit-exact against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from hidet_amd.graph.ops import quant
+from hidet_amd.graph.ops.matmul import matmul_f8 as F8
+from gpu_util import announce, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _near_ties(rng, shape, axis, qmax):
+    """Normal values, half of them replaced by (n + 1/2) * scale of their slice and its two float32 neighbours."""
+    w = (rng.standard_normal(shape) * 0.02).astype(np.float32)
+    s = (np.abs(w).max(axis=axis, keepdims=True) / np.float32(qmax)).astype(np.float32)
+    tie = ((np.floor(w / s).clip(-qmax, qmax - 1) + np.float32(0.5)) * s).astype(np.float32)
+    pick = rng.integers(0, 8, shape)
+    w = np.where(pick == 0, tie, w)
+    w = np.where(pick == 1, np.nextafter(tie, np.float32(1)), w)
+    return np.where(pick == 2, np.nextafter(tie, np.float32(-1)), w).astype(np.float32)
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'float16', 'bfloat16'])
+@pytest.mark.parametrize('shape,dim,codes', [((1, 3), 0, 'int8'), ((63, 255), 0, 'int8'), ((65, 257), 0, 'int16'), ((4100, 1026), 0, 'int8'),
+                                             ((129, 6), 0, 'int8'), ((3, 2049, 130), 1, 'int8'), ((33, 16387), 1, 'int8'), ((5, 4100), 1, 'int16')])
+def test_columns_and_rows_bit_exact(shape, dim, codes, dtype):
+    announce('quantize edges', shape, dim, codes, dtype)
+    w = _near_ties(np.random.default_rng(shape[-1]), shape, dim, 127 if codes == 'int8' else 32767)
+    w.reshape(-1, shape[-1])[:, 0] = 0  # a column of zeros
+    if dtype == 'bfloat16':
+        w = O.to_bf16(w)
+    elif dtype == 'float16':
+        w = w.astype(np.float16)
+    q0, s0 = O.symmetric_quantize(w, codes, dim, dtype=dtype, target='cpu' if dtype == 'float32' else 'gpu')
+    q, s = quant.symmetric_quantize(dev(w).to(getattr(torch, dtype)), codes, dim)
+    assert np.array_equal(host(q), q0)
+    assert np.array_equal(s.float().cpu().numpy(), np.asarray(s0, dtype=np.float32))
+    assert np.array_equal(quant.symmetric_dequantize(q, s, dim).float().cpu().numpy(),
+                          np.asarray(O.symmetric_dequantize(q0, s0, dim, dtype=dtype), dtype=np.float32))
+
+
+@pytest.mark.parametrize('k,n,group', [(4, 2, 4), (96, 258, 32), (66, 254, 33), (128, 1030, 64), (256, 126, 128), (390, 130, 65), (512, 66, 256),
+                                       (514, 6, 257), (1024, 258, 1024)])
+def test_int4_groups_bit_exact(k, n, group):
+    announce('int4 edges', k, n, group)
+    w = _near_ties(np.random.default_rng(k + n), (k // group, group, n), 1, 7).reshape(k, n)
+    packed, scales = quant.symmetric_group_quantize_int4(dev(w), group, 'float16')
+    p0, s0, _ = O.group_quantize_int4(w, group, 'float16')
+    assert np.array_equal(host(packed), p0) and np.array_equal(host(scales).view(np.uint16), s0.view(np.uint16))
+
+
+@pytest.mark.parametrize('numel', [65535, 65537, 8 * 4096 - 4, 4096 * 1024 * 2 + 3])
+def test_fp8_per_tensor_bit_exact(numel):
+    announce('fp8 edges', numel)
+    rng = np.random.default_rng(numel)
+    x = (rng.standard_normal(numel) * 3).astype(np.float32)
+    vals = O.e4m3_decode(np.arange(0, 0x7F, dtype=np.uint8)).astype(np.float64)
+    ties = ((vals[:-1] + vals[1:]) / 2 * (float(np.abs(x).max()) / 448)).astype(np.float32)
+    ties = np.concatenate([ties, np.nextafter(ties, np.float32(0)), np.nextafter(ties, np.float32(9)), np.zeros(5, np.float32)])
+    x[rng.permutation(numel)[:ties.size]] = ties
+    for t in (dev(x), dev(x).bfloat16(), dev(x).half()):
+        codes, scale = F8.fp8_quantize_per_tensor(t)
+        c0, s0 = O.fp8_quantize_per_tensor(t.float().cpu().numpy())
+        assert np.float32(scale.item()) == s0 and np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
