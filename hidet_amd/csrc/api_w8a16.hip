@@ -2,24 +2,132 @@
 #include "common.h"
 
 namespace qmm {
+bool skinny_w8a16_supported(const void *w, const void *scale, const void *bias, int64_t k, int64_t n);
 void skinny_w8a16_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                         int64_t n, int64_t lda, int parallel_k_parts, void *workspace, int64_t workspace_bytes,
-                         bool strict_workspace, hipStream_t stream);
+                         int64_t n, int64_t lda, int64_t n_out, int parallel_k_parts, const Workspace &ws, bool strict_workspace,
+                         hipStream_t stream);
 bool gemm_w8a16_supported(const void *a, const void *w, const void *c, int64_t m, int64_t k, int64_t n, int64_t lda);
 void gemm_w8a16_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                       int64_t n, int64_t lda, void *workspace, int64_t workspace_bytes, hipStream_t stream);
+                       int64_t n, int64_t lda, int64_t n_out, int64_t ldc, const Workspace &ws, hipStream_t stream);
 bool skinny_w8a16_nk_supported(const void *w, int64_t k, int64_t ldw);
 void skinny_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                             int64_t n, int64_t lda, int64_t ldw, hipStream_t stream);
 bool gemm_w8a16_nk_supported(const void *a, const void *w, const void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                              int64_t ldw);
 void gemm_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                          int64_t n, int64_t lda, int64_t ldw, void *workspace, int64_t workspace_bytes, hipStream_t stream);
+                          int64_t n, int64_t lda, int64_t ldw, const Workspace &ws, hipStream_t stream);
 }
 
 using namespace qmm;
 
 namespace {
+
+// ---- operands of sizes or alignments the matrix kernels do not take --------------------------------------------------
+//
+// Copies of the operands with rows of whole 16 (weight, factors) and 64 (activations) elements, zero past the originals,
+// in the scratch memory: columns [n0, n0 + cols) of w[k, n] as [kp, np], the float16 activations [m, k] as [m, kp], the
+// column factors as [np]. One thread per 16 bytes written. 203 rows x 4100 x 4098 take 39 us in all (28 us of them the GEMM),
+// where the element-wise kernel that served such sizes before took 1815 us; one row x 4100 x 4098 20 us.
+struct PadArgs {
+    const int8_t *w;
+    const _Float16 *a, *scale, *bias;
+    int8_t *wp;
+    _Float16 *ap, *scalep, *biasp;
+    int64_t n, lda;
+    int k, kp, n0, cols, np, m;
+    uint32_t w_chunks, a_chunks;  // 16-byte pieces of the copies (none: that operand is left alone)
+};
+__global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p) {
+    uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < p.w_chunks) {
+        const uint32_t per_row = uint32_t(p.np) / 16, row = i / per_row, col = (i - row * per_row) * 16;
+        uint4 v = {0u, 0u, 0u, 0u};
+        if (int(row) < p.k) {
+            const int8_t *src = p.w + int64_t(row) * p.n + p.n0 + col;
+            if (int(col) + 16 <= p.cols) {
+                __builtin_memcpy(&v, src, 16);
+            } else {
+                uint32_t word[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (int(col) + e < p.cols) word[e >> 2] |= uint32_t(uint8_t(src[e])) << (8 * (e & 3));
+                v = uint4{word[0], word[1], word[2], word[3]};
+            }
+        }
+        reinterpret_cast<uint4 *>(p.wp)[i] = v;
+        return;
+    }
+    i -= p.w_chunks;
+    if (i < p.a_chunks) {
+        const uint32_t per_row = uint32_t(p.kp) / 8, row = i / per_row, kk = (i - row * per_row) * 8;
+        half8_t v;
+        const _Float16 *src = p.a + int64_t(row) * p.lda + kk;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = int(kk) + e < p.k ? src[e] : _Float16(0.0f);
+        reinterpret_cast<half8_t *>(p.ap)[i] = v;
+        return;
+    }
+    i -= p.a_chunks;
+    if (p.w_chunks > 0 && i < uint32_t(p.np)) {
+        const bool in = int(i) < p.cols;
+        p.scalep[i] = in ? p.scale[p.n0 + i] : _Float16(0.0f);
+        if (p.bias != nullptr) p.biasp[i] = in ? p.bias[p.n0 + i] : _Float16(0.0f);
+    }
+}
+
+// The matmul on padded copies, in panels of columns and rows that fit the scratch memory (the GEMM; up to 16 rows go to the
+// bandwidth-bound kernel, which reads activations of any alignment, whole): the copies lie at its end, what is before them is left to the GEMM's partial tiles. False: there
+// is not enough of it for a panel.
+bool w8a16_padded(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
+                  int64_t lda, const Workspace &ws, hipStream_t stream) {
+    const bool gemm = m > 16;
+    const int64_t kp = gemm ? cdiv(k, 64) * 64 : k;
+    const bool copy_a = gemm && (kp != k || lda % 8 != 0 || !aligned(a, 16) || (m * lda + k) * 2 >= (int64_t(1) << 31) - (1 << 20));
+    const int64_t room = ws.scratch_bytes / 4 * 3;  // a quarter stays for partial tiles
+    const int64_t rows = copy_a ? std::min<int64_t>(m, room / 3 / (kp * 2) / 128 * 128) : m;
+    if (rows <= 0) return false;
+    const int64_t a_bytes = copy_a ? cdiv(rows * kp * 2, 256) * 256 : 0;
+    int64_t cols = cdiv(n, 16) * 16;  // per panel
+    const int64_t per_col = kp + 4, fixed = a_bytes + 1024;
+    const int64_t most = std::min<int64_t>(room - fixed, int64_t(1) << 30) / per_col;
+    if (cols > most) cols = most / 256 * 256;
+    if (cols <= 0 || (!gemm && cols < n)) return false;  // (the bandwidth-bound kernel writes whole rows: one panel)
+    char *end = ws.scratch + ws.scratch_bytes / 256 * 256;
+    PadArgs p{};
+    p.w = static_cast<const int8_t *>(w);
+    p.scale = static_cast<const _Float16 *>(scale);
+    p.bias = static_cast<const _Float16 *>(bias);
+    p.ap = reinterpret_cast<_Float16 *>(end - a_bytes);
+    p.biasp = reinterpret_cast<_Float16 *>(end - a_bytes - cdiv(cols * 2, 256) * 256);
+    p.scalep = p.biasp - cdiv(cols * 2, 256) * 128;
+    p.wp = reinterpret_cast<int8_t *>(p.scalep) - cdiv(kp * cols, 256) * 256;
+    p.n = n;
+    p.lda = lda;
+    p.k = int(k);
+    p.kp = int(kp);
+    Workspace left = ws;
+    left.scratch_bytes = reinterpret_cast<char *>(p.wp) - ws.scratch;
+    if (left.scratch_bytes < 0) return false;
+    for (int64_t n0 = 0; n0 < n; n0 += cols) {
+        p.n0 = int(n0);
+        p.cols = int(std::min(cols, n - n0));
+        p.np = int(cdiv(p.cols, 16) * 16);
+        for (int64_t m0 = 0; m0 < m; m0 += rows) {
+            p.m = int(std::min(rows, m - m0));
+            p.a = static_cast<const _Float16 *>(a) + m0 * lda;
+            p.w_chunks = m0 == 0 ? uint32_t(kp * p.np / 16) : 0;
+            p.a_chunks = copy_a ? uint32_t(p.m * kp / 8) : 0;
+            const uint64_t threads = uint64_t(p.w_chunks) + p.a_chunks + (p.w_chunks > 0 ? p.np : 0);
+            if (threads > 0) launch_aux(pad_operands_kernel, dim3(uint32_t((threads + 255) / 256)), dim3(256), 0, stream, p);
+            const void *ap = copy_a ? static_cast<const void *>(p.ap) : static_cast<const void *>(p.a);
+            _Float16 *cp = static_cast<_Float16 *>(c) + m0 * n + n0;
+            const void *bp = bias != nullptr ? p.biasp : nullptr;
+            if (gemm) gemm_w8a16_launch(ap, p.wp, p.scalep, bp, cp, p.m, kp, p.np, copy_a ? kp : lda, p.cols, n, left, stream);
+            else skinny_w8a16_launch(ap, p.wp, p.scalep, bp, cp, p.m, k, p.np, lda, p.cols, 0, left, false, stream);
+        }
+    }
+    return true;
+}
 
 // Checks and kernel choice shared by the two row-major entry points. `strict_workspace`: a bandwidth-bound launch whose
 // K split does not fit the scratch memory is an error instead of a launch with fewer K slices.
@@ -33,16 +141,22 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     if (m == 0 || n == 0) return;
     QMM_CHECK(a && w && scale && c, "null tensor pointer");
     QMM_CHECK(aligned(a, 2) && aligned(scale, 2) && aligned(c, 2) && aligned(bias, 2), "float16 tensors must be 2-byte aligned");
+    const Workspace ws = split_workspace(workspace, workspace_bytes);
     // Up to 16 rows one pass of the bandwidth-bound kernel serves; beyond that every 16 rows would cost another pass
     // over the weights, and the MFMA GEMM with its K split and its empty row blocks left out takes over (K=4096, N=11008,
     // weights from HBM: 17 us at M=17..32, 20 us at M=64, 29 us at M=128). For 9 to 16 rows the bandwidth-bound kernel is
     // ahead of the GEMM on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
     // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49).
-    if (m > 16 && k > 0 && gemm_w8a16_supported(a, w, c, m, k, n, lda))
-        gemm_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, workspace, workspace_bytes, stream);
-    else
-        skinny_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, parallel_k_parts, workspace, workspace_bytes, strict_workspace,
-                            stream);
+    if (m > 16 && k > 0 && gemm_w8a16_supported(a, w, c, m, k, n, lda)) {
+        gemm_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, n, ws, stream);
+        return;
+    }
+    // Sizes the GEMM does not take (K no multiple of 64, N of 4): up to 32 rows two passes of the bandwidth-bound kernel,
+    // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the
+    // copy. Tiny matrices are left to the element-wise kernel.
+    const bool skinny = skinny_w8a16_supported(w, scale, bias, k, n);
+    if (k > 0 && (!skinny || m > 32) && m * k * n > (int64_t(1) << 20) && w8a16_padded(a, w, scale, bias, c, m, k, n, lda, ws, stream)) return;
+    skinny_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, parallel_k_parts, ws, strict_workspace, stream);
 }
 
 // Checks and kernel choice shared by the two entry points for K-contiguous weights.
@@ -61,8 +175,7 @@ void w8a16_nk_dispatch(const void *a, const void *w_nk, const void *scale, const
                                                                                                                          << " ldw=" << ldw);
     // more than one pass of 16 rows: the MFMA GEMM reading the same layout, where its conditions hold
     if (m > 16 && gemm_w8a16_nk_supported(a, w_nk, c, m, k, n, lda, ldw))
-        gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, workspace ? workspace : nullptr,
-                             workspace ? workspace_bytes : 0, stream);
+        gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, split_workspace(workspace, workspace_bytes), stream);
     else
         skinny_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, stream);
 }

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
                                                                                  int tiles_m, int tiles_n, int xm, int xn,
                                                                                  int concurrent, int tail_parts, int tail_stride,
                                                                                  float *__restrict__ partials,
-                                                                                 uint32_t *__restrict__ counters) {
+                                                                                 uint32_t *__restrict__ counters, int n_out, int ldc) {
     using Cfg = GemmW8Cfg16<RB, WM, WN>;
     extern __shared__ uint4 lds[];  // no static LDS in this kernel: fragment reads address the ring from 0
     int &s_last = *reinterpret_cast<int *>(lds + Cfg::kRingBytes / 16);
@@ -284,29 +284,45 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
 
     // acc[rb][t][v] = c[m0 + (wm*RB + rb)*16 + 4*kg + v][col + t]
     if (!col_ok) return;
-    float sc[4], bs[4];
+    if (ldc % 4 == 0 && n_out == n && (reinterpret_cast<uintptr_t>(c) & 7) == 0) {
+        float sc[4], bs[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            sc[t] = float(scale[col + t]);
+            bs[t] = bias != nullptr ? float(bias[col + t]) : -0.0f;
+        }
+#pragma unroll
+        for (int rb = 0; rb < RBA; ++rb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = m0 + (wm * RB + rb) * 16 + kg * 4 + v;
+                if (row < m) {
+                    half4_t o;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(acc[rb][t][v], sc[t], bs[t]);
+                    *reinterpret_cast<half4_t *>(c + int64_t(row) * ldc + col) = o;
+                }
+            }
+        return;
+    }
+    // a result whose rows start anywhere and end inside a lane's columns (the weight was copied to padded rows)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        sc[t] = float(scale[col + t]);
-        bs[t] = bias != nullptr ? float(bias[col + t]) : -0.0f;
-    }
+        if (col + t >= n_out) break;
+        const float sc = float(scale[col + t]), bs = bias != nullptr ? float(bias[col + t]) : -0.0f;
 #pragma unroll
-    for (int rb = 0; rb < RBA; ++rb)
+        for (int rb = 0; rb < RBA; ++rb)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int row = m0 + (wm * RB + rb) * 16 + kg * 4 + v;
-            if (row < m) {
-                half4_t o;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(acc[rb][t][v], sc[t], bs[t]);
-                *reinterpret_cast<half4_t *>(c + int64_t(row) * n + col) = o;
+            for (int v = 0; v < 4; ++v) {
+                const int row = m0 + (wm * RB + rb) * 16 + kg * 4 + v;
+                if (row < m) c[int64_t(row) * ldc + col + t] = scaled_biased_f16(acc[rb][t][v], sc, bs);
             }
-        }
+    }
 }
 
 template <int RB, int WM, int WN, int MIN_BLOCKS, int RBA, bool W_NK = false>
 void launch_cfg16(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
-                  int64_t lda, int64_t ldw, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+                  int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, const Workspace &ws, hipStream_t stream) {
     using Cfg = GemmW8Cfg16<RB, WM, WN>;
     const int tiles_m = int(cdiv(m, Cfg::kBM)), tiles_n = int(cdiv(n, Cfg::kBN));
     constexpr int kConcurrent = 32 * MIN_BLOCKS;  // workgroups an XCD (32 CUs) runs at a time
@@ -324,7 +340,6 @@ void launch_cfg16(const void *a, const void *w, const void *scale, const void *b
         tail = make_gemm_tail_by_rounds(tiling, 32, 4, 0.00085 * 4096.0 / double(k));
         split_unit = 32;
     }
-    const Workspace ws = split_workspace(workspace, workspace_bytes);
     while (tail.parts > 1 &&
            (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
         --tail.parts;
@@ -335,7 +350,7 @@ void launch_cfg16(const void *a, const void *w, const void *scale, const void *b
     launch(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, RBA, W_NK>, dim3(uint32_t(grid)), dim3(Cfg::kThreads), size_t(Cfg::kLdsBytes), stream,
            static_cast<const _Float16 *>(a), lda, static_cast<const int8_t *>(w), ldw, static_cast<const _Float16 *>(scale),
            static_cast<const _Float16 *>(bias), static_cast<_Float16 *>(c), int(m), int(k), int(n), tiles_m, tiles_n, tiling.xm, tiling.xn, split_unit, tail.parts, tail.max_tiles,
-           reinterpret_cast<float *>(ws.scratch), ws.counters);
+           reinterpret_cast<float *>(ws.scratch), ws.counters, int(n_out), int(ldc));
 }
 
 }  // namespace
@@ -347,13 +362,14 @@ bool gemm_w8a16_supported(const void *a, const void *w, const void *c, int64_t m
            k * n < (int64_t(1) << 31) - (1 << 20) && (m * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20);
 }
 
+// `n_out` <= n columns of the result are written, at a row stride of ldc.
 void gemm_w8a16_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                       int64_t n, int64_t lda, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+                       int64_t n, int64_t lda, int64_t n_out, int64_t ldc, const Workspace &ws, hipStream_t stream) {
     // waves 128 x 64, workgroup tile 128 x 256; a matrix of at most 32 / 64 / 96 rows leaves the empty row blocks out
-    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2>(a, w, scale, bias, c, m, k, n, lda, n, workspace, workspace_bytes, stream);
-    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4>(a, w, scale, bias, c, m, k, n, lda, n, workspace, workspace_bytes, stream);
-    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6>(a, w, scale, bias, c, m, k, n, lda, n, workspace, workspace_bytes, stream);
-    else launch_cfg16<8, 1, 4, 2, 8>(a, w, scale, bias, c, m, k, n, lda, n, workspace, workspace_bytes, stream);
+    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else launch_cfg16<8, 1, 4, 2, 8>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
 }
 
 // The same kernel on a weight stored K-contiguous (w_nk[col * ldw + k]): 8-byte loads, so rows of w_nk 8-byte aligned.
@@ -365,11 +381,11 @@ bool gemm_w8a16_nk_supported(const void *a, const void *w, const void *c, int64_
 }
 
 void gemm_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                          int64_t n, int64_t lda, int64_t ldw, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
-    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2, true>(a, w, scale, bias, c, m, k, n, lda, ldw, workspace, workspace_bytes, stream);
-    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4, true>(a, w, scale, bias, c, m, k, n, lda, ldw, workspace, workspace_bytes, stream);
-    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6, true>(a, w, scale, bias, c, m, k, n, lda, ldw, workspace, workspace_bytes, stream);
-    else launch_cfg16<8, 1, 4, 2, 8, true>(a, w, scale, bias, c, m, k, n, lda, ldw, workspace, workspace_bytes, stream);
+                          int64_t n, int64_t lda, int64_t ldw, const Workspace &ws, hipStream_t stream) {
+    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else launch_cfg16<8, 1, 4, 2, 8, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
 }
 
 }  // namespace qmm

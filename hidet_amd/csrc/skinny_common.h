@@ -276,14 +276,15 @@ struct SkinnyWord<4> {
     static __device__ __forceinline__ float get(type v, int e) { return __uint_as_float(v[e]); }
 };
 
-template <typename OutT, int WAVES, int CW>
+// RAGGED: n need not be a multiple of 4 (every condition behind the last weight counts, so the others do without)
+template <typename OutT, int WAVES, int CW, bool RAGGED>
 struct SkinnyTail {
     typedef SkinnyWord<CW> W;
     typedef typename W::type Word;
     static constexpr int kThreadsPerRow = kSkinnyTileN / CW;                // 256 or 64
     static constexpr int kRowGroups = WAVES * 64 / kThreadsPerRow;         // rows the workgroup handles at a time
     static_assert(WAVES % 4 == 0, "whole rows of threads");
-    int m, n, row_first, col_in_tile;
+    int m, n, factor_n, row_first, col_in_tile;  // n: columns (and row stride) of the output, factor_n: length of the factor vectors
     int64_t out_col;
     const float *red;
     SkinnyScale factors;
@@ -340,12 +341,13 @@ struct SkinnyTail {
             uint16_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) h[e] = __builtin_bit_cast(uint16_t, finish(x.v[e], e));
-            // 8 bytes at once when the row starts allow it (n a multiple of 4 is given, the base pointer may not be aligned)
-            if ((reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
+            // 8 bytes at once where the row starts allow it (and, RAGGED, the quad does not reach past the row)
+            if ((reinterpret_cast<uintptr_t>(dst) & 7) == 0 && (!RAGGED || out_col + 4 <= n)) {
                 *reinterpret_cast<uint2 *>(dst) = uint2{uint32_t(h[0]) | (uint32_t(h[1]) << 16), uint32_t(h[2]) | (uint32_t(h[3]) << 16)};
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) reinterpret_cast<uint16_t *>(dst)[e] = h[e];
+                for (int e = 0; e < 4; ++e)
+                    if (!RAGGED || out_col + e < n) reinterpret_cast<uint16_t *>(dst)[e] = h[e];
             }
         }
     }
@@ -361,15 +363,15 @@ struct SkinnyTail {
     // past n and a missing vector read as zero bits through the descriptors) and, later, their use.
     __device__ __forceinline__ void fetch_factors() {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(factors.scale), 0,
-                                                                            factors.scale != nullptr ? n * 2 : 0, 0x00020000);
+                                                                            factors.scale != nullptr ? factor_n * 2 : 0, 0x00020000);
         const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(factors.bias), 0,
-                                                                            factors.bias != nullptr ? n * 2 : 0, 0x00020000);
+                                                                            factors.bias != nullptr ? factor_n * 2 : 0, 0x00020000);
         const int off = int(out_col) * 2;
         constexpr bool kBias = !std::is_same<OutT, f16_unbiased_t>::value;
         if constexpr (CW == 1) {
             scale_bits[0] = __builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
             if constexpr (kBias) bias_bits[0] = __builtin_amdgcn_raw_buffer_load_b16(rb, off, 0, 0);
-        } else {  // 8-byte loads: vectors 8-byte aligned, n a multiple of 4
+        } else {  // 8-byte loads: vectors 8-byte aligned, factor_n a multiple of 4
             const auto q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
             scale_bits[0] = q[0];
             scale_bits[1] = q[1];
@@ -546,10 +548,10 @@ struct SkinnyTail {
     }
 };
 
-// A wave's partial sums for one tile into LDS slot `slot` (the layout the tail's readers expect, see kSkinnyRedStride).
-__device__ __forceinline__ void skinny_stash(const float4_t (&res)[16], int m, int slot, float *red) {
-    const int lane = threadIdx.x & 63;
-    const int g = lane >> 4, cl = lane & 15;
+// A wave's partial sums for one tile into LDS slot `slot` (the layout the tail's readers expect, see kSkinnyRedStride). The
+// lane's 16 columns are the tile's chunks of four first_chunk .. + 3, those below the tile's first left out.
+__device__ __forceinline__ void skinny_stash(const float4_t (&res)[16], int m, int slot, float *red, int first_chunk) {
+    const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const int row = 4 * g + v;
@@ -557,21 +559,23 @@ __device__ __forceinline__ void skinny_stash(const float4_t (&res)[16], int m, i
             float *dst = red + (slot * m + row) * kSkinnyRedStride;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                *reinterpret_cast<float4_t *>(dst + skinny_red_chunk(4 * cl + j) * 4) =
-                    float4_t{res[4 * j][v], res[4 * j + 1][v], res[4 * j + 2][v], res[4 * j + 3][v]};
+                if (first_chunk + j >= 0)
+                    *reinterpret_cast<float4_t *>(dst + skinny_red_chunk(first_chunk + j) * 4) =
+                        float4_t{res[4 * j][v], res[4 * j + 1][v], res[4 * j + 2][v], res[4 * j + 3][v]};
         }
     }
 }
 
-template <typename OutT, int WAVES, int CW>
-__device__ __forceinline__ void skinny_tails_as(const SkinnyPlan &plan, const SkinnyWork &wk, const SkinnyRoles &roles, int m, int n,
+template <typename OutT, int WAVES, int CW, bool RAGGED>
+__device__ __forceinline__ void skinny_tails_as(const SkinnyPlan &plan, const SkinnyWork &wk, const SkinnyRoles &roles, int m, int n, int factor_n,
                                                 const SkinnyScale &col_scale, OutT *__restrict__ c, float *__restrict__ mailbox,
                                                 uint32_t *lost_flag, const float *red) {
-    constexpr int kHalf = SkinnyTail<OutT, WAVES, CW>::kRowGroups / 2;
+    constexpr int kHalf = SkinnyTail<OutT, WAVES, CW, RAGGED>::kRowGroups / 2;
     const int tid = threadIdx.x;
-    SkinnyTail<OutT, WAVES, CW> tail;
+    SkinnyTail<OutT, WAVES, CW, RAGGED> tail;
     tail.m = m;
     tail.n = n;
+    tail.factor_n = factor_n;
     tail.red = red;
     tail.c = c;
     tail.lost_flag = lost_flag;
@@ -585,7 +589,6 @@ __device__ __forceinline__ void skinny_tails_as(const SkinnyPlan &plan, const Sk
         tail.row_first = __builtin_amdgcn_readfirstlane(tid >> 6);
         tail.col_in_tile = (tid & 63) * 4;
     }
-    // n is a multiple of 16 where CW is 4: a quad of columns is in or out as a whole
     tail.out_col = int64_t(wk.tile) * kSkinnyTileN + tail.col_in_tile;
     if (tail.out_col >= n) return;  // then the columns of the next tile lie past n as well
     bool send_ok = int64_t(roles.send_tile) * kSkinnyTileN + tail.col_in_tile < n;
@@ -606,14 +609,15 @@ __device__ __forceinline__ void skinny_tails_as(const SkinnyPlan &plan, const Sk
 }
 
 // Everything behind the main loops: call after every wave has stashed its parts (this function holds the barrier).
-// `roles` is skinny_roles_of of this workgroup.
-template <typename OutT, int WAVES>
-__device__ __forceinline__ void skinny_tails(const SkinnyPlan &plan, const SkinnyWork &wk, const SkinnyRoles &roles, int m, int n,
+// `roles` is skinny_roles_of of this workgroup. n: columns and row stride of the output; factor_n: length of the column
+// factors' vectors, a multiple of 4 (n itself, or n rounded up where the operands were copied to padded ones).
+template <typename OutT, int WAVES, bool RAGGED>
+__device__ __forceinline__ void skinny_tails(const SkinnyPlan &plan, const SkinnyWork &wk, const SkinnyRoles &roles, int m, int n, int factor_n,
                                              const SkinnyScale &col_scale, OutT *__restrict__ c, float *__restrict__ mailbox,
                                              uint32_t *lost_flag, const float *red) {
     __syncthreads();
-    if (skinny_column_layout(m, plan.max_others, WAVES)) skinny_tails_as<OutT, WAVES, 1>(plan, wk, roles, m, n, col_scale, c, mailbox, lost_flag, red);
-    else skinny_tails_as<OutT, WAVES, 4>(plan, wk, roles, m, n, col_scale, c, mailbox, lost_flag, red);
+    if (skinny_column_layout(m, plan.max_others, WAVES)) skinny_tails_as<OutT, WAVES, 1, RAGGED>(plan, wk, roles, m, n, factor_n, col_scale, c, mailbox, lost_flag, red);
+    else skinny_tails_as<OutT, WAVES, 4, RAGGED>(plan, wk, roles, m, n, factor_n, col_scale, c, mailbox, lost_flag, red);
 }
 
 // ---- host side: the plan of a launch ------------------------------------------------------------------------------

@@ -24,7 +24,8 @@ constexpr int kDepth = 2;          // 32-row steps fetched together
 // workgroups, non-temporal loads with no condition around them - rows past the wave's range lie outside the buffer and
 // read as zero bytes, which are code 0 - and the exchange of skinny_tails. A step is 32 rows and the group size a
 // multiple of 32, so a step never straddles two groups.
-template <int DT, bool ALIGNED_A, bool BIAS>
+// RAGGED: N is a multiple of 8 only (at least 16): as in the int8 kernel, the last lane with columns takes the row's last 16.
+template <int DT, bool ALIGNED_A, bool BIAS, bool RAGGED>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_w4a16_kernel(int ksteps, uint32_t ksteps_magic, int per_group, int longer, int splits, uint32_t splits_magic,
                                                                         const uint8_t *__restrict__ w, const uint16_t *__restrict__ a,
                                                                         int64_t lda, int m, int k, int n, int group,
@@ -62,7 +63,10 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_w4a16_kernel(int kst
     {
         const int tile = wk.tile + part;
         const int tile_col = tile * kSkinnyTileN;
-        const bool col_ok = tile_col + cl * 16 < n;
+        int lane_col = tile_col + cl * 16;
+        const bool col_ok = lane_col < n;
+        if (RAGGED && col_ok && lane_col + 16 > n) lane_col = n - 16;
+        const int base_col = RAGGED ? 0 : tile_col;  // RAGGED: the lane's columns may start before the tile's
         const int k_begin = (run_lo - tile * plan.ksteps) * 32;
         const int k_end = min(k, (run_hi - tile * plan.ksteps) * 32);
         const int nsteps = run_hi - run_lo;
@@ -77,11 +81,11 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_w4a16_kernel(int kst
 
         // weights: the wave's rows at the tile's first byte column; a lane whose 16 columns lie past N reads the tile's
         // first columns and its results are never stored
-        const int64_t w_bytes = int64_t(k_end - k_begin) * row_bytes - (tile_col >> 1);
+        const int64_t w_bytes = int64_t(k_end - k_begin) * row_bytes - (base_col >> 1);
         const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t *>(w + int64_t(k_begin) * row_bytes + (tile_col >> 1)), 0, int(w_bytes < 0 ? 0 : w_bytes), 0x00020000);
-        uint32_t w_off = uint32_t(8 * g) * uint32_t(row_bytes) + (col_ok ? cl * 8 : 0);
-        const int s_col_off = (tile_col + (col_ok ? cl * 16 : 0)) * 2;
+            const_cast<uint8_t *>(w + int64_t(k_begin) * row_bytes + (base_col >> 1)), 0, int(w_bytes < 0 ? 0 : w_bytes), 0x00020000);
+        uint32_t w_off = uint32_t(8 * g) * uint32_t(row_bytes) + (col_ok ? (lane_col - base_col) >> 1 : 0);
+        const int s_col_off = (col_ok ? lane_col : tile_col) * 2;
         uint4v_t sc_raw[2] = {uint4v_t{0u, 0u, 0u, 0u}, uint4v_t{0u, 0u, 0u, 0u}};
 
         // kDepth 32-row steps are fetched together: a step is only 4 KiB per wave here (8 bytes per lane and row).
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_w4a16_kernel(int kst
                 }
             }
         }
-        skinny_stash(total, m, wave, red);
+        skinny_stash(total, m, wave, red, RAGGED ? (lane_col - tile_col) >> 2 : 4 * cl);
     }
     // no column factor: the group scales are already in the totals; BIAS: the bias (of the output's type) is added to the
     // rounded result, as a matmul followed by an add would. Without one the kernels are the ones that never knew of it.
@@ -169,11 +173,11 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_w4a16_kernel(int kst
     // (worked out here, not inside the loop: there it was measured to cost the loop more than it saves the tail)
     const SkinnyRoles roles = skinny_roles_of(plan, wk, grp, kSkinnyWaves);
     if constexpr (DT == HIDET_QMM_F16)
-        skinny_tails<_Float16, kSkinnyWaves>(plan, wk, roles, m, n, no_scale, reinterpret_cast<_Float16 *>(c), mailbox, lost_flag, red);
+        skinny_tails<_Float16, kSkinnyWaves, false>(plan, wk, roles, m, n, n, no_scale, reinterpret_cast<_Float16 *>(c), mailbox, lost_flag, red);
     else if constexpr (BIAS)
-        skinny_tails<bf16_biased_t, kSkinnyWaves>(plan, wk, roles, m, n, no_scale, reinterpret_cast<bf16_biased_t *>(c), mailbox, lost_flag, red);
+        skinny_tails<bf16_biased_t, kSkinnyWaves, false>(plan, wk, roles, m, n, n, no_scale, reinterpret_cast<bf16_biased_t *>(c), mailbox, lost_flag, red);
     else
-        skinny_tails<uint16_t, kSkinnyWaves>(plan, wk, roles, m, n, no_scale, c, mailbox, lost_flag, red);
+        skinny_tails<uint16_t, kSkinnyWaves, false>(plan, wk, roles, m, n, n, no_scale, c, mailbox, lost_flag, red);
 }
 
 // Any shape the fast kernel cannot take: one thread per output element, serial K, fp32 accumulation.
@@ -204,7 +208,7 @@ __global__ __launch_bounds__(256) void naive_w4a16_kernel(const uint16_t *__rest
 }  // namespace
 
 bool skinny_w4a16_fast(const void *w, const void *scales, int64_t k, int64_t n, int group) {
-    return (n % 16 == 0) && n < (int64_t(1) << 30) && (group % 32 == 0) && aligned(w, 8) && aligned(scales, 16) && k > 0;
+    return (n % 8 == 0) && n >= 16 && n < (int64_t(1) << 30) && (group % 32 == 0) && aligned(w, 4) && aligned(scales, 16) && k > 0;
 }
 
 void skinny_w4a16_launch(const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
@@ -245,23 +249,18 @@ void skinny_w4a16_launch(const void *a, const void *w, const void *scales, const
                    wp, ap0 + m0 * lda, lda, mt, int(k), int(n), group, static_cast<SkinnyPlanRest>(plan), sp, bp, cp0 + m0 * n, ws.mailbox,
                    lost_flag);
         };
-        if (dtype == HIDET_QMM_F16) {
-            if (bias != nullptr) {
-                if (aligned_a) go(skinny_w4a16_kernel<HIDET_QMM_F16, true, true>);
-                else go(skinny_w4a16_kernel<HIDET_QMM_F16, false, true>);
-            } else {
-                if (aligned_a) go(skinny_w4a16_kernel<HIDET_QMM_F16, true, false>);
-                else go(skinny_w4a16_kernel<HIDET_QMM_F16, false, false>);
-            }
-        } else {
-            if (bias != nullptr) {
-                if (aligned_a) go(skinny_w4a16_kernel<HIDET_QMM_BF16, true, true>);
-                else go(skinny_w4a16_kernel<HIDET_QMM_BF16, false, true>);
-            } else {
-                if (aligned_a) go(skinny_w4a16_kernel<HIDET_QMM_BF16, true, false>);
-                else go(skinny_w4a16_kernel<HIDET_QMM_BF16, false, false>);
-            }
-        }
+        auto pick = [&](auto dt, auto ragged_tag) {
+            constexpr int DT = decltype(dt)::value;
+            constexpr bool RAGGED = decltype(ragged_tag)::value;
+            if (bias != nullptr) aligned_a ? go(skinny_w4a16_kernel<DT, true, true, RAGGED>) : go(skinny_w4a16_kernel<DT, false, true, RAGGED>);
+            else aligned_a ? go(skinny_w4a16_kernel<DT, true, false, RAGGED>) : go(skinny_w4a16_kernel<DT, false, false, RAGGED>);
+        };
+        auto pick_type = [&](auto ragged_tag) {
+            if (dtype == HIDET_QMM_F16) pick(std::integral_constant<int, HIDET_QMM_F16>(), ragged_tag);
+            else pick(std::integral_constant<int, HIDET_QMM_BF16>(), ragged_tag);
+        };
+        if (n % 16 != 0 || !aligned(w, 8)) pick_type(std::true_type());
+        else pick_type(std::false_type());
     }
 }
 

@@ -33,13 +33,16 @@ struct SkinnyStep {
     half8_t xa;
 };
 
-template <bool ALIGNED_A, int WAVES, int RING, bool BIAS>
+// RAGGED: N is a multiple of 4 only (at least 16), so the last lane with columns may have fewer than 16 of them: it then takes
+// the last 16 columns of the row instead and shares some with its neighbour (both store the same sums). `n_out` columns of
+// the result are written, at a row stride of n_out.
+template <bool ALIGNED_A, int WAVES, int RING, bool BIAS, bool RAGGED>
 __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_kernel(int ksteps, uint32_t ksteps_magic, int per_group, int longer, int splits, uint32_t splits_magic,
                                                                   const int8_t *__restrict__ w, const _Float16 *__restrict__ a,
                                                                   int64_t lda, int m, int k, int n, SkinnyPlanRest plan_rest,
                                                                   const _Float16 *__restrict__ scale,
                                                                   const _Float16 *__restrict__ bias, _Float16 *__restrict__ c,
-                                                                  float *__restrict__ mailbox, uint32_t *__restrict__ lost_flag) {
+                                                                  float *__restrict__ mailbox, uint32_t *__restrict__ lost_flag, int n_out) {
     extern __shared__ float red[];  // [WAVES][m][kSkinnyRedStride]
 
     const SkinnyPlanHead plan_head = {ksteps, ksteps_magic, per_group, longer, splits, splits_magic};
@@ -86,11 +89,16 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_kernel(int ksteps, ui
     const int k_begin = (run_lo - tile * plan.ksteps) * 32;
     const int k_end = min(k, (run_hi - tile * plan.ksteps) * 32);
     const int ngroups = (run_hi - run_lo + RING - 1) / RING;
-    const int64_t w_bytes = int64_t(k_end - k_begin) * n - tile_col;
+    // (RAGGED: the buffer starts at column 0, the lane's columns may start before the tile's)
+    const int base_col = RAGGED ? 0 : tile_col;
+    const int64_t w_bytes = int64_t(k_end - k_begin) * n - base_col;
     const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t *>(w + int64_t(k_begin) * n + tile_col), 0, int(w_bytes < 0 || ngroups == 0 ? 0 : w_bytes), 0x00020000);
+        const_cast<int8_t *>(w + int64_t(k_begin) * n + base_col), 0, int(w_bytes < 0 || ngroups == 0 ? 0 : w_bytes), 0x00020000);
+    int lane_col = tile_col + cl * 16;
+    if (RAGGED && lane_col < n && lane_col + 16 > n) lane_col = n - 16;
+    const int first_chunk = RAGGED ? (lane_col - tile_col) >> 2 : 4 * cl;
     // offset of row 8g of the next step to be issued; kept opaque so that it stays one register instead of one per load
-    uint32_t w_off = uint32_t(8 * g) * uint32_t(n) + (tile_col + cl * 16 < n ? cl * 16 : 0);
+    uint32_t w_off = uint32_t(8 * g) * uint32_t(n) + (lane_col < n ? lane_col - base_col : 0);
     SkinnyStep ring[RING];
     auto issue = [&](SkinnyStep &st, int step) {
 #pragma unroll
@@ -150,15 +158,16 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_kernel(int ksteps, ui
     for (int t = 0; t < 16; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[t][v] -= 1152.0f * xsum[v];
-    skinny_stash(acc, m, wave, red);
+    skinny_stash(acc, m, wave, red, first_chunk);
     // calls without a bias run the epilogue that never knew of one: every instruction behind the last weight counts
     const SkinnyScale col_scale = {scale, BIAS ? bias : nullptr};
-    if constexpr (BIAS) skinny_tails<_Float16, WAVES>(plan, wk, roles, m, n, col_scale, c, mailbox, lost_flag, red);
-    else skinny_tails<f16_unbiased_t, WAVES>(plan, wk, roles, m, n, col_scale, reinterpret_cast<f16_unbiased_t *>(c), mailbox, lost_flag, red);
+    const int cols = RAGGED ? n_out : n;
+    if constexpr (BIAS) skinny_tails<_Float16, WAVES, RAGGED>(plan, wk, roles, m, cols, n, col_scale, c, mailbox, lost_flag, red);
+    else skinny_tails<f16_unbiased_t, WAVES, RAGGED>(plan, wk, roles, m, cols, n, col_scale, reinterpret_cast<f16_unbiased_t *>(c), mailbox, lost_flag, red);
 }
 
-// Any shape the fast kernel cannot take (N not a multiple of 16, misaligned weights): one thread per
-// output element, serial K, fp32 accumulation.
+// What neither the matrix kernels nor operands copied to padded ones can serve (no room for the copies, tensors beyond 31-bit
+// offsets): one thread per output element, serial K, fp32 accumulation.
 __global__ __launch_bounds__(256) void naive_w8a16_kernel(const _Float16 *__restrict__ a, int64_t lda,
                                                           const int8_t *__restrict__ w, const _Float16 *__restrict__ scale,
                                                           const _Float16 *__restrict__ bias, _Float16 *__restrict__ c, int64_t m,
@@ -173,43 +182,49 @@ __global__ __launch_bounds__(256) void naive_w8a16_kernel(const _Float16 *__rest
 
 }  // namespace
 
+// 16-byte weight loads at the alignment of a dword, 8-byte scale and bias loads, column offsets in bytes below 2^31
+bool skinny_w8a16_supported(const void *w, const void *scale, const void *bias, int64_t k, int64_t n) {
+    return n % 4 == 0 && n >= 16 && n < (int64_t(1) << 30) && aligned(w, 4) && aligned(scale, 8) && aligned(bias, 8) && k > 0;
+}
+
+// `n_out` <= n columns of the result are written, at a row stride of n_out (n_out < n: the weight's rows were padded).
 void skinny_w8a16_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
-                         int64_t n, int64_t lda, int parallel_k_parts, void *workspace, int64_t workspace_bytes,
-                         bool strict_workspace, hipStream_t stream) {
-    // 8-byte scale and bias loads, column offsets in bytes below 2^31
-    const bool fast = (n % 16 == 0) && n < (int64_t(1) << 30) && aligned(w, 16) && aligned(scale, 8) && aligned(bias, 8) && k > 0;
+                         int64_t n, int64_t lda, int64_t n_out, int parallel_k_parts, const Workspace &ws, bool strict_workspace,
+                         hipStream_t stream) {
+    const bool fast = skinny_w8a16_supported(w, scale, bias, k, n);
     constexpr int waves = kWaves;
-    const Workspace ws = split_workspace(workspace, workspace_bytes);
     SkinnyPlan plan;
     if (fast) plan = skinny_make_plan(k, n, parallel_k_parts, int(std::min<int64_t>(16, m)), ws.mailbox_bytes, strict_workspace, /*flat_ok=*/true, device_cus());
     // a wave's run of rows is addressed with 31-bit offsets
     if (!fast || (cdiv(cdiv(skinny_units(plan), plan.groups), waves) * 32 + 160) * n >= (int64_t(1) << 31) - (1 << 20)) {
+        QMM_CHECK(n_out == n, "padded weights of " << k << " x " << n << " cannot be addressed");
         launch(naive_w8a16_kernel, dim3(cdiv(m * n, 256)), dim3(256), 0, stream, static_cast<const _Float16 *>(a), lda,
                static_cast<const int8_t *>(w), static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias),
                static_cast<_Float16 *>(c), m, k, n);
         return;
     }
+    const bool ragged = n % 16 != 0 || !aligned(w, 16) || n_out != n;
     // 16-byte activation loads through a buffer descriptor: aligned rows, offsets below 2^31
     const bool aligned_a = (k % 8 == 0) && (lda % 8 == 0) && aligned(a, 16) && (15 * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20);
     uint32_t *lost_flag = ws.counters != nullptr ? ws.counters + kExchangeLostWord : nullptr;
     for (int64_t m0 = 0; m0 < m; m0 += 16) {
         const int mt = int(std::min<int64_t>(16, m - m0));
         const _Float16 *ap = static_cast<const _Float16 *>(a) + m0 * lda;
-        _Float16 *cp = static_cast<_Float16 *>(c) + m0 * n;
+        _Float16 *cp = static_cast<_Float16 *>(c) + m0 * n_out;
         const size_t shmem = skinny_lds_bytes(mt, waves);
         auto go = [&](auto kern) {
             if (shmem > 65536) allow_dynamic_lds(reinterpret_cast<const void *>(kern), int(skinny_lds_bytes(16, waves)));  // the most any m needs
             launch(kern, dim3(skinny_grid(plan)), dim3(64 * waves), shmem, stream, plan.ksteps, plan.ksteps_magic, plan.per_group, plan.longer, plan.splits, plan.splits_magic,
                    static_cast<const int8_t *>(w), ap, lda, mt, int(k), int(n), static_cast<SkinnyPlanRest>(plan),
-                   static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias), cp, ws.mailbox, lost_flag);
+                   static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias), cp, ws.mailbox, lost_flag, int(n_out));
         };
-        if (bias != nullptr) {
-            if (aligned_a) go(skinny_w8a16_kernel<true, waves, kRing, true>);
-            else go(skinny_w8a16_kernel<false, waves, kRing, true>);
-        } else {
-            if (aligned_a) go(skinny_w8a16_kernel<true, waves, kRing, false>);
-            else go(skinny_w8a16_kernel<false, waves, kRing, false>);
-        }
+        auto with_bias = [&](auto aligned_tag, auto ragged_tag) {
+            constexpr bool ALIGNED = decltype(aligned_tag)::value, RAGGED = decltype(ragged_tag)::value;
+            if (bias != nullptr) go(skinny_w8a16_kernel<ALIGNED, waves, kRing, true, RAGGED>);
+            else go(skinny_w8a16_kernel<ALIGNED, waves, kRing, false, RAGGED>);
+        };
+        if (ragged) aligned_a ? with_bias(std::true_type(), std::true_type()) : with_bias(std::false_type(), std::true_type());
+        else aligned_a ? with_bias(std::true_type(), std::false_type()) : with_bias(std::false_type(), std::false_type());
     }
 }
 

@@ -1,0 +1,61 @@
+"""Sizes off the matrix kernels' tiles: N a multiple of 4 (int4: 8) only, where the last lane with columns shares some of them
+with its neighbour, and K or N that the matrix kernels do not take at all, where they run on padded copies. Small integers and
+powers of two: every sum is exact, the result must equal integer arithmetic with the definition's roundings, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from hidet_amd import ffi
+from hidet_amd.graph.ops import quant
+from gpu_util import announce, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _int8_case(m, k, n, biased):
+    rng = np.random.default_rng(1000 * m + k + n)
+    a = rng.integers(-3, 4, (m, k)).astype(np.float32)
+    w = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    s = (2.0 ** rng.integers(-6, 1, n)).astype(np.float32)
+    with np.errstate(over='ignore'):
+        want = ((a.astype(np.float64) @ w.astype(np.float64)) * s).astype(np.float32).astype(np.float16)
+        b = (rng.integers(-64, 65, n) / 8.0).astype(np.float16) if biased else None
+        if biased:
+            want = (want.astype(np.float32) + b.astype(np.float32)).astype(np.float16)
+    return dev(a.astype(np.float16)), dev(w), dev(s.astype(np.float16)), None if b is None else dev(b), want
+
+
+@pytest.mark.parametrize('m,k,n,biased', [
+    # N a multiple of 4: one short lane in the first tile, a tile of 4 columns behind a whole one, both exchange layouts, K tails
+    (1, 96, 20, False), (3, 4096, 260, True), (16, 4100, 516, False), (1, 4096, 8196, False), (2, 1002, 8204, True), (24, 2050, 276, False),
+    # padded copies: N of no multiple of 4 with one pass of 16 rows and with the GEMM, K of no multiple of 64, several row tiles
+    (1, 4100, 258, False), (16, 1022, 1030, True), (17, 4094, 518, False), (33, 4100, 260, True), (129, 1000, 770, False), (300, 2050, 4098, True)])
+def test_int8_exact(m, k, n, biased):
+    announce('ragged int8', m, k, n, biased)
+    a, w, s, b, want = _int8_case(m, k, n, biased)
+    for _ in range(2):  # the exchange's mailbox is clean again after the first call
+        assert np.array_equal(host(quant.symmetric_quant_matmul(a, w, s, b)), want)
+
+
+@pytest.mark.parametrize('scratch', [1 << 20, 3 << 20])
+def test_int8_in_panels_of_a_small_workspace(scratch):
+    announce('ragged int8 panels', scratch)
+    m, k, n = 270, 1000, 1031
+    a, w, s, _, want = _int8_case(m, k, n, False)
+    c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+    ws = torch.zeros(int(ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(scratch)), dtype=torch.uint8, device='cuda')
+    ffi.call('hidet_symmetric_quant_matmul_f16_i8', a, w, s, c, m, k, n, k, 0, ws, ws.numel(), ffi.current_stream(a.device))
+    assert np.array_equal(host(c), want)
+
+
+@pytest.mark.parametrize('m,k,n,group', [(1, 256, 24, 128), (16, 4096, 264, 128), (3, 1024, 1032, 32), (20, 512, 520, 64)])
+def test_int4_exact(m, k, n, group):
+    announce('ragged int4', m, k, n, group)
+    rng = np.random.default_rng(m + k + n)
+    a = rng.integers(-3, 4, (m, k)).astype(np.float32)
+    q = rng.integers(-7, 8, (k, n)).astype(np.int8)
+    s = rng.integers(1, 4, (k // group, n)).astype(np.float32)
+    want = O.to_bf16((a.astype(np.float64) @ (q.astype(np.float64) * np.repeat(s, group, axis=0))).astype(np.float32))
+    got = quant.symmetric_quant_matmul_w4a16(dev(a, torch.bfloat16), dev(O.pack_int4(q)), dev(s, torch.bfloat16), group)
+    assert np.array_equal(host(got), want)
