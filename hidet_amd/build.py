@@ -1,4 +1,5 @@
-"""Builds libhidet_qmm.so from the HIP sources under csrc/ with hipcc for gfx950.
+"""Builds libhidet_qmm.so from the HIP sources under csrc/ with hipcc for gfx950, and the extension module _front.so (host
+code only, against torch's headers) from csrc/torch_front.cpp.
 
 Plays the part of the reference's compile step for these operators (python/hidet/backend/build.py:206-280,
 `HIPCC.compile`): same compiler, same `--offload-arch`, `-fPIC --shared`; `-ffast-math` is dropped because
@@ -14,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB_DIR = os.path.join(HERE, 'lib')
 LIB_PATH = os.path.join(LIB_DIR, 'libhidet_qmm.so')
+FRONT_PATH = os.path.join(LIB_DIR, '_front.so')
 ARCH = 'gfx950'
 
 FLAGS = [
@@ -47,15 +49,37 @@ def _compile(src, obj, verbose):
         print(out, file=sys.stderr)
 
 
+def _build_front():
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    include = [os.path.join(root, 'include'), os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
+               os.path.join(rocm, 'include'), sysconfig.get_paths()['include']]
+    tmp = FRONT_PATH + '.tmp'
+    cmd = (['g++', '-O2', '-std=c++17', '-fPIC', '-fvisibility=hidden', '-shared', '-w', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+            '-D_GLIBCXX_USE_CXX11_ABI={}'.format(int(torch._C._GLIBCXX_USE_CXX11_ABI))] + ['-I' + i for i in include] +
+           [os.path.join(CSRC, 'torch_front.cpp'), '-o', tmp, '-L' + os.path.join(root, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu',
+            '-ltorch_python', '-ltorch'])
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError('g++ failed on torch_front.cpp:\n' + r.stdout)
+    os.replace(tmp, FRONT_PATH)
+
+
 def build(verbose=False, jobs=8):
-    """Compile every .hip source and link the shared library (always recompiles)."""
+    """Compile every .hip source and link the shared library, and the native front (always recompiles)."""
     obj_dir = os.path.join(HERE, 'build')
     os.makedirs(obj_dir, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     srcs = sources()
     objs = [os.path.join(obj_dir, s[:-4] + '.o') for s in srcs]
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        front = pool.submit(_build_front)
         list(pool.map(lambda so: _compile(so[0], so[1], verbose), zip(srcs, objs)))
+        front.result()
     tmp = LIB_PATH + '.tmp'
     cmd = [hipcc(), '--offload-arch=' + ARCH, '-shared', '-fPIC', '-o', tmp] + objs
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -1,0 +1,270 @@
+// Native front of the decode-sized operators: the argument checks, the output allocation and the call of the library's
+// entry point in one step of compiled code.  A decode loop makes one such call per linear layer and token, and the kernel
+// of a 4096 x 4096 layer runs 6 us; the same work in Python with a ctypes call took 10 us of host time.
+//
+// Every function here takes torch tensors and either does the whole call or returns None, without an effect, when the
+// arguments are not exactly what it handles (another dtype or layout, a subclass, something to be copied, an error to be
+// reported): the Python operators then run their complete path.  Nothing is remembered about a tensor between calls; the
+// workspaces are those of hidet_amd.ffi, looked up by (device, stream) on every call.
+#include <ATen/ATen.h>
+#include <Python.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdint>
+
+#include "../../include/hidet_qmm.h"
+
+namespace {
+
+// Entry points of libhidet_qmm.so, handed over by hidet_amd.ffi (which opened the library), and what errors need.
+struct Library {
+    decltype(&hidet_get_last_error) get_last_error;
+    decltype(&hidet_symmetric_quant_matmul_f16_i8) w8a16;
+    decltype(&hidet_symmetric_quant_matmul_f16_i8_bias) w8a16_bias;
+    decltype(&hidet_symmetric_quant_matmul_f16_i8_nk) w8a16_nk;
+    decltype(&hidet_symmetric_quant_matmul_f16_i8_nk_bias) w8a16_nk_bias;
+    decltype(&hidet_symmetric_quant_matmul_w4a16) w4a16;
+    decltype(&hidet_symmetric_quant_matmul_w4a16_bias) w4a16_bias;
+    decltype(&hidet_fp8_quantize_per_tensor) fp8_quantize;
+    decltype(&hidet_matmul_f8) matmul_f8;
+} lib;
+PyObject *workspaces = nullptr;      // hidet_amd.ffi._WORKSPACES: (device, stream) -> uint8 tensor
+PyObject *new_workspace = nullptr;   // hidet_amd.ffi.workspace(device): makes the entry
+PyObject *backend_error = nullptr;   // hidet_amd.ffi.BackendException
+
+const at::Tensor *tensor(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// A GPU tensor of that type (an argument of these functions: anything else is left to Python).
+const at::Tensor *gpu_tensor(PyObject *o, at::ScalarType type) {
+    const at::Tensor *t = tensor(o);
+    return t != nullptr && t->is_cuda() && t->scalar_type() == type && t->layout() == at::kStrided ? t : nullptr;
+}
+
+bool same_device(const at::Tensor &a, const at::Tensor &b) { return a.get_device() == b.get_device(); }
+
+struct Rows {
+    int64_t m, stride;
+};
+// The leading axes of `a` folded into rows of `k` contiguous elements, where that needs no copy.
+bool as_rows(const at::Tensor &a, int64_t k, Rows *r) {
+    if (a.dim() < 2 || k == 0 || a.size(-1) != k) return false;
+    r->m = a.numel() / k;
+    r->stride = k;
+    if (r->m == 0) return false;
+    if (a.is_contiguous()) return true;
+    if (a.dim() != 2 || a.stride(1) != 1 || a.stride(0) < k) return false;
+    if (r->m > 1) r->stride = a.stride(0);
+    return true;
+}
+
+struct Workspace {
+    void *stream, *ptr;
+    int64_t bytes;
+};
+// The current stream of the tensor's device and its workspace; false with a Python error set.
+bool stream_and_workspace(const at::Tensor &t, Workspace *w) {
+    const auto device = t.get_device();
+    w->stream = c10::hip::getCurrentHIPStream(device).stream();
+    PyObject *key = Py_BuildValue("(iL)", int(device), static_cast<long long>(reinterpret_cast<intptr_t>(w->stream)));
+    if (key == nullptr) return false;
+    PyObject *ws = PyDict_GetItemWithError(workspaces, key);  // borrowed
+    Py_DECREF(key);
+    PyObject *made = nullptr;
+    if (ws == nullptr) {
+        if (PyErr_Occurred()) return false;
+        PyObject *dev = THPDevice_New(t.device());
+        if (dev == nullptr) return false;
+        ws = made = PyObject_CallFunctionObjArgs(new_workspace, dev, nullptr);
+        Py_DECREF(dev);
+        if (made == nullptr) return false;
+    }
+    const at::Tensor &buffer = THPVariable_Unpack(ws);
+    w->ptr = buffer.data_ptr();
+    w->bytes = buffer.numel();
+    Py_XDECREF(made);  // the dictionary holds it
+    return true;
+}
+
+at::Tensor output(const at::Tensor &a, int64_t n, at::ScalarType type) {
+    auto sizes = a.sizes().vec();
+    sizes.back() = n;
+    return at::empty(sizes, a.options().dtype(type).requires_grad(false));
+}
+
+// The result, or the library's error as an exception.
+PyObject *finish(const char *name, PyObject *result) {
+    const char *error = lib.get_last_error();
+    if (error != nullptr) {
+        Py_XDECREF(result);
+        return PyErr_Format(backend_error, "Calling %s failed. error:\n%s", name, error);
+    }
+    return result;
+}
+
+template <typename F>
+PyObject *guarded(F &&f) {
+    try {
+        return f();
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+
+// a, weight, scale, bias or None
+PyObject *w8a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject * {
+        const at::Tensor *a = nargs == 4 ? gpu_tensor(args[0], at::kHalf) : nullptr;
+        const at::Tensor *w = a ? gpu_tensor(args[1], at::kChar) : nullptr;
+        const at::Tensor *scale = w ? gpu_tensor(args[2], at::kHalf) : nullptr;
+        const bool biased = nargs == 4 && args[3] != Py_None;
+        const at::Tensor *bias = scale && biased ? gpu_tensor(args[3], at::kHalf) : nullptr;
+        Rows rows;
+        if (scale == nullptr || (biased && bias == nullptr) || w->dim() != 2 || !same_device(*a, *w) || !same_device(*a, *scale)) Py_RETURN_NONE;
+        const int64_t k = w->size(0), n = w->size(1);
+        if (n == 0 || k % 2 != 0 || n % 2 != 0 || !as_rows(*a, k, &rows) || scale->dim() != 1 || scale->size(0) != n || !scale->is_contiguous()) Py_RETURN_NONE;
+        if (biased && (bias->dim() != 1 || bias->size(0) != n || !bias->is_contiguous() || !same_device(*a, *bias))) Py_RETURN_NONE;
+        const bool row_major = w->is_contiguous();
+        const int64_t ldw = w->stride(1);
+        // the same operand held K-contiguous: up to 16 rows (more rows and everything else: the Python operator)
+        if (!row_major && !(rows.m <= 16 && w->stride(0) == 1 && ldw >= k && ldw % 16 == 0 && k % 16 == 0 && reinterpret_cast<uintptr_t>(w->data_ptr()) % 16 == 0))
+            Py_RETURN_NONE;
+        Workspace ws;
+        if (!stream_and_workspace(*a, &ws)) return nullptr;
+        at::Tensor c = output(*a, n, at::kHalf);
+        const void *ap = a->data_ptr(), *wp = w->data_ptr(), *sp = scale->data_ptr(), *bp = biased ? bias->data_ptr() : nullptr;
+        void *cp = c.data_ptr();
+        if (row_major) {
+            if (biased) lib.w8a16_bias(ap, wp, sp, bp, cp, rows.m, k, n, rows.stride, 0, ws.ptr, ws.bytes, ws.stream);
+            else lib.w8a16(ap, wp, sp, cp, rows.m, k, n, rows.stride, 0, ws.ptr, ws.bytes, ws.stream);
+        } else {
+            if (biased) lib.w8a16_nk_bias(ap, wp, sp, bp, cp, rows.m, k, n, rows.stride, ldw, ws.ptr, ws.bytes, ws.stream);
+            else lib.w8a16_nk(ap, wp, sp, cp, rows.m, k, n, rows.stride, ldw, ws.ptr, ws.bytes, ws.stream);
+        }
+        return finish("hidet_symmetric_quant_matmul_f16_i8", THPVariable_Wrap(std::move(c)));
+    });
+}
+
+// a, packed, scales, group size, bias or None
+PyObject *w4a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject * {
+        const at::Tensor *a = nargs == 5 ? tensor(args[0]) : nullptr;
+        if (a == nullptr || !a->is_cuda() || (a->scalar_type() != at::kHalf && a->scalar_type() != at::kBFloat16)) Py_RETURN_NONE;
+        const at::Tensor *w = gpu_tensor(args[1], at::kByte), *scales = w ? gpu_tensor(args[2], a->scalar_type()) : nullptr;
+        const bool biased = args[4] != Py_None;
+        const at::Tensor *bias = scales && biased ? gpu_tensor(args[4], a->scalar_type()) : nullptr;
+        if (scales == nullptr || (biased && bias == nullptr) || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+        const long group = PyLong_AsLong(args[3]);
+        if (group == -1 && PyErr_Occurred()) return nullptr;
+        if (w->dim() != 2 || scales->dim() != 2 || !w->is_contiguous() || !scales->is_contiguous() || !same_device(*a, *w) || !same_device(*a, *scales)) Py_RETURN_NONE;
+        const int64_t k = w->size(0), n = w->size(1) * 2;
+        Rows rows;
+        if (n == 0 || group <= 0 || group > INT32_MAX || k % group != 0 || scales->size(0) != k / group || scales->size(1) != n || !as_rows(*a, k, &rows)) Py_RETURN_NONE;
+        if (biased && (bias->dim() != 1 || bias->size(0) != n || !bias->is_contiguous() || !same_device(*a, *bias))) Py_RETURN_NONE;
+        Workspace ws;
+        if (!stream_and_workspace(*a, &ws)) return nullptr;
+        at::Tensor c = output(*a, n, a->scalar_type());
+        const int dtype = a->scalar_type() == at::kHalf ? HIDET_QMM_F16 : HIDET_QMM_BF16;
+        if (biased)
+            lib.w4a16_bias(a->data_ptr(), w->data_ptr(), scales->data_ptr(), bias->data_ptr(), c.data_ptr(), rows.m, k, n, rows.stride, int(group), dtype, 0,
+                           ws.ptr, ws.bytes, ws.stream);
+        else
+            lib.w4a16(a->data_ptr(), w->data_ptr(), scales->data_ptr(), c.data_ptr(), rows.m, k, n, rows.stride, int(group), dtype, 0, ws.ptr, ws.bytes, ws.stream);
+        return finish("hidet_symmetric_quant_matmul_w4a16", THPVariable_Wrap(std::move(c)));
+    });
+}
+
+// x -> (codes, scale)
+PyObject *fp8_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject * {
+        const at::Tensor *x = nargs == 1 ? tensor(args[0]) : nullptr;
+        if (x == nullptr || !x->is_cuda() || !x->is_contiguous()) Py_RETURN_NONE;
+        int dtype;
+        switch (x->scalar_type()) {
+            case at::kFloat: dtype = HIDET_QMM_F32; break;
+            case at::kHalf: dtype = HIDET_QMM_F16; break;
+            case at::kBFloat16: dtype = HIDET_QMM_BF16; break;
+            default: Py_RETURN_NONE;
+        }
+        Workspace ws;
+        if (!stream_and_workspace(*x, &ws)) return nullptr;
+        at::Tensor codes = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
+        at::Tensor scale = at::empty({1}, x->options().dtype(at::kFloat).requires_grad(false));
+        lib.fp8_quantize(x->data_ptr(), codes.data_ptr(), scale.data_ptr(), x->numel(), dtype, ws.ptr, ws.bytes, ws.stream);
+        PyObject *pair = PyTuple_New(2);
+        if (pair == nullptr) return nullptr;
+        PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(std::move(codes)));
+        PyTuple_SET_ITEM(pair, 1, THPVariable_Wrap(std::move(scale)));
+        return finish("hidet_fp8_quantize_per_tensor", pair);
+    });
+}
+
+// a, b [N, K] (both float8_e4m3), scale_a, scale_b (float32, one element; both None: unscaled), output dtype
+PyObject *matmul_f8(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject * {
+        const at::Tensor *a = nargs == 5 ? gpu_tensor(args[0], at::kFloat8_e4m3fn) : nullptr, *b = a ? gpu_tensor(args[1], at::kFloat8_e4m3fn) : nullptr;
+        if (b == nullptr || !THPDtype_Check(args[4]) || b->dim() != 2 || !same_device(*a, *b)) Py_RETURN_NONE;
+        const at::Tensor *scale[2] = {nullptr, nullptr};
+        for (int i = 0; i < 2; ++i) {
+            if (args[2 + i] == Py_None) continue;
+            scale[i] = gpu_tensor(args[2 + i], at::kFloat);
+            if (scale[i] == nullptr || scale[i]->numel() != 1 || !same_device(*a, *scale[i])) Py_RETURN_NONE;
+        }
+        const at::ScalarType type = reinterpret_cast<THPDtype *>(args[4])->scalar_type;
+        int out;
+        switch (type) {
+            case at::kFloat: out = HIDET_QMM_F32; break;
+            case at::kHalf: out = HIDET_QMM_F16; break;
+            case at::kBFloat16: out = HIDET_QMM_BF16; break;
+            case at::kFloat8_e4m3fn: out = HIDET_QMM_E4M3; break;
+            default: Py_RETURN_NONE;
+        }
+        const int64_t n = b->size(0), k = b->size(1);
+        Rows rows;
+        if (n == 0 || !as_rows(*a, k, &rows) || (k > 1 && b->stride(1) != 1) || (n > 1 && b->stride(0) < k)) Py_RETURN_NONE;
+        Workspace ws;
+        if (!stream_and_workspace(*a, &ws)) return nullptr;
+        at::Tensor c = output(*a, n, type);
+        lib.matmul_f8(a->data_ptr(), b->data_ptr(), c.data_ptr(), rows.m, n, k, rows.stride, n > 1 ? b->stride(0) : k, out, scale[0] ? scale[0]->data_ptr() : nullptr,
+                      scale[1] ? scale[1]->data_ptr() : nullptr, ws.ptr, ws.bytes, ws.stream);
+        return finish("hidet_matmul_f8", THPVariable_Wrap(std::move(c)));
+    });
+}
+
+// dict of entry point addresses, workspaces, workspace function, exception class
+PyObject *bind(PyObject *, PyObject *args) {
+    PyObject *addresses;
+    if (!PyArg_ParseTuple(args, "O!O!OO", &PyDict_Type, &addresses, &PyDict_Type, &workspaces, &new_workspace, &backend_error)) return nullptr;
+    Py_INCREF(workspaces);
+    Py_INCREF(new_workspace);
+    Py_INCREF(backend_error);
+    auto get = [&](auto &slot, const char *name) {
+        PyObject *v = PyDict_GetItemString(addresses, name);
+        void *p = v != nullptr ? PyLong_AsVoidPtr(v) : nullptr;
+        slot = reinterpret_cast<std::decay_t<decltype(slot)>>(p);
+        if (p == nullptr && !PyErr_Occurred()) PyErr_Format(PyExc_KeyError, "no address for %s", name);
+        return p != nullptr;
+    };
+    const bool ok = get(lib.get_last_error, "hidet_get_last_error") && get(lib.w8a16, "hidet_symmetric_quant_matmul_f16_i8") &&
+                    get(lib.w8a16_bias, "hidet_symmetric_quant_matmul_f16_i8_bias") && get(lib.w8a16_nk, "hidet_symmetric_quant_matmul_f16_i8_nk") &&
+                    get(lib.w8a16_nk_bias, "hidet_symmetric_quant_matmul_f16_i8_nk_bias") && get(lib.w4a16, "hidet_symmetric_quant_matmul_w4a16") &&
+                    get(lib.w4a16_bias, "hidet_symmetric_quant_matmul_w4a16_bias") && get(lib.fp8_quantize, "hidet_fp8_quantize_per_tensor") &&
+                    get(lib.matmul_f8, "hidet_matmul_f8");
+    if (!ok) return nullptr;
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_VARARGS, nullptr},
+    {"w8a16", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(w8a16)), METH_FASTCALL, nullptr},
+    {"w4a16", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(w4a16)), METH_FASTCALL, nullptr},
+    {"fp8_quantize", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fp8_quantize)), METH_FASTCALL, nullptr},
+    {"matmul_f8", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(matmul_f8)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_front", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__front() { return PyModule_Create(&module); }

@@ -7,6 +7,8 @@ python/hidet/ffi/ffi.py:46-60).  There is no CPU fallback: if the library is mis
 a GPU the call fails.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from typing import Dict, Optional, Tuple
 
@@ -14,6 +16,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, 'lib', 'libhidet_qmm.so')
+FRONT_PATH = os.path.join(_HERE, 'lib', '_front.so')
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
 
@@ -168,3 +171,22 @@ def workspace(device: torch.device, nbytes: int = 0) -> torch.Tensor:
         ws = torch.zeros(need, dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
     return ws
+
+
+_FRONT = None
+
+
+def front():
+    """The native front of the decode-sized operators (csrc/torch_front.cpp), bound to the library: each of its functions does a
+    whole call or returns None, and then the Python operator's complete path has to run."""
+    global _FRONT
+    if _FRONT is None:
+        lib = load_library()
+        if not os.path.exists(FRONT_PATH):
+            raise OSError('{} not found: build it with `python -m hidet_amd.build`'.format(FRONT_PATH))
+        loader = importlib.machinery.ExtensionFileLoader('_front', FRONT_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader('_front', loader))
+        loader.exec_module(module)
+        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in SIGNATURES}, _WORKSPACES, workspace, BackendException)
+        _FRONT = module
+    return _FRONT

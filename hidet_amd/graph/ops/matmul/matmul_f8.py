@@ -172,7 +172,8 @@ def _matmul_f8(a, b, is_scaled: bool, scale_a=None, scale_b=None, bias=None, acc
     if not is_scaled:  # checked before: skip building the operator and task records (host time of a decode call)
         out = _VALIDATED.get((a.shape, a.dtype, b.shape, b.dtype, acc_dtype, output_dtype))
         if out is not None:
-            return _run_f8(a, b, out)
+            c = ffi.front().matmul_f8(a, b, None, None, out) if a.is_cuda else None
+            return _run_f8(a, b, out) if c is None else c
     if len(a.shape) < 2 or len(b.shape) < 2:
         raise ValueError('a and b must have at least 2 dimensions, got shape {} and {}'.format(list(a.shape), list(b.shape)))
     if (a.dtype != f8e4m3 or b.dtype != f8e4m3) and (a.dtype != f8e5m2 or b.dtype != f8e5m2):
@@ -207,6 +208,10 @@ def matmul_f8_scaled(a, b, scale_a, scale_b, bias=None, acc_dtype='float32', out
 
 def fp8_quantize_per_tensor(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """(codes float8_e4m3 of x.shape, scale float32 [1]) with scale = max|x| / 448 and codes = e4m3(x / scale)."""
+    if x.is_cuda:
+        out = ffi.front().fp8_quantize(x)
+        if out is not None:
+            return out
     ffi.require_gpu(x)
     if x.dtype not in (torch.float32, torch.float16, torch.bfloat16):
         raise ValueError('fp8_quantize_per_tensor expects float32, float16 or bfloat16, got {}'.format(x.dtype))
@@ -223,6 +228,10 @@ def matmul_f8_per_tensor(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor
                          output_dtype='bfloat16') -> torch.Tensor:
     """cast((a @ b^T) * (scale_a * scale_b)) with fp32 accumulation; the scales are float32 tensors of one
     element on the GPU (as returned by fp8_quantize_per_tensor)."""
+    if a.is_cuda:
+        out = ffi.front().matmul_f8(a, b, scale_a, scale_b, data_type(output_dtype))
+        if out is not None:
+            return out
     if a.dtype != f8e4m3 or b.dtype != f8e4m3:
         raise ValueError('matmul_f8 only supports both operands being f8e4m3 or f8e5m2, got {} and {}'.format(a.dtype, b.dtype))
     if len(a.shape) < 2 or len(b.shape) < 2:

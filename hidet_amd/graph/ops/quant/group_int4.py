@@ -119,6 +119,10 @@ def symmetric_quant_matmul_w4a16(a: torch.Tensor, packed: torch.Tensor, scales: 
     """c[..., M, N] = a @ dequant(packed, scales) with fp32 accumulation; a, scales and c share bfloat16 or float16.
     `bias` ([N], the same type) is added to the rounded result: the bits of the matmul followed by an add, as for the int8
     operator."""
+    if a.is_cuda:
+        out = ffi.front().w4a16(a, packed, scales, group_size, bias)
+        if out is not None:
+            return out
     signature = (a.shape, a.dtype, packed.shape, packed.dtype, scales.shape, scales.dtype, group_size,
                  None if bias is None else (bias.shape, bias.dtype))
     if signature in _VALIDATED:  # checked before: skip building the operator and task records (host time of a decode call)

@@ -149,6 +149,8 @@ class SymmetricQuantizedMatmulOp(Operator):
 # the kernel runs (a 4096 x 11008 GEMV: 11 to 14 us); the device checks and the launch are done on every call.
 _VALIDATED = set()
 
+_LIBRARY_PLANS = ('disabled', 'default')  # values of the parallel_k option that leave the K split to the library
+
 
 def symmetric_quant_matmul(a: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor,
                            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -156,6 +158,10 @@ def symmetric_quant_matmul(a: torch.Tensor, weight: torch.Tensor, scale: torch.T
     does not have, is the fused form of the epilogue its template admits (matmul_f16_i8.py:95-99): a float16 [N] vector
     added to the float16 result (two roundings, as the reference's fused epilogue and the matmul followed by an add
     give): fused and unfused calls return the same bits."""
+    if option.get_parallel_k() in _LIBRARY_PLANS and a.is_cuda:
+        out = ffi.front().w8a16(a, weight, scale, bias)
+        if out is not None:
+            return out
     signature = (a.shape, a.dtype, weight.shape, weight.dtype, scale.shape, scale.dtype,
                  None if bias is None else (bias.shape, bias.dtype))
     if signature in _VALIDATED:

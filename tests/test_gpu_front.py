@@ -1,0 +1,75 @@
+"""The native front of the operators: what it handles equals the Python path bit for bit, and what it does not handle (it
+returns None) still works or raises as before."""
+import pytest
+import torch
+
+from hidet_amd import BackendException, ffi
+from hidet_amd.graph.ops import quant
+from hidet_amd.graph.ops.matmul import matmul_f8 as F8
+from hidet_amd.graph.ops.quant.matmul import run_w8a16
+from hidet_amd.graph.ops.quant.group_int4 import _run_w4a16
+from gpu_util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(m, k, n):
+    g = torch.Generator(device='cuda').manual_seed(m + k + n)
+    x = torch.randn((m, k), generator=g, device='cuda').half()
+    wq, s = quant.symmetric_quantize(torch.randn((k, n), generator=g, device='cuda'), 'int8', 0)
+    return x, wq, s.half(), torch.randn(n, generator=g, device='cuda').half()
+
+
+@pytest.mark.parametrize('m,k,n', [(1, 512, 768), (16, 1024, 512), (70, 256, 320)])
+def test_front_equals_the_python_path(m, k, n):
+    announce('front', m, k, n)
+    x, wq, s, b = _case(m, k, n)
+    wide = torch.randn((m, k + 64), device='cuda').half()[:, :k]  # rows further apart than K
+    nk = quant.to_decode_layout(wq)
+    front = ffi.front()
+    for a in (x, wide, x.reshape(1, m, k)):
+        for w in (wq, nk):
+            for bias in (None, b):
+                got = quant.symmetric_quant_matmul(a, w, s, bias)
+                assert torch.equal(got, run_w8a16(a, w, s, 0, bias)) and got.shape == a.shape[:-1] + (n,)
+        assert front.w8a16(a, wq, s, None) is not None and (front.w8a16(a, nk, s, None) is not None) == (m <= 16)
+    packed, gs = quant.symmetric_group_quantize_int4(torch.randn((k, n), device='cuda'), 128, 'float16')
+    for bias in (None, b):
+        assert torch.equal(quant.symmetric_quant_matmul_w4a16(wide, packed, gs, 128, bias), _run_w4a16(wide, packed, gs, 128, bias))
+    a8, sa = F8.fp8_quantize_per_tensor(x)
+    b8, sb = F8.fp8_quantize_per_tensor(torch.randn((n, k), device='cuda'))
+    assert torch.equal(F8.matmul_f8_per_tensor(a8, b8, sa, sb), F8._run_f8(a8, b8, torch.bfloat16, sa, sb))
+    for _ in range(2):
+        assert torch.equal(F8.matmul_f8(a8, b8, output_dtype='float32'), F8._run_f8(a8, b8, torch.float32))
+
+
+def test_what_the_front_leaves_to_python():
+    announce('front: left to Python')
+    x, wq, s, b = _case(4, 256, 512)
+    front = ffi.front()
+    sparse_rows = torch.randn((4, 512), device='cuda').half()[:, ::2]
+    for args in ((x.float(), wq, s, None), (x, wq.t(), s, None), (x, wq, s.float(), None), (x, wq, s, b[:8]), (x[:, :128], wq, s, None),
+                 (sparse_rows, wq, s, None), (x.cpu(), wq, s, None), (x, wq, s.cpu(), None), (x[0], wq, s, None), (x[:0], wq, s, None)):
+        assert front.w8a16(*args) is None
+    assert torch.equal(quant.symmetric_quant_matmul(sparse_rows, wq, s), quant.symmetric_quant_matmul(sparse_rows.contiguous(), wq, s))
+    assert quant.symmetric_quant_matmul(x[:0], wq, s).shape == (0, 512)
+    with pytest.raises(ValueError):
+        quant.symmetric_quant_matmul(x.float(), wq, s)
+    with pytest.raises(BackendException):
+        quant.symmetric_quant_matmul(x, wq, s.cpu())
+    ffi.load_library().hidet_set_last_error(b'planted')  # an error the library reports surfaces as the exception
+    with pytest.raises(BackendException, match='planted'):
+        quant.symmetric_quant_matmul(x, wq, s)
+
+
+def test_each_stream_has_its_workspace():
+    announce('front: streams')
+    x, wq, s, _ = _case(2, 4096, 8192)
+    want = quant.symmetric_quant_matmul(x, wq, s)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        got = quant.symmetric_quant_matmul(x, wq, s)
+        assert (x.device.index, stream.cuda_stream) in ffi._WORKSPACES
+    stream.synchronize()
+    assert torch.equal(got, want)
