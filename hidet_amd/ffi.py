@@ -177,7 +177,7 @@ _FRONT = None
 
 
 def front():
-    """The native front of the decode-sized operators (csrc/torch_front.cpp), bound to the library: each of its functions does a
+    """The native front of the operators (csrc/torch_front.cpp), bound to the library: each of its functions does a
     whole call or returns None, and then the Python operator's complete path has to run."""
     global _FRONT
     if _FRONT is None:

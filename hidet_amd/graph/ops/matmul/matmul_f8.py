@@ -187,6 +187,10 @@ def _matmul_f8(a, b, is_scaled: bool, scale_a=None, scale_b=None, bias=None, acc
     if output_dtype not in _OUT_TYPES or (output_dtype in (f8e4m3, f8e5m2) and output_dtype != a.dtype):
         raise ValueError('unsupported output dtype {} for operands of {}'.format(output_dtype, a.dtype))
     if is_scaled:
+        if bias is None and a.is_cuda:
+            c = ffi.front().matmul_f8_scaled(a, b, scale_a, scale_b, output_dtype)
+            if c is not None:
+                return c
         return MatmulF8ScaledOperator(a, b, scale_a, scale_b, acc_dtype, output_dtype, bias).outputs[0]
     c = MatmulF8Operator(a, b, acc_dtype, output_dtype).outputs[0]
     _VALIDATED[signature] = output_dtype

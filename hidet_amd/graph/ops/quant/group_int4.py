@@ -49,6 +49,10 @@ def symmetric_group_quantize_int4(w: torch.Tensor, group_size: int = 128, scale_
         raise ValueError('symmetric_group_quantize_int4 expects float32 weights, got {}'.format(w.dtype))
     if scale_dtype not in (torch.bfloat16, torch.float16):
         raise ValueError('scale dtype must be bfloat16 or float16, got {}'.format(scale_dtype))
+    if w.is_cuda:
+        out = ffi.front().quantize_int4(w, group_size, scale_dtype)
+        if out is not None:
+            return out
     op = SymmetricGroupQuantizationInt4Op(w, group_size, scale_dtype)
     return op.outputs[0], op.outputs[1]
 
@@ -159,6 +163,10 @@ def symmetric_quant_matmul_w4a16_decode(a: torch.Tensor, packed_nk: torch.Tensor
     """`symmetric_quant_matmul_w4a16` on a weight repacked with `to_decode_layout_int4` ([N, K/2]); `scales` stay
     [K/group, N]. For decode: up to 16 rows of `a` per pass over the weights. K a multiple of 128, group size 128 times
     a power of two."""
+    if a.is_cuda:
+        out = ffi.front().w4a16_decode(a, packed_nk, scales, group_size)
+        if out is not None:
+            return out
     if len(a.shape) < 2 or len(packed_nk.shape) != 2 or len(scales.shape) != 2:
         raise ValueError('expect a[..., M, K], packed_nk[N, K/2], scales[K/g, N], got {}, {} and {}'.format(
             list(a.shape), list(packed_nk.shape), list(scales.shape)))

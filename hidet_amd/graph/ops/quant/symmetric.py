@@ -121,6 +121,10 @@ def symmetric_quantize(w: torch.Tensor, quant_type='int8', dims: Union[int, List
         raise ValueError('symmetric_quantize supports int8 and int16, got {}'.format(quant_type))
     if w.dtype not in _FLOATS:
         raise ValueError('symmetric_quantize expects a float32, float16 or bfloat16 tensor, got {}'.format(w.dtype))
+    if w.is_cuda:
+        out = ffi.front().quantize(w, quant_type, dims)
+        if out is not None:
+            return out
     op = SymmetricQuantizationOp(w, quant_type, dims=dims)
     return op.outputs[0], op.outputs[1]
 
@@ -130,4 +134,8 @@ def symmetric_dequantize(wq: torch.Tensor, scale: torch.Tensor, dims: Union[int,
         raise ValueError('symmetric_dequantize expects int8 or int16 codes, got {}'.format(wq.dtype))
     if scale.dtype not in _FLOATS:
         raise ValueError('symmetric_dequantize expects a float32, float16 or bfloat16 scale, got {}'.format(scale.dtype))
+    if wq.is_cuda:
+        out = ffi.front().dequantize(wq, scale, dims)
+        if out is not None:
+            return out
     return SymmetricDeQuantizationOp(wq, scale, dims).outputs[0]

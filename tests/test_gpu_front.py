@@ -6,6 +6,7 @@ import torch
 from hidet_amd import BackendException, ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as F8
+from hidet_amd.graph.ops.quant import group_int4, symmetric
 from hidet_amd.graph.ops.quant.matmul import run_w8a16
 from hidet_amd.graph.ops.quant.group_int4 import _run_w4a16
 from gpu_util import announce
@@ -41,6 +42,34 @@ def test_front_equals_the_python_path(m, k, n):
     assert torch.equal(F8.matmul_f8_per_tensor(a8, b8, sa, sb), F8._run_f8(a8, b8, torch.bfloat16, sa, sb))
     for _ in range(2):
         assert torch.equal(F8.matmul_f8(a8, b8, output_dtype='float32'), F8._run_f8(a8, b8, torch.float32))
+
+
+@pytest.mark.parametrize('shape,dim', [((96, 200), 0), ((33, 260), -1), ((3, 40, 24), [1]), ((3, 40, 24), 0)])
+def test_quantizers_equal_the_python_path(shape, dim):
+    announce('front quantizers', shape, dim)
+    w = torch.randn(shape, device='cuda')
+    for dtype in (torch.float32, torch.bfloat16):
+        for codes in ('int8', 'int16'):
+            q, s = quant.symmetric_quantize(w.to(dtype), codes, dim)
+            op = symmetric.SymmetricQuantizationOp(w.to(dtype), getattr(torch, codes), dims=dim)
+            assert torch.equal(q, op.outputs[0]) and torch.equal(s, op.outputs[1])
+            assert torch.equal(quant.symmetric_dequantize(q, s, dim), symmetric.SymmetricDeQuantizationOp(q, s, dim).outputs[0])
+
+
+def test_int4_and_block_scaled_equal_the_python_path():
+    announce('front int4 and block scaled')
+    w = torch.randn((512, 264), device='cuda')
+    p, s = quant.symmetric_group_quantize_int4(w, 128, 'bfloat16')
+    op = group_int4.SymmetricGroupQuantizationInt4Op(w, 128, torch.bfloat16)
+    assert torch.equal(p, op.outputs[0]) and torch.equal(s, op.outputs[1])
+    x, nk = torch.randn((3, 512), device='cuda').bfloat16(), quant.to_decode_layout_int4(p)
+    out = quant.symmetric_quant_matmul_w4a16_decode(x, nk, s)
+    # the same values through a view that the front leaves to Python (no 16-byte aligned rows)
+    assert torch.equal(out, quant.symmetric_quant_matmul_w4a16_decode(torch.nn.functional.pad(x, (1, 0))[:, 1:], nk, s))
+    a, b = torch.randn((40, 256), device='cuda').to(F8.f8e4m3), torch.randn((384, 256), device='cuda').to(F8.f8e4m3)
+    sa, sb = torch.rand((2, 40), device='cuda'), torch.rand((3, 2), device='cuda')
+    want = F8.MatmulF8ScaledOperator(a, b, sa, sb, torch.float32, torch.bfloat16).outputs[0]
+    assert torch.equal(F8.matmul_f8_scaled(a, b, sa, sb, output_dtype='bfloat16'), want)
 
 
 def test_what_the_front_leaves_to_python():
