@@ -14,6 +14,9 @@ void skinny_w8a16_nk_launch(const void *a, const void *w, const void *scale, con
                             int64_t n, int64_t lda, int64_t ldw, hipStream_t stream);
 bool gemm_w8a16_nk_supported(const void *a, const void *w, const void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                              int64_t ldw);
+bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
+                      int64_t n, int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, double limit_us, const Workspace &ws, hipStream_t stream);
+double gemm_w8a16_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws);
 void gemm_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                           int64_t n, int64_t lda, int64_t ldw, const Workspace &ws, hipStream_t stream);
 }
@@ -22,11 +25,13 @@ using namespace qmm;
 
 namespace {
 
+constexpr int64_t kMidRows = 1024;  // above, the prefill GEMM's tiles fill the chip on every shape
+
 // ---- operands of sizes or alignments the matrix kernels do not take --------------------------------------------------
 //
 // Copies of the operands with rows of whole 16 (weight, factors) and 64 (activations) elements, zero past the originals,
 // in the scratch memory: columns [n0, n0 + cols) of w[k, n] as [kp, np], the float16 activations [m, k] as [m, kp], the
-// column factors as [np]. One thread per 16 bytes written. 203 rows x 4100 x 4098 take 39 us in all (28 us of them the GEMM),
+// column factors as [np]. One thread per 16 bytes written. 203 rows x 4100 x 4098 take 29 us in all (18 us of them the GEMM),
 // where the element-wise kernel that served such sizes before took 1815 us; one row x 4100 x 4098 20 us.
 struct PadArgs {
     const int8_t *w;
@@ -122,6 +127,10 @@ bool w8a16_padded(const void *a, const void *w, const void *scale, const void *b
             const void *ap = copy_a ? static_cast<const void *>(p.ap) : static_cast<const void *>(p.a);
             _Float16 *cp = static_cast<_Float16 *>(c) + m0 * n + n0;
             const void *bp = bias != nullptr ? p.biasp : nullptr;
+            if (gemm && p.m <= kMidRows &&
+                mid_w8a16_launch(ap, p.wp, false, p.scalep, bp, cp, p.m, kp, p.np, copy_a ? kp : lda, p.np, p.cols, n,
+                                 gemm_w8a16_estimate_us(p.m, kp, p.np, left), left, stream))
+                continue;
             if (gemm) gemm_w8a16_launch(ap, p.wp, p.scalep, bp, cp, p.m, kp, p.np, copy_a ? kp : lda, p.cols, n, left, stream);
             else skinny_w8a16_launch(ap, p.wp, p.scalep, bp, cp, p.m, k, p.np, lda, p.cols, 0, left, false, stream);
         }
@@ -143,13 +152,19 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     QMM_CHECK(aligned(a, 2) && aligned(scale, 2) && aligned(c, 2) && aligned(bias, 2), "float16 tensors must be 2-byte aligned");
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     // Up to 16 rows one pass of the bandwidth-bound kernel serves; beyond that every 16 rows would cost another pass
-    // over the weights, and the MFMA GEMM with its K split and its empty row blocks left out takes over (K=4096, N=11008,
-    // weights from HBM: 17 us at M=17..32, 20 us at M=64, 29 us at M=128). For 9 to 16 rows the bandwidth-bound kernel is
+    // over the weights, and the GEMMs take over: narrow tiles (gemm_mid.h) or the prefill tiles, whichever is estimated to be
+    // the faster (K=4096, N=11008, weights from HBM: narrow 14.9 / 18.8 / 24.3 / 36.6 us at M=17 / 64 / 128 / 256, prefill tiles 17.2 /
+    // 20.5 / 30.1 / 39.8; at M=512 64 against 58.5). For 9 to 16 rows the bandwidth-bound kernel is
     // ahead of the GEMM on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
     // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49).
-    if (m > 16 && k > 0 && gemm_w8a16_supported(a, w, c, m, k, n, lda)) {
-        gemm_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, n, ws, stream);
-        return;
+    if (m > 16 && k > 0) {
+        const bool gemm = gemm_w8a16_supported(a, w, c, m, k, n, lda);
+        const double limit = gemm ? gemm_w8a16_estimate_us(m, k, n, ws) : 1e29;
+        if (m <= kMidRows && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, limit, ws, stream)) return;
+        if (gemm) {
+            gemm_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, n, ws, stream);
+            return;
+        }
     }
     // Sizes the GEMM does not take (K no multiple of 64, N of 4): up to 32 rows two passes of the bandwidth-bound kernel,
     // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the
@@ -173,7 +188,9 @@ void w8a16_nk_dispatch(const void *a, const void *w_nk, const void *scale, const
     QMM_CHECK(skinny_w8a16_nk_supported(w_nk, k, ldw),
               "K-contiguous weights need K and the row stride to be multiples of 16 and a 16-byte aligned pointer, got K=" << k
                                                                                                                          << " ldw=" << ldw);
-    // more than one pass of 16 rows: the MFMA GEMM reading the same layout, where its conditions hold
+    // More than one pass of 16 rows: the narrow tiles reading the same layout (4096 x 4096, 49 rows: 12.3 us, the prefill tiles 21.3),
+    // beyond 64 rows the prefill tiles, where their conditions hold.
+    if (m > 16 && m <= 64 && k > 0 && mid_w8a16_launch(a, w_nk, true, scale, bias, c, m, k, n, lda, ldw, n, n, 1e29, split_workspace(workspace, workspace_bytes), stream)) return;
     if (m > 16 && gemm_w8a16_nk_supported(a, w_nk, c, m, k, n, lda, ldw))
         gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, split_workspace(workspace, workspace_bytes), stream);
     else

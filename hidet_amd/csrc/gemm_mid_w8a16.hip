@@ -1,0 +1,210 @@
+// W8A16 on gemm_mid.h: c[m, n] = (sum_k a[m, k] * w[k, n]) * scale[n] (+ bias[n]), int8 weights widened exactly to float16
+// (0x6400 | (q ^ 0x80) is 1152 + q, one packed subtract removes the 1152), float16 MFMA, fp32 sums.
+#include "gemm_mid.h"
+
+namespace qmm {
+namespace {
+
+struct MidW8Args {
+    const _Float16 *scale, *bias;
+    _Float16 *c;
+    int ldc, n_out;
+    int vector_out;    // rows of c start at multiples of 8 bytes and end with a lane's four columns
+};
+
+template <bool NK>
+struct MidW8 {
+    using Args = MidW8Args;
+    // Row-major: a stage is 32 rows of 128 columns, so that memory is read in whole 128-byte lines (64-byte pieces reached
+    // half the rate: 3 TB/s), and goes through LDS to the two waves of a group. K-contiguous: 64 k, 16 bytes of each of a
+    // lane's 4 columns, straight into its registers.
+    static constexpr int kElementBytes = 2;
+    static constexpr int kStageK = NK ? 64 : 32;
+    static constexpr int kGroupWaves = NK ? 1 : 2;
+    static constexpr int kWLdsBytes = NK ? 0 : 32 * 128;
+    static constexpr int kRowBytes = kStageK * 2;
+    static constexpr int kAChunks = NK ? 2 : 1;
+    static constexpr int kWLoads = NK ? 4 : 2;
+    struct Weights {
+        uint32_t u[NK ? 16 : 1];
+        uint64_t pair[4];
+    };
+    struct Fragments {
+        half8_t h[kAChunks][4];
+    };
+    static constexpr int kWidenOps = 48;  // VALU instructions of widen()
+    int side_;
+    __amdgpu_buffer_rsrc_t rsrc;
+    int w_stage;       // bytes from one stage to the next
+    int w_off[NK ? 4 : 2];
+    uint32_t w_read;   // LDS address of this lane's first dword in a slot's weights (row-major)
+    uint32_t sel[4];   // byte gathers of the columns
+    const MidW8Args &args;
+    int k;
+    half4_t scale4, bias4;
+
+    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int n, int n0, int side, int lane) : side_(side), args(x), k(depth) {
+        const int kg = lane >> 4, ns = lane & 15;
+        if constexpr (NK) {
+            const int base = n0 < n - 4 ? n0 : n - 4, col = n0 + ns * 4 < n - 4 ? n0 + ns * 4 : n - 4;
+            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(w) + int64_t(base) * ldw, 0, (n - 1 - base < 63 ? n - 1 - base : 63) * ldw + k, 0x00020000);
+            w_stage = 64;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) w_off[t] = (col + t - base) * ldw + kg * 16;
+        } else {
+            // Instruction b = 2 side + i brings rows 8 b .. 8 b + 7, the rows of the lanes with kg = b: its LDS position p (16
+            // bytes each) holds chunk x % 8 of row x / 8, x = p ^ 4 b. A read of one row per kg, 64 bytes each, then
+            // touches every bank once; kg 2 and 3 find the rows of a pair the other way round, which the gather undoes.
+            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(w), 0, k * n, 0x00020000);  // rows past K read as code 0
+            w_stage = 32 * n;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int blk = 2 * side + i, at = lane ^ (4 * blk);
+                w_off[i] = (8 * blk + (at >> 3)) * n + n0 + (at & 7) * 16;
+            }
+            w_read = uint32_t(kg * 1024 + ((side * 4 + (ns >> 2)) ^ ((kg & 1) * 4)) * 16 + (ns & 3) * 4);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sel[t] = 0x0c000c00u | (kg >= 2 ? (uint32_t(t) << 16) | uint32_t(4 + t) : (uint32_t(4 + t) << 16) | uint32_t(t));
+        }
+    }
+    __device__ __forceinline__ void load(Weights &dst, uint32_t at) const {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const uint4v_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, int(uint32_t(w_off[t]) + at), 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst.u[4 * t + e] = v[e];
+        }
+    }
+    __device__ __forceinline__ void load(uint4 *lds, uint32_t slot, uint32_t at) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) buffer_load_to_lds_b128(rsrc, lds + (slot + (2 * side_ + i) * 1024) / 16, int(uint32_t(w_off[i]) + at), 0);
+    }
+    __device__ __forceinline__ void factors(int col) {
+        bias4 = half4_t{_Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f)};
+        scale4 = bias4;
+        if (col >= args.n_out) return;
+        if (args.vector_out) {
+            __builtin_memcpy(&scale4, args.scale + col, 8);
+            if (args.bias != nullptr) __builtin_memcpy(&bias4, args.bias + col, 8);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (col + t < args.n_out) {
+                    scale4[t] = args.scale[col + t];
+                    if (args.bias != nullptr) bias4[t] = args.bias[col + t];
+                }
+        }
+    }
+    // rows j and j + 1 of the lane's eight, 128 bytes apart
+    __device__ __forceinline__ void read(Weights &dst, uint32_t at) const {
+        uint64_t v[4];
+        asm volatile("ds_read2_b32 %0, %1 offset0:0 offset1:32" : "=v"(v[0]) : "v"(w_read + at));
+        asm volatile("ds_read2_b32 %0, %1 offset0:64 offset1:96" : "=v"(v[1]) : "v"(w_read + at));
+        asm volatile("ds_read2_b32 %0, %1 offset0:128 offset1:160" : "=v"(v[2]) : "v"(w_read + at));
+        asm volatile("ds_read2_b32 %0, %1 offset0:192 offset1:224" : "=v"(v[3]) : "v"(w_read + at));
+#pragma unroll
+        for (int p = 0; p < 4; ++p) dst.pair[p] = v[p];
+    }
+    static __device__ __forceinline__ half8_t minus_1152(const uint32_t (&u)[4]) {
+        half8_t out;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const half2_t v = __builtin_bit_cast(half2_t, u[p] ^ 0x64806480u) - half2_t{_Float16(1152.0f), _Float16(1152.0f)};
+            out[2 * p] = v[0];
+            out[2 * p + 1] = v[1];
+        }
+        return out;
+    }
+    template <int NEWER>
+    static __device__ __forceinline__ void settle(Weights &raw) {
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]) : "n"(NEWER));
+    }
+    __device__ __forceinline__ void widen(const Weights &raw, Fragments &b, int) const {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            uint32_t u[4];
+            if constexpr (NK) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {  // bytes 8 q .. 8 q + 7 of the lane's sixteen
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        const uint32_t src = raw.u[4 * t + 2 * q + p / 2];
+                        u[p] = __builtin_amdgcn_perm(src, src, (p & 1) ? 0x0c030c02u : 0x0c010c00u);
+                    }
+                    b.h[q][t] = minus_1152(u);
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) u[p] = __builtin_amdgcn_perm(uint32_t(raw.pair[p] >> 32), uint32_t(raw.pair[p]), sel[t]);
+                b.h[0][t] = minus_1152(u);
+            }
+        }
+    }
+    // zero what a fragment holds past K (the next row's values, which may be anything)
+    __device__ __forceinline__ void mask(int4v_t (&af)[kAChunks], int st, int kg) const {
+#pragma unroll
+        for (int q = 0; q < kAChunks; ++q) {
+            const int left = k - (st * kStageK + (kg * kAChunks + q) * 8);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t keep = left >= 2 * e + 2 ? 0xFFFFFFFFu : left == 2 * e + 1 ? 0xFFFFu : 0u;
+                af[q][e] = int(uint32_t(af[q][e]) & keep);
+            }
+        }
+    }
+    static __device__ __forceinline__ void multiply(const int4v_t (&af)[kAChunks], const Fragments &b, float4_t (&acc)[4]) {
+#pragma unroll
+        for (int q = 0; q < kAChunks; ++q)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, af[q]), b.h[q][t], acc[t], 0, 0, 0);
+    }
+    __device__ __forceinline__ void store(int row, int col, const float (&v)[4]) const {
+        if (col >= args.n_out) return;
+        half4_t o;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t], float(scale4[t]), float(bias4[t]));
+        _Float16 *dst = args.c + int64_t(row) * args.ldc + col;
+        if (args.vector_out) {
+            *reinterpret_cast<half4_t *>(dst) = o;
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (col + t < args.n_out) dst[t] = o[t];
+        }
+    }
+};
+
+}  // namespace
+
+// Per shape and row count the tile and the K split of the smallest estimated time. `limit_us`: no launch and false where that
+// exceeds it - or where the operands have a form this kernel does not take.
+// `n_out` <= n columns of the result are written, at a row stride of ldc.
+bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
+                      int64_t n, int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, double limit_us, const Workspace &ws, hipStream_t stream) {
+    const MidW8Args args{static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias), static_cast<_Float16 *>(c), int(ldc), int(n_out),
+                         n_out % 4 == 0 && ldc % 4 == 0 && aligned(c, 8)};
+    // four columns of a lane are all inside the matrix; loads start at multiples of four bytes; what a tile reads lies within
+    // 2 GiB (kMidOutside)
+    constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
+    if (n % 4 != 0 || lda % 2 != 0 || !aligned(a, 4) || !aligned(w, 4) || lda * 256 + k * 2 >= kMost || ldc >= kMost) return false;
+    const int64_t las = lda * 2;
+    if (nk) {
+        if (ldw % 4 != 0 || ldw * 64 + k >= kMost) return false;
+        const MidChoice c2 = mid_choose<MidW8<true>, 2, 4>({5.5, 1.4, 1.5, 0.3}, ws, m, n, k), c4 = mid_choose<MidW8<true>, 4, 2>({6.0, 1.6, 1.5, 0.4}, ws, m, n, k);
+        if (std::min(c2.us, c4.us) > limit_us) return false;
+        if (c2.us < c4.us) mid_launch<MidW8<true>, 2, 4>(c2, a, w, las, ldw, args, m, n, k, ws, stream);
+        else mid_launch<MidW8<true>, 4, 2>(c4, a, w, las, ldw, args, m, n, k, ws, stream);
+        return true;
+    }
+    if ((k + 64) * n >= kMost) return false;
+    const MidChoice c2 = mid_choose<MidW8<false>, 2, 6>({5.5, 0.36, 1.4, 0.4}, ws, m, n, k), c4 = mid_choose<MidW8<false>, 4, 4>({6.0, 0.5, 1.5, 0.5}, ws, m, n, k),
+                    c8 = mid_choose<MidW8<false>, 8, 3>({6.5, 0.8, 1.8, 1.0}, ws, m, n, k);
+    const double us = std::min({c2.us, c4.us, c8.us});
+    if (us > limit_us) return false;
+    if (us == c2.us) mid_launch<MidW8<false>, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
+    else if (us == c4.us) mid_launch<MidW8<false>, 4, 4>(c4, a, w, las, n, args, m, n, k, ws, stream);
+    else mid_launch<MidW8<false>, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);
+    return true;
+}
+
+}  // namespace qmm

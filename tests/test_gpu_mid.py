@@ -1,0 +1,48 @@
+"""The narrow-tile GEMMs that serve 17 to about 1000 rows, at the edges of their tiles, K stages and K splits.
+
+Operands are small integers and the column factors powers of two, so that every product and sum is exact in float32 and the
+only rounding is that of the result: the expected values are computed in float64 and rounded the same way."""
+import pytest
+import torch
+
+from hidet_amd.graph.ops import quant
+
+pytestmark = pytest.mark.gpu
+
+
+def _ints(g, shape, lo, hi):
+    return torch.randint(lo, hi + 1, shape, generator=g, device='cuda')
+
+
+# rows around the 32 / 64 / 128 of the tiles; K off the 32 of a stage (and odd multiples of 2), from less than one stage to
+# eight pieces; N off the 128 of a tile, down to one chunk
+@pytest.mark.parametrize('m,k,n', [(17, 256, 4), (31, 4098, 132), (32, 64, 128), (33, 96, 260), (48, 64, 64), (64, 11008, 516), (65, 34, 516),
+                                   (70, 66, 20), (127, 1000, 1028), (129, 4096, 384), (203, 4100, 4098), (512, 4096, 1024),
+                                   (300, 96, 200), (700, 2048, 4096)])
+def test_w8a16_rows_of_a_batch(m, k, n):
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m * 31 + k + n)
+    x, w = _ints(g, (m, k), -3, 3).half(), _ints(g, (k, n), -7, 7).to(torch.int8)
+    scale = (2.0 ** _ints(g, (n,), -4, 0).float()).half()
+    bias = _ints(g, (n,), -4, 4).half()
+    want = ((x.double() @ w.double()) * scale.double()).half()
+    layouts = [w]
+    if m <= 64 and k % 64 == 0 and n % 4 == 0:
+        layouts.append(quant.to_decode_layout(w))
+    for weight in layouts:
+        for _ in range(2):  # the exchange's counters are back at zero for the second call
+            assert torch.equal(quant.symmetric_quant_matmul(x, weight, scale), want)
+        assert torch.equal(quant.symmetric_quant_matmul(x, weight, scale, bias), (want.float() + bias.float()).half())
+
+
+def test_w8a16_values_past_k_do_not_reach_the_result():
+    """A K stage that ends inside the matrix reads the next row's activations too: NaN and infinities there stay out."""
+    g = torch.Generator(device='cuda')
+    g.manual_seed(5)
+    m, k, n = 40, 70, 256
+    wide = torch.full((m, 96), float('nan'), device='cuda', dtype=torch.float16)
+    wide[:, ::2] = float('inf')
+    wide[:, :k] = _ints(g, (m, k), -3, 3).half()
+    x, w = wide[:, :k], _ints(g, (k, n), -7, 7).to(torch.int8)
+    scale = torch.ones(n, device='cuda', dtype=torch.float16)
+    assert torch.equal(quant.symmetric_quant_matmul(x, w, scale), (x.double() @ w.double()).half())
