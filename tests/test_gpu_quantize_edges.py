@@ -65,3 +65,18 @@ def test_fp8_per_tensor_bit_exact(numel):
         codes, scale = F8.fp8_quantize_per_tensor(t)
         c0, s0 = O.fp8_quantize_per_tensor(t.float().cpu().numpy())
         assert np.float32(scale.item()) == s0 and np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
+
+
+# one value, around a workgroup's 4096 elements, the last size of the single launch and the first behind it; the largest value
+# at the end, where only the last workgroup converts it
+@pytest.mark.parametrize('numel', [4, 4092, 4096, 4100, 20000, 65536, 65540])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_fp8_per_tensor_of_a_few_rows(numel, dtype):
+    announce('fp8 few rows', numel, dtype)
+    x = np.random.default_rng(numel).standard_normal(numel).astype(np.float32)
+    x[-1] = 9.0
+    t = dev(x).to(dtype)
+    codes, scale = F8.fp8_quantize_per_tensor(t)
+    c0, s0 = O.fp8_quantize_per_tensor(t.float().cpu().numpy())
+    assert np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
+    assert scale.item() == float(np.asarray(s0).reshape(-1)[0])
