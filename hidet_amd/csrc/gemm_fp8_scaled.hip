@@ -419,6 +419,30 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
 
 }  // namespace
 
+// Tail split (tiles that do not fill a round of one workgroup per CU are computed in K ranges and summed in range
+// order by the last workgroup to arrive): at most 4 ranges of at least 4 k blocks, and only with a workspace that
+// holds the partial tiles (8 XCDs x their tail tiles x parts) in its scratch part.
+static GemmTail tail8_of(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
+    GemmTail tail = make_gemm_tail(tiling, 32, 32, 4);
+    if (ws.scratch == nullptr) tail.parts = 1;
+    while (tail.parts > 1 &&
+           (k / 128 < 4 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * kM8 * kN8 * 4))
+        --tail.parts;
+    return tail;
+}
+
+// Estimated time in microseconds of the tiled kernels, for the choice between them and the narrow tiles of gemm_mid.h: a fixed
+// part, 1.0 us per k block and round of 256 x 128 tiles and what an exchange of K ranges costs; where K is no multiple of 128
+// (the register-staged 256 x 256 kernel) 3.5 us per k block and round.
+double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, void *workspace, int64_t workspace_bytes) {
+    if (k % 128 != 0) return 8.0 + double(cdiv(cdiv(m, 256) * cdiv(n, 256), 256)) * 3.5 * double(cdiv(k, 128));
+    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, kM8)), int(cdiv(n, kN8)), 32);
+    const GemmTail tail = tail8_of(tiling, k, split_workspace(workspace, workspace_bytes));
+    const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
+    const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);
+    return 7.0 + rounds * double(k) / 128.0 + (tail.parts > 1 ? 5.0 + 0.4 * tail.parts : 0.0);
+}
+
 // Launch of the 8-wave kernel; SCALED selects block scales (scale_a [K/128, M], scale_b [N/128, K/128]) or optional
 // per-tensor scales.
 template <bool SCALED, int FMT = 0>
@@ -427,15 +451,8 @@ static void launch_kernel8(const void *a, int64_t lda, const void *b, int64_t ld
                            hipStream_t stream) {
     const int tiles_m = int(cdiv(m, kM8)), tiles_n = int(cdiv(n, kN8));
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, 32);
-    // Tail split (tiles that do not fill a round of one workgroup per CU are computed in K ranges and summed in range
-    // order by the last workgroup to arrive): at most 4 ranges of at least 4 k blocks, and only with a workspace that
-    // holds the partial tiles (8 XCDs x their tail tiles x parts) in its scratch part.
-    GemmTail tail = make_gemm_tail(tiling, 32, 32, 4);
     const Workspace ws = split_workspace(workspace, workspace_bytes);
-    if (ws.scratch == nullptr) tail.parts = 1;
-    while (tail.parts > 1 &&
-           (k / 128 < 4 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * kM8 * kN8 * 4))
-        --tail.parts;
+    const GemmTail tail = tail8_of(tiling, k, ws);
     const int64_t grid = gemm_grid_with_tail(tiling, 32, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
     auto go = [&](auto kern) {

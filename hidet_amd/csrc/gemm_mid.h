@@ -87,9 +87,11 @@ __device__ __forceinline__ int mid_key(int row) {
 
 template <class Op, int RB, int DEPTH>
 struct MidCfg {
-    static constexpr int kGroupWaves = Op::kGroupWaves;        // waves side by side (64 columns each) on one K stage
+    static constexpr int kGroupWaves = Op::kGroupWaves;        // waves side by side on one K stage,
+    static constexpr int kFrags = Op::kFrags;                  // each with so many 16-column blocks, kFrags columns to a lane
     static constexpr int kGroups = kMidWaves / kGroupWaves;
-    static constexpr int kCols = kGroupWaves * 64;
+    static constexpr int kWaveCols = kFrags * 16;
+    static constexpr int kCols = kGroupWaves * kWaveCols;
     static constexpr int kRowBytes = Op::kRowBytes;            // bytes of an activation row per stage
     static constexpr int kChunks = kRowBytes / 16;
     static constexpr int kABytes = RB * 16 * kRowBytes;
@@ -101,11 +103,13 @@ struct MidCfg {
     static constexpr int kHalves = RB / kHalfRows;
     static constexpr int kPlanes = kMidWaves / (kHalfRows * kGroupWaves);
     static constexpr int kWidth = 4 / kPlanes;                 // accumulator rows a thread sums
-    static constexpr int kMeetBytes = kGroups * kHalfRows * kGroupWaves * 4096;
+    static constexpr int kMeetBytes = kGroups * kHalfRows * kGroupWaves * kFrags * 1024;
+    static constexpr int kVecs = kFrags * kWidth / 4;          // float4 sums of a thread and half
     static constexpr int kLdsMain = kRingBytes > kMeetBytes ? kRingBytes : kMeetBytes;
     static constexpr int kLdsBytes = kLdsMain + 16;            // + the exchange's flag
     static constexpr int kTileFloats = RB * 16 * kCols;
     static_assert(kALoads * 1024 * kGroupWaves == kABytes, "whole load instructions");
+    static_assert(kVecs * 4 == kFrags * kWidth, "whole float4 sums");
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
     static_assert(kLoads * (DEPTH - 1) <= 63, "vmcnt range");
 };
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
     const int rows = plan.m - m0 < RB * 16 ? plan.m - m0 : RB * 16;
 
     // ---- main loop ----------------------------------------------------------------------------------------------
-    Op op(args, w, w_stride, k, n, n0, side, lane);
+    Op op(args, w, w_stride, k, m, n, m0, n0, side, lane);
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char *>(a) + int64_t(m0) * a_stride, 0, (rows - 1) * a_stride + k * Op::kElementBytes, 0x00020000);
     int a_off[Cfg::kALoads];
@@ -145,11 +149,11 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
     for (int q = 0; q < Op::kAChunks; ++q)
         af_addr[q] = ring + uint32_t(ns * Cfg::kRowBytes + (((kg * Op::kAChunks + q) ^ mid_key<Cfg::kRowBytes>(ns)) * 16));
 
-    float4_t acc[RB][4];
+    float4_t acc[RB][Cfg::kFrags];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[rb][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < Cfg::kFrags; ++t) acc[rb][t] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     // Every load of a stage past the end of the piece goes past the end of its buffer: it returns zeros without touching
     // memory, so the number of loads in flight is always the same. Activation rows past the matrix read as zeros. (All
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
             if constexpr (Op::kAChunks == 1) lds_wait_keep_newer<NEWER>(af[R][0]);
             else lds_wait_keep_newer<NEWER>(af[R][0], af[R][1]);
             if (st * Op::kStageK + Op::kStageK > k) op.mask(af[R], st, kg);  // the stage that K ends in
-            op.multiply(af[R], bf, acc[R]);
+            op.multiply(af[R], bf, acc[R], r);
         });
     };
     if constexpr (Cfg::kGroupWaves == 1) {
@@ -256,12 +260,12 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
             read_a(af[B ^ 1], slot);
             __builtin_amdgcn_sched_barrier(0);
             constexpr int kAhead = RB / 4 > 0 ? RB / 4 : 1;  // row blocks whose MFMAs cover the reads' latency
-            mid_for<0, kAhead>([&](auto r) { op.multiply(af[B][decltype(r)::value], bf[B], acc[decltype(r)::value]); });
+            mid_for<0, kAhead>([&](auto r) { op.multiply(af[B][decltype(r)::value], bf[B], acc[decltype(r)::value], r); });
             __builtin_amdgcn_sched_barrier(0);
             op.template settle<RB * Op::kAChunks>(raw);
             op.widen(raw, bf[B ^ 1], st);
-            mid_for<kAhead, RB>([&](auto r) { op.multiply(af[B][decltype(r)::value], bf[B], acc[decltype(r)::value]); });
-            constexpr int kLeft = (RB - kAhead) * 4 * Op::kAChunks;
+            mid_for<kAhead, RB>([&](auto r) { op.multiply(af[B][decltype(r)::value], bf[B], acc[decltype(r)::value], r); });
+            constexpr int kLeft = (RB - kAhead) * Op::kMfmas;
             mid_for<0, kLeft>([&](auto) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, (Op::kWidenOps + kLeft - 1) / kLeft, 0);
@@ -277,24 +281,24 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // nothing may land in LDS past this point
     asm volatile("" ::: "memory");
 
-    op.factors(n0 + (wave / Cfg::kPlanes % Cfg::kGroupWaves) * 64 + ns * 4);  // on their way while the sums come together
+    op.factors(n0 + (wave / Cfg::kPlanes % Cfg::kGroupWaves) * Cfg::kWaveCols + ns * Cfg::kFrags);  // on their way while the sums come together
 
-    // ---- the groups meet: thread (unit, lane) sums four columns x kWidth rows of a row block ------------------------
-    float4_t sum[Cfg::kHalves][Cfg::kWidth];  // [half][.]: flat index t * kWidth + row
+    // ---- the groups meet: thread (unit, lane) sums kFrags columns x kWidth rows of a row block ------------------------
+    float4_t sum[Cfg::kHalves][Cfg::kVecs];  // [half][.]: flat index t * kWidth + row
     float *meet = reinterpret_cast<float *>(lds);
     const int plane = wave % Cfg::kPlanes, side_u = wave / Cfg::kPlanes % Cfg::kGroupWaves, rbu = wave / (Cfg::kPlanes * Cfg::kGroupWaves);
     typedef float width_t __attribute__((ext_vector_type(Cfg::kWidth)));
     static_assert(Cfg::kHalfRows * Cfg::kGroupWaves * Cfg::kPlanes == kMidWaves, "one unit per wave");
     // [group][side][plane][row block][t][lane]
     auto meet_at = [&](int g, int sd, int p, int f) {
-        return reinterpret_cast<width_t *>(meet + ((((g * Cfg::kGroupWaves + sd) * Cfg::kPlanes + p) * (Cfg::kHalfRows * 4) + f) * 64 + lane) * Cfg::kWidth);
+        return reinterpret_cast<width_t *>(meet + ((((g * Cfg::kGroupWaves + sd) * Cfg::kPlanes + p) * (Cfg::kHalfRows * Cfg::kFrags) + f) * 64 + lane) * Cfg::kWidth);
     };
     mid_for<0, Cfg::kHalves>([&](auto h_tag) {
         constexpr int H = decltype(h_tag)::value;
         __syncthreads();
-        mid_for<0, Cfg::kHalfRows * 4>([&](auto f_tag) {
+        mid_for<0, Cfg::kHalfRows * Cfg::kFrags>([&](auto f_tag) {
             constexpr int F = decltype(f_tag)::value;
-            const float4_t v = acc[H * Cfg::kHalfRows + F / 4][F % 4];
+            const float4_t v = acc[H * Cfg::kHalfRows + F / Cfg::kFrags][F % Cfg::kFrags];
 #pragma unroll
             for (int p = 0; p < Cfg::kPlanes; ++p) {
                 width_t part;
@@ -304,26 +308,26 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
             }
         });
         __syncthreads();
-        float total[4 * Cfg::kWidth];
+        float total[Cfg::kFrags * Cfg::kWidth];
 #pragma unroll
-        for (int e = 0; e < 4 * Cfg::kWidth; ++e) total[e] = 0.f;
+        for (int e = 0; e < Cfg::kFrags * Cfg::kWidth; ++e) total[e] = 0.f;
 #pragma unroll
         for (int g = 0; g < Cfg::kGroups; ++g)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const width_t part = *meet_at(g, side_u, plane, rbu * 4 + t);
+            for (int t = 0; t < Cfg::kFrags; ++t) {
+                const width_t part = *meet_at(g, side_u, plane, rbu * Cfg::kFrags + t);
 #pragma unroll
                 for (int e = 0; e < Cfg::kWidth; ++e) total[t * Cfg::kWidth + e] += part[e];
             }
 #pragma unroll
-        for (int e = 0; e < 4 * Cfg::kWidth; ++e) sum[H][e / 4][e % 4] = total[e];
+        for (int e = 0; e < Cfg::kFrags * Cfg::kWidth; ++e) sum[H][e / 4][e % 4] = total[e];
     });
 
     // ---- the pieces of a tile meet: the last to arrive adds them in the order of K --------------------------------
     bool finish = true;
     if (parts > 1) {
         constexpr int kAgentScope = 1 << 4;  // sc1
-        constexpr int kVec = Cfg::kHalves * Cfg::kWidth;
+        constexpr int kVec = Cfg::kHalves * Cfg::kVecs;
         constexpr int kOutside = 0x7FFFFFF0;
         auto store_of = [&](int p) {
             return partials + int64_t(item.tile * parts + p) * Cfg::kTileFloats;
@@ -333,8 +337,8 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
         for (int h = 0; h < Cfg::kHalves; ++h) {
             const int off = (h * Cfg::kHalfRows + rbu) * 16 < rows ? tid * 16 : kOutside;
 #pragma unroll
-            for (int e = 0; e < Cfg::kWidth; ++e)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v_t, sum[h][e]), own, off, (h * Cfg::kWidth + e) * (kMidThreads * 16), kAgentScope);
+            for (int e = 0; e < Cfg::kVecs; ++e)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v_t, sum[h][e]), own, off, (h * Cfg::kVecs + e) * (kMidThreads * 16), kAgentScope);
         }
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // every store of this lane has been acknowledged (they write through)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -354,7 +358,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 #pragma unroll
             for (int h = 0; h < Cfg::kHalves; ++h)
 #pragma unroll
-                for (int e = 0; e < Cfg::kWidth; ++e) sum[h][e] = float4_t{0.f, 0.f, 0.f, 0.f};
+                for (int e = 0; e < Cfg::kVecs; ++e) sum[h][e] = float4_t{0.f, 0.f, 0.f, 0.f};
             for (int p0 = 0; p0 < parts; p0 += kBatch) {
                 uint4v_t v[kBatch][kVec];
 #pragma unroll
@@ -365,8 +369,8 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
                     for (int h = 0; h < Cfg::kHalves; ++h) {
                         const int off = in && (h * Cfg::kHalfRows + rbu) * 16 < rows ? tid * 16 : kOutside;
 #pragma unroll
-                        for (int e = 0; e < Cfg::kWidth; ++e)
-                            v[b][h * Cfg::kWidth + e] = __builtin_amdgcn_raw_buffer_load_b128(from, off, (h * Cfg::kWidth + e) * (kMidThreads * 16), kAgentScope);
+                        for (int e = 0; e < Cfg::kVecs; ++e)
+                            v[b][h * Cfg::kVecs + e] = __builtin_amdgcn_raw_buffer_load_b128(from, off, (h * Cfg::kVecs + e) * (kMidThreads * 16), kAgentScope);
                     }
                 }
 #pragma unroll
@@ -374,7 +378,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 #pragma unroll
                     for (int h = 0; h < Cfg::kHalves; ++h)
 #pragma unroll
-                        for (int e = 0; e < Cfg::kWidth; ++e) sum[h][e] += __builtin_bit_cast(float4_t, v[b][h * Cfg::kWidth + e]);
+                        for (int e = 0; e < Cfg::kVecs; ++e) sum[h][e] += __builtin_bit_cast(float4_t, v[b][h * Cfg::kVecs + e]);
             }
         }
     }
@@ -384,10 +388,10 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 #pragma unroll
             for (int r = 0; r < Cfg::kWidth; ++r) {
                 const int row = (h * Cfg::kHalfRows + rbu) * 16 + 4 * kg + plane * Cfg::kWidth + r;
-                float four[4];
+                float out[Cfg::kFrags];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) four[t] = sum[h][(t * Cfg::kWidth + r) / 4][(t * Cfg::kWidth + r) % 4];
-                if (row < rows) op.store(m0 + row, n0 + side_u * 64 + ns * 4, four);
+                for (int t = 0; t < Cfg::kFrags; ++t) out[t] = sum[h][(t * Cfg::kWidth + r) / 4][(t * Cfg::kWidth + r) % 4];
+                if (row < rows) op.store(m0 + row, n0 + side_u * Cfg::kWaveCols + ns * Cfg::kFrags, out);
             }
     }
 }

@@ -21,6 +21,7 @@ struct MidW8 {
     static constexpr int kElementBytes = 2;
     static constexpr int kStageK = NK ? 64 : 32;
     static constexpr int kGroupWaves = NK ? 1 : 2;
+    static constexpr int kFrags = 4;
     static constexpr int kWLdsBytes = NK ? 0 : 32 * 128;
     static constexpr int kRowBytes = kStageK * 2;
     static constexpr int kAChunks = NK ? 2 : 1;
@@ -32,6 +33,7 @@ struct MidW8 {
     struct Fragments {
         half8_t h[kAChunks][4];
     };
+    static constexpr int kMfmas = 4;      // per row block
     static constexpr int kWidenOps = 48;  // VALU instructions of widen()
     int side_;
     __amdgpu_buffer_rsrc_t rsrc;
@@ -43,7 +45,7 @@ struct MidW8 {
     int k;
     half4_t scale4, bias4;
 
-    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int n, int n0, int side, int lane) : side_(side), args(x), k(depth) {
+    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int, int n, int, int n0, int side, int lane) : side_(side), args(x), k(depth) {
         const int kg = lane >> 4, ns = lane & 15;
         if constexpr (NK) {
             const int base = n0 < n - 4 ? n0 : n - 4, col = n0 + ns * 4 < n - 4 ? n0 + ns * 4 : n - 4;
@@ -152,7 +154,8 @@ struct MidW8 {
             }
         }
     }
-    static __device__ __forceinline__ void multiply(const int4v_t (&af)[kAChunks], const Fragments &b, float4_t (&acc)[4]) {
+    template <typename R>
+    static __device__ __forceinline__ void multiply(const int4v_t (&af)[kAChunks], const Fragments &b, float4_t (&acc)[4], R) {
 #pragma unroll
         for (int q = 0; q < kAChunks; ++q)
 #pragma unroll

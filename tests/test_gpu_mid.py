@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from hidet_amd.graph.ops import quant
+from hidet_amd.graph.ops.matmul import matmul_f8 as f8
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +47,30 @@ def test_w8a16_values_past_k_do_not_reach_the_result():
     x, w = wide[:, :k], _ints(g, (k, n), -7, 7).to(torch.int8)
     scale = torch.ones(n, device='cuda', dtype=torch.float16)
     assert torch.equal(quant.symmetric_quant_matmul(x, w, scale), (x.double() @ w.double()).half())
+
+
+# rows around the 32 / 64 of the tiles; K of less than one 128-deep stage, off the stages (multiples of 16), of many pieces; N
+# off the 128 of a tile
+@pytest.mark.parametrize('m,k,n', [(17, 128, 4), (31, 144, 60), (33, 272, 132), (64, 4096, 4096), (65, 1040, 516), (100, 16, 4), (200, 2048, 68),
+                                   (256, 7168, 640), (1000, 512, 256)])
+def test_fp8_rows_of_a_batch(m, k, n):
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m + k + n)
+    a, b = _ints(g, (m, k), -3, 3).float().to(torch.float8_e4m3fn), _ints(g, (n, k), -3, 3).float().to(torch.float8_e4m3fn)
+    half, quarter = torch.tensor(0.5, device='cuda'), torch.tensor(0.25, device='cuda')
+    exact = (a.double() @ b.double().t()) * 0.125
+    for dtype in (torch.float32, torch.float16, torch.bfloat16, torch.float32):
+        assert torch.equal(f8.matmul_f8_per_tensor(a, b, half, quarter, output_dtype=dtype), exact.to(dtype))
+
+
+@pytest.mark.parametrize('m,k,n', [(17, 128, 128), (64, 7168, 512), (65, 1024, 256), (130, 2048, 1536), (513, 512, 384)])
+def test_fp8_block_scaled_rows_of_a_batch(m, k, n):
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m + k + n)
+    a, b = _ints(g, (m, k), -3, 3).float().to(torch.float8_e4m3fn), _ints(g, (n, k), -3, 3).float().to(torch.float8_e4m3fn)
+    scale_a, scale_b = 2.0 ** _ints(g, (k // 128, m), -3, 0).float(), 2.0 ** _ints(g, (n // 128, k // 128), -3, 0).float()
+    af = (a.double().view(m, k // 128, 128) * scale_a.t().double()[:, :, None]).view(m, k)
+    bf = (b.double().view(n // 128, 128, k // 128, 128) * scale_b.double()[:, None, :, None]).view(n, k)
+    want = (af @ bf.t()).float()
+    for _ in range(2):
+        assert torch.equal(f8.matmul_f8_scaled(a, b, scale_a, scale_b, output_dtype='float32'), want)
