@@ -12,6 +12,9 @@ void gemm_w4a16_launch(const void *a, const void *w, const void *scales, void *c
 bool skinny_w4a16_nk_supported(const void *a, const void *w, int64_t k, int64_t lda, int64_t ldw, int group);
 void skinny_w4a16_nk_launch(const void *a, const void *w, const void *scales, void *c, int64_t m, int64_t k, int64_t n,
                             int64_t lda, int64_t ldw, int group, int dtype, hipStream_t stream);
+bool mid_w4a16_launch(const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
+                      int group, int dtype, double limit_us, void *workspace, int64_t workspace_bytes, hipStream_t stream);
+double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n);
 }  // namespace qmm
 
 using namespace qmm;
@@ -71,9 +74,14 @@ void w4a16_dispatch(const void *a, const void *w, const void *scales, const void
     if (m == 0 || n == 0) return;
     QMM_CHECK(a && c && (k == 0 || (w && scales)), "null tensor pointer");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    // one or two 16-row passes of the bandwidth-bound kernel (19 us each at K=4096, N=11008) beat the MFMA GEMM
-    // (46 us up to M=128); beyond 32 rows the GEMM wins
-    if (m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size)) {
+    // Beyond one 16-row pass of the bandwidth-bound kernel the narrow tiles (gemm_mid.h) or, where those are estimated to take
+    // longer, the MFMA GEMM on tall ones (K = 4096, N = 11008: 128 / 256 / 512 rows narrow 34.7 / 67 / 101 us, tall 36.9 / 48.5 / 76). What
+    // neither takes is done in passes of 16 rows.
+    const bool gemm = m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size);
+    if (m > 16 && m <= 1024 &&
+        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype, gemm ? gemm_w4a16_estimate_us(m, k, n) : 1e29, workspace, workspace_bytes, stream))
+        return;
+    if (gemm) {
         gemm_w4a16_launch(a, w, scales, c, m, k, n, lda, group_size, dtype, workspace, workspace_bytes, stream);
         if (bias != nullptr) {
             // a few microseconds next to a GEMM of 35 and more; the decode-sized calls below add the bias in their epilogue

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 #pragma unroll
         for (int i = 0; i < Cfg::kALoads; ++i)
             buffer_load_to_lds_b128(rsrc_a, lds + (ring + slot_bytes + (side * Cfg::kALoads + i) * 1024) / 16, int(uint32_t(a_off[i]) + at), 0);
-        load_w(on ? uint32_t(st) * uint32_t(op.w_stage) : kMidOutside);
+        load_w(on ? uint32_t(st) * uint32_t(op.w_stage) : kMidOutside, st);
     };
     auto multiply_all = [&](auto &af, auto &bf, int st) {
         mid_for<0, RB>([&](auto r) {
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
         int s = item.s_begin + group;
         mid_for<0, DEPTH>([&](auto d) {
             constexpr int D = decltype(d)::value;
-            issue(D * Cfg::kSlotBytes, s + D * Cfg::kGroups, [&](uint32_t at) { op.load(wr[D], at); });
+            issue(D * Cfg::kSlotBytes, s + D * Cfg::kGroups, [&](uint32_t at, int) { op.load(wr[D], at); });
         });
         for (; s < item.s_end; s += DEPTH * Cfg::kGroups) {
             mid_for<0, DEPTH>([&](auto d_tag) {
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
                     multiply_all(af, bf, st);
                     asm volatile("" ::: "memory");
                     __builtin_amdgcn_sched_barrier(0);
-                    issue(D * Cfg::kSlotBytes, st + DEPTH * Cfg::kGroups, [&](uint32_t at) { op.load(wr[D], at); });
+                    issue(D * Cfg::kSlotBytes, st + DEPTH * Cfg::kGroups, [&](uint32_t at, int) { op.load(wr[D], at); });
                 }
             });
         }
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
         int st = item.s_begin + group;
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d)
-            issue(d * Cfg::kSlotBytes, st + d * Cfg::kGroups, [&](uint32_t at) { op.load(lds, ring + d * Cfg::kSlotBytes + Cfg::kABytes, at); });
+            issue(d * Cfg::kSlotBytes, st + d * Cfg::kGroups, [&](uint32_t at, int nst) { op.load(lds, ring + d * Cfg::kSlotBytes + Cfg::kABytes, at, nst); });
         typename Op::Fragments bf[2];
         int4v_t af[2][RB][Op::kAChunks];
         typename Op::Weights raw;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
         auto round = [&](auto b_tag) {
             constexpr int B = decltype(b_tag)::value;
             arrive(MidStatic<DEPTH - 2>());
-            issue(slot, st + DEPTH * Cfg::kGroups, [&](uint32_t at) { op.load(lds, ring + slot + Cfg::kABytes, at); });
+            issue(slot, st + DEPTH * Cfg::kGroups, [&](uint32_t at, int nst) { op.load(lds, ring + slot + Cfg::kABytes, at, nst); });
             slot = slot + Cfg::kSlotBytes == DEPTH * Cfg::kSlotBytes ? 0 : slot + Cfg::kSlotBytes;
             st += Cfg::kGroups;
             op.read(raw, ring + slot + Cfg::kABytes);

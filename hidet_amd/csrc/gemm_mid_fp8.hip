@@ -72,7 +72,7 @@ struct MidF8 {
             sa_read = uint32_t(128 * 128 + side * kFactorBytes + kg * 16);
         }
     }
-    __device__ __forceinline__ void load(uint4 *lds, uint32_t slot, uint32_t at) const {
+    __device__ __forceinline__ void load(uint4 *lds, uint32_t slot, uint32_t at, int) const {
 #pragma unroll
         for (int j = 0; j < 4; ++j) buffer_load_to_lds_b128(rsrc, lds + (slot + (side * 4 + j) * 1024) / 16, int(uint32_t(w_off[j]) + at), 0);
         if constexpr (SCALED) {

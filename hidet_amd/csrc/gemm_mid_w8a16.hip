@@ -77,7 +77,7 @@ struct MidW8 {
             for (int e = 0; e < 4; ++e) dst.u[4 * t + e] = v[e];
         }
     }
-    __device__ __forceinline__ void load(uint4 *lds, uint32_t slot, uint32_t at) const {
+    __device__ __forceinline__ void load(uint4 *lds, uint32_t slot, uint32_t at, int) const {
 #pragma unroll
         for (int i = 0; i < 2; ++i) buffer_load_to_lds_b128(rsrc, lds + (slot + (2 * side_ + i) * 1024) / 16, int(uint32_t(w_off[i]) + at), 0);
     }

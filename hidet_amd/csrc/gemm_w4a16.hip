@@ -909,6 +909,14 @@ bool gemm_w4a16_supported(const void *a, const void *w, const void *scales, cons
            aligned(scales, 16) && aligned(c, 16);
 }
 
+// Estimated time in microseconds, for the choice between these kernels and the narrow tiles of gemm_mid.h: a fixed part, 1.06 us
+// per 64-deep stage of a 256 x 256 tile, cut into K ranges while that leaves at most half the CUs busy, and the exchange of
+// those. On the low side where the tiles of 128 rows or a general kernel run instead.
+double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n) {
+    const int64_t tiles = cdiv(m, 256) * cdiv(n, 256), parts = std::max<int64_t>(1, std::min<int64_t>(4, 128 / tiles));
+    return 8.0 + double(cdiv(tiles, 256)) * 1.06 * double(k) / 64.0 / double(parts) + (parts > 1 ? 3.0 * double(parts) : 0.0);
+}
+
 void gemm_w4a16_launch(const void *a, const void *w, const void *scales, void *c, int64_t m, int64_t k, int64_t n,
                        int64_t lda, int group, int dtype, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
     const bool fast = (k % kBK == 0) && (group % kBK == 0) && k * (n / 2) < (int64_t(1) << 31) - (1 << 20) &&

@@ -74,3 +74,38 @@ def test_fp8_block_scaled_rows_of_a_batch(m, k, n):
     want = (af @ bf.t()).float()
     for _ in range(2):
         assert torch.equal(f8.matmul_f8_scaled(a, b, scale_a, scale_b, output_dtype='float32'), want)
+
+
+def _int4(g, k, n, group, dtype):
+    """Packed codes of small integers with scales that are powers of two, and the weights they stand for."""
+    q = _ints(g, (k, n), -8, 7)
+    packed = ((q[:, 0::2] & 0xF) | ((q[:, 1::2] & 0xF) << 4)).to(torch.uint8)
+    scales = 2.0 ** _ints(g, (k // group, n), -3, 0).double()
+    return packed, scales.to(dtype), q.double() * scales.repeat_interleave(group, 0)
+
+
+# rows around the 32 / 64 of the tiles, K of one 32-deep stage and of many pieces, N off the 128 of a tile, every kind of group
+@pytest.mark.parametrize('m,k,n,group', [(17, 32, 8, 32), (31, 128, 136, 128), (33, 192, 1032, 64), (64, 11008, 264, 128), (65, 96, 72, 96), (70, 4096, 4096, 128),
+                                         (200, 2048, 520, 64), (300, 512, 128, 256)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_w4a16_rows_of_a_batch(m, k, n, group, dtype):
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m + k + n)
+    x = _ints(g, (m, k), -2, 2).to(dtype)
+    packed, scales, w = _int4(g, k, n, group, dtype)
+    want = (x.double() @ w).to(dtype)
+    for _ in range(2):
+        assert torch.equal(quant.symmetric_quant_matmul_w4a16(x, packed, scales, group), want)
+
+
+def test_w4a16_infinite_and_large_activations():
+    g = torch.Generator(device='cuda')
+    g.manual_seed(8)
+    m, k, n = 40, 256, 128
+    x = _ints(g, (m, k), -2, 2).to(torch.bfloat16)
+    x[3, 17] = float('inf')
+    x[4] = 0
+    x[4, 0] = 2.0 ** 124
+    packed, scales, w = _int4(g, k, n, 128, torch.bfloat16)
+    want = (x.double() @ w).to(torch.bfloat16)  # row 3: infinities, NaN where the code is zero
+    assert torch.equal(quant.symmetric_quant_matmul_w4a16(x, packed, scales, 128).nan_to_num(nan=-1.0), want.nan_to_num(nan=-1.0))
