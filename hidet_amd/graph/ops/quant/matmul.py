@@ -40,7 +40,7 @@ class SymmetricQuantizedMatmulTask(Task):
                          outputs=[TensorSpec('c', 'float16', c_shape)], attrs={})
 
 
-_NK_MAX_ROWS = 16  # one pass of the bandwidth-bound kernels for K-contiguous weights; more rows go to the MFMA GEMM
+_NK_MAX_ROWS = 16  # one pass of the bandwidth-bound kernels for K-contiguous weights; more rows go to the narrow-tile GEMM
 # The GEMM that reads K-contiguous weights gathers 8 bytes per lane from 16 rows of the stored matrix per load and runs
 # about a third slower than the row-major one at prefill sizes (2048 x 4096 x 11008: 214 against 157 us; 64 rows: 25 against
 # 20 us).  Batched decode (17 to 64 rows) uses it, so a model that only decodes never makes a second copy of its weights;
