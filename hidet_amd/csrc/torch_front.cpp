@@ -272,11 +272,12 @@ bool view_of(const at::Tensor &t, PyObject *dims, View *v) {
     if (PyList_CheckExact(dims) && PyList_GET_SIZE(dims) == 1) dims = PyList_GET_ITEM(dims, 0);
     if (!PyLong_CheckExact(dims)) return false;
     v->axis = PyLong_AsLong(dims);
-    if (v->axis < 0) v->axis += t.dim();
-    if (v->axis < 0 || v->axis >= t.dim()) {
+    if (v->axis == -1 && PyErr_Occurred()) {  // no long holds it
         PyErr_Clear();
         return false;
     }
+    if (v->axis < 0) v->axis += t.dim();
+    if (v->axis < 0 || v->axis >= t.dim()) return false;
     v->outer = v->inner = 1;
     for (int64_t d = 0; d < v->axis; ++d) v->outer *= t.size(d);
     for (int64_t d = v->axis + 1; d < t.dim(); ++d) v->inner *= t.size(d);

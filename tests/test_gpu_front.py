@@ -86,6 +86,10 @@ def test_what_the_front_leaves_to_python():
         quant.symmetric_quant_matmul(x.float(), wq, s)
     with pytest.raises(BackendException):
         quant.symmetric_quant_matmul(x, wq, s.cpu())
+    for axis in (2, -3, 2 ** 70):
+        assert front.quantize(x, torch.int8, axis) is None
+        with pytest.raises((ValueError, IndexError)):
+            quant.symmetric_quantize(x, 'int8', axis)
     ffi.load_library().hidet_set_last_error(b'planted')  # an error the library reports surfaces as the exception
     with pytest.raises(BackendException, match='planted'):
         quant.symmetric_quant_matmul(x, wq, s)
