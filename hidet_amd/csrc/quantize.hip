@@ -1,8 +1,8 @@
 // Quantization kernels: symmetric int8/int16 quantize + dequantize over a [outer, reduce, inner]
 // view, group-wise signed int4 with nibble packing, and per-tensor float8 e4m3.
 //
-// Every division and rounding here is IEEE (no fast-math, no reciprocal approximation): the codes
-// and scales must match the CPU definition bit for bit.
+// Codes and scales match the CPU definition (IEEE division, then rounding) bit for bit. A product with the reciprocal stands in
+// for a division only where it provably rounds alike (round_quotients_f32, round_quotients_16, e4m3_codes4).
 #include "common.h"
 #include "numeric.h"
 
@@ -220,6 +220,38 @@ __global__ __launch_bounds__(64 * kAmaxLanes) void amax_strided_kernel(const voi
     }
 }
 
+// The same for a short innermost axis (narrow_inner, at most 256): the threads of a workgroup take consecutive elements of
+// whole rows, eight loads in flight each, so that a thread stays on one column and no lane is idle for want of columns.
+template <int DT>
+__global__ __launch_bounds__(256) void amax_narrow_kernel(const void *__restrict__ w, float *__restrict__ amax, int64_t R, int64_t inner_,
+                                                          int64_t rows_per_range, int64_t nscale) {
+    __shared__ float red[256];
+    const int t = threadIdx.x, inner = int(inner_), lanes = 256 / inner, span = lanes * inner;
+    const int64_t o = blockIdx.z, r0 = int64_t(blockIdx.y) * rows_per_range;
+    const int64_t base = (o * R + r0) * inner, count = (min(R, r0 + rows_per_range) - r0) * inner;
+    float m = 0.0f;
+    if (t < span) {
+        int64_t i = t;
+        for (; i + 7 * span < count; i += 8 * span) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = load_as_f32<DT>(w, base + i + j * span);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[j]));
+        }
+        for (; i < count; i += span) m = fmaxf(m, fabsf(load_as_f32<DT>(w, base + i)));
+    }
+    red[t] = m;
+    __syncthreads();
+    int step = 1;
+    while (2 * step < lanes) step *= 2;
+    for (; step > 0; step >>= 1) {
+        if (t < step * inner && t + step * inner < span) red[t] = fmaxf(red[t], red[t + step * inner]);
+        __syncthreads();
+    }
+    if (t < inner) amax[int64_t(blockIdx.y) * nscale + o * inner + t] = red[t];
+}
+
 // amax over the last axis of [outer, R] (inner == 1): one wave per row, 4 rows per block.
 template <int DT>
 __global__ __launch_bounds__(256) void amax_contig_kernel(const void *__restrict__ w, float *__restrict__ amax,
@@ -394,6 +426,71 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const void *__rest
         for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * s[e]);
         store_upto4<ST>(w, i, count, out);
     }
+}
+
+// [outer, R, inner] with a short innermost axis (narrow_inner), or more slices than a grid has layers: four consecutive elements
+// per thread, each with the scale of its own column. The kernels above give a column quad to a lane, so of a row of 9
+// elements (a 3 x 3 filter) they use 3 lanes in 64. Bound by memory and, where rows are no multiple of four, by the gathers of
+// the scales. float32, quad kernels -> these, us: quantize 4096 x 256 x 9 193 -> 30, 4096 x 256 x 32 155 -> 71, 2048 x 128 x 64
+// 46.4 -> 36.3; dequantize 68 -> 12, 65 -> 27, 20.6 -> 15.6.
+template <typename F>
+__device__ __forceinline__ void for_columns4(int64_t i, int64_t R, int64_t inner, F &&f) {  // f(e, column of the scales, row)
+    int64_t row, o;
+    if (((i | R | inner) >> 32) == 0) {
+        row = uint32_t(i) / uint32_t(inner);
+        o = uint32_t(row) / uint32_t(R);
+    } else {
+        row = i / inner;
+        o = row / R;
+    }
+    int64_t r = row - o * R, c = i - row * inner;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        f(e, o * inner + c, r);
+        if (++c == inner) {
+            c = 0;
+            if (++r == R) r = 0, ++o;
+        }
+    }
+}
+// Entries of `p`, one per column, of the `count` elements from i on (four at most).
+template <int DT>
+__device__ __forceinline__ void load_columns4(const void *p, int64_t i, int64_t count, int64_t R, int64_t inner, float (&v)[4]) {
+    if (inner % 4 == 0) {  // a quad lies in one row, and so does the last
+        for_columns4(i, R, inner, [&](int e, int64_t column, int64_t) {
+            if (e == 0) load_upto4<DT>(p, column, 4, v);
+        });
+        return;
+    }
+    for_columns4(i, R, inner, [&](int e, int64_t column, int64_t) { v[e] = e < count ? load_as_f32<DT>(p, column) : 0.0f; });
+}
+template <int DT, int QT>
+__global__ __launch_bounds__(256) void quantize_flat_kernel(const void *__restrict__ w, const float *__restrict__ amax, void *__restrict__ q,
+                                                            void *__restrict__ scale, int64_t R, int64_t inner, int64_t total) {
+    const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4, count = total - i;
+    if (count <= 0) return;
+    float x[4], m[4], s[4], inv[4];
+    load_upto4<DT>(w, i, count, x);
+    load_columns4<HIDET_QMM_F32>(amax, i, count, R, inner, m);
+    const bool fast = scales4<DT, QT>(m, s, inv);
+    for_columns4(i, R, inner, [&](int e, int64_t column, int64_t r) {
+        if (e < count && r == 0) store_from_f32<DT>(scale, column, s[e]);
+    });
+    uint32_t code[4];
+    codes4<DT, QT>(x, s, inv, fast, code);
+    store_codes_upto4<QT>(q, i, count, code);
+}
+template <int QT, int ST>
+__global__ __launch_bounds__(256) void dequantize_flat_kernel(const void *__restrict__ q, const void *__restrict__ scale, void *__restrict__ w,
+                                                              int64_t R, int64_t inner, int64_t total) {
+    const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4, count = total - i;
+    if (count <= 0) return;
+    float code[4], s[4], out[4];
+    load_codes_upto4<QT>(q, i, count, code);
+    load_columns4<ST>(scale, i, count, R, inner, s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * s[e]);
+    store_upto4<ST>(w, i, count, out);
 }
 
 // inner == 1: one scale per row. Block x counts blocks of 4096 elements within a row, then rows.
@@ -658,6 +755,10 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restric
     }
 }
 
+// Rows of which the column-quad kernels would use less than three eighths of a wave's lanes: at 64 the flat kernels are the
+// faster ones for every type, at 96 float32 quantizes slower in them (2048 x 128 x 96 48.5 -> 52.5 us, bfloat16 52.0 -> 46.4).
+inline bool narrow_inner(int64_t inner) { return inner < 96; }
+
 template <typename F>
 void dispatch_float(int dt, F &&f) {
     switch (dt) {
@@ -720,8 +821,16 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
         int64_t ranges = std::min(512 / std::min<int64_t>(512, col_blocks * outer), cdiv(reduce, 64));
         ranges = std::max<int64_t>(1, std::min<int64_t>({ranges, kMaxRanges, ws.scratch_bytes / (nscale * 4)}));
         const int64_t rows_per_range = cdiv(reduce, ranges);
-        launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
-               rows_per_range, nscale);
+        if (narrow_inner(inner))
+            launch(amax_narrow_kernel<DT>, dim3(1, uint32_t(ranges), uint32_t(outer)), dim3(256), 0, stream, w, amax, reduce, inner, rows_per_range, nscale);
+        else
+            launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
+                   rows_per_range, nscale);
+        if (narrow_inner(inner) && ranges == 1 && cdiv(total, 1024) < (int64_t(1) << 31)) {
+            go(quantize_flat_kernel<DT, HIDET_QMM_I8>, quantize_flat_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(cdiv(total, 1024))), 256, w, amax, wq, scale, reduce,
+               inner, total);
+            return;
+        }
         go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
            dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
     });
@@ -756,7 +865,13 @@ HIDET_API void hidet_symmetric_dequantize(const void *wq, const void *scale, voi
             else launch(dequantize_long_row_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, uint32_t(blocks));
             return;
         }
-        QMM_CHECK(outer <= 65535, "outer extent " << outer << " exceeds the grid limit");
+        if (narrow_inner(inner) || outer > 65535) {
+            QMM_CHECK(cdiv(total, 1024) < (int64_t(1) << 31), "tensor too large for one launch");
+            const dim3 grid{uint32_t(cdiv(total, 1024))};
+            if (q_dtype == HIDET_QMM_I8) launch(dequantize_flat_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
+            else launch(dequantize_flat_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
+            return;
+        }
         const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kDequantRows);
         QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
         const dim3 grid(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer));

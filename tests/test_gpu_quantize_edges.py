@@ -25,7 +25,8 @@ def _near_ties(rng, shape, axis, qmax):
 
 @pytest.mark.parametrize('dtype', ['float32', 'float16', 'bfloat16'])
 @pytest.mark.parametrize('shape,dim,codes', [((1, 3), 0, 'int8'), ((63, 255), 0, 'int8'), ((65, 257), 0, 'int16'), ((4100, 1026), 0, 'int8'),
-                                             ((129, 6), 0, 'int8'), ((3, 2049, 130), 1, 'int8'), ((33, 16387), 1, 'int8'), ((5, 4100), 1, 'int16')])
+                                             ((129, 6), 0, 'int8'), ((3, 2049, 130), 1, 'int8'), ((33, 16387), 1, 'int8'), ((5, 4100), 1, 'int16'),
+                                             ((520, 66, 9), 1, 'int8'), ((521, 3, 7), 1, 'int16'), ((9, 130, 63), 1, 'int8'), ((513, 5, 64), 1, 'int8'), ((513, 300, 2), 1, 'int8'), ((3, 2100, 95), 1, 'int8'), ((600, 9, 96), 1, 'int8')])
 def test_columns_and_rows_bit_exact(shape, dim, codes, dtype):
     announce('quantize edges', shape, dim, codes, dtype)
     w = _near_ties(np.random.default_rng(shape[-1]), shape, dim, 127 if codes == 'int8' else 32767)
@@ -40,6 +41,17 @@ def test_columns_and_rows_bit_exact(shape, dim, codes, dtype):
     assert np.array_equal(s.float().cpu().numpy(), np.asarray(s0, dtype=np.float32))
     assert np.array_equal(quant.symmetric_dequantize(q, s, dim).float().cpu().numpy(),
                           np.asarray(O.symmetric_dequantize(q0, s0, dim, dtype=dtype), dtype=np.float32))
+
+
+# more slices than a grid has layers
+@pytest.mark.parametrize('shape', [(65536, 3, 5), (65537, 2, 64)])
+def test_dequantize_of_many_slices(shape):
+    announce('dequantize of many slices', shape)
+    rng = np.random.default_rng(shape[2])
+    q = rng.integers(-127, 128, shape).astype(np.int8)
+    s = rng.random((shape[0], shape[2])).astype(np.float32)
+    got = quant.symmetric_dequantize(dev(q), dev(s), 1).cpu().numpy()
+    assert np.array_equal(got, q.astype(np.float32) * s[:, None, :])
 
 
 @pytest.mark.parametrize('k,n,group', [(4, 2, 4), (96, 258, 32), (66, 254, 33), (128, 1030, 64), (256, 126, 128), (390, 130, 65), (512, 66, 256),
