@@ -653,10 +653,11 @@ __global__ __launch_bounds__(256) void amax_all_kernel(const void *__restrict__ 
 }
 
 // e4m3 codes of four values: the quotient by the scale, clamped to +-448 (what saturation means for a format whose largest
-// finite value is 448), converted by the hardware's round-to-nearest-even OCP conversion. The product with the reciprocal,
-// within 2^-22 of the quotient, converts alike unless a rounding boundary of the format lies between them; those have at
+// finite value is 448), converted by the hardware's round-to-nearest-even OCP conversion; NaN becomes NaN of the same sign. The product with the
+// reciprocal, within 2^-22 of the quotient, converts alike unless a rounding boundary of the format lies between them; those have at
 // most four significant bits, so a product whose low 19 bits are not within 8 of zero (or that is too small for any code
-// but zero) needs no division.
+// but zero) needs no division. 448 is such a boundary and no quotient by a precise scale exceeds it by as much as 8 units
+// in the last place, so only divided values need the clamp.
 __device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, float inv, bool fast) {
     if (s == 0.0f) return 0u;
     float q[4];
@@ -668,13 +669,17 @@ __device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, fl
     }
     if (__builtin_expect(!fast || nearest <= 16u, 0)) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[e] = x[e] / s;
+        for (int e = 0; e < 4; ++e)  // (these two keep a NaN, where the median of three hides it)
+            q[e] = __builtin_elementwise_minimum(__builtin_elementwise_maximum(x[e] / s, -448.0f), 448.0f);
     }
+    uint32_t p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+    p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], int(p), true);
+    if (__builtin_expect(__builtin_isunordered(q[0], q[1]) || __builtin_isunordered(q[2], q[3]), 0)) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) q[e] = __builtin_amdgcn_fmed3f(q[e], -448.0f, 448.0f);
-    int p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
-    p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], p, true);
-    return uint32_t(p);
+        for (int e = 0; e < 4; ++e)  // (the conversion drops a NaN's sign)
+            if (q[e] != q[e]) p = (p & ~(0xFFu << (8 * e))) | ((0x7Fu | ((__float_as_uint(q[e]) >> 24) & 0x80u)) << (8 * e));
+    }
+    return p;
 }
 
 // Small tensors (the activations of a decode step), up to 65536 elements, in one launch: a workgroup of 1024 threads looks at
