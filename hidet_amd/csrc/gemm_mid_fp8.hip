@@ -110,7 +110,9 @@ struct MidF8 {
     __device__ __forceinline__ void widen(const Weights &raw, Fragments &b, int st) const {
         b = raw;
         if constexpr (SCALED) {
-            b.col_scale = col_scales[st < args.k_blocks ? st : 0];
+            // a stage past the end adds nothing, whatever the scales are: its products and row factors are zeros, so is this
+            const float f = col_scales[st < args.k_blocks ? st : 0];
+            b.col_scale = st < args.k_blocks ? f : 0.0f;
         } else if (st * 128 + 128 > k) {
             mask(b.half[0], st, kg);
             mask(b.half[1], st, kg);

@@ -40,3 +40,21 @@ def test_fp8_quantization_of_infinities_and_subnormal_scales():
     codes, scale = F8.fp8_quantize_per_tensor(dev(tiny))
     c0, s0 = O.fp8_quantize_per_tensor(tiny)
     assert np.float32(scale.item()) == s0 and np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
+
+
+# an odd number of k blocks: a group of waves has a stage past the end in its last round; one and several pieces of K
+@pytest.mark.parametrize('m,k,n', [(17, 128, 128), (40, 384, 256), (64, 7040, 384), (130, 1152, 512)])
+def test_block_scaled_fp8_with_infinite_scales(m, k, n):
+    announce('fp8 block scales inf', m, k, n)
+    g = torch.Generator(device='cuda').manual_seed(m + k)
+    a = torch.randint(1, 4, (m, k), generator=g, device='cuda').float()
+    a[::3] *= -1
+    b = torch.randint(1, 4, (n, k), generator=g, device='cuda').float()
+    scale_a, scale_b = torch.full((k // 128, m), 0.5, device='cuda'), torch.full((n // 128, k // 128), 0.25, device='cuda')
+    scale_b[0, 0] = float('inf')
+    scale_a[-1, 5] = float('inf')
+    part = torch.matmul(a.view(m, k // 128, 128).transpose(0, 1).double().contiguous(), b.view(n, k // 128, 128).permute(1, 2, 0).double().contiguous())
+    want = (part * scale_a.double()[:, :, None] * scale_b.double().repeat_interleave(128, 0).t()[:, None, :]).sum(0).float()
+    assert not want.isnan().any() and want.isinf().any()
+    for _ in range(2):
+        assert torch.equal(F8.matmul_f8_scaled(a.to(F8.f8e4m3), b.to(F8.f8e4m3), scale_a, scale_b, output_dtype='float32'), want)
