@@ -223,6 +223,7 @@ PyObject *matmul_f8(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         const at::Tensor *a = nargs == 5 ? gpu_tensor(args[0], at::kFloat8_e4m3fn) : nullptr, *b = a ? gpu_tensor(args[1], at::kFloat8_e4m3fn) : nullptr;
         if (b == nullptr || !THPDtype_Check(args[4]) || b->dim() != 2 || !same_device(*a, *b)) Py_RETURN_NONE;
         const at::Tensor *scale[2] = {nullptr, nullptr};
+        if ((args[2] == Py_None) != (args[3] == Py_None)) Py_RETURN_NONE;
         for (int i = 0; i < 2; ++i) {
             if (args[2 + i] == Py_None) continue;
             scale[i] = gpu_tensor(args[2 + i], at::kFloat);

@@ -232,7 +232,7 @@ def matmul_f8_per_tensor(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor
                          output_dtype='bfloat16') -> torch.Tensor:
     """cast((a @ b^T) * (scale_a * scale_b)) with fp32 accumulation; the scales are float32 tensors of one
     element on the GPU (as returned by fp8_quantize_per_tensor)."""
-    if a.is_cuda:
+    if a.is_cuda and scale_a is not None and scale_b is not None:  # (to the front two None mean an unscaled product)
         out = ffi.front().matmul_f8(a, b, scale_a, scale_b, data_type(output_dtype))
         if out is not None:
             return out

@@ -106,3 +106,15 @@ def test_each_stream_has_its_workspace():
         assert (x.device.index, stream.cuda_stream) in ffi._WORKSPACES
     stream.synchronize()
     assert torch.equal(got, want)
+
+
+def test_a_missing_scale_is_an_error():
+    announce('front: missing scales')
+    a, sa = F8.fp8_quantize_per_tensor(torch.randn((3, 64), device='cuda'))
+    b, sb = F8.fp8_quantize_per_tensor(torch.randn((32, 64), device='cuda'))
+    for scales in ((None, sb), (sa, None), (None, None)):
+        with pytest.raises(AttributeError):
+            F8.matmul_f8_per_tensor(a, b, *scales)
+    for scales in ((None, sb), (sa, None)):
+        assert ffi.front().matmul_f8(a, b, *scales, torch.float32) is None
+    assert torch.equal(ffi.front().matmul_f8(a, b, None, None, torch.float32), F8.matmul_f8(a, b, output_dtype='float32'))
