@@ -192,9 +192,12 @@ void skinny_w8a16_launch(const void *a, const void *w, const void *scale, const 
                          int64_t n, int64_t lda, int64_t n_out, int parallel_k_parts, const Workspace &ws, bool strict_workspace,
                          hipStream_t stream) {
     const bool fast = skinny_w8a16_supported(w, scale, bias, k, n);
+    const bool ragged = n % 16 != 0 || !aligned(w, 16) || n_out != n;
     constexpr int waves = kWaves;
     SkinnyPlan plan;
-    if (fast) plan = skinny_make_plan(k, n, parallel_k_parts, int(std::min<int64_t>(16, m)), ws.mailbox_bytes, strict_workspace, /*flat_ok=*/true, device_cus());
+    // (a K split that does not fit the scratch memory is an error only for operands that need no ragged form: the others run
+    // with whatever there is)
+    if (fast) plan = skinny_make_plan(k, n, parallel_k_parts, int(std::min<int64_t>(16, m)), ws.mailbox_bytes, strict_workspace && !ragged, /*flat_ok=*/true, device_cus());
     // a wave's run of rows is addressed with 31-bit offsets
     if (!fast || (cdiv(cdiv(skinny_units(plan), plan.groups), waves) * 32 + 160) * n >= (int64_t(1) << 31) - (1 << 20)) {
         QMM_CHECK(n_out == n, "padded weights of " << k << " x " << n << " cannot be addressed");
@@ -203,7 +206,6 @@ void skinny_w8a16_launch(const void *a, const void *w, const void *scale, const 
                static_cast<_Float16 *>(c), m, k, n);
         return;
     }
-    const bool ragged = n % 16 != 0 || !aligned(w, 16) || n_out != n;
     // 16-byte activation loads through a buffer descriptor: aligned rows, offsets below 2^31
     const bool aligned_a = (k % 8 == 0) && (lda % 8 == 0) && aligned(a, 16) && (15 * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20);
     uint32_t *lost_flag = ws.counters != nullptr ? ws.counters + kExchangeLostWord : nullptr;

@@ -163,3 +163,15 @@ def test_task_library_launch_matches_the_operator(tmp_path):
     want = quant.symmetric_quant_matmul(da, dq, ds)
     assert torch.equal(c, want)
     assert O.max_rel_err(host(c), clib.quant_matmul_f32acc(a, q, s)) <= 1e-2
+
+
+def test_static_scratch_takes_any_k_split_on_sizes_off_the_tiles():
+    """N a multiple of 4 but not of 16: a number of K slices that does not fit the static array is a launch with fewer of them."""
+    for m, k, n, parts in ((16, 4096, 4100, 16), (9, 2048, 16388, 64)):
+        announce('static scratch, ragged with K slices', m, k, n, parts)
+        rng = np.random.default_rng(n)
+        a = rng.integers(-3, 4, (m, k)).astype(np.float16)
+        q = rng.integers(-7, 8, (k, n)).astype(np.int8)
+        want = a.astype(np.float32) @ q.astype(np.float32)  # small integers: every sum is exact
+        got = host(_static(dev(a), dev(q), dev(np.ones(n, np.float16)), parts))
+        assert np.array_equal(got, want.astype(np.float16))
