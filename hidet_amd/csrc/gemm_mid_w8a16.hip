@@ -142,14 +142,14 @@ struct MidW8 {
             }
         }
     }
-    // zero what a fragment holds past K (the next row's values, which may be anything)
+    // zero what a fragment holds past K (the next row's values, which may be anything); K is even
     __device__ __forceinline__ void mask(int4v_t (&af)[kAChunks], int st, int kg) const {
 #pragma unroll
         for (int q = 0; q < kAChunks; ++q) {
             const int left = k - (st * kStageK + (kg * kAChunks + q) * 8);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const uint32_t keep = left >= 2 * e + 2 ? 0xFFFFFFFFu : left == 2 * e + 1 ? 0xFFFFu : 0u;
+                const uint32_t keep = left > 2 * e ? 0xFFFFFFFFu : 0u;
                 af[q][e] = int(uint32_t(af[q][e]) & keep);
             }
         }
@@ -186,10 +186,11 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
                       int64_t n, int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, double limit_us, const Workspace &ws, hipStream_t stream) {
     const MidW8Args args{static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias), static_cast<_Float16 *>(c), int(ldc), int(n_out),
                          n_out % 4 == 0 && ldc % 4 == 0 && aligned(c, 8)};
-    // four columns of a lane are all inside the matrix; loads start at multiples of four bytes; what a tile reads lies within
-    // 2 GiB (kMidOutside)
+    // four columns of a lane are all inside the matrix; loads start at multiples of four bytes, and no dword of the
+    // activations lies half outside their buffer (it would read as zero: K is even); what a tile reads lies within 2 GiB
+    // (kMidOutside)
     constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
-    if (n % 4 != 0 || lda % 2 != 0 || !aligned(a, 4) || !aligned(w, 4) || lda * 256 + k * 2 >= kMost || ldc >= kMost) return false;
+    if (n % 4 != 0 || k % 2 != 0 || lda % 2 != 0 || !aligned(a, 4) || !aligned(w, 4) || lda * 256 + k * 2 >= kMost || ldc >= kMost) return false;
     const int64_t las = lda * 2;
     if (nk) {
         if (ldw % 4 != 0 || ldw * 64 + k >= kMost) return false;

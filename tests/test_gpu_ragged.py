@@ -59,3 +59,18 @@ def test_int4_exact(m, k, n, group):
     want = O.to_bf16((a.astype(np.float64) @ (q.astype(np.float64) * np.repeat(s, group, axis=0))).astype(np.float32))
     got = quant.symmetric_quant_matmul_w4a16(dev(a, torch.bfloat16), dev(O.pack_int4(q)), dev(s, torch.bfloat16), group)
     assert np.array_equal(host(got), want)
+
+
+# K odd, rows of an even stride (what a C caller may pass): the last element of the last row counts, the one behind it does not
+@pytest.mark.parametrize('m,k,n', [(17, 129, 256), (31, 4097, 260), (33, 1001, 512), (64, 63, 1024), (130, 2047, 388)])
+def test_int8_odd_k(m, k, n):
+    announce('ragged int8 odd k', m, k, n)
+    a, w, s, _, _ = _int8_case(m, k, n, False)
+    a[-1, -1], w[-1] = 3, 100
+    wide = torch.full((m, k + 1), float('nan'), dtype=torch.float16, device='cuda')
+    wide[:, :k] = a
+    want = ((a.double() @ w.double()) * s.double()).float().half()
+    c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+    ws = ffi.workspace(a.device)
+    ffi.call('hidet_symmetric_quant_matmul_f16_i8', wide, w, s, c, m, k, n, k + 1, 0, ws, ws.numel(), ffi.current_stream(a.device))
+    assert torch.equal(c, want)
