@@ -96,7 +96,9 @@ bool w8a16_padded(const void *a, const void *w, const void *scale, const void *b
     const int64_t per_col = kp + 4, fixed = a_bytes + 1024;
     const int64_t most = std::min<int64_t>(room - fixed, int64_t(1) << 30) / per_col;
     if (cols > most) cols = most / 256 * 256;
-    if (cols <= 0 || (!gemm && cols < n)) return false;  // (the bandwidth-bound kernel writes whole rows: one panel)
+    if (cols <= 0) return false;
+    // the bandwidth-bound kernel writes whole rows (one panel) and addresses a wave's rows with 31-bit offsets
+    if (!gemm && (cols < n || (k + 192) * cols >= (int64_t(1) << 31) - (1 << 20))) return false;
     char *end = ws.scratch + ws.scratch_bytes / 256 * 256;
     PadArgs p{};
     p.w = static_cast<const int8_t *>(w);

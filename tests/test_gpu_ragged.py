@@ -74,3 +74,15 @@ def test_int8_odd_k(m, k, n):
     ws = ffi.workspace(a.device)
     ffi.call('hidet_symmetric_quant_matmul_f16_i8', wide, w, s, c, m, k, n, k + 1, 0, ws, ws.numel(), ffi.current_stream(a.device))
     assert torch.equal(c, want)
+
+
+def test_int8_rows_beyond_31_bit_offsets():
+    """So wide that 160 rows of the weight take more than 2 GiB, N no multiple of 4: neither the bandwidth-bound kernel nor its
+    padded copies can address it."""
+    m, k, n = 1, 2, 13_500_002
+    announce('ragged int8 wide', m, k, n)
+    g = torch.Generator(device='cuda').manual_seed(3)
+    a = torch.tensor([[3.0, -2.0]], device='cuda').half()
+    w = torch.randint(-127, 128, (k, n), generator=g, device='cuda', dtype=torch.int8)
+    s = torch.full((n,), 0.5, device='cuda', dtype=torch.float16)
+    assert torch.equal(quant.symmetric_quant_matmul(a, w, s), ((3.0 * w[0].float() - 2.0 * w[1].float()) * 0.5).half()[None])
