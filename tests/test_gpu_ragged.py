@@ -85,4 +85,9 @@ def test_int8_rows_beyond_31_bit_offsets():
     a = torch.tensor([[3.0, -2.0]], device='cuda').half()
     w = torch.randint(-127, 128, (k, n), generator=g, device='cuda', dtype=torch.int8)
     s = torch.full((n,), 0.5, device='cuda', dtype=torch.float16)
-    assert torch.equal(quant.symmetric_quant_matmul(a, w, s), ((3.0 * w[0].float() - 2.0 * w[1].float()) * 0.5).half()[None])
+    want = ((3.0 * w[0].float() - 2.0 * w[1].float()) * 0.5).half()[None]
+    c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+    for scratch in (64 << 20, 160 << 20):  # without and with room for a copy of the weight
+        ws = torch.zeros(int(ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(scratch)), dtype=torch.uint8, device='cuda')
+        ffi.call('hidet_symmetric_quant_matmul_f16_i8', a, w, s, c, m, k, n, k, 0, ws, ws.numel(), ffi.current_stream(a.device))
+        assert torch.equal(c, want)
