@@ -10,9 +10,10 @@ namespace qmm {
 namespace {
 
 
-__global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v) {
+template <typename T>
+__global__ void zero_kernel(T *p, int64_t n) {
     int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    if (i < n) p[i] = 0;
 }
 
 // Nearest integer (ties to even) of v, |v| < 2^21, in the low bits of the returned word.
@@ -797,9 +798,13 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
     float *amax = reinterpret_cast<float *>(ws.scratch);
     dispatch_float(w_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (total == 0) return;
         const int esize = DT == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
         QMM_CHECK(aligned(w, esize) && aligned(wq, qsize) && aligned(scale, esize), "a tensor is not aligned to its element type");
+        if (total == 0) {  // no elements (reduce is 0): the scales still have to be written
+            if (DT == HIDET_QMM_F32) launch_aux(zero_kernel<uint32_t>, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, static_cast<uint32_t *>(scale), nscale);
+            else launch_aux(zero_kernel<uint16_t>, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, static_cast<uint16_t *>(scale), nscale);
+            return;
+        }
         auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) {
             if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), 0, stream, args...);
             else launch(i16, grid, dim3(threads), 0, stream, args...);
@@ -839,14 +844,6 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
         go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
            dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
     });
-    if (reduce == 0) {
-        // no elements: scale = 0 still has to be written
-        dispatch_float(w_dtype, [&](auto dt) {
-            constexpr int DT = decltype(dt)::value;
-            if (DT == HIDET_QMM_F32) launch_aux(fill_u32_kernel, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, static_cast<uint32_t *>(scale), nscale, 0u);
-            else launch_aux(fill_u32_kernel, dim3(cdiv(cdiv(nscale, 2), 256)), dim3(256), 0, stream, static_cast<uint32_t *>(scale), cdiv(nscale, 2), 0u);
-        });
-    }
     QMM_ENTRY_END
 }
 

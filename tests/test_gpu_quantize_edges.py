@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
+from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as F8
 from gpu_util import announce, dev, host
@@ -92,3 +93,20 @@ def test_fp8_per_tensor_of_a_few_rows(numel, dtype):
     c0, s0 = O.fp8_quantize_per_tensor(t.float().cpu().numpy())
     assert np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
     assert scale.item() == float(np.asarray(s0).reshape(-1)[0])
+
+
+# an empty reduction: scales of zero, and nothing behind the last of them (a number of 16-bit scales that fills no whole word)
+@pytest.mark.parametrize('count', [1, 3, 256, 257])
+@pytest.mark.parametrize('start', [0, 1])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+def test_scales_of_an_empty_reduction(count, start, dtype):
+    announce('empty reduction', count, start, dtype)
+    buf = torch.full((count + 4,), 7.0, dtype=dtype, device='cuda')
+    scale = buf[start:start + count]
+    ws = ffi.workspace(buf.device)
+    none = torch.empty((0,), dtype=torch.int8, device='cuda')
+    ffi.call('hidet_symmetric_quantize', none, none, scale, 1, 0, count, ffi.DTYPE_CODE[dtype], ffi.DTYPE_CODE[torch.int8], ws, ws.numel(),
+             ffi.current_stream(buf.device))
+    want = torch.full_like(buf, 7.0)
+    want[start:start + count] = 0
+    assert torch.equal(buf, want)
