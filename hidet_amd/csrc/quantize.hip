@@ -765,6 +765,54 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restric
 // faster ones for every type, at 96 float32 quantizes slower in them (2048 x 128 x 96 48.5 -> 52.5 us, bfloat16 52.0 -> 46.4).
 inline bool narrow_inner(int64_t inner) { return inner < 96; }
 
+// The quantizer's launches for [outer, reduce, inner], no extent zero, outer at most quantize_slices_most(reduce, inner).
+template <int DT>
+void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_t reduce, int64_t inner, int q_dtype, float *amax, int64_t scratch_bytes,
+                     hipStream_t stream) {
+    const int64_t total = outer * reduce * inner, nscale = outer * inner;
+    const int esize = DT == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
+    auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) {
+        if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), 0, stream, args...);
+        else launch(i16, grid, dim3(threads), 0, stream, args...);
+    };
+    if (inner == 1) {
+        // rows that fit a workgroup's registers: one pass
+        if (reduce % 4 == 0 && reduce <= 256 * 4 * 16 && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
+            const dim3 grid{uint32_t(outer)};
+            if (reduce <= 256 * 4 * 4) go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 4>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 4>, grid, 256, w, wq, scale, reduce / 4);
+            else go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 16>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 16>, grid, 256, w, wq, scale, reduce / 4);
+            return;
+        }
+        launch(amax_contig_kernel<DT>, dim3(cdiv(outer, 4)), dim3(256), 0, stream, w, amax, outer, reduce);
+        const int64_t blocks = cdiv(reduce, 1024);
+        go(quantize_long_row_kernel<DT, HIDET_QMM_I8>, quantize_long_row_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(blocks * outer)), 256, w, amax, wq, scale,
+           reduce, uint32_t(blocks));
+        return;
+    }
+    const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kQuantRows);
+    QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
+    // enough row ranges for two workgroups per CU, of 64 rows at least, and as many as the scratch memory holds maxima of
+    int64_t ranges = std::min(512 / std::min<int64_t>(512, col_blocks * outer), cdiv(reduce, 64));
+    ranges = std::max<int64_t>(1, std::min<int64_t>({ranges, kMaxRanges, scratch_bytes / (nscale * 4)}));
+    const int64_t rows_per_range = cdiv(reduce, ranges);
+    if (narrow_inner(inner))
+        launch(amax_narrow_kernel<DT>, dim3(1, uint32_t(ranges), uint32_t(outer)), dim3(256), 0, stream, w, amax, reduce, inner, rows_per_range, nscale);
+    else
+        launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
+               rows_per_range, nscale);
+    if (narrow_inner(inner) && ranges == 1 && cdiv(total, 1024) < (int64_t(1) << 24)) {
+        go(quantize_flat_kernel<DT, HIDET_QMM_I8>, quantize_flat_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(cdiv(total, 1024))), 256, w, amax, wq, scale, reduce,
+           inner, total);
+        return;
+    }
+    go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
+       dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
+}
+// Slices of a launch: a grid has 65535 layers, and 2^32 threads along x.
+inline int64_t quantize_slices_most(int64_t reduce, int64_t inner) {
+    return inner > 1 ? 65535 : std::max<int64_t>(1, ((int64_t(1) << 24) - 1) / cdiv(reduce, 1024));
+}
+
 template <typename F>
 void dispatch_float(int dt, F &&f) {
     switch (dt) {
@@ -790,7 +838,7 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
     const int64_t nscale = outer * inner;
     if (nscale == 0) return;
     QMM_CHECK(scale && (total == 0 || (w && wq)), "null tensor pointer");
-    QMM_CHECK(inner < (int64_t(1) << 31) * 64 && outer < 65536 * int64_t(4), "extent too large");
+    QMM_CHECK(inner < (int64_t(1) << 31) * 64, "extent too large");
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     QMM_CHECK(ws.scratch_bytes >= nscale * 4, "workspace too small: its scratch part (three quarters of what follows the first 64 KiB) must hold "
                                                   << nscale * 4 << " bytes, got a workspace of " << workspace_bytes);
@@ -805,44 +853,10 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
             else launch_aux(zero_kernel<uint16_t>, dim3(cdiv(nscale, 256)), dim3(256), 0, stream, static_cast<uint16_t *>(scale), nscale);
             return;
         }
-        auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) {
-            if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), 0, stream, args...);
-            else launch(i16, grid, dim3(threads), 0, stream, args...);
-        };
-        if (inner == 1) {
-            // rows that fit a workgroup's registers: one pass
-            if (reduce % 4 == 0 && reduce <= 256 * 4 * 16 && outer < (int64_t(1) << 31) && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
-                const dim3 grid{uint32_t(outer)};
-                if (reduce <= 256 * 4 * 4) go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 4>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 4>, grid, 256, w, wq, scale, reduce / 4);
-                else go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 16>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 16>, grid, 256, w, wq, scale, reduce / 4);
-                return;
-            }
-            launch(amax_contig_kernel<DT>, dim3(cdiv(outer, 4)), dim3(256), 0, stream, w, amax, outer, reduce);
-            const int64_t blocks = cdiv(reduce, 1024);
-            QMM_CHECK(blocks * outer < (int64_t(1) << 31), "tensor too large for one launch");
-            go(quantize_long_row_kernel<DT, HIDET_QMM_I8>, quantize_long_row_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(blocks * outer)), 256, w, amax, wq, scale,
-               reduce, uint32_t(blocks));
-            return;
-        }
-        QMM_CHECK(outer <= 65535, "outer extent " << outer << " exceeds the grid limit");
-        const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kQuantRows);
-        QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
-        // enough row ranges for two workgroups per CU, of 64 rows at least, and as many as the scratch memory holds maxima of
-        int64_t ranges = std::min(512 / std::min<int64_t>(512, col_blocks * outer), cdiv(reduce, 64));
-        ranges = std::max<int64_t>(1, std::min<int64_t>({ranges, kMaxRanges, ws.scratch_bytes / (nscale * 4)}));
-        const int64_t rows_per_range = cdiv(reduce, ranges);
-        if (narrow_inner(inner))
-            launch(amax_narrow_kernel<DT>, dim3(1, uint32_t(ranges), uint32_t(outer)), dim3(256), 0, stream, w, amax, reduce, inner, rows_per_range, nscale);
-        else
-            launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
-                   rows_per_range, nscale);
-        if (narrow_inner(inner) && ranges == 1 && cdiv(total, 1024) < (int64_t(1) << 31)) {
-            go(quantize_flat_kernel<DT, HIDET_QMM_I8>, quantize_flat_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(cdiv(total, 1024))), 256, w, amax, wq, scale, reduce,
-               inner, total);
-            return;
-        }
-        go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
-           dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
+        const int64_t step = quantize_slices_most(reduce, inner);
+        for (int64_t o = 0; o < outer; o += step)  // (one launch after the other: they share the scratch memory)
+            quantize_slices<DT>(static_cast<const char *>(w) + o * reduce * inner * esize, static_cast<char *>(wq) + o * reduce * inner * qsize,
+                                static_cast<char *>(scale) + o * inner * esize, std::min(step, outer - o), reduce, inner, q_dtype, amax, ws.scratch_bytes, stream);
     });
     QMM_ENTRY_END
 }

@@ -55,6 +55,18 @@ def test_dequantize_of_many_slices(shape):
     assert np.array_equal(got, q.astype(np.float32) * s[:, None, :])
 
 
+# the same for the quantizer, whose slices then take several launches, and rows of more than one launch's threads
+@pytest.mark.parametrize('shape', [(65535, 3, 5), (65536, 3, 5), (131071, 2, 9), (65537, 2, 100), (262144, 6), (262145, 7), ((1 << 24) + 3, 4)])
+def test_quantize_of_many_slices(shape):
+    announce('quantize of many slices', shape)
+    w = torch.randn(shape, generator=torch.Generator(device='cuda').manual_seed(shape[0]), device='cuda')
+    q, s = quant.symmetric_quantize(w, 'int8', 1)
+    for part in (slice(0, 1000), slice(65000, 66000), slice(shape[0] - 1000, shape[0])):
+        q0, s0 = O.symmetric_quantize(host(w[part]), 'int8', 1)
+        assert np.array_equal(host(q[part]), q0) and np.array_equal(host(s[part]), s0)
+    assert torch.equal(s, w.abs().amax(1) / torch.full_like(s, 127))  # (by a number torch multiplies with its reciprocal)
+
+
 @pytest.mark.parametrize('k,n,group', [(4, 2, 4), (96, 258, 32), (66, 254, 33), (128, 1030, 64), (256, 126, 128), (390, 130, 65), (512, 66, 256),
                                        (514, 6, 257), (1024, 258, 1024)])
 def test_int4_groups_bit_exact(k, n, group):
