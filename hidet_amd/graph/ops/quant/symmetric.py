@@ -73,7 +73,7 @@ class SymmetricQuantizationOp(Operator):
         wq = torch.empty(src.shape, dtype=quant_type, device=w.device)
         scale_shape = [s for i, s in enumerate(shape) if i not in dims]
         scale = torch.empty(scale_shape, dtype=w.dtype, device=w.device)
-        ws = ffi.workspace(w.device, (64 << 10) + 4 * outer * inner)
+        ws = ffi.workspace(w.device, ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(4 * outer * inner))  # one maximum per scale
         ffi.call('hidet_symmetric_quantize', src, wq, scale, outer, reduce, inner, ffi.DTYPE_CODE[w.dtype],
                  ffi.DTYPE_CODE[quant_type], ws, ws.numel(), ffi.current_stream(w.device))
         if perm is not None:

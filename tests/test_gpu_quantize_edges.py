@@ -67,6 +67,15 @@ def test_quantize_of_many_slices(shape):
     assert torch.equal(s, w.abs().amax(1) / torch.full_like(s, 127))  # (by a number torch multiplies with its reciprocal)
 
 
+def test_more_scales_than_the_standing_workspace_holds():
+    announce('quantize with 22 million scales')
+    w = torch.randn((2, 22_000_000), device='cuda')
+    q, s = quant.symmetric_quantize(w, 'int8', 0)
+    assert torch.equal(s, w.abs().amax(0) / torch.full_like(s, 127))
+    for part in (slice(0, 1000), slice(-1000, None)):
+        assert np.array_equal(host(q[:, part]), O.symmetric_quantize(host(w[:, part]), 'int8', 0)[0])
+
+
 @pytest.mark.parametrize('k,n,group', [(4, 2, 4), (96, 258, 32), (66, 254, 33), (128, 1030, 64), (256, 126, 128), (390, 130, 65), (512, 66, 256),
                                        (514, 6, 257), (1024, 258, 1024)])
 def test_int4_groups_bit_exact(k, n, group):
