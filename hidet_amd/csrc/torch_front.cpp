@@ -172,6 +172,14 @@ PyObject *w8a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     });
 }
 
+// A group size; false where it is no int, not positive or more than the ABI's type holds.
+bool group_of(PyObject *o, int64_t *group) {
+    if (!PyLong_CheckExact(o)) return false;
+    *group = PyLong_AsLong(o);
+    if (*group == -1) PyErr_Clear();  // (set where no long holds it)
+    return *group > 0 && *group <= INT32_MAX;
+}
+
 // a, packed, scales, group size, bias or None
 PyObject *w4a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject * {
@@ -180,13 +188,12 @@ PyObject *w4a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         const at::Tensor *w = gpu_tensor(args[1], at::kByte), *scales = w ? gpu_tensor(args[2], a->scalar_type()) : nullptr;
         const bool biased = args[4] != Py_None;
         const at::Tensor *bias = scales && biased ? gpu_tensor(args[4], a->scalar_type()) : nullptr;
-        if (scales == nullptr || (biased && bias == nullptr) || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
-        const long group = PyLong_AsLong(args[3]);
-        if (group == -1 && PyErr_Occurred()) return nullptr;
+        int64_t group;
+        if (scales == nullptr || (biased && bias == nullptr) || !group_of(args[3], &group)) Py_RETURN_NONE;
         if (w->dim() != 2 || scales->dim() != 2 || !w->is_contiguous() || !scales->is_contiguous() || !same_device(*a, *w) || !same_device(*a, *scales)) Py_RETURN_NONE;
         const int64_t k = w->size(0), n = w->size(1) * 2;
         Rows rows;
-        if (n == 0 || group <= 0 || group > INT32_MAX || k % group != 0 || scales->size(0) != k / group || scales->size(1) != n || !as_rows(*a, k, &rows)) Py_RETURN_NONE;
+        if (n == 0 || k % group != 0 || scales->size(0) != k / group || scales->size(1) != n || !as_rows(*a, k, &rows)) Py_RETURN_NONE;
         if (biased && (bias->dim() != 1 || bias->size(0) != n || !bias->is_contiguous() || !same_device(*a, *bias))) Py_RETURN_NONE;
         Workspace ws;
         if (!stream_and_workspace(*a, &ws)) return nullptr;
@@ -331,12 +338,11 @@ PyObject *dequantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 PyObject *quantize_int4(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject * {
         const at::Tensor *w = nargs == 3 ? gpu_tensor(args[0], at::kFloat) : nullptr;
-        if (w == nullptr || w->dim() != 2 || !w->is_contiguous() || w->numel() == 0 || !PyLong_CheckExact(args[1]) || !THPDtype_Check(args[2])) Py_RETURN_NONE;
-        const long group = PyLong_AsLong(args[1]);
-        if (group == -1 && PyErr_Occurred()) return nullptr;
+        int64_t group;
+        if (w == nullptr || w->dim() != 2 || !w->is_contiguous() || w->numel() == 0 || !group_of(args[1], &group) || !THPDtype_Check(args[2])) Py_RETURN_NONE;
         const at::ScalarType type = reinterpret_cast<THPDtype *>(args[2])->scalar_type;
         const int64_t k = w->size(0), n = w->size(1);
-        if (group <= 0 || group > INT32_MAX || k % group != 0 || n % 2 != 0 || (type != at::kHalf && type != at::kBFloat16)) Py_RETURN_NONE;
+        if (k % group != 0 || n % 2 != 0 || (type != at::kHalf && type != at::kBFloat16)) Py_RETURN_NONE;
         at::Tensor packed = at::empty({k, n / 2}, w->options().dtype(at::kByte).requires_grad(false));
         at::Tensor scales = at::empty({k / group, n}, w->options().dtype(type).requires_grad(false));
         lib.quantize_int4(w->data_ptr(), packed.data_ptr(), scales.data_ptr(), k, n, int(group), HIDET_QMM_F32, type == at::kHalf ? HIDET_QMM_F16 : HIDET_QMM_BF16,
@@ -351,14 +357,13 @@ PyObject *w4a16_decode(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         const at::Tensor *a = nargs == 4 ? tensor(args[0]) : nullptr;
         if (a == nullptr || !a->is_cuda() || (a->scalar_type() != at::kHalf && a->scalar_type() != at::kBFloat16)) Py_RETURN_NONE;
         const at::Tensor *w = gpu_tensor(args[1], at::kByte), *scales = w ? gpu_tensor(args[2], a->scalar_type()) : nullptr;
-        if (scales == nullptr || !PyLong_CheckExact(args[3]) || w->dim() != 2 || scales->dim() != 2 || !w->is_contiguous() || !scales->is_contiguous() ||
+        int64_t group;
+        if (scales == nullptr || !group_of(args[3], &group) || w->dim() != 2 || scales->dim() != 2 || !w->is_contiguous() || !scales->is_contiguous() ||
             !same_device(*a, *w) || !same_device(*a, *scales))
             Py_RETURN_NONE;
-        const long group = PyLong_AsLong(args[3]);
-        if (group == -1 && PyErr_Occurred()) return nullptr;
         const int64_t n = w->size(0), k = w->size(1) * 2;
         Rows rows;
-        if (n == 0 || group <= 0 || group > INT32_MAX || k % group != 0 || scales->size(0) != k / group || scales->size(1) != n || !as_rows(*a, k, &rows)) Py_RETURN_NONE;
+        if (n == 0 || k % group != 0 || scales->size(0) != k / group || scales->size(1) != n || !as_rows(*a, k, &rows)) Py_RETURN_NONE;
         if (rows.stride % 8 != 0 || reinterpret_cast<uintptr_t>(a->data_ptr()) % 16 != 0) Py_RETURN_NONE;
         at::Tensor c = output(*a, n, a->scalar_type());
         lib.w4a16_nk(a->data_ptr(), w->data_ptr(), scales->data_ptr(), c.data_ptr(), rows.m, k, n, rows.stride, k / 2, int(group),

@@ -118,3 +118,17 @@ def test_a_missing_scale_is_an_error():
     for scales in ((None, sb), (sa, None)):
         assert ffi.front().matmul_f8(a, b, *scales, torch.float32) is None
     assert torch.equal(ffi.front().matmul_f8(a, b, None, None, torch.float32), F8.matmul_f8(a, b, output_dtype='float32'))
+
+
+def test_a_group_size_no_integer_type_holds():
+    announce('front: group sizes')
+    w = torch.randn((256, 64), device='cuda')
+    p, s = quant.symmetric_group_quantize_int4(w, 128, 'float16')
+    x, nk, front = torch.randn((2, 256), device='cuda').half(), quant.to_decode_layout_int4(p), ffi.front()
+    for group in (2 ** 70, -2 ** 70, 2 ** 40, -1, 0):
+        assert front.quantize_int4(w, group, torch.float16) is None and front.w4a16(x, p, s, group, None) is None
+        assert front.w4a16_decode(x, nk, s, group) is None
+    for call in (lambda: quant.symmetric_group_quantize_int4(w, 2 ** 70), lambda: quant.symmetric_quant_matmul_w4a16(x, p, s, 2 ** 70),
+                 lambda: quant.symmetric_quant_matmul_w4a16_decode(x, nk, s, 2 ** 70)):
+        with pytest.raises((ValueError, AssertionError)):
+            call()
