@@ -38,7 +38,7 @@ struct Library {
 } lib;
 PyObject *workspaces = nullptr;      // hidet_amd.ffi._WORKSPACES: (device, stream) -> uint8 tensor
 PyObject *new_workspace = nullptr;   // hidet_amd.ffi.workspace(device): makes the entry
-PyObject *backend_error = nullptr;   // hidet_amd.ffi.BackendException
+PyObject *failure = nullptr;         // hidet_amd.ffi.failure(entry point, arguments, error): the exception to raise
 
 const at::Tensor *tensor(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
@@ -99,14 +99,23 @@ at::Tensor output(const at::Tensor &a, int64_t n, at::ScalarType type) {
     return at::empty(sizes, a.options().dtype(type).requires_grad(false));
 }
 
-// The result, or the library's error as an exception.
-PyObject *finish(const char *name, PyObject *result) {
+// The result, or the library's error as an exception that names the entry point and describes the arguments.
+PyObject *finish(const char *name, PyObject *const *args, Py_ssize_t nargs, PyObject *result) {
     const char *error = lib.get_last_error();
-    if (error != nullptr) {
-        Py_XDECREF(result);
-        return PyErr_Format(backend_error, "Calling %s failed. error:\n%s", name, error);
+    if (error == nullptr) return result;
+    Py_XDECREF(result);
+    PyObject *list = PyTuple_New(nargs);
+    if (list == nullptr) return nullptr;
+    for (Py_ssize_t i = 0; i < nargs; ++i) {
+        Py_INCREF(args[i]);
+        PyTuple_SET_ITEM(list, i, args[i]);
     }
-    return result;
+    PyObject *exception = PyObject_CallFunction(failure, "sOs", name, list, error);
+    Py_DECREF(list);
+    if (exception == nullptr) return nullptr;
+    PyErr_SetObject(reinterpret_cast<PyObject *>(Py_TYPE(exception)), exception);
+    Py_DECREF(exception);
+    return nullptr;
 }
 
 PyObject *pair(at::Tensor first, at::Tensor second) {
@@ -168,7 +177,9 @@ PyObject *w8a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             if (biased) lib.w8a16_nk_bias(ap, wp, sp, bp, cp, rows.m, k, n, rows.stride, ldw, ws.ptr, ws.bytes, ws.stream);
             else lib.w8a16_nk(ap, wp, sp, cp, rows.m, k, n, rows.stride, ldw, ws.ptr, ws.bytes, ws.stream);
         }
-        return finish("hidet_symmetric_quant_matmul_f16_i8", THPVariable_Wrap(std::move(c)));
+        const char *name = row_major ? (biased ? "hidet_symmetric_quant_matmul_f16_i8_bias" : "hidet_symmetric_quant_matmul_f16_i8")
+                                     : (biased ? "hidet_symmetric_quant_matmul_f16_i8_nk_bias" : "hidet_symmetric_quant_matmul_f16_i8_nk");
+        return finish(name, args, nargs, THPVariable_Wrap(std::move(c)));
     });
 }
 
@@ -204,7 +215,7 @@ PyObject *w4a16(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                            ws.ptr, ws.bytes, ws.stream);
         else
             lib.w4a16(a->data_ptr(), w->data_ptr(), scales->data_ptr(), c.data_ptr(), rows.m, k, n, rows.stride, int(group), dtype, 0, ws.ptr, ws.bytes, ws.stream);
-        return finish("hidet_symmetric_quant_matmul_w4a16", THPVariable_Wrap(std::move(c)));
+        return finish(biased ? "hidet_symmetric_quant_matmul_w4a16_bias" : "hidet_symmetric_quant_matmul_w4a16", args, nargs, THPVariable_Wrap(std::move(c)));
     });
 }
 
@@ -220,7 +231,7 @@ PyObject *fp8_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor codes = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
         at::Tensor scale = at::empty({1}, x->options().dtype(at::kFloat).requires_grad(false));
         lib.fp8_quantize(x->data_ptr(), codes.data_ptr(), scale.data_ptr(), x->numel(), dtype, ws.ptr, ws.bytes, ws.stream);
-        return finish("hidet_fp8_quantize_per_tensor", pair(std::move(codes), std::move(scale)));
+        return finish("hidet_fp8_quantize_per_tensor", args, nargs, pair(std::move(codes), std::move(scale)));
     });
 }
 
@@ -247,7 +258,7 @@ PyObject *matmul_f8(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor c = output(*a, n, type);
         lib.matmul_f8(a->data_ptr(), b->data_ptr(), c.data_ptr(), rows.m, n, k, rows.stride, n > 1 ? b->stride(0) : k, out, scale[0] ? scale[0]->data_ptr() : nullptr,
                       scale[1] ? scale[1]->data_ptr() : nullptr, ws.ptr, ws.bytes, ws.stream);
-        return finish("hidet_matmul_f8", THPVariable_Wrap(std::move(c)));
+        return finish("hidet_matmul_f8", args, nargs, THPVariable_Wrap(std::move(c)));
     });
 }
 
@@ -268,7 +279,7 @@ PyObject *matmul_f8_scaled(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
         if (!stream_and_workspace(*a, &ws)) return nullptr;
         at::Tensor c = output(*a, n, type);
         lib.matmul_f8_scaled(a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), c.data_ptr(), m, n, k, out, ws.ptr, ws.bytes, ws.stream);
-        return finish("hidet_matmul_f8_scaled", THPVariable_Wrap(std::move(c)));
+        return finish("hidet_matmul_f8_scaled", args, nargs, THPVariable_Wrap(std::move(c)));
     });
 }
 
@@ -311,7 +322,7 @@ PyObject *quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor scale = at::empty(kept, w->options().requires_grad(false));
         lib.quantize(w->data_ptr(), codes.data_ptr(), scale.data_ptr(), v.outer, v.reduce, v.inner, dtype, type == at::kChar ? HIDET_QMM_I8 : HIDET_QMM_I16, ws.ptr,
                      ws.bytes, ws.stream);
-        return finish("hidet_symmetric_quantize", pair(std::move(codes), std::move(scale)));
+        return finish("hidet_symmetric_quantize", args, nargs, pair(std::move(codes), std::move(scale)));
     });
 }
 
@@ -330,7 +341,7 @@ PyObject *dequantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor w = at::empty(q->sizes(), scale->options().requires_grad(false));
         lib.dequantize(q->data_ptr(), scale->data_ptr(), w.data_ptr(), v.outer, v.reduce, v.inner, q->scalar_type() == at::kChar ? HIDET_QMM_I8 : HIDET_QMM_I16, dtype,
                        c10::hip::getCurrentHIPStream(q->get_device()).stream());
-        return finish("hidet_symmetric_dequantize", THPVariable_Wrap(std::move(w)));
+        return finish("hidet_symmetric_dequantize", args, nargs, THPVariable_Wrap(std::move(w)));
     });
 }
 
@@ -347,7 +358,7 @@ PyObject *quantize_int4(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor scales = at::empty({k / group, n}, w->options().dtype(type).requires_grad(false));
         lib.quantize_int4(w->data_ptr(), packed.data_ptr(), scales.data_ptr(), k, n, int(group), HIDET_QMM_F32, type == at::kHalf ? HIDET_QMM_F16 : HIDET_QMM_BF16,
                           c10::hip::getCurrentHIPStream(w->get_device()).stream());
-        return finish("hidet_group_quantize_int4", pair(std::move(packed), std::move(scales)));
+        return finish("hidet_group_quantize_int4", args, nargs, pair(std::move(packed), std::move(scales)));
     });
 }
 
@@ -368,17 +379,17 @@ PyObject *w4a16_decode(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         at::Tensor c = output(*a, n, a->scalar_type());
         lib.w4a16_nk(a->data_ptr(), w->data_ptr(), scales->data_ptr(), c.data_ptr(), rows.m, k, n, rows.stride, k / 2, int(group),
                      a->scalar_type() == at::kHalf ? HIDET_QMM_F16 : HIDET_QMM_BF16, c10::hip::getCurrentHIPStream(a->get_device()).stream());
-        return finish("hidet_symmetric_quant_matmul_w4a16_nk", THPVariable_Wrap(std::move(c)));
+        return finish("hidet_symmetric_quant_matmul_w4a16_nk", args, nargs, THPVariable_Wrap(std::move(c)));
     });
 }
 
-// dict of entry point addresses, workspaces, workspace function, exception class
+// dict of entry point addresses, workspaces, workspace function, function that makes exceptions
 PyObject *bind(PyObject *, PyObject *args) {
     PyObject *addresses;
-    if (!PyArg_ParseTuple(args, "O!O!OO", &PyDict_Type, &addresses, &PyDict_Type, &workspaces, &new_workspace, &backend_error)) return nullptr;
+    if (!PyArg_ParseTuple(args, "O!O!OO", &PyDict_Type, &addresses, &PyDict_Type, &workspaces, &new_workspace, &failure)) return nullptr;
     Py_INCREF(workspaces);
     Py_INCREF(new_workspace);
-    Py_INCREF(backend_error);
+    Py_INCREF(failure);
     auto get = [&](auto &slot, const char *name) {
         PyObject *v = PyDict_GetItemString(addresses, name);
         void *p = v != nullptr ? PyLong_AsVoidPtr(v) : nullptr;

@@ -102,6 +102,12 @@ def _describe(arg) -> str:
     return str(arg)
 
 
+def failure(name: str, args, status: str) -> BackendException:
+    """The exception for the error `status` that entry point `name` reported."""
+    return BackendException('Calling {} with arguments ({}) failed. error:\n{}\nFunction @ {}'.format(
+        name, ', '.join(_describe(a) for a in args), status, LIB_PATH))
+
+
 _FUNCS: Dict[str, object] = {}
 _Tensor = torch.Tensor
 
@@ -128,8 +134,7 @@ def call(name: str, *args):
     ret = fn(*cargs)
     status = _FUNCS['hidet_get_last_error']()
     if status is not None:
-        raise BackendException('Calling {} with arguments ({}) failed. error:\n{}\nFunction @ {}'.format(
-            name, ', '.join(_describe(a) for a in args), status.decode('utf-8'), LIB_PATH))
+        raise failure(name, args, status.decode('utf-8'))
     return ret
 
 
@@ -187,6 +192,6 @@ def front():
         loader = importlib.machinery.ExtensionFileLoader('_front', FRONT_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader('_front', loader))
         loader.exec_module(module)
-        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in SIGNATURES}, _WORKSPACES, workspace, BackendException)
+        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in SIGNATURES}, _WORKSPACES, workspace, failure)
         _FRONT = module
     return _FRONT

@@ -132,3 +132,18 @@ def test_a_group_size_no_integer_type_holds():
                  lambda: quant.symmetric_quant_matmul_w4a16_decode(x, nk, s, 2 ** 70)):
         with pytest.raises((ValueError, AssertionError)):
             call()
+
+
+def test_an_error_names_the_entry_point_and_the_arguments():
+    announce('front: errors')
+    x, wq, s, b = _case(2, 256, 512)
+    nk, lib = quant.to_decode_layout(wq), ffi.load_library()
+    for w, bias, name in ((wq, None, 'i8'), (wq, b, 'i8_bias'), (nk, None, 'i8_nk'), (nk, b, 'i8_nk_bias')):
+        lib.hidet_set_last_error(b'planted')
+        with pytest.raises(BackendException) as e:
+            quant.symmetric_quant_matmul(x, w, s, bias)
+        text = str(e.value)
+        assert 'Calling hidet_symmetric_quant_matmul_f16_' + name + ' with' in text and 'planted' in text
+        assert 'shape=(2, 256), dtype=torch.float16' in text and text.endswith(ffi.LIB_PATH)
+    with pytest.raises(BackendException, match=r'shape=\(32, 64\)(.|\n)*8-byte aligned'):  # the library's own check
+        quant.symmetric_group_quantize_int4(torch.randn(32 * 64 + 1, device='cuda')[1:].view(32, 64), 32)
