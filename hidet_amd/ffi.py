@@ -10,6 +10,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 from typing import Dict, Optional, Tuple
 
 import torch
@@ -178,20 +179,32 @@ def workspace(device: torch.device, nbytes: int = 0) -> torch.Tensor:
     return ws
 
 
+class _NoFront:
+    """In the place of the native front where it cannot be loaded: it handles nothing, every operator runs its Python path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _FRONT = None
 
 
 def front():
     """The native front of the operators (csrc/torch_front.cpp), bound to the library: each of its functions does a
-    whole call or returns None, and then the Python operator's complete path has to run."""
+    whole call or returns None, and then the Python operator's complete path has to run.  That path calls the same kernels, so
+    a front that is missing or was built for another torch costs host time and no operator."""
     global _FRONT
     if _FRONT is None:
         lib = load_library()
-        if not os.path.exists(FRONT_PATH):
-            raise OSError('{} not found: build it with `python -m hidet_amd.build`'.format(FRONT_PATH))
-        loader = importlib.machinery.ExtensionFileLoader('_front', FRONT_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader('_front', loader))
-        loader.exec_module(module)
+        try:
+            loader = importlib.machinery.ExtensionFileLoader('_front', FRONT_PATH)
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader('_front', loader))
+            loader.exec_module(module)
+        except ImportError as e:  # (a file that is missing is one too)
+            warnings.warn('{} cannot be loaded ({}): the operators take their Python path, with about 10 us more host time per '
+                          'call; build it with `python -m hidet_amd.build`'.format(FRONT_PATH, e), RuntimeWarning, stacklevel=2)
+            _FRONT = _NoFront()
+            return _FRONT
         module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in SIGNATURES}, _WORKSPACES, workspace, failure)
         _FRONT = module
     return _FRONT
