@@ -88,8 +88,15 @@ TimingSlot &timing_slot();
 // true while this thread's last-error string has not been read (it stays set)
 bool error_pending();
 
+// Along an axis a launch has fewer than 2^32 threads: of a larger grid the runtime runs the remainder, without an error.
+inline void check_grid(const dim3 &grid, const dim3 &block) {
+    QMM_CHECK(((uint64_t(grid.x) * block.x | uint64_t(grid.y) * block.y | uint64_t(grid.z) * block.z) >> 32) == 0,
+              "tensor too large for one launch: " << grid.x << " x " << grid.y << " x " << grid.z << " workgroups of " << block.x << " threads");
+}
+
 template <typename... KArgs, typename... Args>
 inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t shmem, hipStream_t stream, Args... args) {
+    check_grid(grid, block);
     TimingSlot &ts = timing_slot();
     if (ts.start != nullptr) {
         hipEvent_t s = ts.start, e = ts.stop;
@@ -132,6 +139,7 @@ inline int device_cus() {
 // Helper kernels (fills, conversions) never consume the timing slot.
 template <typename... KArgs, typename... Args>
 inline void launch_aux(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t shmem, hipStream_t stream, Args... args) {
+    check_grid(grid, block);
     hipLaunchKernelGGL(kernel, grid, block, shmem, stream, static_cast<KArgs>(args)...);
     QMM_HIP(hipGetLastError());
 }
