@@ -175,35 +175,37 @@ __device__ __forceinline__ void load_codes_upto4(const void *p, int64_t i, int64
     }
 }
 
-// Maxima over the middle axis of [outer, R, inner], inner > 1 (strided reduction): kAmaxLanes row lanes x 64 column quads,
+// Maxima over the middle axis of [outer, R, inner], inner > 1 (strided reduction): 1024 / QUADS row lanes x QUADS column quads,
 // 4 rows of 16 bytes (float32) in flight per thread. Block x = column block, y = row range, z = outer: the ranges of one
 // column leave their maxima in rows of their own of `amax` [ranges, outer * inner], which the quantizing kernel takes
 // together (one atomic per range and column instead wants the array cleared by a launch of its own). Bound by memory: K = 4096,
 // N = 11008, float32 in 37 - 38 us = 4.8 TB/s, what a copy reaches (4-byte loads, 64 columns per workgroup, and the
 // clearing launch in front: 40.6 us and 2 - 5 us).
-constexpr int kAmaxLanes = 16, kAmaxRows = 4;
-template <int DT>
-__global__ __launch_bounds__(64 * kAmaxLanes) void amax_strided_kernel(const void *__restrict__ w, float *__restrict__ amax, int64_t R,
-                                                                       int64_t inner, int64_t rows_per_range, int64_t nscale) {
-    __shared__ float4_t red[kAmaxLanes][64];
-    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // a wave's row is a scalar
-    const int64_t col = int64_t(blockIdx.x) * 256 + 4 * tx;
+constexpr int kAmaxThreads = 1024, kAmaxRows = 4;
+template <int DT, int QUADS>
+__global__ __launch_bounds__(kAmaxThreads) void amax_strided_kernel(const void *__restrict__ w, float *__restrict__ amax, int64_t R,
+                                                                    int64_t inner, int64_t rows_per_range, int64_t nscale) {
+    constexpr int kLanes = kAmaxThreads / QUADS;
+    __shared__ float4_t red[kLanes][QUADS];
+    const int tx = threadIdx.x % QUADS;
+    const int ty = QUADS == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / QUADS) : threadIdx.x / QUADS;  // (64: a wave's row is a scalar)
+    const int64_t col = int64_t(blockIdx.x) * (4 * QUADS) + 4 * tx;
     const int64_t o = blockIdx.z, count = inner - col;
     const int64_t r1 = min(R, (int64_t(blockIdx.y) + 1) * rows_per_range);
     float m[4] = {0.f, 0.f, 0.f, 0.f};
     if (count > 0) {
         const int64_t base = o * R * inner;
         int64_t r = int64_t(blockIdx.y) * rows_per_range + ty;
-        for (; r + kAmaxLanes * (kAmaxRows - 1) < r1; r += kAmaxLanes * kAmaxRows) {
+        for (; r + kLanes * (kAmaxRows - 1) < r1; r += kLanes * kAmaxRows) {
             float v[kAmaxRows][4];
 #pragma unroll
-            for (int i = 0; i < kAmaxRows; ++i) load_upto4<DT>(w, base + (r + kAmaxLanes * i) * inner + col, count, v[i]);
+            for (int i = 0; i < kAmaxRows; ++i) load_upto4<DT>(w, base + (r + kLanes * i) * inner + col, count, v[i]);
 #pragma unroll
             for (int i = 0; i < kAmaxRows; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[i][e]));
         }
-        for (; r < r1; r += kAmaxLanes) {
+        for (; r < r1; r += kLanes) {
             float v[4];
             load_upto4<DT>(w, base + r * inner + col, count, v);
 #pragma unroll
@@ -212,9 +214,18 @@ __global__ __launch_bounds__(64 * kAmaxLanes) void amax_strided_kernel(const voi
     }
     red[ty][tx] = float4_t{m[0], m[1], m[2], m[3]};
     __syncthreads();
+    if constexpr (kLanes > 16) {  // 16 rows of maxima are left to the first threads
+        if (ty < 16) {
+            for (int t = ty + 16; t < kLanes; t += 16)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t][tx][e]);
+            red[ty][tx] = float4_t{m[0], m[1], m[2], m[3]};
+        }
+        __syncthreads();
+    }
     if (ty == 0 && count > 0) {
 #pragma unroll 4
-        for (int t = 1; t < kAmaxLanes; ++t)
+        for (int t = 1; t < 16; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t][tx][e]);
         store_upto4<HIDET_QMM_F32>(amax, int64_t(blockIdx.y) * nscale + o * inner + col, count, m);
@@ -222,10 +233,11 @@ __global__ __launch_bounds__(64 * kAmaxLanes) void amax_strided_kernel(const voi
 }
 
 // The same for a short innermost axis (narrow_inner, at most 256): the threads of a workgroup take consecutive elements of
-// whole rows, eight loads in flight each, so that a thread stays on one column and no lane is idle for want of columns.
+// whole rows, eight loads in flight each, so that a thread stays on one column and no lane is idle for want of columns. The
+// maxima of the ranges form a tensor [outer, ranges, inner], which a second launch of this kernel takes together.
 template <int DT>
 __global__ __launch_bounds__(256) void amax_narrow_kernel(const void *__restrict__ w, float *__restrict__ amax, int64_t R, int64_t inner_,
-                                                          int64_t rows_per_range, int64_t nscale) {
+                                                          int64_t rows_per_range) {
     __shared__ float red[256];
     const int t = threadIdx.x, inner = int(inner_), lanes = 256 / inner, span = lanes * inner;
     const int64_t o = blockIdx.z, r0 = int64_t(blockIdx.y) * rows_per_range;
@@ -250,7 +262,7 @@ __global__ __launch_bounds__(256) void amax_narrow_kernel(const void *__restrict
         if (t < step * inner && t + step * inner < span) red[t] = fmaxf(red[t], red[t + step * inner]);
         __syncthreads();
     }
-    if (t < inner) amax[int64_t(blockIdx.y) * nscale + o * inner + t] = red[t];
+    if (t < inner) amax[(o * gridDim.y + blockIdx.y) * inner + t] = red[t];
 }
 
 // amax over the last axis of [outer, R] (inner == 1): one wave per row, 4 rows per block.
@@ -429,11 +441,11 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const void *__rest
     }
 }
 
-// [outer, R, inner] with a short innermost axis (narrow_inner), or more slices than a grid has layers: four consecutive elements
+// [outer, R, inner] with a short innermost axis, or more slices than a grid has layers: four consecutive elements
 // per thread, each with the scale of its own column. The kernels above give a column quad to a lane, so of a row of 9
 // elements (a 3 x 3 filter) they use 3 lanes in 64. Bound by memory and, where rows are no multiple of four, by the gathers of
-// the scales. float32, quad kernels -> these, us: quantize 4096 x 256 x 9 193 -> 30, 4096 x 256 x 32 155 -> 71, 2048 x 128 x 64
-// 46.4 -> 36.3; dequantize 68 -> 12, 65 -> 27, 20.6 -> 15.6.
+// the scales. float32, element-wise kernels on 64-bit indexes -> these, us: quantize 4096 x 256 x 9 40.6 -> 28.7, 1000000 x 9 53 -> 30,
+// 64 x 4096 x 32 49 -> 23, 1000000 x 64 202 -> 154; dequantize 19.1 -> 11.5, 19.0 -> 11.9, 11.6 -> 8.5, 64 -> 64.
 template <typename F>
 __device__ __forceinline__ void for_columns4(int64_t i, int64_t R, int64_t inner, F &&f) {  // f(e, column of the scales, row)
     int64_t row, o;
@@ -487,6 +499,16 @@ __global__ __launch_bounds__(256) void dequantize_flat_kernel(const void *__rest
     const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4, count = total - i;
     if (count <= 0) return;
     float code[4], s[4], out[4];
+    if (ST == HIDET_QMM_F32 && inner % 4 == 0) {  // whole quads: no branch between the two loads
+        load_codes_upto4<QT>(q, i, 4, code);
+        for_columns4(i, R, inner, [&](int e, int64_t column, int64_t) {
+            if (e == 0) load_upto4<ST>(scale, column, 4, s);
+        });
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = round_to<ST>(code[e] * s[e]);
+        store_upto4<ST>(w, i, 4, out);
+        return;
+    }
     load_codes_upto4<QT>(q, i, count, code);
     load_columns4<ST>(scale, i, count, R, inner, s);
 #pragma unroll
@@ -685,7 +707,7 @@ __device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, fl
 
 // Small tensors (the activations of a decode step), up to 65536 elements, in one launch: a workgroup of 1024 threads looks at
 // the whole tensor for its maximum and converts 4096 elements of it. One workgroup that converted all of it was bound by its
-// vector ALU (65536 elements 17 us, the two launches of larger tensors 7 us); looking at everything 16 times costs little
+// vector ALU (bfloat16, 65536 elements 10.5 us, the two launches of larger tensors 7); looking at everything 16 times costs little
 // beside that. Same arithmetic as fp8_quantize_kernel.
 template <int DT>
 __global__ __launch_bounds__(1024) void fp8_quantize_small_kernel(const void *__restrict__ x, uint32_t *__restrict__ codes,
@@ -761,9 +783,14 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restric
     }
 }
 
-// Rows of which the column-quad kernels would use less than three eighths of a wave's lanes: at 64 the flat kernels are the
-// faster ones for every type, at 96 float32 quantizes slower in them (2048 x 128 x 96 48.5 -> 52.5 us, bfloat16 52.0 -> 46.4).
+// Rows of which the quantizing column-quad kernel would use less than three eighths of a wave's lanes: at 64 the flat kernel is the
+// faster one for every type, at 96 float32 quantizes slower in it (2048 x 128 x 96 48.5 -> 52.5 us, bfloat16 52.0 -> 46.4).
 inline bool narrow_inner(int64_t inner) { return inner < 96; }
+constexpr int64_t kNarrowGroups = 1024;
+
+// Elements of a workgroup's share of the maxima from which more than kMaxRanges row ranges pay for the launch that puts them
+// together (float32, kMaxRanges -> more: 16384 x 128, 32768 elements, 12.0 -> 13.2 us; 65536 x 128, 131072 elements, 30.4 -> 20.6).
+constexpr int64_t kCombineFrom = 65536;
 
 // The quantizer's launches for [outer, reduce, inner], no extent zero, outer at most quantize_slices_most(reduce, inner).
 template <int DT>
@@ -791,19 +818,42 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
     }
     const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kQuantRows);
     QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
-    // enough row ranges for two workgroups per CU, of 64 rows at least, and as many as the scratch memory holds maxima of
-    int64_t ranges = std::min(512 / std::min<int64_t>(512, col_blocks * outer), cdiv(reduce, 64));
-    ranges = std::max<int64_t>(1, std::min<int64_t>({ranges, kMaxRanges, scratch_bytes / (nscale * 4)}));
-    const int64_t rows_per_range = cdiv(reduce, ranges);
-    if (narrow_inner(inner))
-        launch(amax_narrow_kernel<DT>, dim3(1, uint32_t(ranges), uint32_t(outer)), dim3(256), 0, stream, w, amax, reduce, inner, rows_per_range, nscale);
-    else
-        launch(amax_strided_kernel<DT>, dim3(uint32_t(col_blocks), uint32_t(ranges), uint32_t(outer)), dim3(64 * kAmaxLanes), 0, stream, w, amax, reduce, inner,
-               rows_per_range, nscale);
-    if (narrow_inner(inner) && ranges == 1 && cdiv(total, 1024) < (int64_t(1) << 24)) {
-        go(quantize_flat_kernel<DT, HIDET_QMM_I8>, quantize_flat_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(cdiv(total, 1024))), 256, w, amax, wq, scale, reduce,
-           inner, total);
+    const int64_t spare = scratch_bytes / (nscale * 4) - 1;  // rows of maxima the scratch memory holds beside the final ones
+    float *partials = amax + nscale;
+    if (narrow_inner(inner)) {
+        // Four workgroups per CU, of 2048 elements at least (1000000 x 9, float32: 32 workgroups and the column-quad kernel 216 us, these
+        // and the flat one 30).
+        int64_t ranges = std::min<int64_t>({kNarrowGroups / std::min<int64_t>(kNarrowGroups, outer), reduce * inner / 2048, spare});
+        const int64_t rows_per_range = cdiv(reduce, std::max<int64_t>(1, ranges));
+        ranges = cdiv(reduce, rows_per_range);
+        launch(amax_narrow_kernel<DT>, dim3(1, uint32_t(ranges), uint32_t(outer)), dim3(256), 0, stream, w, ranges > 1 ? partials : amax, reduce, inner, rows_per_range);
+        if (ranges > 1) launch(amax_narrow_kernel<HIDET_QMM_F32>, dim3(1, 1, uint32_t(outer)), dim3(256), 0, stream, partials, amax, ranges, inner, ranges);
+        if (cdiv(total, 1024) < (int64_t(1) << 24)) {
+            go(quantize_flat_kernel<DT, HIDET_QMM_I8>, quantize_flat_kernel<DT, HIDET_QMM_I16>, dim3(uint32_t(cdiv(total, 1024))), 256, w, amax, wq, scale, reduce,
+               inner, total);
+            return;
+        }
+        go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
+           dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, 1, nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
         return;
+    }
+    // Workgroups of 256 columns where kMaxRanges row ranges of them are two workgroups per CU, else of 64 (float32, 256 -> 64:
+    // 16384 x 1024 42.8 -> 34.8 us, 65536 x 1024 150 -> 122, 65536 x 512 103 -> 56; bfloat16 65536 x 1024 120 -> 82). Ranges of 64 rows at
+    // least, as many as two workgroups per CU take and the scratch memory holds maxima of. Up to
+    // kMaxRanges of them are put together by the quantizing kernel; more, which a launch of its own puts together, where they
+    // take that from the maxima's time.
+    const bool wide = col_blocks * outer * kMaxRanges >= 512;
+    const int64_t amax_blocks = wide ? col_blocks : cdiv(inner, 64), groups = amax_blocks * outer;
+    int64_t ranges = std::min(512 / std::min<int64_t>(512, groups), cdiv(reduce, 64));
+    if (ranges > kMaxRanges && total / (kMaxRanges * groups) < kCombineFrom) ranges = kMaxRanges;
+    ranges = std::max<int64_t>(1, std::min(ranges, ranges > kMaxRanges ? spare : spare + 1));
+    const bool combine = ranges > kMaxRanges;
+    const dim3 grid{uint32_t(amax_blocks), uint32_t(ranges), uint32_t(outer)};
+    if (wide) launch(amax_strided_kernel<DT, 64>, grid, dim3(kAmaxThreads), 0, stream, w, combine ? partials : amax, reduce, inner, cdiv(reduce, ranges), nscale);
+    else launch(amax_strided_kernel<DT, 16>, grid, dim3(kAmaxThreads), 0, stream, w, combine ? partials : amax, reduce, inner, cdiv(reduce, ranges), nscale);
+    if (combine) {
+        launch(amax_strided_kernel<HIDET_QMM_F32, 16>, dim3(uint32_t(cdiv(nscale, 64))), dim3(kAmaxThreads), 0, stream, partials, amax, ranges, nscale, ranges, nscale);
+        ranges = 1;
     }
     go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
        dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
@@ -881,7 +931,12 @@ HIDET_API void hidet_symmetric_dequantize(const void *wq, const void *scale, voi
             else launch(dequantize_long_row_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, uint32_t(blocks));
             return;
         }
-        if (narrow_inner(inner) || outer > 65535) {
+        // The kernel that gives a column quad to a lane where nine tenths of its lanes have one and, in float32, there are workgroups
+        // for four rounds of the chip's at a time (a thread's eight rows are a chain). us, flat against that: float32 400000 x 192 76 and 77, 200000 x 384
+        // 76 and 90, 4096 x 4096 13.5 and 16.2, 250000 x 256 64 and 55, 4096 x 11008 42 and 37; bfloat16 500000 x 128 50 and 64,
+        // 200000 x 320 50 and 59, 250000 x 256 50 and 39, 4096 x 4096 13.6 and 9.6.
+        const int64_t lanes = cdiv(inner, 256) * 256, groups = cdiv(inner, 256) * cdiv(reduce, kDequantRows) * outer;
+        if (outer > 65535 || ((inner * 10 < lanes * 9 || (ST == HIDET_QMM_F32 && groups < 4096)) && cdiv(total, 1024) < (int64_t(1) << 24))) {
             QMM_CHECK(cdiv(total, 1024) < (int64_t(1) << 31), "tensor too large for one launch");
             const dim3 grid{uint32_t(cdiv(total, 1024))};
             if (q_dtype == HIDET_QMM_I8) launch(dequantize_flat_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, total);

@@ -8,7 +8,7 @@ from oracle import oracle as O
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as F8
-from gpu_util import announce, dev, host
+from gpu_util import announce, dev, fastest_ms, host
 
 pytestmark = pytest.mark.gpu
 
@@ -27,7 +27,10 @@ def _near_ties(rng, shape, axis, qmax):
 @pytest.mark.parametrize('dtype', ['float32', 'float16', 'bfloat16'])
 @pytest.mark.parametrize('shape,dim,codes', [((1, 3), 0, 'int8'), ((63, 255), 0, 'int8'), ((65, 257), 0, 'int16'), ((4100, 1026), 0, 'int8'),
                                              ((129, 6), 0, 'int8'), ((3, 2049, 130), 1, 'int8'), ((33, 16387), 1, 'int8'), ((5, 4100), 1, 'int16'),
-                                             ((520, 66, 9), 1, 'int8'), ((521, 3, 7), 1, 'int16'), ((9, 130, 63), 1, 'int8'), ((513, 5, 64), 1, 'int8'), ((513, 300, 2), 1, 'int8'), ((3, 2100, 95), 1, 'int8'), ((600, 9, 96), 1, 'int8')])
+                                             ((520, 66, 9), 1, 'int8'), ((521, 3, 7), 1, 'int16'), ((9, 130, 63), 1, 'int8'), ((513, 5, 64), 1, 'int8'), ((513, 300, 2), 1, 'int8'), ((3, 2100, 95), 1, 'int8'), ((600, 9, 96), 1, 'int8'),
+                                             # tall: many row ranges, whose maxima one more launch puts together
+                                             ((50001, 9), 0, 'int8'), ((2, 30000, 3), 1, 'int16'), ((20000, 95), 0, 'int8'), ((70001, 66), 0, 'int8'), ((70000, 130), 0, 'int8'),
+                                             ((2, 20000, 260), 1, 'int8'), ((2, 66000, 96), 1, 'int8')])
 def test_columns_and_rows_bit_exact(shape, dim, codes, dtype):
     announce('quantize edges', shape, dim, codes, dtype)
     w = _near_ties(np.random.default_rng(shape[-1]), shape, dim, 127 if codes == 'int8' else 32767)
@@ -131,3 +134,12 @@ def test_scales_of_an_empty_reduction(count, start, dtype):
     want = torch.full_like(buf, 7.0)
     want[start:start + count] = 0
     assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize('inner', [9, 64, 128])
+def test_tall_weights_cost_no_more_than_others(inner):
+    """Maxima over a long axis of a few columns keep the whole chip at work (32 workgroups took ten times as long)."""
+    announce('quantize tall', inner)
+    rows = (1 << 24) // inner
+    tall, square = torch.randn((rows, inner), device='cuda'), torch.randn((4096, 4096), device='cuda')
+    assert fastest_ms(lambda: quant.symmetric_quantize(tall, 'int8', 0)) < 3 * fastest_ms(lambda: quant.symmetric_quantize(square, 'int8', 0))
