@@ -837,12 +837,12 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
            dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, 1, nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
         return;
     }
-    // Workgroups of 256 columns where kMaxRanges row ranges of them are two workgroups per CU, else of 64 (float32, 256 -> 64:
-    // 16384 x 1024 42.8 -> 34.8 us, 65536 x 1024 150 -> 122, 65536 x 512 103 -> 56; bfloat16 65536 x 1024 120 -> 82). Ranges of 64 rows at
-    // least, as many as two workgroups per CU take and the scratch memory holds maxima of. Up to
-    // kMaxRanges of them are put together by the quantizing kernel; more, which a launch of its own puts together, where they
-    // take that from the maxima's time.
-    const bool wide = col_blocks * outer * kMaxRanges >= 512;
+    // Workgroups of 256 columns where 16 row ranges of them are two workgroups per CU, else of 64, which need a quarter of the
+    // ranges (float32, 256 -> 64: 4096 x 4096 35.3 -> 29.4 us, 16384 x 1024 42.8 -> 34.8, 65536 x 1024 150 -> 122, 65536 x 512 103 -> 56, but 16384 x 4096 106 -> 110;
+    // bfloat16 65536 x 1024 120 -> 82). Ranges of 64 rows at least, as many as two workgroups per CU take and the scratch memory holds
+    // maxima of. Up to kMaxRanges of them are put together by the quantizing kernel; more, which a launch of its own puts together,
+    // where they take that from the maxima's time.
+    const bool wide = col_blocks * outer >= 32;
     const int64_t amax_blocks = wide ? col_blocks : cdiv(inner, 64), groups = amax_blocks * outer;
     int64_t ranges = std::min(512 / std::min<int64_t>(512, groups), cdiv(reduce, 64));
     if (ranges > kMaxRanges && total / (kMaxRanges * groups) < kCombineFrom) ranges = kMaxRanges;
