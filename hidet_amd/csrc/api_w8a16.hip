@@ -25,6 +25,7 @@ using namespace qmm;
 
 namespace {
 
+constexpr int64_t kPanelK = 256;    // from this depth on panels of a padded weight beat the element-wise kernel on few rows
 constexpr int64_t kMidRows = 1024;  // above, the prefill GEMM's tiles fill the chip on every shape
 
 // ---- operands of sizes or alignments the matrix kernels do not take --------------------------------------------------
@@ -80,12 +81,11 @@ __global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p) {
     }
 }
 
-// The matmul on padded copies, in panels of columns and rows that fit the scratch memory (the GEMM; up to 16 rows go to the
-// bandwidth-bound kernel, which reads activations of any alignment, whole): the copies lie at its end, what is before them is left to the GEMM's partial tiles. False: there
+// The matmul on padded copies, in panels of columns and rows that fit the scratch memory (the GEMM; without `gemm`, for up to 16 rows,
+// the bandwidth-bound kernel, which reads activations of any alignment, on one panel): the copies lie at its end, what is before them is left to the GEMM's partial tiles. False: there
 // is not enough of it for a panel.
-bool w8a16_padded(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
+bool w8a16_padded(bool gemm, const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
                   int64_t lda, const Workspace &ws, hipStream_t stream) {
-    const bool gemm = m > 16;
     const int64_t kp = gemm ? cdiv(k, 64) * 64 : k;
     const bool copy_a = gemm && (kp != k || lda % 8 != 0 || !aligned(a, 16) || (m * lda + k) * 2 >= (int64_t(1) << 31) - (1 << 20));
     const int64_t room = ws.scratch_bytes / 4 * 3;  // a quarter stays for partial tiles
@@ -172,7 +172,12 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the
     // copy. Tiny matrices are left to the element-wise kernel.
     const bool skinny = skinny_w8a16_supported(w, scale, bias, k, n);
-    if (k > 0 && (!skinny || m > 32) && m * k * n > (int64_t(1) << 20) && w8a16_padded(a, w, scale, bias, c, m, k, n, lda, ws, stream)) return;
+    if (k > 0 && (!skinny || m > 32) && m * k * n > (int64_t(1) << 20)) {
+        if (m <= 16 && w8a16_padded(false, a, w, scale, bias, c, m, k, n, lda, ws, stream)) return;
+        // Up to 16 rows of a weight whose copy does not fit the scratch memory whole: panels for the GEMM (8192 x 8190, one row: 52 us,
+        // element by element 3037; 256 x 300002 60 and 101; at a depth of 64 such a weight has threads enough for the latter).
+        if ((m > 16 || k >= kPanelK) && w8a16_padded(true, a, w, scale, bias, c, m, k, n, lda, ws, stream)) return;
+    }
     skinny_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, parallel_k_parts, ws, strict_workspace, stream);
 }
 

@@ -8,7 +8,7 @@ import torch
 from oracle import oracle as O
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
-from gpu_util import announce, dev, host
+from gpu_util import announce, dev, fastest_ms, host
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +47,33 @@ def test_int8_in_panels_of_a_small_workspace(scratch):
     ws = torch.zeros(int(ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(scratch)), dtype=torch.uint8, device='cuda')
     ffi.call('hidet_symmetric_quant_matmul_f16_i8', a, w, s, c, m, k, n, k, 0, ws, ws.numel(), ffi.current_stream(a.device))
     assert np.array_equal(host(c), want)
+
+
+# up to 16 rows of a weight whose padded copy does not fit the workspace whole: panels, as for more rows
+@pytest.mark.parametrize('m,k,n,biased', [(1, 1000, 1031, False), (16, 1022, 4099, True), (3, 256, 9002, True)])
+def test_int8_decode_in_panels_of_a_small_workspace(m, k, n, biased):
+    announce('ragged int8 decode panels', m, k, n, biased)
+    a, w, s, b, want = _int8_case(m, k, n, biased)
+    ws = torch.zeros(int(ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(1 << 20)), dtype=torch.uint8, device='cuda')
+    for _ in range(2):
+        c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+        args = (a, w, s, b, c) if biased else (a, w, s, c)
+        ffi.call('hidet_symmetric_quant_matmul_f16_i8' + ('_bias' if biased else ''), *args, m, k, n, k, 0, ws, ws.numel(), ffi.current_stream(a.device))
+        assert np.array_equal(host(c), want)
+
+
+@pytest.mark.parametrize('m', [1, 16])
+def test_int8_decode_of_a_large_ragged_weight_costs_no_more_than_more_rows(m):
+    """8192 x 8190 does not fit the standing workspace: in panels it takes what 17 rows take, element by element fifty times that."""
+    announce('ragged int8 decode, large', m)
+    k, n = 8192, 8190
+    w = torch.randint(-7, 8, (k, n), device='cuda', dtype=torch.int8)
+    x = torch.randint(-3, 4, (17, k), device='cuda').half()
+    s = torch.ones(n, device='cuda', dtype=torch.float16)
+
+    want = (x.float() @ w.float()).half()
+    assert torch.equal(quant.symmetric_quant_matmul(x[:m], w, s), want[:m])
+    assert fastest_ms(lambda: quant.symmetric_quant_matmul(x[:m], w, s)) < 8 * fastest_ms(lambda: quant.symmetric_quant_matmul(x, w, s))
 
 
 @pytest.mark.parametrize('m,k,n,group', [(1, 256, 24, 128), (16, 4096, 264, 128), (3, 1024, 1032, 32), (20, 512, 520, 64)])
