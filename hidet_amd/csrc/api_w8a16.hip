@@ -17,6 +17,7 @@ bool gemm_w8a16_nk_supported(const void *a, const void *w, const void *c, int64_
 bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                       int64_t n, int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, double limit_us, const Workspace &ws, hipStream_t stream);
 double gemm_w8a16_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws);
+double gemm_w8a16_nk_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws);
 void gemm_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                           int64_t n, int64_t lda, int64_t ldw, const Workspace &ws, hipStream_t stream);
 }
@@ -155,8 +156,8 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     // Up to 16 rows one pass of the bandwidth-bound kernel serves; beyond that every 16 rows would cost another pass
     // over the weights, and the GEMMs take over: narrow tiles (gemm_mid.h) or the prefill tiles, whichever is estimated to be
-    // the faster (K=4096, N=11008, weights from HBM: narrow 14.9 / 18.8 / 24.3 / 36.6 us at M=17 / 64 / 128 / 256, prefill tiles 17.2 /
-    // 20.5 / 30.1 / 39.8; at M=512 64 against 58.5). For 9 to 16 rows the bandwidth-bound kernel is
+    // the faster (K=4096, N=11008, weights from HBM: narrow 14.6 / 18.3 / 24.1 / 34.6 us at M=17 / 64 / 128 / 256, prefill tiles 17.0 /
+    // 20.6 / 29.2 / 39.1; at M=512 64 against 57; a wide weight, 4096 x 57344: narrow 54 / 65 us at M=17 / 64, prefill tiles 46 / 52). For 9 to 16 rows the bandwidth-bound kernel is
     // ahead of the GEMM on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
     // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49).
     if (m > 16 && k > 0) {
@@ -195,11 +196,15 @@ void w8a16_nk_dispatch(const void *a, const void *w_nk, const void *scale, const
     QMM_CHECK(skinny_w8a16_nk_supported(w_nk, k, ldw),
               "K-contiguous weights need K and the row stride to be multiples of 16 and a 16-byte aligned pointer, got K=" << k
                                                                                                                          << " ldw=" << ldw);
-    // More than one pass of 16 rows: the narrow tiles reading the same layout (4096 x 4096, 49 rows: 12.3 us, the prefill tiles 21.3),
-    // beyond 64 rows the prefill tiles, where their conditions hold.
-    if (m > 16 && m <= 64 && k > 0 && mid_w8a16_launch(a, w_nk, true, scale, bias, c, m, k, n, lda, ldw, n, n, 1e29, split_workspace(workspace, workspace_bytes), stream)) return;
-    if (m > 16 && gemm_w8a16_nk_supported(a, w_nk, c, m, k, n, lda, ldw))
-        gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, split_workspace(workspace, workspace_bytes), stream);
+    // More than one pass of 16 rows: up to 64 the narrow tiles reading the same layout (4096 x 4096, 49 rows: 12.3 us, the prefill
+    // tiles 19.9) unless they are estimated to take longer, which they do on very wide weights (1024 x 131072, 33 rows: 61 us
+    // against 47; 4096 x 57344, 64 rows: 84 against 78); else the prefill tiles, where their conditions hold.
+    const Workspace ws = split_workspace(workspace, workspace_bytes);
+    const bool gemm = m > 16 && gemm_w8a16_nk_supported(a, w_nk, c, m, k, n, lda, ldw);
+    if (m > 16 && m <= 64 && k > 0 &&
+        mid_w8a16_launch(a, w_nk, true, scale, bias, c, m, k, n, lda, ldw, n, n, gemm ? gemm_w8a16_nk_estimate_us(m, k, n, ws) : 1e29, ws, stream))
+        return;
+    if (gemm) gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, ws, stream);
     else
         skinny_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, stream);
 }

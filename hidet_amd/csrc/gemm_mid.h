@@ -399,13 +399,16 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 // What a launch costs in microseconds: the workgroups of a CU one after the other, each with its fixed part, its rounds of
 // the groups and, where K is cut, the exchange of `parts` partial tiles. The coefficients come from K = 4096 and 11008, N = 4096
 // and 11008, 17 to 400 rows, 1 to 8 pieces, and give those times to about 15 %.
+// `full_round` (0: not known) is the least a round takes with every CU at work: the weights of a round then come at the
+// rate of the memory.
 struct MidCost {
-    double fixed, round, exchange, exchange_part;
+    double fixed, round, exchange, exchange_part, full_round;
 };
 
 struct MidChoice {
     int64_t parts = 0, share = 0;
     double us = 1e30;
+    double busy_us = 1e30;  // the same with full_round, for the comparison with another kernel
 };
 // The K split of the smallest cost. Without a workspace (or too little of it) the tiles are computed whole.
 template <class Op, int RB, int DEPTH>
@@ -418,8 +421,13 @@ MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_
     MidChoice best;
     for (int64_t p = 1; p <= std::max<int64_t>(1, most); ++p) {
         const int64_t rounds = cdiv(cdiv(stages, p), Cfg::kGroups), share = rounds * Cfg::kGroups, parts = cdiv(stages, share);
-        const double us = double(cdiv(tiles * parts, cus)) * (cost.fixed + double(rounds) * cost.round + (parts > 1 ? cost.exchange + double(parts) * cost.exchange_part : 0.0));
-        if (us < best.us) best = MidChoice{parts, share, us};
+        const double rest = cost.fixed + (parts > 1 ? cost.exchange + double(parts) * cost.exchange_part : 0.0);
+        const double us = double(cdiv(tiles * parts, cus)) * (rest + double(rounds) * cost.round);
+        if (us >= best.us) continue;
+        const auto batch = [&](int64_t active) {  // workgroups side by side
+            return active == 0 ? 0.0 : rest + double(rounds) * std::max(cost.round, cost.full_round * double(active) / double(cus));
+        };
+        best = MidChoice{parts, share, us, double(tiles * parts / cus) * batch(cus) + batch(tiles * parts % cus)};
     }
     return best;
 }

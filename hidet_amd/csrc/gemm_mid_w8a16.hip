@@ -201,10 +201,11 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
         return true;
     }
     if ((k + 64) * n >= kMost) return false;
-    const MidChoice c2 = mid_choose<MidW8<false>, 2, 6>({5.5, 0.36, 1.4, 0.4}, ws, m, n, k), c4 = mid_choose<MidW8<false>, 4, 4>({6.0, 0.5, 1.5, 0.5}, ws, m, n, k),
-                    c8 = mid_choose<MidW8<false>, 8, 3>({6.5, 0.8, 1.8, 1.0}, ws, m, n, k);
+    constexpr double kFullRound = 0.62;  // 256 pieces of 16 KiB at 6.8 TB/s
+    const MidChoice c2 = mid_choose<MidW8<false>, 2, 6>({5.5, 0.36, 1.4, 0.4, kFullRound}, ws, m, n, k), c4 = mid_choose<MidW8<false>, 4, 4>({6.0, 0.5, 1.5, 0.5, kFullRound}, ws, m, n, k),
+                    c8 = mid_choose<MidW8<false>, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
     const double us = std::min({c2.us, c4.us, c8.us});
-    if (us > limit_us) return false;
+    if ((us == c2.us ? c2 : us == c4.us ? c4 : c8).busy_us > limit_us) return false;
     if (us == c2.us) mid_launch<MidW8<false>, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
     else if (us == c4.us) mid_launch<MidW8<false>, 4, 4>(c4, a, w, las, n, args, m, n, k, ws, stream);
     else mid_launch<MidW8<false>, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);

@@ -19,7 +19,8 @@
 // ahead into the registers they were just dequantised from.  The activation tile goes global -> LDS
 // directly (buffer_load ... lds, no registers) into a three-slot ring of 16-byte chunks XOR-swizzled by
 // row (the swizzle is applied on the global side), two stages ahead; one barrier per 64 k.  The per-column
-// scale is applied to the fp32 accumulators in the epilogue.
+// scale is applied to the fp32 accumulators in the epilogue.  Matrices of at most 96 rows run the same tile with the
+// row blocks that cannot hold a row left out at compile time (template parameter RBA).
 #include "common.h"
 #include "gemm_tiling.h"
 
@@ -38,9 +39,11 @@ struct GemmW8Cfg16 {
     static constexpr int kLdsBytes = kRingBytes + 16;  // + the fix-up's flag; the ring must start at LDS address 0
 };
 
+// RBA <= RB: row blocks (of 16 rows) per wave that can hold rows of the matrix. A short matrix (M <= 16 RBA) runs the same
+// tile with the activation loads, fragment reads and MFMAs of the other row blocks left out.
 // W_NK: the weight is stored K-contiguous, w[col * ldw + k] (the [N, K] storage of nn.Linear); a lane then loads the 8
 // consecutive k of one of its 4 columns with one 8-byte load and widens byte pairs instead of gathering rows.
-template <int RB, int WM, int WN, int MIN_BLOCKS, bool W_NK = false>
+template <int RB, int WM, int WN, int MIN_BLOCKS, int RBA, bool W_NK = false>
 __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(const _Float16 *__restrict__ a, int64_t lda,
                                                                                  const int8_t *__restrict__ w, int64_t ldw,
                                                                                  const _Float16 *__restrict__ scale,
@@ -108,10 +111,12 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
     };
     BFrag bq[2][4];
 
-    static_assert(WM == 1, "a wave has all rows of the tile");
+    // instruction j brings tile rows j * kThreads / 8 ..: only those below 16 RBA are needed
+    static_assert(WM == 1 && (RBA * 16 * 8) % Cfg::kThreads == 0, "whole load instructions per active row range");
+    constexpr int kAChunksActive = RBA * 16 * 8 / Cfg::kThreads;
     auto load_a = [&](int st, int slot) {
 #pragma unroll
-        for (int j = 0; j < Cfg::kAChunks; ++j)
+        for (int j = 0; j < kAChunksActive; ++j)
             buffer_load_to_lds_b128(rsrc_a, lds + slot * Cfg::kBM * 8 + j * Cfg::kThreads + wave * 64, a_off[j],
                                     (st < stages ? st : stages - 1) * (kBK * 2));  // the scalar offset is not range-checked
     };
@@ -167,11 +172,11 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
         const uint32_t slot_off = uint32_t(slot * Cfg::kBM * 128);
         const uint32_t addr0 = af_addr[0] + slot_off, addr1 = af_addr[1] + slot_off;
         // A fragments are read from LDS three fragments (12 MFMAs) ahead of their use, through a ring of four
-        // (fragment index = k-step * RB + row block)
+        // (fragment index = k-step * RBA + row block, over the active row blocks only)
         int4v_t af[4];
         auto issue = [&](auto idx_tag) {
             constexpr int IDX = decltype(idx_tag)::value;
-            if constexpr (IDX < 2 * RB) af[IDX & 3] = lds_read_b128_early<(IDX % RB) * 2048>(IDX / RB ? addr1 : addr0);
+            if constexpr (IDX < 2 * RBA) af[IDX & 3] = lds_read_b128_early<(IDX % RBA) * 2048>(IDX / RBA ? addr1 : addr0);
         };
         issue(std::integral_constant<int, 0>());
         issue(std::integral_constant<int, 1>());
@@ -181,8 +186,8 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
         auto block = [&](auto idx_tag) {
             constexpr int IDX = decltype(idx_tag)::value;
             constexpr int Q = IDX / RB, RBI = IDX % RB;
-            constexpr int AI = Q * RB + RBI;  // fragment index
-            issue(std::integral_constant<int, AI + 3>());
+            constexpr int AI = Q * RBA + RBI;  // fragment index, if the row block is active
+            if constexpr (RBI < RBA) issue(std::integral_constant<int, AI + 3>());
             if constexpr (W_NK) {
                 constexpr int T = RBI / 2;  // column of the next k-step's block; this block widens one of its two dwords
                 const uint32_t src = w_raw[Q ^ 1][2 * T + (RBI & 1)];
@@ -220,8 +225,8 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
                     w_raw[Q ^ 1][2 * P + 1] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_w, w_off[2 * P + 1], soff, 0);
                 }
             }
-            {
-                constexpr int NEWER = (2 * RB - 1 - AI) < 3 ? (2 * RB - 1 - AI) : 3;
+            if constexpr (RBI < RBA) {
+                constexpr int NEWER = (2 * RBA - 1 - AI) < 3 ? (2 * RBA - 1 - AI) : 3;
                 lds_wait_keep_newer<NEWER>(af[AI & 3]);
                 const half8_t afrag = __builtin_bit_cast(half8_t, af[AI & 3]);
 #pragma unroll
@@ -245,8 +250,8 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
         kstep(std::integral_constant<int, 0>());
         kstep(std::integral_constant<int, 1>());
         // the loads of stage s + 1 (issued one stage ago) must have landed in LDS before anyone reads them; the
-        // loads issued during this stage (Cfg::kAChunks + kWLoadsPerStage of them) may stay in flight
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(Cfg::kAChunks + kWLoadsPerStage));
+        // loads issued during this stage (kAChunksActive + kWLoadsPerStage of them) may stay in flight
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kAChunksActive + kWLoadsPerStage));
         __syncthreads();
     };
 
@@ -270,8 +275,9 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
     if (parts > 1) {
         uint32_t rows_valid = 0;  // row blocks of this wave that reach into the matrix
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) rows_valid |= uint32_t(m0 + (wm * RB + rb) * 16 < m) << rb;
-        if (!gemm_k_split_fixup<Cfg::kThreads>(acc, item, partials, counters, &s_last,
+        for (int rb = 0; rb < RBA; ++rb) rows_valid |= uint32_t(m0 + (wm * RB + rb) * 16 < m) << rb;
+        // only the active row blocks take part (every workgroup of a launch has the same RBA)
+        if (!gemm_k_split_fixup<Cfg::kThreads>(reinterpret_cast<float4_t(&)[RBA][4]>(acc), item, partials, counters, &s_last,
                                                rows_valid))
             return;
     }
@@ -286,7 +292,7 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
             bs[t] = bias != nullptr ? float(bias[col + t]) : -0.0f;
         }
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RBA; ++rb)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int row = m0 + (wm * RB + rb) * 16 + kg * 4 + v;
@@ -305,7 +311,7 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
         if (col + t >= n_out) break;
         const float sc = float(scale[col + t]), bs = bias != nullptr ? float(bias[col + t]) : -0.0f;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RBA; ++rb)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int row = m0 + (wm * RB + rb) * 16 + kg * 4 + v;
@@ -319,11 +325,12 @@ __global__ __launch_bounds__(WM * WN * 64, MIN_BLOCKS) void gemm_w8a16_kernel16(
 // per CU. The tiles past a whole number of such rounds share their CUs with another workgroup or run in a round of their own;
 // cut into K ranges they finish sooner when they are few (K = 4096, N = 11008: M = 768 / 896 / 1024: 96 / 94.5 / 96 -> 88 / 84 /
 // 91.5 us, M = 1536 / 1792: 149.5 / 153 -> 133 / 140 us; up to 8 ranges instead of 4: no further gain).
-template <class Cfg, int CONCURRENT>
+// (Light workgroups, of at most 4 active row blocks, are worth up to 8 ranges: measured.)
+template <class Cfg, int CONCURRENT, int RBA>
 GemmTail tail_of(const GemmTiling &tiling, int64_t k, const Workspace &ws, int *split_unit) {
-    GemmTail tail = make_gemm_tail(tiling, CONCURRENT, 32, 4);
+    GemmTail tail = make_gemm_tail(tiling, CONCURRENT, 32, RBA <= 4 ? 8 : 4);
     *split_unit = CONCURRENT;
-    if (tail.parts == 1) {
+    if (RBA == 8 && tail.parts == 1) {
         tail = make_gemm_tail_by_rounds(tiling, 32, 4, 0.00085 * 4096.0 / double(k));
         *split_unit = 32;
     }
@@ -333,7 +340,7 @@ GemmTail tail_of(const GemmTiling &tiling, int64_t k, const Workspace &ws, int *
     return tail;
 }
 
-template <int RB, int WM, int WN, int MIN_BLOCKS, bool W_NK = false>
+template <int RB, int WM, int WN, int MIN_BLOCKS, int RBA, bool W_NK = false>
 void launch_cfg16(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
                   int64_t lda, int64_t ldw, int64_t n_out, int64_t ldc, const Workspace &ws, hipStream_t stream) {
     using Cfg = GemmW8Cfg16<RB, WM, WN>;
@@ -341,15 +348,31 @@ void launch_cfg16(const void *a, const void *w, const void *scale, const void *b
     constexpr int kConcurrent = 32 * MIN_BLOCKS;  // workgroups an XCD (32 CUs) runs at a time
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, kConcurrent);
     int split_unit;
-    const GemmTail tail = tail_of<Cfg, kConcurrent>(tiling, k, ws, &split_unit);
+    const GemmTail tail = tail_of<Cfg, kConcurrent, RBA>(tiling, k, ws, &split_unit);
     static_assert(8 * kConcurrent * 4 <= kCounterBytes, "one counter per tail tile");
     const int64_t grid = gemm_grid_with_tail(tiling, split_unit, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
-    allow_dynamic_lds(reinterpret_cast<const void *>(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, W_NK>), Cfg::kLdsBytes);
-    launch(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, W_NK>, dim3(uint32_t(grid)), dim3(Cfg::kThreads), size_t(Cfg::kLdsBytes), stream,
+    allow_dynamic_lds(reinterpret_cast<const void *>(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, RBA, W_NK>), Cfg::kLdsBytes);
+    launch(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, RBA, W_NK>, dim3(uint32_t(grid)), dim3(Cfg::kThreads), size_t(Cfg::kLdsBytes), stream,
            static_cast<const _Float16 *>(a), lda, static_cast<const int8_t *>(w), ldw, static_cast<const _Float16 *>(scale),
            static_cast<const _Float16 *>(bias), static_cast<_Float16 *>(c), int(m), int(k), int(n), tiles_m, tiles_n, tiling.xm, tiling.xn, split_unit, tail.parts, tail.max_tiles,
            reinterpret_cast<float *>(ws.scratch), ws.counters, int(n_out), int(ldc));
+}
+
+// Time of a launch with a number of active row blocks: `stage` microseconds per stage and round of one workgroup per CU, a fixed part
+// and what an exchange of K ranges costs. Tiles past a whole number of rounds that are not cut share their CUs with others,
+// which hides some of their time where a workgroup is bound by its MFMAs.
+template <int RBA>
+double estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws, double stage) {
+    using Cfg = GemmW8Cfg16<8, 1, 4>;
+    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, Cfg::kBM)), int(cdiv(n, Cfg::kBN)), 64);
+    int unit;
+    const GemmTail tail = tail_of<Cfg, 64, RBA>(tiling, k, ws, &unit);
+    const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
+    double rounds = whole;
+    if (rest > 0 && (tail.parts > 1 || whole == 0)) rounds += double((rest * tail.parts + 31) / 32) / tail.parts;
+    else if (rest > 0) rounds = RBA < 8 ? whole + 1.0 : std::max(whole + 0.62, tiling.region_tiles / 32.0 * 0.69);
+    return 8.0 + rounds * stage * double(k) / kBK + (tail.parts > 1 ? 6.1 + 0.85 * tail.parts : 0.0);
 }
 
 }  // namespace
@@ -361,22 +384,29 @@ bool gemm_w8a16_supported(const void *a, const void *w, const void *c, int64_t m
            k * n < (int64_t(1) << 31) - (1 << 20) && (m * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20);
 }
 
-// Estimated time in microseconds (to about 15 %), for the choice between this kernel and the narrow tiles of gemm_mid.h:
-// a fixed part, 0.77 us per stage and round of one workgroup per CU, and what an exchange of K ranges costs.
+// Estimated time in microseconds, for the choice between this kernel and the narrow tiles of gemm_mid.h, with which it was
+// fitted to 17 layers of 15 to 235 MB at 16 row counts from 17 to 512 (the narrow tiles' estimate, with their memory rate, against
+// 0.85 of this one: the slower kernel is taken in 5 of those 304 cases, by 3 to 8 %).
 double gemm_w8a16_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws) {
-    using Cfg = GemmW8Cfg16<8, 1, 4>;
-    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, Cfg::kBM)), int(cdiv(n, Cfg::kBN)), 64);
-    int unit;
-    const GemmTail tail = tail_of<Cfg, 64>(tiling, k, ws, &unit);
-    const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
-    const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);
-    return 8.0 + rounds * 0.77 * double(k) / kBK + (tail.parts > 1 ? 5.0 + 0.8 * tail.parts : 0.0);
+    if (m <= 32) return 0.85 * estimate_us<2>(m, k, n, ws, 0.36);
+    if (m <= 64) return 0.85 * estimate_us<4>(m, k, n, ws, 0.456);
+    if (m <= 96) return 0.85 * estimate_us<6>(m, k, n, ws, 0.544);
+    return 0.85 * estimate_us<8>(m, k, n, ws, 0.814);
+}
+// The same for the weight stored K-contiguous, up to 64 rows: a stage takes the same whatever the rows, as long as its loads
+// of 32 bytes per column take.
+double gemm_w8a16_nk_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws) {
+    return m <= 32 ? estimate_us<2>(m, k, n, ws, 1.04) : estimate_us<4>(m, k, n, ws, 1.04);
 }
 
 // `n_out` <= n columns of the result are written, at a row stride of ldc.
 void gemm_w8a16_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                        int64_t n, int64_t lda, int64_t n_out, int64_t ldc, const Workspace &ws, hipStream_t stream) {
-    launch_cfg16<8, 1, 4, 2>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);  // waves 128 x 64, workgroup tile 128 x 256
+    // waves 128 x 64, workgroup tile 128 x 256; a matrix of at most 32 / 64 / 96 rows leaves the empty row blocks out
+    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
+    else launch_cfg16<8, 1, 4, 2, 8>(a, w, scale, bias, c, m, k, n, lda, n, n_out, ldc, ws, stream);
 }
 
 // The same kernel on a weight stored K-contiguous (w_nk[col * ldw + k]): 8-byte loads, so rows of w_nk 8-byte aligned.
@@ -389,7 +419,10 @@ bool gemm_w8a16_nk_supported(const void *a, const void *w, const void *c, int64_
 
 void gemm_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                           int64_t n, int64_t lda, int64_t ldw, const Workspace &ws, hipStream_t stream) {
-    launch_cfg16<8, 1, 4, 2, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    if (m <= 32) launch_cfg16<8, 1, 4, 2, 2, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else if (m <= 64) launch_cfg16<8, 1, 4, 2, 4, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else if (m <= 96) launch_cfg16<8, 1, 4, 2, 6, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
+    else launch_cfg16<8, 1, 4, 2, 8, true>(a, w, scale, bias, c, m, k, n, lda, ldw, n, n, ws, stream);
 }
 
 }  // namespace qmm

@@ -5,8 +5,10 @@ only rounding is that of the result: the expected values are computed in float64
 import pytest
 import torch
 
+from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as f8
+from gpu_util import announce
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +111,26 @@ def test_w4a16_infinite_and_large_activations():
     packed, scales, w = _int4(g, k, n, 128, torch.bfloat16)
     want = (x.double() @ w).to(torch.bfloat16)  # row 3: infinities, NaN where the code is zero
     assert torch.equal(quant.symmetric_quant_matmul_w4a16(x, packed, scales, 128).nan_to_num(nan=-1.0), want.nan_to_num(nan=-1.0))
+
+
+# a weight so wide that the tall tiles fill the chip: short matrices leave their empty row blocks out (one, two, three of four
+# pairs of blocks at work), rows at both edges of each form, a last tile of 8 columns
+@pytest.mark.parametrize('m', [17, 32, 33, 64, 65, 96, 97])
+@pytest.mark.parametrize('nk', [False, True])
+def test_w8a16_few_rows_of_a_wide_weight(m, nk):
+    announce('wide w8a16', m, nk)
+    k, n = 320, 131080
+    g = torch.Generator(device='cuda').manual_seed(m)
+    a = torch.randint(-3, 4, (m, k), generator=g, device='cuda').half()
+    w = torch.randint(-7, 8, (k, n), generator=g, device='cuda', dtype=torch.int8)
+    s = 2.0 ** torch.randint(-3, 1, (n,), generator=g, device='cuda').half()
+    b = torch.randint(-8, 9, (n,), generator=g, device='cuda').half()
+    want = ((a.float() @ w.float()) * s.float()).half()  # small integers: every sum and product is exact
+    c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+    ws = ffi.workspace(a.device)
+    weight = w.t().contiguous() if nk else w
+    for bias in (None, b):
+        name = 'hidet_symmetric_quant_matmul_f16_i8' + ('_nk' if nk else '') + ('_bias' if bias is not None else '')
+        operands = (a, weight, s) + ((bias,) if bias is not None else ()) + (c,)
+        ffi.call(name, *operands, m, k, n, k, k if nk else 0, ws, ws.numel(), ffi.current_stream(a.device))
+        assert torch.equal(c, want if bias is None else (want.float() + b.float()).half())
