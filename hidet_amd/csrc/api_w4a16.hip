@@ -14,7 +14,7 @@ void skinny_w4a16_nk_launch(const void *a, const void *w, const void *scales, vo
                             int64_t lda, int64_t ldw, int group, int dtype, hipStream_t stream);
 bool mid_w4a16_launch(const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                       int group, int dtype, double limit_us, void *workspace, int64_t workspace_bytes, hipStream_t stream);
-double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n);
+double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n, int64_t lda, int group, bool biased, void *workspace, int64_t workspace_bytes);
 }  // namespace qmm
 
 using namespace qmm;
@@ -79,7 +79,8 @@ void w4a16_dispatch(const void *a, const void *w, const void *scales, const void
     // neither takes is done in passes of 16 rows.
     const bool gemm = m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size);
     if (m > 16 && m <= 1024 &&
-        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype, gemm ? gemm_w4a16_estimate_us(m, k, n) : 1e29, workspace, workspace_bytes, stream))
+        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype,
+                         gemm ? gemm_w4a16_estimate_us(m, k, n, lda, group_size, bias != nullptr, workspace, workspace_bytes) : 1e29, workspace, workspace_bytes, stream))
         return;
     if (gemm) {
         gemm_w4a16_launch(a, w, scales, c, m, k, n, lda, group_size, dtype, workspace, workspace_bytes, stream);

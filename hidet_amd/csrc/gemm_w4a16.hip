@@ -854,6 +854,27 @@ __global__ __launch_bounds__(512, 1) void gemm_w4a16_lds_kernel(
     }
 }
 
+// One part of one tile exchanged = 256 KiB through memory, about 0.05 us of the chip's bandwidth; a tile's compute
+// time is about 74 us at K = 4096 (measured: M = 512, all 172 tiles in 4 parts: 82 -> 104 us; M = 1024, 88 tail
+// tiles in 2 parts: 146 -> 121 us).
+GemmTail lds_tail_of(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
+    using Cfg = GemmW4LdsCfg;
+    GemmTail tail = make_gemm_tail_by_rounds(tiling, 32, 4, 0.0007 * 4096.0 / double(k));
+    while (tail.parts > 1 &&
+           (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
+        --tail.parts;
+    return tail;
+}
+
+// The kernels in whole 64-deep stages, for groups of whole stages and tensors of 31-bit offsets.
+bool whole_stages(int64_t m, int64_t k, int64_t n, int64_t lda, int group) {
+    return (k % kBK == 0) && (group % kBK == 0) && k * (n / 2) < (int64_t(1) << 31) - (1 << 20) && (m * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20) &&
+           (k / group) * n * 2 < (int64_t(1) << 31);
+}
+// Measured on K = 4096, N = 11008, M = 33 .. 4096: of those the kernel that widens once per workgroup (256-row tiles) is
+// ahead except where its tall tiles leave a second or third tile row mostly empty (3 or 5 tile rows of 128).
+bool tall_tiles(int64_t m, int64_t n) { return n % 32 == 0 && cdiv(m, 128) != 3 && cdiv(m, 128) != 5; }
+
 template <int DT>
 void launch_lds(const void *a, const void *w, const void *scales, void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                 int group, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -861,14 +882,8 @@ void launch_lds(const void *a, const void *w, const void *scales, void *c, int64
     const int tiles_m = int(cdiv(m, Cfg::kBM)), tiles_n = int(cdiv(n, Cfg::kBN));
     constexpr int kConcurrent = 32;
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, kConcurrent);
-    // one part of one tile exchanged = 256 KiB through memory, about 0.05 us of the chip's bandwidth; a tile's compute
-    // time is about 74 us at K = 4096 (measured: M = 512, all 172 tiles in 4 parts: 82 -> 104 us; M = 1024, 88 tail
-    // tiles in 2 parts: 146 -> 121 us)
-    GemmTail tail = make_gemm_tail_by_rounds(tiling, kConcurrent, 4, 0.0007 * 4096.0 / double(k));
     const Workspace ws = split_workspace(workspace, workspace_bytes);
-    while (tail.parts > 1 &&
-           (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
-        --tail.parts;
+    const GemmTail tail = lds_tail_of(tiling, k, ws);
     const int64_t grid = gemm_grid_with_tail(tiling, kConcurrent, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
     // Runs across the tiles instead (gemm_tiling.h), one workgroup per CU, when the busiest XCD has a few tiles more than
@@ -909,22 +924,30 @@ bool gemm_w4a16_supported(const void *a, const void *w, const void *scales, cons
            aligned(scales, 16) && aligned(c, 16);
 }
 
-// Estimated time in microseconds, for the choice between these kernels and the narrow tiles of gemm_mid.h: a fixed part, 1.06 us
-// per 64-deep stage of a 256 x 256 tile, cut into K ranges while that leaves at most half the CUs busy, and the exchange of
-// those. On the low side where the tiles of 128 rows or a general kernel run instead.
-double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n) {
-    const int64_t tiles = cdiv(m, 256) * cdiv(n, 256), parts = std::max<int64_t>(1, std::min<int64_t>(4, 128 / tiles));
-    return 8.0 + double(cdiv(tiles, 256)) * 1.06 * double(k) / 64.0 / double(parts) + (parts > 1 ? 3.0 * double(parts) : 0.0);
+// Estimated time in microseconds, for the choice between these kernels and the narrow tiles of gemm_mid.h: a fixed part, what a
+// 64-deep stage takes with so many rows in the last tile row, and the exchange of K ranges; 0.98 of that where they tie. From K = 4096 and 11008, N = 4096 and 11008, 33 to 1024
+// rows (4096 x 11008, 128 / 160 rows: narrow 34.7 / 51.5 us, these 36.5 / 43.3). Groups that are no whole stages (32, 96) run
+// on the kernel that takes any, at 0.077 us per k whatever the rows (4096 x 11008, 512 rows: 346 us, narrow 101).
+double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n, int64_t lda, int group, bool biased, void *workspace, int64_t workspace_bytes) {
+    const double bias = biased ? 4.0 + double(m * n) * 1e-6 : 0.0;  // a pass over the result
+    if (!whole_stages(m, k, n, lda, group)) return 0.98 * (5.0 + 0.077 * double(k) * double(cdiv(cdiv(m, 64) * cdiv(n, 256), 512)) + bias);
+    const double stages = double(k) / kBK;
+    if (!tall_tiles(m, n)) {
+        const int64_t tiles = cdiv(m, 128) * cdiv(n, 256), parts = std::max<int64_t>(1, std::min<int64_t>(4, 192 / tiles));
+        return 0.98 * (8.0 + double(cdiv(tiles, 512)) * (parts > 1 ? 1.3 : 0.98) * stages / double(parts) + (parts > 1 ? 2.7 * double(parts) : 0.0) + bias);
+    }
+    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, GemmW4LdsCfg::kBM)), int(cdiv(n, GemmW4LdsCfg::kBN)), 32);
+    const GemmTail tail = lds_tail_of(tiling, k, split_workspace(workspace, workspace_bytes));
+    const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
+    const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);
+    const double stage = m <= 64 ? 0.64 : m <= 128 ? 0.74 : m <= 192 ? 0.97 : 1.06;
+    return 0.98 * (8.0 + rounds * stage * stages + (tail.parts > 1 ? 2.0 * tail.parts : 0.0) + bias);
 }
 
 void gemm_w4a16_launch(const void *a, const void *w, const void *scales, void *c, int64_t m, int64_t k, int64_t n,
                        int64_t lda, int group, int dtype, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
-    const bool fast = (k % kBK == 0) && (group % kBK == 0) && k * (n / 2) < (int64_t(1) << 31) - (1 << 20) &&
-                      (m * lda + k) * 2 < (int64_t(1) << 31) - (1 << 20) && (k / group) * n * 2 < (int64_t(1) << 31);
-    // Measured on K = 4096, N = 11008, M = 33 .. 4096: the kernel that widens once per workgroup (256-row tiles) is
-    // ahead except where its tall tiles leave a second or third tile row mostly empty (3 or 5 tile rows of 128).
-    const int64_t rows128 = cdiv(m, 128);
-    if (fast && n % 32 == 0 && rows128 != 3 && rows128 != 5) {
+    const bool fast = whole_stages(m, k, n, lda, group);
+    if (fast && tall_tiles(m, n)) {
         if (dtype == HIDET_QMM_F16) launch_lds<HIDET_QMM_F16>(a, w, scales, c, m, k, n, lda, group, workspace, workspace_bytes, stream);
         else launch_lds<HIDET_QMM_BF16>(a, w, scales, c, m, k, n, lda, group, workspace, workspace_bytes, stream);
         return;

@@ -8,7 +8,7 @@ import torch
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as f8
-from gpu_util import announce
+from gpu_util import announce, fastest_ms
 
 pytestmark = pytest.mark.gpu
 
@@ -111,6 +111,24 @@ def test_w4a16_infinite_and_large_activations():
     packed, scales, w = _int4(g, k, n, 128, torch.bfloat16)
     want = (x.double() @ w).to(torch.bfloat16)  # row 3: infinities, NaN where the code is zero
     assert torch.equal(quant.symmetric_quant_matmul_w4a16(x, packed, scales, 128).nan_to_num(nan=-1.0), want.nan_to_num(nan=-1.0))
+
+
+# groups that are no whole stages of the tall tiles, from where their general kernel took over; edges of the tiles in M and N
+@pytest.mark.parametrize('m,k,n,group', [(192, 1024, 1032, 32), (257, 96, 264, 96), (513, 192, 136, 96), (1000, 256, 520, 32), (1024, 64, 8, 32)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_w4a16_small_groups_of_many_rows(m, k, n, group, dtype):
+    test_w4a16_rows_of_a_batch(m, k, n, group, dtype)
+
+
+def test_w4a16_small_groups_cost_no_more_than_large_ones():
+    """Groups of 32 run on the narrow tiles wherever those are the faster; the general kernel took four times as long."""
+    announce('w4a16 groups of 32')
+    m, k, n = 512, 4096, 11008
+    packed = torch.randint(0, 256, (k, n // 2), device='cuda', dtype=torch.uint8)
+    x = torch.randn((m, k), device='cuda').bfloat16()
+    scales = {group: torch.ones((k // group, n), device='cuda', dtype=torch.bfloat16) for group in (32, 128)}
+    small, large = (fastest_ms(lambda: quant.symmetric_quant_matmul_w4a16(x, packed, scales[group], group)) for group in (32, 128))
+    assert small < 2 * large
 
 
 # a weight so wide that the tall tiles fill the chip: short matrices leave their empty row blocks out (one, two, three of four
