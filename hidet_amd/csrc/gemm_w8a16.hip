@@ -386,7 +386,7 @@ bool gemm_w8a16_supported(const void *a, const void *w, const void *c, int64_t m
 
 // Estimated time in microseconds, for the choice between this kernel and the narrow tiles of gemm_mid.h, with which it was
 // fitted to 17 layers of 15 to 235 MB at 16 row counts from 17 to 512 (the narrow tiles' estimate, with their memory rate, against
-// 0.85 of this one: the slower kernel is taken in 5 of those 304 cases, by 3 to 8 %).
+// 0.85 of this one: the slower kernel is taken in 7 of those 272 cases, by 3 to 8 %).
 double gemm_w8a16_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws) {
     if (m <= 32) return 0.85 * estimate_us<2>(m, k, n, ws, 0.36);
     if (m <= 64) return 0.85 * estimate_us<4>(m, k, n, ws, 0.456);

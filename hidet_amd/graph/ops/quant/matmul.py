@@ -41,10 +41,10 @@ class SymmetricQuantizedMatmulTask(Task):
 
 
 _NK_MAX_ROWS = 16  # one pass of the bandwidth-bound kernels for K-contiguous weights; more rows go to the narrow-tile GEMM
-# The GEMM that reads K-contiguous weights gathers 8 bytes per lane from 16 rows of the stored matrix per load and runs
-# about a third slower than the row-major one at prefill sizes (2048 x 4096 x 11008: 214 against 157 us; 64 rows: 25 against
-# 20 us).  Batched decode (17 to 64 rows) uses it, so a model that only decodes never makes a second copy of its weights;
-# longer prompts use the row-major copy.
+# The tall-tile GEMM that reads K-contiguous weights gathers 8 bytes per lane from 16 rows of the stored matrix per load and
+# runs about a third slower than the row-major one at prefill sizes (2048 x 4096 x 11008: 214 against 157 us).  Batched decode
+# (17 to 64 rows) runs on the narrow tiles that read this layout, so a model that only decodes never makes a second copy of
+# its weights; longer prompts use the row-major copy.
 _NK_GEMM_MAX_ROWS = 64
 
 
@@ -52,7 +52,7 @@ def to_decode_layout(wq: torch.Tensor) -> torch.Tensor:
     """The same [K, N] int8 weight, stored K-contiguous (a view with strides (1, K) of a fresh [N, K] tensor).
 
     `symmetric_quant_matmul` on such a weight with up to 16 activation rows runs the kernel that
-    reduces along the contiguous axis (no exchange between workgroups), with up to 64 the MFMA GEMM that reads this layout;
+    reduces along the contiguous axis (no exchange between workgroups), with up to 64 the narrow tiles that read this layout;
     it is what `nn.Linear` stores, so `linear.weight` quantized with `dims=1` and viewed with `.t()` is already in this
     layout.  A call with more rows makes a row-major copy of the weight the first time and keeps it for as long as the
     weight tensor lives.
@@ -102,7 +102,7 @@ def run_w8a16(a: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, parall
     scale = scale.contiguous()
     c = torch.empty((m, n), dtype=torch.float16, device=a.device)
     # A [K, N] weight held K-contiguous (strides (1, ldw): `wq_nk.t()` of an [N, K] tensor, see `to_decode_layout`) goes to
-    # the entry point for that layout: the bandwidth-bound kernels up to 16 rows, the MFMA GEMM reading the same layout up
+    # the entry point for that layout: the bandwidth-bound kernels up to 16 rows, the narrow tiles reading the same layout up
     # to 64 (K a multiple of 64, N of 4).  What neither takes uses a row-major copy, as any non-contiguous operand does.
     if (k > 1 and n > 1 and weight.stride(0) == 1 and weight.stride(1) >= k and weight.stride(1) % 16 == 0
             and k % 16 == 0 and weight.data_ptr() % 16 == 0
