@@ -152,3 +152,18 @@ def test_w8a16_few_rows_of_a_wide_weight(m, nk):
         operands = (a, weight, s) + ((bias,) if bias is not None else ()) + (c,)
         ffi.call(name, *operands, m, k, n, k, k if nk else 0, ws, ws.numel(), ffi.current_stream(a.device))
         assert torch.equal(c, want if bias is None else (want.float() + b.float()).half())
+
+
+# the same forms on padded copies: rows of the result that start anywhere and end inside a lane's columns
+@pytest.mark.parametrize('m', [17, 50, 96])
+def test_w8a16_few_rows_of_a_wide_ragged_weight(m):
+    announce('wide ragged w8a16', m)
+    k, n = 322, 131078
+    g = torch.Generator(device='cuda').manual_seed(m)
+    a = torch.randint(-3, 4, (m, k), generator=g, device='cuda').half()
+    w = torch.randint(-7, 8, (k, n), generator=g, device='cuda', dtype=torch.int8)
+    s = 2.0 ** torch.randint(-3, 1, (n,), generator=g, device='cuda').half()
+    b = torch.randint(-8, 9, (n,), generator=g, device='cuda').half()
+    want = ((a.float() @ w.float()) * s.float()).half()
+    assert torch.equal(quant.symmetric_quant_matmul(a, w, s), want)
+    assert torch.equal(quant.symmetric_quant_matmul(a, w, s, b), (want.float() + b.float()).half())
