@@ -839,12 +839,14 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
     }
     // Workgroups of 256 columns where 16 row ranges of them are two workgroups per CU, else of 64, which need a quarter of the
     // ranges (float32, 256 -> 64: 4096 x 4096 35.3 -> 29.4 us, 16384 x 1024 42.8 -> 34.8, 65536 x 1024 150 -> 122, 65536 x 512 103 -> 56, but 16384 x 4096 106 -> 110;
-    // bfloat16 65536 x 1024 120 -> 82). Ranges of 64 rows at least, as many as two workgroups per CU take and the scratch memory holds
-    // maxima of. Up to kMaxRanges of them are put together by the quantizing kernel; more, which a launch of its own puts together,
+    // bfloat16 65536 x 1024 120 -> 82). Ranges of 64 (128) rows at least, as many as two workgroups per CU take and the scratch memory
+    // holds maxima of. Up to kMaxRanges of them are put together by the quantizing kernel; more, which a launch of its own puts together,
     // where they take that from the maxima's time.
-    const bool wide = col_blocks * outer >= 32;
+    // (Rows that do not start on whole cache lines give short segments away: bfloat16 960 x 6410 26.3 us with 256, 29.5 with 64.)
+    const int64_t blocks = col_blocks * outer;
+    const bool wide = blocks >= 32 || (blocks >= 16 && inner * esize % 64 != 0);
     const int64_t amax_blocks = wide ? col_blocks : cdiv(inner, 64), groups = amax_blocks * outer;
-    int64_t ranges = std::min(512 / std::min<int64_t>(512, groups), cdiv(reduce, 64));
+    int64_t ranges = std::min(512 / std::min<int64_t>(512, groups), cdiv(reduce, wide ? 64 : 128));
     if (ranges > kMaxRanges && total / (kMaxRanges * groups) < kCombineFrom) ranges = kMaxRanges;
     ranges = std::max<int64_t>(1, std::min(ranges, ranges > kMaxRanges ? spare : spare + 1));
     const bool combine = ranges > kMaxRanges;
@@ -936,7 +938,7 @@ HIDET_API void hidet_symmetric_dequantize(const void *wq, const void *scale, voi
         // 76 and 90, 4096 x 4096 13.5 and 16.2, 250000 x 256 64 and 55, 4096 x 11008 42 and 37; bfloat16 500000 x 128 50 and 64,
         // 200000 x 320 50 and 59, 250000 x 256 50 and 39, 4096 x 4096 13.6 and 9.6.
         const int64_t lanes = cdiv(inner, 256) * 256, groups = cdiv(inner, 256) * cdiv(reduce, kDequantRows) * outer;
-        if (outer > 65535 || ((inner * 10 < lanes * 9 || (ST == HIDET_QMM_F32 && groups < 4096)) && cdiv(total, 1024) < (int64_t(1) << 24))) {
+        if (outer > 65535 || ((inner * 10 < lanes * 9 || (ST == HIDET_QMM_F32 && inner % 4 == 0 && groups < 4096)) && cdiv(total, 1024) < (int64_t(1) << 24))) {
             QMM_CHECK(cdiv(total, 1024) < (int64_t(1) << 31), "tensor too large for one launch");
             const dim3 grid{uint32_t(cdiv(total, 1024))};
             if (q_dtype == HIDET_QMM_I8) launch(dequantize_flat_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
