@@ -6,13 +6,17 @@
 // the running sum with its two scales on the vector ALU: one fma per accumulator element and k block, which the MFMA
 // cannot absorb (its built-in block scales are powers of two).
 //
-// gemm_fp8_scaled_kernel8 (tensors below 1 GiB, 16-byte aligned): workgroup tile 256 x 128 (one scale_b entry per k
-// block), eight waves of 64 x 64 - two per SIMD, so that one wave's folding overlaps the other's MFMAs; in a single
-// wave the two do not overlap - operand tiles straight into a three-slot LDS ring (buffer_load ... lds) two k blocks
-// ahead, one barrier per k block, hand-placed fragment reads, the scratch accumulator double-buffered per row block so
-// that the fold of row block i runs behind the MFMAs of row block i + 1. The running sums live in VGPRs (the VALU cannot
-// read accumulation registers). gemm_fp8_scaled_kernel (128 x 128 tile, register-staged double-buffered LDS) takes
-// the rest.
+// gemm_fp8_kernel8 (tensors below 1 GiB, 16-byte aligned): workgroup tile 256 x 128 (one scale_b entry per k block), eight
+// waves of 64 x 64, two per SIMD, operand tiles and the block's row scales straight into a three-slot LDS ring
+// (buffer_load ... lds) three k blocks ahead, one barrier per k block in the middle of its MFMAs, fragments fetched half a block
+// ahead, the scratch accumulator double-buffered per row block so that the fold of row block i - 1 runs behind the MFMAs of row
+// block i. The running sums live in VGPRs (the VALU cannot read accumulation registers). What bounds it: on real operands the
+// power limit (16384 x 7168 x 1536 179 us, on zeros 150: before the scales came through the LDS, the barrier moved and the tiles were
+// dealt by bytes 188 and 163; 2048 x 7168 x 4096 62.0 -> 58.6, 8192 x 2048 x 1024 28.4 -> 23.3; without scales 16384 x 7168 x 1536 151 ->
+// 142, 1536 x 4096 x 4096 28.6 -> 27.2, 8192 x 2048 x 1024 27.0 -> 19.9). Matrix and vector instructions of a SIMD hardly overlap, also between its two
+// waves. Measured and dropped: single MFMAs alternating with their folds (fewer cycles but 226 us: the clock falls), 32 x 32 x 64
+// MFMAs (on zeros 139, on real operands 180; without scales 149), raised priority during the MFMAs (180; 150).
+// gemm_fp8_scaled_kernel (128 x 128 tile, register-staged double-buffered LDS) takes the rest.
 #include "common.h"
 #include "gemm_tiling.h"
 #include "numeric.h"
@@ -162,16 +166,28 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_scaled_kernel(const uint
 
 constexpr int kM8 = 256, kN8 = 128;           // workgroup tile
 constexpr int kThreads8 = 512;
-constexpr int kSlotChunks8 = (kM8 + kN8) * 8;  // 16-byte chunks of one k block: A rows then B rows
-constexpr int kLoads8 = kSlotChunks8 / kThreads8;  // 6 direct-to-LDS loads per thread and k block
-constexpr int kRingBytes8 = 3 * kSlotChunks8 * 16;  // 144 KiB
+constexpr int kOperandChunks8 = (kM8 + kN8) * 8;       // 16-byte chunks of one k block: A rows then B rows
+constexpr int kSlotChunks8 = kOperandChunks8 + kM8 / 4;  // + the block's scales of the rows
+constexpr int kLoads8 = kOperandChunks8 / kThreads8;  // 6 direct-to-LDS loads per thread and k block
+constexpr int kRingBytes8 = 3 * kSlotChunks8 * 16;  // 147 KiB
 constexpr int kLdsBytes8 = kRingBytes8 + 16;       // + the K-split fix-up's flag; the ring must start at LDS address 0
 
 template <int FMT>
-__device__ __forceinline__ float4_t mfma_fp8_k128_fresh(const int4v_t &r0, const int4v_t &r1, const int4v_t &c0, const int4v_t &c1) {
-    const int8v_t rv = __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
-    const int8v_t cv = __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rv, cv, float4_t{0.f, 0.f, 0.f, 0.f}, FMT, FMT, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+__device__ __forceinline__ float4_t mfma_fp8_k128(const int4v_t (&r)[2], const int4v_t (&c)[2], const float4_t &acc) {
+    const int8v_t rv = __builtin_shufflevector(r[0], r[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    const int8v_t cv = __builtin_shufflevector(c[0], c[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rv, cv, acc, FMT, FMT, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+}
+
+// sum += part * factor, at its place among the instructions around it.
+__device__ __forceinline__ void fold_row_block(float4_t (&part)[4], float4_t (&sum)[4], float factor) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        asm volatile("" : "+v"(part[j]));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sum[j][v] = __builtin_fmaf(part[j][v], factor, sum[j][v]);
+        asm volatile("" : "+v"(sum[j]));
+    }
 }
 
 // SCALED: scale_a / scale_b are the block scales described at the top of the file. !SCALED: plain a x b^T with optional
@@ -182,12 +198,12 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
                                                                  const float *__restrict__ scale_a,
                                                                  const float *__restrict__ scale_b, void *__restrict__ c,
                                                                  int m, int n, int k, int tiles_m, int tiles_n, int xm, int xn,
-                                                                 int tail_parts, int tail_stride, float *__restrict__ partials,
+                                                                 int tail_parts, int tail_stride, int panel, float *__restrict__ partials,
                                                                  uint32_t *__restrict__ counters) {
     extern __shared__ uint4 lds[];  // [3][kSlotChunks8]; no static LDS: fragment reads address the ring from 0
     int &s_last = *reinterpret_cast<int *>(lds + kRingBytes8 / 16);
     GemmWorkItem item;
-    if (!gemm_work_item(tiles_m, tiles_n, xm, xn, 32, tail_parts, tail_stride, &item)) return;
+    if (!gemm_work_item(tiles_m, tiles_n, xm, xn, 32, tail_parts, tail_stride, &item, panel)) return;
     const int tile_m = item.tile_m, tile_n = item.tile_n;
     const int m0 = tile_m * kM8, n0 = tile_n * kN8;
     const int kblocks = k / 128;
@@ -211,8 +227,6 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(b), 0, int(int64_t(n - 1) * ldb + k), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_sa = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float *>(scale_a), 0, SCALED ? int(int64_t(kblocks) * m * 4) : 0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc_sb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(scale_b), 0, SCALED ? int(int64_t(n / 128) * kblocks * 4) : 0, 0x00020000);
 
     // Load instruction j of a wave fills chunk slots j * 512 + wave * 64 .. + 63 of a k block: tile row j * 64 + tid / 8
     // (A rows for j < 4, B rows after), position tid % 8, which holds chunk (tid % 8) ^ key(row). Rows past the end of a
@@ -226,6 +240,10 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
         if (j < 4) voff[j] = m0 + r < m ? int(int64_t(m0 + r) * lda) + chunk * 16 : kOutside;
         else voff[j] = n0 + r - kM8 < n ? int(int64_t(n0 + r - kM8) * ldb) + chunk * 16 : kOutside;
     }
+    // The row scales of a k block lie next to each other: one more direct-to-LDS load per wave (64 rows, four waves would do; the
+    // same number of loads in every wave keeps the waits alike). Fetched per lane and block instead, four rows and the column
+    // factor, they took the vector memory path about as long as the operands: 174 against 134 us with the MFMAs left out.
+    const int sa_row = m0 + (wave & 3) * 64 + lane, sa_off = sa_row < m ? sa_row * 4 : kOutside;
     // A short matrix leaves most of the 256 tile rows empty: load instructions whose 64 rows all lie past M are left
     // out (a_cnt of the 4 stay; the same for every wave), and a wave whose 64 output rows do skips its fragment reads
     // and MFMAs.
@@ -233,50 +251,55 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
 #pragma unroll
     for (int j = 0; j < 4; ++j) a_cnt += int(m0 + j * 64 < m);
     const bool wave_active = m0 + wm * 64 < m;
-    // (all_tag: the tile is full - no conditions in the loop)
-    auto load_tiles = [&](int kb, int slot, auto all_tag) {
+    constexpr int kBlockLoads = kLoads8 + (SCALED ? 1 : 0);
+    auto load_one = [&](auto j_tag, int kb, int slot) {  // one of the kBlockLoads instructions of a k block
+        constexpr int J = decltype(j_tag)::value;
         // the scalar offset is not part of the buffer's range check: a prefetch past the end of K re-reads the last block
         const int kbc = kb < kblocks ? kb : kblocks - 1;
-        uint4 *dst = lds + slot * kSlotChunks8 + wave * 64;
-#pragma unroll
-        for (int j = 0; j < kLoads8; ++j)
-            if (decltype(all_tag)::value || j >= 4 || j < a_cnt)
-                buffer_load_to_lds_b128(j < 4 ? rsrc_a : rsrc_b, dst + j * kThreads8, voff[j], kbc * 128);
+        uint4 *dst = lds + slot * kSlotChunks8;
+        if constexpr (J < kLoads8) buffer_load_to_lds_b128(J < 4 ? rsrc_a : rsrc_b, dst + wave * 64 + J * kThreads8, voff[J], kbc * 128);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sa, (__attribute__((address_space(3))) void *)(dst + kOperandChunks8 + (wave & 3) * 16), 4,
+                                                     sa_off, kbc * m * 4, 0, 0);
     };
-    auto load_tile_one = [&](auto j_tag, int kb, int slot) {  // one of the kLoads8 instructions of load_tiles, full tiles
-        constexpr int J = decltype(j_tag)::value;
-        const int kbc = kb < kblocks ? kb : kblocks - 1;
-        buffer_load_to_lds_b128(J < 4 ? rsrc_a : rsrc_b, lds + slot * kSlotChunks8 + wave * 64 + J * kThreads8, voff[J], kbc * 128);
+    using i0 = std::integral_constant<int, 0>;
+    using i1 = std::integral_constant<int, 1>;
+    using i2 = std::integral_constant<int, 2>;
+    using i3 = std::integral_constant<int, 3>;
+    using i4 = std::integral_constant<int, 4>;
+    using i5 = std::integral_constant<int, 5>;
+    using i6 = std::integral_constant<int, 6>;
+    using i7 = std::integral_constant<int, 7>;
+    auto load_tiles = [&](int kb, int slot) {
+        load_one(i0(), kb, slot);
+        if (a_cnt > 1) load_one(i1(), kb, slot);
+        if (a_cnt > 2) load_one(i2(), kb, slot);
+        if (a_cnt > 3) load_one(i3(), kb, slot);
+        load_one(i4(), kb, slot);
+        load_one(i5(), kb, slot);
+        if constexpr (SCALED) load_one(i6(), kb, slot);
     };
-    auto wait_older_tiles = [&](auto all_tag) {  // everything but the loads of the last load_scales + load_tiles has landed
-        constexpr int kScaleLoads = SCALED ? 5 : 0;
-        if (decltype(all_tag)::value) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm(kScaleLoads + kLoads8));
-            return;
-        }
+    auto wait_older_tiles = [&]() {  // everything but the loads of the last load_tiles has landed
         switch (a_cnt) {
-            case 1: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kScaleLoads + 3)); break;
-            case 2: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kScaleLoads + 4)); break;
-            case 3: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kScaleLoads + 5)); break;
-            default: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kScaleLoads + 6)); break;
+            case 1: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kBlockLoads - 3)); break;
+            case 2: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kBlockLoads - 2)); break;
+            case 3: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kBlockLoads - 1)); break;
+            default: __builtin_amdgcn_s_waitcnt(waitcnt_vm(kBlockLoads)); break;
         }
     };
-    // scales of a k block: the lane's 4 rows (one per row block) and the tile's column block
-    int sa_off[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = m0 + wm * 64 + i * 16 + ls;
-        sa_off[i] = row < m ? row * 4 : kOutside;
-    }
-    const int sb_off = tile_n * kblocks * 4;
-    float sa_next[4] = {1.f, 1.f, 1.f, 1.f}, sb_next = 1.f;
-    auto load_scales = [&](int kb) {
-        if constexpr (!SCALED) return;
-        const int kbc = kb < kblocks ? kb : kblocks - 1;  // scalar offsets are not range-checked: stay inside
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sa_next[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_sa, sa_off[i], kbc * m * 4, 0));
-        sb_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_sb, sb_off, kbc * 4, 0));
+    // The column factor of 64 k blocks at a time, one per lane (lane s % 64 that of block s).
+    const float *const col_scale = SCALED ? scale_b + int64_t(tile_n) * kblocks : nullptr;
+    float sb_lane = 1.0f;
+    auto column_factors_at = [&](int kb) {
+        const int at = (kb & ~63) + lane;
+        return col_scale + (at < kblocks ? at : kblocks - 1);
     };
+    auto fetch_column_factors = [&](int kb) {  // (load and wait by hand: a load that the compiler knows of would be waited for in every block)
+        asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(sb_lane) : "v"(column_factors_at(kb)) : "memory");
+    };
+    auto column_factor = [&](int kb) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sb_lane), kb & 63)); };
+    if constexpr (SCALED) sb_lane = *column_factors_at(kb_begin);
+    __builtin_amdgcn_sched_barrier(0);  // (in front of the tiles' loads: it is waited for together with the first of them)
 
     // LDS byte addresses of this lane's two 16-byte fragment halves in block 0 of its wave, ring slot 0; block i adds
     // i * 16 rows = i * 2048 bytes
@@ -289,101 +312,197 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
             b_addr[h] = uint32_t((rb * 8 + ((2 * kg + h) ^ lds_swizzle_key_step2(rb))) * 16);
         }
     }
+    const uint32_t sa_addr = uint32_t(kOperandChunks8 * 16 + (wm * 64 + ls) * 4);
     constexpr uint32_t kSlotBytes = kSlotChunks8 * 16;
-
-    load_scales(kb_begin);
-    load_tiles(kb_begin, 0, std::false_type());
-    load_tiles(kb_begin + 1, 1, std::false_type());
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    __builtin_amdgcn_s_barrier();
-
-    auto k_loop = [&](auto all_tag) {
-    for (int s = kb_begin, slot = 0; s < kb_end; ++s) {
-        float f[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) f[i] = sa_next[i] * sb_next;
-        load_scales(s + 1);                           // issued before the tile loads: waiting for them later does not
-        // wait for these. Slot (s + 2) % 3 was last read in k block s - 1. Full tiles issue the six load instructions two,
-        // two, one and one at a time between the row blocks instead of in one burst behind the barrier (every wave of the
-        // workgroup would queue its burst at the same moment, in front of its MFMAs).
-        constexpr bool kSpread = decltype(all_tag)::value;
-        const int slot_in = slot >= 1 ? slot - 1 : 2;
-        if constexpr (kSpread) {
-            load_tile_one(std::integral_constant<int, 0>(), s + 2, slot_in);
-            load_tile_one(std::integral_constant<int, 1>(), s + 2, slot_in);
-        } else {
-            load_tiles(s + 2, slot_in, all_tag);
-        }
-        if (decltype(all_tag)::value || wave_active) {
-        const uint32_t so = uint32_t(slot) * kSlotBytes;
-        const uint32_t aa0 = a_addr[0] + so, aa1 = a_addr[1] + so, ba0 = b_addr[0] + so, ba1 = b_addr[1] + so;
-        int4v_t bf[4][2], af[4][2];
-        bf[0][0] = lds_read_b128_early<0>(ba0);        bf[0][1] = lds_read_b128_early<0>(ba1);
-        af[0][0] = lds_read_b128_early<0>(aa0);        af[0][1] = lds_read_b128_early<0>(aa1);
-        bf[1][0] = lds_read_b128_early<2048>(ba0);     bf[1][1] = lds_read_b128_early<2048>(ba1);
-        bf[2][0] = lds_read_b128_early<4096>(ba0);     bf[2][1] = lds_read_b128_early<4096>(ba1);
-        bf[3][0] = lds_read_b128_early<6144>(ba0);     bf[3][1] = lds_read_b128_early<6144>(ba1);
-        af[1][0] = lds_read_b128_early<2048>(aa0);     af[1][1] = lds_read_b128_early<2048>(aa1);
-        af[2][0] = lds_read_b128_early<4096>(aa0);     af[2][1] = lds_read_b128_early<4096>(aa1);
-        af[3][0] = lds_read_b128_early<6144>(aa0);     af[3][1] = lds_read_b128_early<6144>(aa1);
-        __builtin_amdgcn_sched_barrier(0);
-        float4_t part[2][4];  // scratch accumulators of two consecutive row blocks
-        // row block 0: fragments arrive in issue order b0, a0, b1, b2, b3 (then a1 .. a3: 6 reads)
-        lds_wait_keep_newer<12>(bf[0][0], bf[0][1]);
-        lds_wait_keep_newer<12>(af[0][0], af[0][1]);
-        auto mm = [&](float4_t &dst_scaled, float4_t &dst_plain, const int4v_t &r0, const int4v_t &r1, const int4v_t &c0, const int4v_t &c1) {
-            if constexpr (SCALED) dst_scaled = mfma_fp8_k128_fresh<FMT>(r0, r1, c0, c1);
-            else {
-                const int8v_t rv = __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
-                const int8v_t cv = __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7);
-                dst_plain = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rv, cv, dst_plain, FMT, FMT, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
-            }
-        };
-        mm(part[0][0], total[0][0], bf[0][0], bf[0][1], af[0][0], af[0][1]);
-        lds_wait_keep_newer<10>(bf[1][0], bf[1][1]);
-        mm(part[0][1], total[0][1], bf[1][0], bf[1][1], af[0][0], af[0][1]);
-        lds_wait_keep_newer<8>(bf[2][0], bf[2][1]);
-        mm(part[0][2], total[0][2], bf[2][0], bf[2][1], af[0][0], af[0][1]);
-        lds_wait_keep_newer<6>(bf[3][0], bf[3][1]);
-        mm(part[0][3], total[0][3], bf[3][0], bf[3][1], af[0][0], af[0][1]);
-        if constexpr (kSpread) {
-            load_tile_one(std::integral_constant<int, 2>(), s + 2, slot_in);
-            load_tile_one(std::integral_constant<int, 3>(), s + 2, slot_in);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        auto row_block = [&](auto i_tag) {  // MFMAs of row block I, then the fold of row block I - 1 behind them
-            constexpr int I = decltype(i_tag)::value;
-            lds_wait_keep_newer<2 * (3 - I)>(af[I][0], af[I][1]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mm(part[I & 1][j], total[I][j], bf[j][0], bf[j][1], af[I][0], af[I][1]);
-            if constexpr (kSpread && I <= 2) load_tile_one(std::integral_constant<int, 3 + I>(), s + 2, slot_in);
-            if constexpr (SCALED) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) total[I - 1][j][v] = __builtin_fmaf(part[(I - 1) & 1][j][v], f[I - 1], total[I - 1][j][v]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        row_block(std::integral_constant<int, 1>());
-        row_block(std::integral_constant<int, 2>());
-        row_block(std::integral_constant<int, 3>());
-        if constexpr (SCALED) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) total[3][j][v] = __builtin_fmaf(part[1][j][v], f[3], total[3][j][v]);
-        }
-        }
-        // the tiles of k block s + 1 (issued one block ago) must have landed before anyone reads them; the scale loads
-        // and tile loads issued in this block may stay in flight
-        wait_older_tiles(all_tag);
-        __builtin_amdgcn_s_barrier();
-        slot = slot == 2 ? 0 : slot + 1;
-    }
+    int4v_t af[4][2], bf[4][2];        // [16-row or 16-column block][half]
+    uint64_t sa_pair[2] = {0, 0};      // factors of this lane's rows, blocks 0 and 1, 2 and 3
+    auto read_a = [&](auto i_tag, uint32_t so) {
+        constexpr int I = decltype(i_tag)::value;
+        af[I][0] = lds_read_b128_early<I * 2048>(a_addr[0] + so);
+        af[I][1] = lds_read_b128_early<I * 2048>(a_addr[1] + so);
     };
-    if (a_cnt == 4) k_loop(std::true_type());
-    else k_loop(std::false_type());
+    auto read_b = [&](auto j_tag, uint32_t so) {
+        constexpr int J = decltype(j_tag)::value;
+        bf[J][0] = lds_read_b128_early<J * 2048>(b_addr[0] + so);
+        bf[J][1] = lds_read_b128_early<J * 2048>(b_addr[1] + so);
+    };
+    auto read_row_factors = [&](uint32_t so) {
+        if constexpr (!SCALED) return;
+        asm volatile("ds_read2_b32 %0, %1 offset0:0 offset1:16" : "=v"(sa_pair[0]) : "v"(sa_addr + so));
+        asm volatile("ds_read2_b32 %0, %1 offset0:32 offset1:48" : "=v"(sa_pair[1]) : "v"(sa_addr + so));
+    };
+    float f[4] = {0.f, 0.f, 0.f, 0.f};  // factors of the k block at hand, per row block
+    auto take_factors = [&](int kb) {   // (behind the wait for sa_pair)
+        asm volatile("" : "+v"(sa_pair[0]), "+v"(sa_pair[1]));
+        const float sb = column_factor(kb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = __builtin_bit_cast(float, uint32_t(sa_pair[i >> 1] >> (32 * (i & 1)))) * sb;
+    };
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+
+    if (a_cnt == 4) {
+        // Full tiles. One barrier per k block, in the middle of its MFMAs: in front of it everything of this block has been
+        // read (its slot is free for block s + 3) and every wave's loads of block s + 1 have landed, behind it the fragments
+        // of block s + 1 are fetched as those of this block have had their last use. The four MFMAs of a row block run as one
+        // burst and the sums of the row block before are folded behind them. `keep` fixes that order: left to itself the
+        // compiler folds a row block right behind its own MFMAs, which then wait for one another.
+        float4_t part[2][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[0][j] = zero, part[1][j] = zero;
+        auto keep = [](auto &v) { asm volatile("" : "+v"(v)); };
+        load_tiles(kb_begin, 0);
+        load_tiles(kb_begin + 1, 1);
+        load_tiles(kb_begin + 2, 2);
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kBlockLoads));
+        asm volatile("" : "+v"(sb_lane) :: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read_a(i0(), 0);
+        read_a(i1(), 0);
+        read_row_factors(0);
+        read_a(i2(), 0);
+        lds_wait_keep_newer<2>(af[0][0], af[1][0]);  // (no more than 15 reads can be counted)
+        read_b(i0(), 0);
+        read_b(i1(), 0);
+        read_b(i2(), 0);
+        read_b(i3(), 0);
+        read_a(i3(), 0);
+        __builtin_amdgcn_sched_barrier(0);
+        int slot = 0;
+        for (int s = kb_begin; s < kb_end; ++s) {
+            const int next = slot == 2 ? 0 : slot + 1;
+            const uint32_t so = uint32_t(next) * kSlotBytes;
+            auto row_block = [&](auto i_tag) {
+                constexpr int I = decltype(i_tag)::value, O = (I + 3) % 4;
+                // reads in flight, oldest first: a0 a1 factors a2 | b0 b1 b2 b3 a3, two each
+                if constexpr (I == 0) {
+                    lds_wait_keep_newer<8>(af[0][0], af[0][1]);
+                    lds_wait_keep_newer<8>(bf[0][0], bf[0][1]);
+                }
+                auto mm = [&](auto j_tag) {
+                    constexpr int J = decltype(j_tag)::value;
+                    if constexpr (I == 0 && J > 0) lds_wait_keep_newer<8 - 2 * J>(bf[J][0], bf[J][1]);
+                    else keep(af[I][0]);
+                    if constexpr (SCALED) {
+                        part[I & 1][J] = mfma_fp8_k128<FMT>(bf[J], af[I], zero);
+                        keep(part[I & 1][J]);
+                    } else {
+                        total[I][J] = mfma_fp8_k128<FMT>(bf[J], af[I], total[I][J]);
+                        keep(total[I][J]);
+                    }
+                };
+                mm(i0());
+                mm(i1());
+                mm(i2());
+                mm(i3());
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (I == 1) {
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kBlockLoads));
+                    lds_wait_keep_newer<0>(af[2][0], af[2][1]);
+                    lds_wait_keep_newer<0>(af[3][0], af[3][1]);
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                    read_a(i0(), so);
+                    read_a(i1(), so);
+                    read_row_factors(so);
+                    load_one(i0(), s + 3, slot), load_one(i1(), s + 3, slot);
+                }
+                if constexpr (I == 2) {
+                    read_a(i2(), so);
+                    load_one(i2(), s + 3, slot), load_one(i3(), s + 3, slot), load_one(i4(), s + 3, slot);
+                }
+                if constexpr (I == 3) {
+                    lds_wait_keep_newer<2>(af[0][0], af[1][0]);
+                    read_b(i0(), so);
+                    read_b(i1(), so);
+                    read_b(i2(), so);
+                    read_b(i3(), so);
+                    read_a(i3(), so);
+                    load_one(i5(), s + 3, slot);
+                    if constexpr (SCALED) load_one(i6(), s + 3, slot);
+                }
+                if constexpr (SCALED) {
+                    fold_row_block(part[O & 1], total[O], f[O]);
+                    if constexpr (I == 0) {
+                        take_factors(s);
+                        keep(f[0]), keep(f[1]), keep(f[2]), keep(f[3]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            row_block(i0());
+            row_block(i1());
+            row_block(i2());
+            row_block(i3());
+            slot = next;
+            if constexpr (SCALED)
+                if (((s + 1) & 63) == 0) fetch_column_factors(s + 1);
+        }
+        if constexpr (SCALED) fold_row_block(part[1], total[3], f[3]);
+        // the fragments of a block past the end must not land in registers that have another use by then
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            lds_wait_keep_newer<0>(af[i][0], af[i][1]);
+            lds_wait_keep_newer<0>(bf[i][0], bf[i][1]);
+        }
+        asm volatile("" : "+v"(sa_pair[0]), "+v"(sa_pair[1]));
+    } else {
+        load_tiles(kb_begin, 0);
+        load_tiles(kb_begin + 1, 1);
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        asm volatile("" : "+v"(sb_lane) :: "memory");
+        __builtin_amdgcn_s_barrier();
+        for (int s = kb_begin, slot = 0; s < kb_end; ++s) {
+            load_tiles(s + 2, slot >= 1 ? slot - 1 : 2);  // slot (s + 2) % 3 was last read in k block s - 1
+            if (wave_active) {
+                const uint32_t so = uint32_t(slot) * kSlotBytes;
+                read_row_factors(so);
+                read_b(i0(), so);
+                read_a(i0(), so);
+                read_b(i1(), so);
+                read_b(i2(), so);
+                read_b(i3(), so);
+                lds_wait_keep_newer<6>(af[0][0], bf[0][0]);  // (no more than 15 reads can be counted)
+                read_a(i1(), so);
+                read_a(i2(), so);
+                read_a(i3(), so);
+                __builtin_amdgcn_sched_barrier(0);
+                lds_wait_keep_newer<12>(af[0][0], af[0][1]);
+                lds_wait_keep_newer<12>(bf[0][0], bf[0][1]);
+                if constexpr (SCALED) take_factors(s);
+                lds_wait_keep_newer<6>(bf[1][0], bf[1][1]);
+                lds_wait_keep_newer<6>(bf[2][0], bf[2][1]);
+                lds_wait_keep_newer<6>(bf[3][0], bf[3][1]);
+                auto row_block = [&](auto i_tag) {
+                    constexpr int I = decltype(i_tag)::value;
+                    if constexpr (I > 0) lds_wait_keep_newer<2 * (3 - I)>(af[I][0], af[I][1]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if constexpr (SCALED) {
+                            const float4_t sum = mfma_fp8_k128<FMT>(bf[j], af[I], zero);
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) total[I][j][v] = __builtin_fmaf(sum[v], f[I], total[I][j][v]);
+                        } else {
+                            total[I][j] = mfma_fp8_k128<FMT>(bf[j], af[I], total[I][j]);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                row_block(i0());
+                row_block(i1());
+                row_block(i2());
+                row_block(i3());
+            }
+            if constexpr (SCALED)
+                if (((s + 1) & 63) == 0) fetch_column_factors(s + 1);
+            // the tiles of k block s + 1 (issued one block ago) must have landed before anyone reads them; the loads issued
+            // in this block may stay in flight
+            wait_older_tiles();
+            __builtin_amdgcn_s_barrier();
+            slot = slot == 2 ? 0 : slot + 1;
+        }
+    }
     // LDS must not be released with tile loads in flight
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
 
@@ -436,7 +555,7 @@ static GemmTail tail8_of(const GemmTiling &tiling, int64_t k, const Workspace &w
 // (the register-staged 256 x 256 kernel) 3.5 us per k block and round.
 double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, void *workspace, int64_t workspace_bytes) {
     if (k % 128 != 0) return 8.0 + double(cdiv(cdiv(m, 256) * cdiv(n, 256), 256)) * 3.5 * double(cdiv(k, 128));
-    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, kM8)), int(cdiv(n, kN8)), 32);
+    const GemmTiling tiling = make_gemm_tiling_weighted(int(cdiv(m, kM8)), int(cdiv(n, kN8)), 32, kM8, kN8);
     const GemmTail tail = tail8_of(tiling, k, split_workspace(workspace, workspace_bytes));
     const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
     const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);
@@ -450,7 +569,7 @@ static void launch_kernel8(const void *a, int64_t lda, const void *b, int64_t ld
                            void *c, int64_t m, int64_t n, int64_t k, int out_dtype, void *workspace, int64_t workspace_bytes,
                            hipStream_t stream) {
     const int tiles_m = int(cdiv(m, kM8)), tiles_n = int(cdiv(n, kN8));
-    const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, 32);
+    const GemmTiling tiling = make_gemm_tiling_weighted(tiles_m, tiles_n, 32, kM8, kN8);
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     const GemmTail tail = tail8_of(tiling, k, ws);
     const int64_t grid = gemm_grid_with_tail(tiling, 32, tail);
@@ -459,7 +578,7 @@ static void launch_kernel8(const void *a, int64_t lda, const void *b, int64_t ld
         allow_dynamic_lds(reinterpret_cast<const void *>(kern), kLdsBytes8);
         launch(kern, dim3(uint32_t(grid)), dim3(kThreads8), size_t(kLdsBytes8), stream, static_cast<const uint8_t *>(a), lda,
                static_cast<const uint8_t *>(b), ldb, static_cast<const float *>(scale_a), static_cast<const float *>(scale_b), c,
-               int(m), int(n), int(k), tiles_m, tiles_n, tiling.xm, tiling.xn, tail.parts, tail.max_tiles,
+               int(m), int(n), int(k), tiles_m, tiles_n, tiling.xm, tiling.xn, tail.parts, tail.max_tiles, tiling.panel,
                reinterpret_cast<float *>(ws.scratch), ws.counters);
     };
     constexpr int kOut8 = FMT == 1 ? HIDET_QMM_E5M2 : HIDET_QMM_E4M3;  // the 8-bit output type is the operands' own

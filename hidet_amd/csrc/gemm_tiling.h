@@ -17,6 +17,7 @@ struct GemmTiling {
     int tiles_m, tiles_n;
     int xm, xn;         // XCD grid
     int region_tiles;   // largest number of tiles any XCD owns
+    int panel;          // tile columns of a panel
     int64_t grid() const { return int64_t(8) * region_tiles; }
 };
 
@@ -39,7 +40,7 @@ __host__ __device__ constexpr int lds_swizzle_key_step2(int row) { return (row &
 
 // `concurrent` = workgroups one XCD runs at a time (32 CUs x workgroups per CU).
 inline GemmTiling make_gemm_tiling(int tiles_m, int tiles_n, int concurrent) {
-    GemmTiling best{tiles_m, tiles_n, 1, 8, 0};
+    GemmTiling best{tiles_m, tiles_n, 1, 8, 0, kPanelCols};
     int64_t best_cost = -1;
     for (int xm = 1; xm <= 8; xm *= 2) {
         const int xn = 8 / xm;
@@ -61,6 +62,34 @@ inline GemmTiling make_gemm_tiling(int tiles_m, int tiles_n, int concurrent) {
     return best;
 }
 
+// The same for tiles whose two operand slices differ in size (`row_bytes` and `col_bytes` of a tile's slices per step of K, in any
+// common unit): regions and panels so that the workgroups an XCD runs together pull the fewest bytes into its L2, `panel` columns x
+// concurrent / panel rows at a time. (FP8 tiles of 256 x 128: 8192 x 2048 x 1024 29.0 -> 23.3 us, 16384 x 7168 x 1536 190 -> 187 against
+// make_gemm_tiling; what an L2 misses comes from the last-level cache at about the rate that a copy has.)
+inline GemmTiling make_gemm_tiling_weighted(int tiles_m, int tiles_n, int concurrent, int row_bytes, int col_bytes) {
+    GemmTiling best{tiles_m, tiles_n, 1, 8, 0, kPanelCols};
+    int64_t best_rounds = 0, best_bytes = -1;
+    for (int xm = 1; xm <= 8; xm *= 2) {
+        const int xn = 8 / xm;
+        const int rr = (tiles_m + xm - 1) / xm, rc = (tiles_n + xn - 1) / xn;
+        const int64_t rounds = (int64_t(rr) * rc + concurrent - 1) / concurrent;
+        for (int panel = 1; panel <= concurrent; panel *= 2) {
+            const int width = panel < rc ? panel : rc, full = rc / width;  // panels of `width` columns and a last narrower one
+            auto bytes_of = [&](int w) {  // of one panel: its rows in batches, each with the panel's columns
+                if (w == 0) return int64_t(0);
+                const int batch = (concurrent + w - 1) / w < rr ? (concurrent + w - 1) / w : rr;
+                return int64_t(rr) * row_bytes + int64_t((rr + batch - 1) / batch) * w * col_bytes;
+            };
+            const int64_t bytes = full * bytes_of(width) + bytes_of(rc - full * width);
+            if (best_bytes >= 0 && (rounds > best_rounds || (rounds == best_rounds && bytes >= best_bytes))) continue;
+            best_rounds = rounds;
+            best_bytes = bytes;
+            best = GemmTiling{tiles_m, tiles_n, xm, xn, rr * rc, panel};
+        }
+    }
+    return best;
+}
+
 struct GemmRegion {
     int row_begin, col_begin, rows, cols;
 };
@@ -73,20 +102,20 @@ __host__ __device__ __forceinline__ GemmRegion gemm_region_of_xcd(int tiles_m, i
 }
 
 // Tile (row, column) number `local` of a region in panel order; false past the end of the region.
-__host__ __device__ __forceinline__ bool gemm_tile_of_region(const GemmRegion &reg, int local, int *tile_m, int *tile_n) {
+__host__ __device__ __forceinline__ bool gemm_tile_of_region(const GemmRegion &reg, int local, int *tile_m, int *tile_n, int panel_cols = kPanelCols) {
     const int rr = reg.rows, rc = reg.cols;
     if (local >= rr * rc) return false;
-    const int full_panels = rc / kPanelCols;
-    const int full_tiles = full_panels * rr * kPanelCols;
+    const int full_panels = rc / panel_cols;
+    const int full_tiles = full_panels * rr * panel_cols;
     int row, col;
     if (local < full_tiles) {
-        const int panel = local / (rr * kPanelCols), rem = local % (rr * kPanelCols);
-        row = rem / kPanelCols;
-        col = panel * kPanelCols + rem % kPanelCols;
+        const int panel = local / (rr * panel_cols), rem = local % (rr * panel_cols);
+        row = rem / panel_cols;
+        col = panel * panel_cols + rem % panel_cols;
     } else {
-        const int rem = local - full_tiles, w = rc - full_panels * kPanelCols;
+        const int rem = local - full_tiles, w = rc - full_panels * panel_cols;
         row = rem / w;
-        col = full_panels * kPanelCols + rem % w;
+        col = full_panels * panel_cols + rem % w;
     }
     *tile_m = reg.row_begin + row;
     *tile_n = reg.col_begin + col;
@@ -139,7 +168,7 @@ struct GemmWorkItem {
 // (Workgroup `block` of the launch; a pure function so that the host can enumerate a launch, as the tests do.)
 __host__ __device__ __forceinline__ bool gemm_work_item_of_block(int block, int tiles_m, int tiles_n, int xm, int xn,
                                                                  int concurrent, int tail_parts, int tail_stride,
-                                                                 GemmWorkItem *item) {
+                                                                 GemmWorkItem *item, int panel_cols = kPanelCols) {
     const GemmRegion reg = gemm_region_of_xcd(tiles_m, tiles_n, xm, xn, block & 7);
     const int region_tiles = reg.rows * reg.cols;
     const int whole = tail_parts > 1 ? (region_tiles / concurrent) * concurrent : region_tiles;
@@ -154,12 +183,12 @@ __host__ __device__ __forceinline__ bool gemm_work_item_of_block(int block, int 
         item->parts = tail_parts;
         item->slot = (block & 7) * tail_stride + j / tail_parts;
     }
-    return gemm_tile_of_region(reg, local, &item->tile_m, &item->tile_n);
+    return gemm_tile_of_region(reg, local, &item->tile_m, &item->tile_n, panel_cols);
 }
 
 __device__ __forceinline__ bool gemm_work_item(int tiles_m, int tiles_n, int xm, int xn, int concurrent, int tail_parts,
-                                               int tail_stride, GemmWorkItem *item) {
-    return gemm_work_item_of_block(int(blockIdx.x), tiles_m, tiles_n, xm, xn, concurrent, tail_parts, tail_stride, item);
+                                               int tail_stride, GemmWorkItem *item, int panel_cols = kPanelCols) {
+    return gemm_work_item_of_block(int(blockIdx.x), tiles_m, tiles_n, xm, xn, concurrent, tail_parts, tail_stride, item, panel_cols);
 }
 
 // Fix-up of a tile computed in K ranges by item.parts workgroups of THREADS threads, each holding R x T float4
