@@ -88,6 +88,22 @@ __device__ __forceinline__ bool scales4(const float (&amax)[4], float (&s)[4], f
     return fast;
 }
 
+// Largest of a wave's values, in every lane (no LDS: the six exchanges of a shuffled tree are 0.3 us of a kernel that runs for 3).
+__device__ __forceinline__ float wave_max(float m) {
+    auto step = [&m](auto ctrl, auto rows) {  // (lanes that the move does not reach keep their own value)
+        const int v = __float_as_int(m);
+        m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(v, v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false)));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0xB1>(), integral_constant<int, 0xF>());   // quads: neighbours
+    step(integral_constant<int, 0x4E>(), integral_constant<int, 0xF>());   // quads: pairs
+    step(integral_constant<int, 0x141>(), integral_constant<int, 0xF>());  // half rows of 16 lanes, mirrored
+    step(integral_constant<int, 0x140>(), integral_constant<int, 0xF>());  // rows, mirrored
+    step(integral_constant<int, 0x142>(), integral_constant<int, 0xA>());  // lane 15 of rows 0, 2 to rows 1, 3
+    step(integral_constant<int, 0x143>(), integral_constant<int, 0xC>());  // lane 31 to rows 2, 3
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 63));
+}
+
 // Four elements at the alignment of one: rows of an odd length start anywhere (the hardware takes such accesses whole).
 typedef float float4_at4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint16_t half4_at2_t __attribute__((ext_vector_type(4), aligned(2)));
@@ -651,6 +667,9 @@ __device__ __forceinline__ float vector_element(const uint4v_t &v, int e) {
     return DT == HIDET_QMM_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
 }
 constexpr int kChunkLoads = 4, kChunkVectors = 256 * kChunkLoads;  // 16 KiB of 16-byte vectors: one trip of a workgroup
+constexpr int kAmaxPartials = 1024;
+// Vectors of 256 threads up to which a thread converts one of them (bfloat16, one and four: 512 x 4096 4.4 and 5.4 us, 2048 x 4096 5.9 and 6.1, 4096 x 8192 18.6 and 13.6).
+constexpr int kFineChunks = 2048;
 
 // Largest magnitude of each workgroup's share of a tensor, one float per workgroup (an atomic on a single word takes
 // longer than the reads, and the word has to be cleared by a launch of its own).
@@ -668,65 +687,87 @@ __global__ __launch_bounds__(256) void amax_all_kernel(const void *__restrict__ 
 #pragma unroll
             for (int e = 0; e < V; ++e) m = fmaxf(m, fabsf(vector_element<DT>(v[j], e)));
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    m = wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) amax[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 // e4m3 codes of four values: the quotient by the scale, clamped to +-448 (what saturation means for a format whose largest
-// finite value is 448), converted by the hardware's round-to-nearest-even OCP conversion; NaN becomes NaN of the same sign. The product with the
-// reciprocal, within 2^-22 of the quotient, converts alike unless a rounding boundary of the format lies between them; those have at
-// most four significant bits, so a product whose low 19 bits are not within 8 of zero (or that is too small for any code
-// but zero) needs no division. 448 is such a boundary and no quotient by a precise scale exceeds it by as much as 8 units
-// in the last place, so only divided values need the clamp.
-__device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, float inv, bool fast) {
-    if (s == 0.0f) return 0u;
+// finite value is 448), converted by the hardware's round-to-nearest-even OCP conversion; NaN becomes NaN of the same sign.
+__device__ __forceinline__ uint32_t e4m3_codes4_divided(const float (&x)[4], float s) {
     float q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)  // (these two keep a NaN, where the median of three hides it)
+        q[e] = s == 0.0f ? 0.0f : __builtin_elementwise_minimum(__builtin_elementwise_maximum(x[e] / s, -448.0f), 448.0f);
+    uint32_t p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+    p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], int(p), true);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)  // (the conversion drops a NaN's sign)
+        if (q[e] != q[e]) p = (p & ~(0xFFu << (8 * e))) | ((0x7Fu | ((__float_as_uint(q[e]) >> 24) & 0x80u)) << (8 * e));
+    return p;
+}
+
+// The same without the division where its result provably converts alike; `fast`: the reciprocal of the scale is precise.
+// float32: the product with the reciprocal, within 2^-22 of the quotient, converts alike unless a rounding boundary of the format lies
+// between them; those have at most five significant bits, so a product whose low 19 bits are not within 8 of zero (or that is too
+// small for any code but zero) needs no division. 448 is such a boundary and no quotient by a precise scale exceeds it by
+// as much as 8 units in the last place, so only divided values need the clamp.
+// 16-bit types: there that test fails for one element in 128 or so (448 / 2^j times a maximum of few bits, and often 3/4 of that),
+// which sends nearly every wave through the division (4096 x 8192: 23 us, of which 10 for this). One correction with the remainder
+// instead leaves Q (1 + h), |h| < 2^-45, rounded once. It differs from the rounded quotient Q only next to a midpoint of two
+// float32 numbers, and matters only where one of those is a boundary B: where x = s T (1 + h) with T = B +- half a unit. With s = N 2^b,
+// N of 24 bits, and B = beta 2^c, 16 <= beta < 32, x and s T differ by |J -+ N / 2^20| 2^(b+c) for an integer J, out of at most 2^29 2^(b+c): h would
+// have to be below 2^-45, so N within 2^-16 of a multiple of 2^20. But N is (maximum / 7) times a power of two, rounded: the low bits of a
+// multiple of 1/7 repeat with period three and never come near zero, and where seven divides the maximum N has at most nine bits, a
+// multiple of 2^15; N / 2^20 is then an integer (x = s T would need 25 bits) or 2^-5 away from one. (tests/host/e4m3_quotients.cpp: every pair.)
+template <int DT>
+__device__ __forceinline__ uint32_t e4m3_codes4(const float (&x)[4], float s, float inv, bool fast) {
+    float q[4];
+    bool sure = fast;
     uint32_t nearest = 0xFFFFFFFFu;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         q[e] = x[e] * inv;
-        nearest = min(nearest, (__float_as_uint(fmaxf(fabsf(q[e]), 0x1.1p-12f + 0x1p-20f)) + 8u) & 0x7FFFFu);
+        if constexpr (DT == HIDET_QMM_F32) nearest = min(nearest, (__float_as_uint(fmaxf(fabsf(q[e]), 0x1.1p-12f + 0x1p-20f)) + 8u) & 0x7FFFFu);
+        else q[e] = __builtin_fmaf(-__builtin_fmaf(q[e], s, -x[e]), inv, q[e]);  // (in this form a zero keeps its sign)
     }
-    if (__builtin_expect(!fast || nearest <= 16u, 0)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)  // (these two keep a NaN, where the median of three hides it)
-            q[e] = __builtin_elementwise_minimum(__builtin_elementwise_maximum(x[e] / s, -448.0f), 448.0f);
-    }
+    if constexpr (DT == HIDET_QMM_F32) sure = sure && nearest > 16u;
+    sure = sure && !(__builtin_isunordered(q[0], q[1]) || __builtin_isunordered(q[2], q[3]));
     uint32_t p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
     p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], int(p), true);
-    if (__builtin_expect(__builtin_isunordered(q[0], q[1]) || __builtin_isunordered(q[2], q[3]), 0)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)  // (the conversion drops a NaN's sign)
-            if (q[e] != q[e]) p = (p & ~(0xFFu << (8 * e))) | ((0x7Fu | ((__float_as_uint(q[e]) >> 24) & 0x80u)) << (8 * e));
-    }
+    if (__builtin_expect(!sure, 0)) p = e4m3_codes4_divided(x, s);
     return p;
 }
 
 // Small tensors (the activations of a decode step), up to 65536 elements, in one launch: a workgroup of 1024 threads looks at
 // the whole tensor for its maximum and converts 4096 elements of it. One workgroup that converted all of it was bound by its
 // vector ALU (bfloat16, 65536 elements 10.5 us, the two launches of larger tensors 7); looking at everything 16 times costs little
-// beside that. Same arithmetic as fp8_quantize_kernel.
+// beside that. What bounds it is the launch and code that comes from memory line by line, so the loops stay rolled up. Same
+// arithmetic as fp8_quantize_kernel.
 template <int DT>
 __global__ __launch_bounds__(1024) void fp8_quantize_small_kernel(const void *__restrict__ x, uint32_t *__restrict__ codes,
                                                                   float *__restrict__ scale, int numel4) {
     __shared__ float red[16];
-    const int tid = threadIdx.x, own = blockIdx.x * 1024 + tid;
-    float mine[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (own < numel4) load4_as_f32<DT>(x, own, mine);
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int i = j * 1024 + tid;
-        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (i < numel4) load4_as_f32<DT>(x, i, v);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[e]));
+    const int tid = threadIdx.x, own = blockIdx.x * 1024 + tid, last = numel4 - 1;
+    if (numel4 == 0) {
+        if (tid == 0) *scale = 0.0f;
+        return;
     }
+    float mine[4];
+    load4_as_f32<DT>(x, min(own, last), mine);
+    float m = 0.0f;
+#pragma unroll 1
+    for (int j = tid; j < numel4; j += 4096) {
+        float v[4][4];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+        for (int i = 0; i < 4; ++i) load4_as_f32<DT>(x, min(j + i * 1024, last), v[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[i][e]));
+    }
+    m = wave_max(m);
     if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
     m = red[0];
@@ -735,26 +776,33 @@ __global__ __launch_bounds__(1024) void fp8_quantize_small_kernel(const void *__
     const float s = m / 448.0f, inv = __builtin_amdgcn_rcpf(s);
     const bool fast = reciprocal_is_precise(s);
     if (own == 0) *scale = s;
-    if (own < numel4) codes[own] = e4m3_codes4(mine, s, inv, fast);
+    if (own < numel4) codes[own] = e4m3_codes4<DT>(mine, s, inv, fast);
 }
 
-// One chunk (16 KiB) per workgroup. The loads go out first; the workgroups' maxima (amax_all_kernel) are put together
-// while they are under way. Chunks are taken from the end of the tensor, where the maximum pass read last, each on the
+// LOADS * 4 KiB per workgroup. The loads go out first; the workgroups' maxima (amax_all_kernel) are put together
+// while they are under way. Chunks of 16 KiB are taken from the end of the tensor, where the maximum pass read last, each on the
 // XCD that read it then: what is still in that L2 does not come from memory again. 4096 x 8192
-// bfloat16: maxima 11 us (15.4 with atomics, + a clearing launch), codes 22 us (23.7; 27.5 with 32 KiB per workgroup).
-template <int DT>
+// bfloat16: maxima 11 us (15.4 with atomics, + a clearing launch), codes 14 us (13 with no arithmetic at all). A tensor of which one
+// vector per thread already fills the chip takes that: what bounds it is the launch and the code, which comes from memory line by line (4 -> 1
+// vectors: 64 x 4096 5.6 -> 2.8 us, 512 x 4096 5.2 -> 4.0).
+template <int DT, int LOADS>
 __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restrict__ x, const float *__restrict__ amax, int partials,
                                                            uint8_t *__restrict__ codes, float *__restrict__ scale, int64_t numel, int64_t chunks8) {
     constexpr int V = DT == HIDET_QMM_F32 ? 4 : 8;
     __shared__ float red[4];
     const int64_t c = (chunks8 - 1 - int64_t(blockIdx.x >> 3)) * 8 + (blockIdx.x & 7);
-    uint4v_t v[kChunkLoads];
+    uint4v_t v[LOADS];
 #pragma unroll
-    for (int j = 0; j < kChunkLoads; ++j) v[j] = load_vector<DT>(x, (c * kChunkVectors + j * 256 + threadIdx.x) * V, numel);
+    for (int j = 0; j < LOADS; ++j) v[j] = load_vector<DT>(x, (c * (256 * LOADS) + j * 256 + threadIdx.x) * V, numel);
     float m = 0.0f;
-    for (int i = threadIdx.x; i < partials; i += 256) m = fmaxf(m, amax[i]);
+    {
+        float a[kAmaxPartials / 256];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+        for (int i = 0; i < kAmaxPartials / 256; ++i) a[i] = amax[min(int(threadIdx.x) + i * 256, partials - 1)];
+#pragma unroll
+        for (int i = 0; i < kAmaxPartials / 256; ++i) m = fmaxf(m, a[i]);
+    }
+    m = wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -762,8 +810,8 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restric
     const bool fast = reciprocal_is_precise(s);
     if (blockIdx.x == 0 && threadIdx.x == 0) *scale = s;
 #pragma unroll
-    for (int j = 0; j < kChunkLoads; ++j) {
-        const int64_t i = (c * kChunkVectors + j * 256 + threadIdx.x) * V;
+    for (int j = 0; j < LOADS; ++j) {
+        const int64_t i = (c * (256 * LOADS) + j * 256 + threadIdx.x) * V;
         if (i >= numel) continue;
         uint32_t out[V / 4];
 #pragma unroll
@@ -771,7 +819,7 @@ __global__ __launch_bounds__(256) void fp8_quantize_kernel(const void *__restric
             float t[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) t[e] = vector_element<DT>(v[j], 4 * h + e);
-            out[h] = e4m3_codes4(t, s, inv, fast);
+            out[h] = e4m3_codes4<DT>(t, s, inv, fast);
         }
         if (i + V <= numel) {
             __builtin_memcpy(codes + i, out, V);
@@ -1002,10 +1050,13 @@ HIDET_API void hidet_fp8_quantize_per_tensor(const void *x, void *codes, void *s
         QMM_CHECK(chunks8 * 8 < (int64_t(1) << 31), "tensor too large for one launch");
         // four workgroups per CU, a multiple of the XCDs (a chunk is then converted on the XCD that looked at it); fewer where the
         // scratch memory holds fewer maxima
-        const int64_t partials = std::min<int64_t>({chunks, 1024, ws.scratch_bytes / 4});
+        const int64_t partials = std::min<int64_t>({chunks, kAmaxPartials, ws.scratch_bytes / 4});
         launch(amax_all_kernel<DT>, dim3(uint32_t(partials)), dim3(256), 0, stream, x, amax, numel, chunks);
-        launch(fp8_quantize_kernel<DT>, dim3(uint32_t(chunks8 * 8)), dim3(256), 0, stream, x, amax, int(partials), static_cast<uint8_t *>(codes),
-               static_cast<float *>(scale), numel, chunks8);
+        const int64_t fine8 = cdiv(cdiv(numel, int64_t(256) * (16 / esize)), 8);
+        if (fine8 * 8 <= kFineChunks) launch(fp8_quantize_kernel<DT, 1>, dim3(uint32_t(fine8 * 8)), dim3(256), 0, stream, x, amax, int(partials), static_cast<uint8_t *>(codes),
+                                      static_cast<float *>(scale), numel, fine8);
+        else launch(fp8_quantize_kernel<DT, kChunkLoads>, dim3(uint32_t(chunks8 * 8)), dim3(256), 0, stream, x, amax, int(partials), static_cast<uint8_t *>(codes),
+                    static_cast<float *>(scale), numel, chunks8);
     });
     QMM_ENTRY_END
 }

@@ -119,6 +119,23 @@ def test_fp8_per_tensor_of_a_few_rows(numel, dtype):
     assert scale.item() == float(np.asarray(s0).reshape(-1)[0])
 
 
+# 16-bit inputs whose quotients are often rounding boundaries of the format (448 or 3/4 of it, by powers of two) or one float32 away
+# from one; the largest sizes of one launch and of one vector per thread, and the first behind them
+@pytest.mark.parametrize('numel', [65536, 65544, 2048 * 2048, 2048 * 2048 + 8])
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_fp8_per_tensor_of_ties(numel, dtype):
+    announce('fp8 ties', numel, dtype)
+    rng = np.random.default_rng(numel)
+    for amax in (5.125, 3.5, 7.9375, 1.0):
+        x = amax * np.exp2(-rng.integers(0, 19, numel)) * rng.choice([1, 3 / 4, 1 / 2, 17 / 28, 5 / 7, 25 / 28, 31 / 32, 0.9], numel)
+        x = (x * rng.choice([-1, 1], numel)).astype(np.float32)
+        x[numel // 2] = amax
+        t = dev(x).to(dtype)
+        codes, scale = F8.fp8_quantize_per_tensor(t)
+        c0, s0 = O.fp8_quantize_per_tensor(t.float().cpu().numpy())
+        assert np.float32(scale.item()) == s0 and np.array_equal(codes.view(torch.uint8).cpu().numpy(), c0)
+
+
 # an empty reduction: scales of zero, and nothing behind the last of them (a number of 16-bit scales that fills no whole word)
 @pytest.mark.parametrize('count', [1, 3, 256, 257])
 @pytest.mark.parametrize('start', [0, 1])
