@@ -324,19 +324,29 @@ __device__ __forceinline__ void load4_as_f32(const void *p, int64_t i4, float (&
 
 // Columns of [outer, R, inner] quantized from their maxima (`ranges` <= kMaxRanges rows of them, amax_strided_kernel):
 // kQuantLanes row lanes x 64 column quads. The workgroup puts its columns' maxima together, a thread works out the scales
-// of its four columns once and takes 8 rows, four 16-byte loads in flight together. Block x counts column blocks, then row
-// blocks of kQuantRows; z = outer. 64 rows per workgroup pay for the maxima and scales (16: 51 us); all eight loads of a
+// of its four columns once and takes TRIPS times TRIP rows, a trip's 16-byte loads in flight together (a single trip's go out before
+// the maxima are read). Block x counts column blocks, then row blocks of kQuantLanes * TRIP * TRIPS; z = outer. Of a large matrix 64 rows per workgroup pay for
+// the maxima and scales (16: 40 - 51 us); all eight loads of a
 // thread at once cost the occupancy that hides them (16-bit types: 44 instead of 28 us). K = 4096, N = 11008: float32 35 - 36 us
 // (the second read comes from the last-level cache: 6.3 TB/s), bfloat16 36 -> 28 us (the divisions).
 constexpr int kQuantLanes = 8, kQuantTrip = 4, kQuantRows = 2 * kQuantLanes * kQuantTrip, kMaxRanges = 32;
-template <int DT, int QT>
+template <int DT, int QT, int TRIP, int TRIPS>
 __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const void *__restrict__ w, const float *__restrict__ amax, int ranges,
                                                                          int64_t nscale, void *__restrict__ q, void *__restrict__ scale,
                                                                          int64_t R, int64_t inner, uint32_t col_blocks) {
     __shared__ float4_t red[kQuantLanes][64];
+    constexpr int kRows = kQuantLanes * TRIP * TRIPS;
     const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // a wave's row is a scalar
-    const int64_t col = int64_t(blockIdx.x % col_blocks) * 256 + 4 * tx, row0 = int64_t(blockIdx.x / col_blocks) * kQuantRows;
-    const int64_t o = blockIdx.z, count = inner - col;
+    const int64_t col = int64_t(blockIdx.x % col_blocks) * 256 + 4 * tx, row0 = int64_t(blockIdx.x / col_blocks) * kRows;
+    const int64_t o = blockIdx.z, count = inner - col, r_end = min(R, row0 + kRows);
+    int64_t r = row0 + ty;
+    float x[TRIP][4];
+    auto load = [&] {
+#pragma unroll
+        for (int j = 0; j < TRIP; ++j)
+            if (count > 0 && r + kQuantLanes * j < r_end) load_upto4<DT>(w, (o * R + r + kQuantLanes * j) * inner + col, count, x[j]);
+    };
+    if constexpr (TRIPS == 1) load();
     float m[4] = {0.f, 0.f, 0.f, 0.f};
     if (count > 0) {
         for (int i = ty; i < ranges; i += kQuantLanes) {
@@ -356,20 +366,16 @@ __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const v
     float s[4], inv[4];
     const bool fast = scales4<DT, QT>(m, s, inv);
     if (row0 == 0 && ty == 0) store_upto4<DT>(scale, o * inner + col, count, s);
-    const int64_t r_end = min(R, row0 + kQuantRows);
-    for (int64_t r = row0 + ty; r < r_end; r += kQuantLanes * kQuantTrip) {
-        const int64_t base = (o * R + r) * inner;
-        float x[kQuantTrip][4];
+    for (; r < r_end; r += kQuantLanes * TRIP) {
+        if constexpr (TRIPS > 1) load();
 #pragma unroll
-        for (int j = 0; j < kQuantTrip; ++j)
-            if (r + kQuantLanes * j < r_end) load_upto4<DT>(w, base + kQuantLanes * j * inner + col, count, x[j]);
-#pragma unroll
-        for (int j = 0; j < kQuantTrip; ++j) {
+        for (int j = 0; j < TRIP; ++j) {
             if (r + kQuantLanes * j >= r_end) break;
             uint32_t code[4];
             codes4<DT, QT>(x[j], s, inv, fast, code);
-            store_codes_upto4<QT>(q, base + kQuantLanes * j * inner + col, count, code);
+            store_codes_upto4<QT>(q, (o * R + r + kQuantLanes * j) * inner + col, count, code);
         }
+        if constexpr (TRIPS == 1) break;
     }
 }
 
@@ -393,36 +399,37 @@ __global__ __launch_bounds__(256) void quantize_long_row_kernel(const void *__re
 }
 
 // inner == 1 (one scale per row, e.g. an embedding table): one workgroup per row keeps the whole row in registers
-// between the amax pass and the quantization, so the tensor is read once. Rows of up to 256 * 4 * NV elements, a
+// between the amax pass and the quantization, so the tensor is read once. Rows of up to T * 4 * NV elements, a
 // multiple of 4, 16-byte aligned. Same arithmetic as above.
-template <int DT, int QT, int NV>
-__global__ __launch_bounds__(256) void quantize_row_fused_kernel(const void *__restrict__ w, void *__restrict__ q,
+template <int DT, int QT, int T, int NV>
+__global__ __launch_bounds__(T) void quantize_row_fused_kernel(const void *__restrict__ w, void *__restrict__ q,
                                                                  void *__restrict__ scale, int64_t R4) {
-    __shared__ float red[4];
+    __shared__ float red[T / 64];
     const int tid = threadIdx.x;
     const int64_t base4 = int64_t(blockIdx.x) * R4;
     float x[NV][4];
     float m = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int64_t j = int64_t(v) * 256 + tid;
+        const int64_t j = int64_t(v) * T + tid;
         x[v][0] = x[v][1] = x[v][2] = x[v][3] = 0.0f;
         if (j < R4) load4_as_f32<DT>(w, base4 + j, x[v]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(x[v][e]));
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    m = wave_max(m);
     if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < T / 64; ++i) m = fmaxf(m, red[i]);
     const float mm[4] = {m, m, m, m};
     float s[4], inv[4];
     const bool fast = scales4<DT, QT>(mm, s, inv);
     if (tid == 0) store_from_f32<DT>(scale, blockIdx.x, s[0]);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int64_t j = int64_t(v) * 256 + tid;
+        const int64_t j = int64_t(v) * T + tid;
         if (j >= R4) continue;
         uint32_t code[4];
         codes4<DT, QT>(x[v], s, inv, fast, code);
@@ -852,10 +859,18 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
     };
     if (inner == 1) {
         // rows that fit a workgroup's registers: one pass
-        if (reduce % 4 == 0 && reduce <= 256 * 4 * 16 && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
+        if (reduce % 4 == 0 && reduce <= 4 * 4 * 1024 && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
             const dim3 grid{uint32_t(outer)};
-            if (reduce <= 256 * 4 * 4) go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 4>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 4>, grid, 256, w, wq, scale, reduce / 4);
-            else go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, 16>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, 16>, grid, 256, w, wq, scale, reduce / 4);
+            auto run = [&](auto threads, auto vectors) {
+                constexpr int T = decltype(threads)::value, NV = decltype(vectors)::value;
+                go(quantize_row_fused_kernel<DT, HIDET_QMM_I8, T, NV>, quantize_row_fused_kernel<DT, HIDET_QMM_I16, T, NV>, grid, T, w, wq, scale, reduce / 4);
+            };
+            using std::integral_constant;
+            // (four quads per thread: sixteen of 256 threads are code that comes from memory line by line; 4096 x 11008 bfloat16 40 -> 33.5 us,
+            // 512 x 11008 10.2 -> 7.0, 1024 x 6144 9.6 -> 7.3; float32 56.8 -> 50, 8.2 -> 8.0, 10.8 -> 8.6)
+            if (reduce <= 4 * 4 * 256) run(integral_constant<int, 256>(), integral_constant<int, 4>());
+            else if (reduce <= 4 * 4 * 512) run(integral_constant<int, 512>(), integral_constant<int, 4>());
+            else run(integral_constant<int, 1024>(), integral_constant<int, 4>());
             return;
         }
         launch(amax_contig_kernel<DT>, dim3(cdiv(outer, 4)), dim3(256), 0, stream, w, amax, outer, reduce);
@@ -868,6 +883,19 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
     QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
     const int64_t spare = scratch_bytes / (nscale * 4) - 1;  // rows of maxima the scratch memory holds beside the final ones
     float *partials = amax + nscale;
+    auto quantize = [&](int ranges) {
+        auto run = [&](auto i8, auto i16, int64_t rows) {
+            go(i8, i16, dim3(uint32_t(col_blocks * cdiv(reduce, rows)), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, ranges, nscale, wq, scale, reduce, inner,
+               uint32_t(col_blocks));
+        };
+        // Small matrices: more workgroups, each a shorter chain with its loads in front of the maxima, until what every workgroup
+        // spends on maxima and scales costs more (16, 32 and 64 rows, float32: 600 x 600 3.9, 4.4, 5.4 us; 1024 x 1024 4.3, 4.8, 5.8; 2048 x 4096
+        // 9.8, 9.0, 8.8; bfloat16: 1500 x 2432 7.0, 6.4, 8.4; 4096 x 4096 17.6, 14.5, 12.7).
+        const int64_t groups = col_blocks * row_blocks * outer;
+        if (groups <= 128) run(quantize_rows_kernel<DT, HIDET_QMM_I8, 2, 1>, quantize_rows_kernel<DT, HIDET_QMM_I16, 2, 1>, 2 * kQuantLanes);
+        else if (groups <= 384) run(quantize_rows_kernel<DT, HIDET_QMM_I8, 4, 1>, quantize_rows_kernel<DT, HIDET_QMM_I16, 4, 1>, 4 * kQuantLanes);
+        else run(quantize_rows_kernel<DT, HIDET_QMM_I8, kQuantTrip, 2>, quantize_rows_kernel<DT, HIDET_QMM_I16, kQuantTrip, 2>, kQuantRows);
+    };
     if (narrow_inner(inner)) {
         // Four workgroups per CU, of 2048 elements at least (1000000 x 9, float32: 32 workgroups and the column-quad kernel 216 us, these
         // and the flat one 30).
@@ -881,8 +909,7 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
                inner, total);
             return;
         }
-        go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
-           dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, 1, nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
+        quantize(1);
         return;
     }
     // Workgroups of 256 columns where 16 row ranges of them are two workgroups per CU, else of 64, which need a quarter of the
@@ -905,8 +932,7 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
         launch(amax_strided_kernel<HIDET_QMM_F32, 16>, dim3(uint32_t(cdiv(nscale, 64))), dim3(kAmaxThreads), 0, stream, partials, amax, ranges, nscale, ranges, nscale);
         ranges = 1;
     }
-    go(quantize_rows_kernel<DT, HIDET_QMM_I8>, quantize_rows_kernel<DT, HIDET_QMM_I16>,
-       dim3(uint32_t(col_blocks * row_blocks), 1, uint32_t(outer)), 64 * kQuantLanes, w, amax, int(ranges), nscale, wq, scale, reduce, inner, uint32_t(col_blocks));
+    quantize(int(ranges));
 }
 // Slices of a launch: a grid has 65535 layers, and 2^32 threads along x.
 inline int64_t quantize_slices_most(int64_t reduce, int64_t inner) {

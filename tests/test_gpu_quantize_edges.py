@@ -27,7 +27,9 @@ def _near_ties(rng, shape, axis, qmax):
 @pytest.mark.parametrize('dtype', ['float32', 'float16', 'bfloat16'])
 @pytest.mark.parametrize('shape,dim,codes', [((1, 3), 0, 'int8'), ((63, 255), 0, 'int8'), ((65, 257), 0, 'int16'), ((4100, 1026), 0, 'int8'),
                                              ((129, 6), 0, 'int8'), ((3, 2049, 130), 1, 'int8'), ((33, 16387), 1, 'int8'), ((5, 4100), 1, 'int16'),
-                                             ((520, 66, 9), 1, 'int8'), ((521, 3, 7), 1, 'int16'), ((9, 130, 63), 1, 'int8'), ((513, 5, 64), 1, 'int8'), ((513, 300, 2), 1, 'int8'), ((3, 2100, 95), 1, 'int8'), ((600, 9, 96), 1, 'int8'),
+                                             ((520, 66, 9), 1, 'int8'), ((521, 3, 7), 1, 'int16'), ((9, 130, 63), 1, 'int8'), ((513, 5, 64), 1, 'int8'), ((513, 300, 2), 1, 'int8'), ((3, 4096), 1, 'int8'), ((3, 8192), 1, 'int16'), ((3, 8196), 1, 'int8'), ((2, 16384), 1, 'int8'), ((2, 16388), 1, 'int8'),
+                                             # 2, 4 and 8 rows per thread: the last matrices of one form and the first of the next
+                                             ((17, 1026), 0, 'int8'), ((8192, 256), 0, 'int8'), ((8193, 256), 0, 'int16'), ((1025, 6144), 0, 'int8'), ((1024, 6146), 0, 'int8'), ((2, 65, 514), 1, 'int8'), ((3, 2100, 95), 1, 'int8'), ((600, 9, 96), 1, 'int8'),
                                              # tall: many row ranges, whose maxima one more launch puts together
                                              ((50001, 9), 0, 'int8'), ((2, 30000, 3), 1, 'int16'), ((20000, 95), 0, 'int8'), ((70001, 66), 0, 'int8'), ((70000, 130), 0, 'int8'),
                                              ((2, 20000, 260), 1, 'int8'), ((2, 66000, 96), 1, 'int8')])
