@@ -1007,12 +1007,13 @@ HIDET_API void hidet_symmetric_dequantize(const void *wq, const void *scale, voi
             else launch(dequantize_long_row_kernel<HIDET_QMM_I16, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, uint32_t(blocks));
             return;
         }
-        // The kernel that gives a column quad to a lane where nine tenths of its lanes have one and, in float32, there are workgroups
-        // for four rounds of the chip's at a time (a thread's eight rows are a chain). us, flat against that: float32 400000 x 192 76 and 77, 200000 x 384
+        // The kernel that gives a column quad to a lane where nine tenths of its lanes have one and there are workgroups enough: a
+        // thread's eight rows are a chain, in float32 for four rounds of the chip's at a time. us, flat against that: float32 400000 x 192 76 and 77, 200000 x 384
         // 76 and 90, 4096 x 4096 13.5 and 16.2, 250000 x 256 64 and 55, 4096 x 11008 42 and 37; bfloat16 500000 x 128 50 and 64,
-        // 200000 x 320 50 and 59, 250000 x 256 50 and 39, 4096 x 4096 13.6 and 9.6.
+        // 200000 x 320 50 and 59, 250000 x 256 50 and 39, 4096 x 4096 13.6 and 9.6, 2048 x 4096 8.2 and 7.7, 1500 x 2432 4.9 and 5.4,
+        // 1024 x 1024 2.8 and 5.0.
         const int64_t lanes = cdiv(inner, 256) * 256, groups = cdiv(inner, 256) * cdiv(reduce, kDequantRows) * outer;
-        if (outer > 65535 || ((inner * 10 < lanes * 9 || (ST == HIDET_QMM_F32 && inner % 4 == 0 && groups < 4096)) && cdiv(total, 1024) < (int64_t(1) << 24))) {
+        if (outer > 65535 || ((inner * 10 < lanes * 9 || (inner % 4 == 0 && groups < (ST == HIDET_QMM_F32 ? 4096 : 512))) && cdiv(total, 1024) < (int64_t(1) << 24))) {
             QMM_CHECK(cdiv(total, 1024) < (int64_t(1) << 31), "tensor too large for one launch");
             const dim3 grid{uint32_t(cdiv(total, 1024))};
             if (q_dtype == HIDET_QMM_I8) launch(dequantize_flat_kernel<HIDET_QMM_I8, ST>, grid, dim3(256), 0, stream, wq, scale, w, reduce, inner, total);
