@@ -27,14 +27,15 @@ using namespace qmm;
 namespace {
 
 constexpr int64_t kPanelK = 256;    // from this depth on panels of a padded weight beat the element-wise kernel on few rows
+constexpr int64_t kElementWise = int64_t(1) << 20;  // products up to which a matrix is tiny
 constexpr int64_t kMidRows = 1024;  // above, the prefill GEMM's tiles fill the chip on every shape
 
 // ---- operands of sizes or alignments the matrix kernels do not take --------------------------------------------------
 //
 // Copies of the operands with rows of whole 16 (weight, factors) and 64 (activations) elements, zero past the originals,
 // in the scratch memory: columns [n0, n0 + cols) of w[k, n] as [kp, np], the float16 activations [m, k] as [m, kp], the
-// column factors as [np]. One thread per 16 bytes written. 203 rows x 4100 x 4098 take 29 us in all (18 us of them the GEMM),
-// where the element-wise kernel that served such sizes before took 1815 us; one row x 4100 x 4098 20 us.
+// column factors as [np]. One thread per 16 bytes written. For odd N or K, and for N = 4 i + 2 above kMidRows: 203 rows x 4100 x 4098 took 29 us
+// in all this way (18 us of them the GEMM; 20 as they lie on the narrow tiles), element by element 1815.
 struct PadArgs {
     const int8_t *w;
     const _Float16 *a, *scale, *bias;
@@ -141,6 +142,11 @@ bool w8a16_padded(bool gemm, const void *a, const void *w, const void *scale, co
     return true;
 }
 
+// What the copy and the prefill tiles take together (the copy: 4100 x 4098 10.9 us, 1026 x 2050 4.0).
+double padded_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws) {
+    return 3.0 + double(k) * double(n) / 2.15e6 + gemm_w8a16_estimate_us(m, cdiv(k, 64) * 64, cdiv(n, 16) * 16, ws);
+}
+
 // Checks and kernel choice shared by the two row-major entry points. `strict_workspace`: a bandwidth-bound launch whose
 // K split does not fit the scratch memory is an error instead of a launch with fewer K slices.
 void w8a16_dispatch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
@@ -160,7 +166,7 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     // 20.6 / 29.2 / 39.1; at M=512 64 against 57; a wide weight, 4096 x 57344: narrow 54 / 65 us at M=17 / 64, prefill tiles 46 / 52). For 9 to 16 rows the bandwidth-bound kernel is
     // ahead of the GEMM on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
     // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49).
-    if (m > 16 && k > 0) {
+    if (m > 16 && k > 0 && n % 4 != 2) {
         const bool gemm = gemm_w8a16_supported(a, w, c, m, k, n, lda);
         const double limit = gemm ? gemm_w8a16_estimate_us(m, k, n, ws) : 1e29;
         if (m <= kMidRows && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, limit, ws, stream)) return;
@@ -169,11 +175,18 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
             return;
         }
     }
+    // N = 4 i + 2 on the narrow tiles as it lies, also for one pass of 16 rows (which the bandwidth-bound kernel takes on a copy only),
+    // unless the copy and the prefill tiles are estimated to take less. us, on copies against that: 1 x 1026 x 2050 14.0 and 7.6, 16 x 4096 x 4098
+    // 21.3 and 11.1, 203 x 4096 x 4098 27.9 and 20.4, 600 x 4096 x 4098 45 and 37, 16 x 8192 x 8190 35 and 18; 1 x 2002 x 514 element by element 193
+    // and 7.7 (0.1 us per k whatever else).
+    if (n % 4 == 2 && k > 0 && m <= kMidRows && (k >= 64 || m * k * n > kElementWise) &&
+        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, padded_estimate_us(m, k, n, ws), ws, stream))
+        return;
     // Sizes the GEMM does not take (K no multiple of 64, N of 4): up to 32 rows two passes of the bandwidth-bound kernel,
     // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the
     // copy. Tiny matrices are left to the element-wise kernel.
     const bool skinny = skinny_w8a16_supported(w, scale, bias, k, n);
-    if (k > 0 && (!skinny || m > 32) && m * k * n > (int64_t(1) << 20)) {
+    if (k > 0 && (!skinny || m > 32) && m * k * n > kElementWise) {
         if (m <= 16 && w8a16_padded(false, a, w, scale, bias, c, m, k, n, lda, ws, stream)) return;
         // Up to 16 rows of a weight whose copy does not fit the scratch memory whole: panels for the GEMM (8192 x 8190, one row: 52 us,
         // element by element 3037; 256 x 300002 60 and 101; at a depth of 64 such a weight has threads enough for the latter).

@@ -92,6 +92,7 @@ struct MidCfg {
     static constexpr int kGroups = kMidWaves / kGroupWaves;
     static constexpr int kWaveCols = kFrags * 16;
     static constexpr int kCols = kGroupWaves * kWaveCols;
+    static constexpr int kPitch = kCols - Op::kSpare;          // columns from one tile to the next
     static constexpr int kRowBytes = Op::kRowBytes;            // bytes of an activation row per stage
     static constexpr int kChunks = kRowBytes / 16;
     static constexpr int kABytes = RB * 16 * kRowBytes;
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 
     MidItem item;
     if (!mid_item(plan, int(blockIdx.x), &item)) return;
-    const int m0 = item.tile_m * (RB * 16), n0 = item.tile_n * Cfg::kCols;
+    const int m0 = item.tile_m * (RB * 16), n0 = item.tile_n * Cfg::kPitch;
     const int rows = plan.m - m0 < RB * 16 ? plan.m - m0 : RB * 16;
 
     // ---- main loop ----------------------------------------------------------------------------------------------
@@ -414,7 +415,7 @@ struct MidChoice {
 template <class Op, int RB, int DEPTH>
 MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_t n, int64_t k) {
     using Cfg = MidCfg<Op, RB, DEPTH>;
-    const int64_t tiles = cdiv(m, RB * 16) * cdiv(n, Cfg::kCols), stages = cdiv(k, Op::kStageK), cus = std::max(1, device_cus());
+    const int64_t tiles = cdiv(m, RB * 16) * cdiv(n, Cfg::kPitch), stages = cdiv(k, Op::kStageK), cus = std::max(1, device_cus());
     int64_t most = 8;
     if (ws.counters == nullptr || tiles > cus) most = 1;
     else most = std::min(most, ws.scratch_bytes / (tiles * Cfg::kTileFloats * 4));
@@ -436,7 +437,7 @@ template <class Op, int RB, int DEPTH>
 void mid_launch(const MidChoice &choice, const void *a, const void *w, int64_t a_stride, int64_t w_stride, const typename Op::Args &args,
                 int64_t m, int64_t n, int64_t k, const Workspace &ws, hipStream_t stream) {
     using Cfg = MidCfg<Op, RB, DEPTH>;
-    const int64_t tiles_m = cdiv(m, RB * 16), tiles_n = cdiv(n, Cfg::kCols), items = tiles_m * tiles_n * choice.parts;
+    const int64_t tiles_m = cdiv(m, RB * 16), tiles_n = cdiv(n, Cfg::kPitch), items = tiles_m * tiles_n * choice.parts;
     QMM_CHECK(items < (int64_t(1) << 28), "problem too large for one launch");
     static_assert(256 * 4 * 4 <= kCounterBytes / 2, "one counter per tile that is cut");
     allow_dynamic_lds(reinterpret_cast<const void *>(gemm_mid_kernel<Op, RB, DEPTH>), Cfg::kLdsBytes);

@@ -26,6 +26,7 @@ struct MidF8 {
     static constexpr int kStageK = 128;
     static constexpr int kGroupWaves = 4;
     static constexpr int kFrags = 2;
+    static constexpr int kSpare = 0;
     static constexpr int kFactorBytes = SCALED ? 256 * ((RB + 3) / 4) : 0;  // of a wave: the stage's factors of its rows
     static constexpr int kWLdsBytes = 128 * 128 + kGroupWaves * kFactorBytes;
     static constexpr int kRowBytes = 128;

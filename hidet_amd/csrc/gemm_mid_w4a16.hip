@@ -30,6 +30,7 @@ struct MidW4 {
     static constexpr int kStageK = 32;
     static constexpr int kGroupWaves = 2;
     static constexpr int kFrags = 4;
+    static constexpr int kSpare = 0;
     static constexpr int kCodeBytes = 32 * 64;                     // 32 rows of 128 columns
     static constexpr int kWLdsBytes = kCodeBytes + kGroupWaves * 256;  // and the scales of each wave's 64 columns
     static constexpr int kRowBytes = 64;

@@ -12,7 +12,10 @@ struct MidW8Args {
     int vector_out;    // rows of c start at multiples of 8 bytes and end with a lane's four columns
 };
 
-template <bool NK>
+// SHIFTED: row-major weights of N = 4 i + 2. Their odd rows start between two dwords, which direct-to-LDS loads cannot; they are loaded
+// from two bytes in front, so that in LDS a lane's four columns of an odd row lie across two dwords. The second of them is one more read, and the
+// last lane's is missing: a tile has 124 columns. (A copy of the weight with rows of whole dwords, for the plain form: 4100 x 4098 11 us.)
+template <bool NK, bool SHIFTED = false>
 struct MidW8 {
     using Args = MidW8Args;
     // Row-major: a stage is 32 rows of 128 columns, so that memory is read in whole 128-byte lines (64-byte pieces reached
@@ -22,30 +25,33 @@ struct MidW8 {
     static constexpr int kStageK = NK ? 64 : 32;
     static constexpr int kGroupWaves = NK ? 1 : 2;
     static constexpr int kFrags = 4;
+    static constexpr int kSpare = SHIFTED ? 4 : 0;
     static constexpr int kWLdsBytes = NK ? 0 : 32 * 128;
     static constexpr int kRowBytes = kStageK * 2;
     static constexpr int kAChunks = NK ? 2 : 1;
     static constexpr int kWLoads = NK ? 4 : 2;
     struct Weights {
         uint32_t u[NK ? 16 : 1];
-        uint64_t pair[4];
+        uint64_t pair[SHIFTED ? 6 : 4];
     };
     struct Fragments {
         half8_t h[kAChunks][4];
     };
     static constexpr int kMfmas = 4;      // per row block
-    static constexpr int kWidenOps = 48;  // VALU instructions of widen()
+    static constexpr int kWidenOps = SHIFTED ? 52 : 48;  // VALU instructions of widen()
     int side_;
     __amdgpu_buffer_rsrc_t rsrc;
     int w_stage;       // bytes from one stage to the next
     int w_off[NK ? 4 : 2];
     uint32_t w_read;   // LDS address of this lane's first dword in a slot's weights (row-major)
     uint32_t sel[4];   // byte gathers of the columns
+    uint32_t w_odd, w_next;  // SHIFTED: addresses of the lane's dword in the first odd row and of the one behind it
+    int limit;         // columns from here on are not this tile's
     const MidW8Args &args;
     int k;
     half4_t scale4, bias4;
 
-    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int, int n, int, int n0, int side, int lane) : side_(side), args(x), k(depth) {
+    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int, int n, int, int n0, int side, int lane) : side_(side), limit(SHIFTED && x.n_out > n0 + 124 ? n0 + 124 : x.n_out), args(x), k(depth) {
         const int kg = lane >> 4, ns = lane & 15;
         if constexpr (NK) {
             const int base = n0 < n - 4 ? n0 : n - 4, col = n0 + ns * 4 < n - 4 ? n0 + ns * 4 : n - 4;
@@ -62,9 +68,18 @@ struct MidW8 {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int blk = 2 * side + i, at = lane ^ (4 * blk);
-                w_off[i] = (8 * blk + (at >> 3)) * n + n0 + (at & 7) * 16;
+                w_off[i] = (8 * blk + (at >> 3)) * n + n0 + (at & 7) * 16 - (SHIFTED ? 2 * ((at >> 3) & 1) : 0);
             }
-            w_read = uint32_t(kg * 1024 + ((side * 4 + (ns >> 2)) ^ ((kg & 1) * 4)) * 16 + (ns & 3) * 4);
+            auto position = [&](int row, int dword) { return uint32_t(kg * 1024 + row * 128 + ((dword >> 2) ^ ((kg & 1) * 4)) * 16 + (dword & 3) * 4); };
+            const int dword = side * 16 + ns, swapped = kg >> 1;
+            w_read = position(SHIFTED ? swapped : 0, dword);
+            if constexpr (SHIFTED) {
+                w_odd = position(swapped ^ 1, dword);
+                w_next = position(swapped ^ 1, dword < 31 ? dword + 1 : dword);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sel[t] = 0x0c000c00u | (uint32_t(4 + t) << 16) | uint32_t(t);
+                return;
+            }
 #pragma unroll
             for (int t = 0; t < 4; ++t) sel[t] = 0x0c000c00u | (kg >= 2 ? (uint32_t(t) << 16) | uint32_t(4 + t) : (uint32_t(4 + t) << 16) | uint32_t(t));
         }
@@ -84,8 +99,15 @@ struct MidW8 {
     __device__ __forceinline__ void factors(int col) {
         bias4 = half4_t{_Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f)};
         scale4 = bias4;
-        if (col >= args.n_out) return;
-        if (args.vector_out) {
+        if (col >= limit) return;
+        if (SHIFTED) {
+#pragma unroll
+            for (int t = 0; t < 4; t += 2)
+                if (col + t < limit) {  // (N is even)
+                    __builtin_memcpy(reinterpret_cast<_Float16 *>(&scale4) + t, args.scale + col + t, 4);
+                    if (args.bias != nullptr) __builtin_memcpy(reinterpret_cast<_Float16 *>(&bias4) + t, args.bias + col + t, 4);
+                }
+        } else if (args.vector_out) {
             __builtin_memcpy(&scale4, args.scale + col, 8);
             if (args.bias != nullptr) __builtin_memcpy(&bias4, args.bias + col, 8);
         } else {
@@ -97,8 +119,20 @@ struct MidW8 {
                 }
         }
     }
-    // rows j and j + 1 of the lane's eight, 128 bytes apart
+    // rows j and j + 1 of the lane's eight, 128 bytes apart; SHIFTED: rows 0, 2 and 4, 6, then 1, 3 and 5, 7 and the dwords behind those
     __device__ __forceinline__ void read(Weights &dst, uint32_t at) const {
+        if constexpr (SHIFTED) {
+            const uint32_t from[3] = {w_read + at, w_odd + at, w_next + at};
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                uint64_t lo, hi;
+                asm volatile("ds_read2_b32 %0, %1 offset0:0 offset1:64" : "=v"(lo) : "v"(from[i]));
+                asm volatile("ds_read2_b32 %0, %1 offset0:128 offset1:192" : "=v"(hi) : "v"(from[i]));
+                dst.pair[2 * i] = lo;
+                dst.pair[2 * i + 1] = hi;
+            }
+            return;
+        }
         uint64_t v[4];
         asm volatile("ds_read2_b32 %0, %1 offset0:0 offset1:32" : "=v"(v[0]) : "v"(w_read + at));
         asm volatile("ds_read2_b32 %0, %1 offset0:64 offset1:96" : "=v"(v[1]) : "v"(w_read + at));
@@ -119,9 +153,18 @@ struct MidW8 {
     }
     template <int NEWER>
     static __device__ __forceinline__ void settle(Weights &raw) {
-        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]) : "n"(NEWER));
+        if constexpr (SHIFTED)
+            asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]), "+v"(raw.pair[4]), "+v"(raw.pair[5]) : "n"(NEWER));
+        else
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]) : "n"(NEWER));
     }
     __device__ __forceinline__ void widen(const Weights &raw, Fragments &b, int) const {
+        auto dword = [&](int i, int p) { return uint32_t(p & 1 ? raw.pair[i + p / 2] >> 32 : raw.pair[i + p / 2]); };
+        uint32_t odd[4];
+        if constexpr (SHIFTED) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) odd[p] = __builtin_amdgcn_alignbyte(dword(4, p), dword(2, p), 2);
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             uint32_t u[4];
@@ -137,7 +180,8 @@ struct MidW8 {
                 }
             } else {
 #pragma unroll
-                for (int p = 0; p < 4; ++p) u[p] = __builtin_amdgcn_perm(uint32_t(raw.pair[p] >> 32), uint32_t(raw.pair[p]), sel[t]);
+                for (int p = 0; p < 4; ++p)
+                    u[p] = SHIFTED ? __builtin_amdgcn_perm(odd[p], dword(0, p), sel[t]) : __builtin_amdgcn_perm(uint32_t(raw.pair[p] >> 32), uint32_t(raw.pair[p]), sel[t]);
                 b.h[0][t] = minus_1152(u);
             }
         }
@@ -162,12 +206,16 @@ struct MidW8 {
             for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, af[q]), b.h[q][t], acc[t], 0, 0, 0);
     }
     __device__ __forceinline__ void store(int row, int col, const float (&v)[4]) const {
-        if (col >= args.n_out) return;
+        if (col >= limit) return;
         half4_t o;
 #pragma unroll
         for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t], float(scale4[t]), float(bias4[t]));
         _Float16 *dst = args.c + int64_t(row) * args.ldc + col;
-        if (args.vector_out) {
+        if (SHIFTED) {
+#pragma unroll
+            for (int t = 0; t < 4; t += 2)
+                if (col + t < limit) __builtin_memcpy(dst + t, reinterpret_cast<const _Float16 *>(&o) + t, 4);
+        } else if (args.vector_out) {
             *reinterpret_cast<half4_t *>(dst) = o;
         } else {
 #pragma unroll
@@ -175,6 +223,11 @@ struct MidW8 {
                 if (col + t < args.n_out) dst[t] = o[t];
         }
     }
+};
+
+template <typename T>
+struct Form {
+    using type = T;
 };
 
 }  // namespace
@@ -190,7 +243,8 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
     // activations lies half outside their buffer (it would read as zero: K is even); what a tile reads lies within 2 GiB
     // (kMidOutside)
     constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
-    if (n % 4 != 0 || k % 2 != 0 || lda % 2 != 0 || !aligned(a, 4) || !aligned(w, 4) || lda * 256 + k * 2 >= kMost || ldc >= kMost) return false;
+    const bool shifted = !nk && n % 4 == 2 && n_out == n;
+    if ((n % 4 != 0 && !shifted) || k % 2 != 0 || lda % 2 != 0 || !aligned(a, 4) || !aligned(w, 4) || lda * 256 + k * 2 >= kMost || ldc >= kMost) return false;
     const int64_t las = lda * 2;
     if (nk) {
         if (ldw % 4 != 0 || ldw * 64 + k >= kMost) return false;
@@ -202,14 +256,18 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
     }
     if ((k + 64) * n >= kMost) return false;
     constexpr double kFullRound = 0.62;  // 256 pieces of 16 KiB at 6.8 TB/s
-    const MidChoice c2 = mid_choose<MidW8<false>, 2, 6>({5.5, 0.36, 1.4, 0.4, kFullRound}, ws, m, n, k), c4 = mid_choose<MidW8<false>, 4, 4>({6.0, 0.5, 1.5, 0.5, kFullRound}, ws, m, n, k),
-                    c8 = mid_choose<MidW8<false>, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
-    const double us = std::min({c2.us, c4.us, c8.us});
-    if ((us == c2.us ? c2 : us == c4.us ? c4 : c8).busy_us > limit_us) return false;
-    if (us == c2.us) mid_launch<MidW8<false>, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
-    else if (us == c4.us) mid_launch<MidW8<false>, 4, 4>(c4, a, w, las, n, args, m, n, k, ws, stream);
-    else mid_launch<MidW8<false>, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);
-    return true;
+    auto run = [&](auto form) {
+        using Op = typename decltype(form)::type;
+        const MidChoice c2 = mid_choose<Op, 2, 6>({5.5, 0.36, 1.4, 0.4, kFullRound}, ws, m, n, k), c4 = mid_choose<Op, 4, 4>({6.0, 0.5, 1.5, 0.5, kFullRound}, ws, m, n, k),
+                        c8 = mid_choose<Op, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
+        const double us = std::min({c2.us, c4.us, c8.us});
+        if ((us == c2.us ? c2 : us == c4.us ? c4 : c8).busy_us > limit_us) return false;
+        if (us == c2.us) mid_launch<Op, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
+        else if (us == c4.us) mid_launch<Op, 4, 4>(c4, a, w, las, n, args, m, n, k, ws, stream);
+        else mid_launch<Op, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);
+        return true;
+    };
+    return shifted ? run(Form<MidW8<false, true>>()) : run(Form<MidW8<false>>());
 }
 
 }  // namespace qmm

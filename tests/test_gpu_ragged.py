@@ -38,6 +38,24 @@ def test_int8_exact(m, k, n, biased):
         assert np.array_equal(host(quant.symmetric_quant_matmul(a, w, s, b)), want)
 
 
+# N = 4 i + 2 on the narrow tiles as it lies: one column pair to spare, one short of a tile and one more, two tiles and a pair; one to three
+# row blocks per wave group, K of less than a stage, of several pieces, ending inside a stage. Rows of the activations are followed by NaN, which
+# the last stage's reads bring along.
+@pytest.mark.parametrize('m,k,n,biased', [(1, 64, 2, False), (3, 66, 6, True), (17, 26, 4094, False), (1, 16390, 122, True), (2, 4096, 126, False), (16, 4098, 250, True), (33, 1030, 374, False),
+                                          (64, 2048, 1022, True), (65, 994, 2050, False), (128, 1000, 126, True), (131, 3000, 498, False), (1000, 130, 4098, True)])
+def test_int8_rows_off_the_dwords(m, k, n, biased):
+    announce('ragged int8 off the dwords', m, k, n, biased)
+    a, w, s, b, want = _int8_case(m, k, n, biased)
+    wide = torch.full((m, k + 6), float('nan'), dtype=torch.float16, device='cuda')
+    wide[:, :k] = a
+    ws = ffi.workspace(a.device)
+    for _ in range(2):
+        c = torch.full((m + 1, n), 7.0, dtype=torch.float16, device='cuda')
+        args = (wide, w, s, b, c) if biased else (wide, w, s, c)
+        ffi.call('hidet_symmetric_quant_matmul_f16_i8' + ('_bias' if biased else ''), *args, m, k, n, k + 6, 0, ws, ws.numel(), ffi.current_stream(a.device))
+        assert np.array_equal(host(c[:m]), want) and bool((c[m] == 7.0).all())
+
+
 @pytest.mark.parametrize('scratch', [1 << 20, 3 << 20])
 def test_int8_in_panels_of_a_small_workspace(scratch):
     announce('ragged int8 panels', scratch)
