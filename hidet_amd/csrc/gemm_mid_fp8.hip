@@ -24,6 +24,7 @@ struct MidF8 {
     using Args = MidF8Args;
     static constexpr int kElementBytes = 1;
     static constexpr int kStageK = 128;
+    static constexpr bool kKeep = false;
     static constexpr int kGroupWaves = 4;
     static constexpr int kFrags = 2;
     static constexpr int kSpare = 0;

@@ -23,6 +23,7 @@ struct MidW8 {
     // lane's 4 columns, straight into its registers.
     static constexpr int kElementBytes = 2;
     static constexpr int kStageK = NK ? 64 : 32;
+    static constexpr bool kKeep = false;
     static constexpr int kGroupWaves = NK ? 1 : 2;
     static constexpr int kFrags = 4;
     static constexpr int kSpare = SHIFTED ? 4 : 0;
