@@ -47,12 +47,12 @@ struct MidW8 {
     uint32_t w_read;   // LDS address of this lane's first dword in a slot's weights (row-major)
     uint32_t sel[4];   // byte gathers of the columns
     uint32_t w_odd, w_next;  // SHIFTED: addresses of the lane's dword in the first odd row and of the one behind it
-    int limit;         // columns from here on are not this tile's
+    int last_out;      // SHIFTED: columns from here on are not this tile's
     const MidW8Args &args;
     int k;
     half4_t scale4, bias4;
 
-    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int, int n, int, int n0, int side, int lane) : side_(side), limit(SHIFTED && x.n_out > n0 + 124 ? n0 + 124 : x.n_out), args(x), k(depth) {
+    __device__ __forceinline__ MidW8(const MidW8Args &x, const char *w, int ldw, int depth, int, int n, int, int n0, int side, int lane) : side_(side), args(x), k(depth) {
         const int kg = lane >> 4, ns = lane & 15;
         if constexpr (NK) {
             const int base = n0 < n - 4 ? n0 : n - 4, col = n0 + ns * 4 < n - 4 ? n0 + ns * 4 : n - 4;
@@ -71,20 +71,23 @@ struct MidW8 {
                 const int blk = 2 * side + i, at = lane ^ (4 * blk);
                 w_off[i] = (8 * blk + (at >> 3)) * n + n0 + (at & 7) * 16 - (SHIFTED ? 2 * ((at >> 3) & 1) : 0);
             }
-            auto position = [&](int row, int dword) { return uint32_t(kg * 1024 + row * 128 + ((dword >> 2) ^ ((kg & 1) * 4)) * 16 + (dword & 3) * 4); };
-            const int dword = side * 16 + ns, swapped = kg >> 1;
-            w_read = position(SHIFTED ? swapped : 0, dword);
             if constexpr (SHIFTED) {
+                last_out = x.n_out > n0 + 124 ? n0 + 124 : x.n_out;
+                auto position = [&](int row, int dword) { return uint32_t(kg * 1024 + row * 128 + ((dword >> 2) ^ ((kg & 1) * 4)) * 16 + (dword & 3) * 4); };
+                const int dword = side * 16 + ns, swapped = kg >> 1;
+                w_read = position(swapped, dword);
                 w_odd = position(swapped ^ 1, dword);
                 w_next = position(swapped ^ 1, dword < 31 ? dword + 1 : dword);
 #pragma unroll
                 for (int t = 0; t < 4; ++t) sel[t] = 0x0c000c00u | (uint32_t(4 + t) << 16) | uint32_t(t);
                 return;
             }
+            w_read = uint32_t(kg * 1024 + ((side * 4 + (ns >> 2)) ^ ((kg & 1) * 4)) * 16 + (ns & 3) * 4);
 #pragma unroll
             for (int t = 0; t < 4; ++t) sel[t] = 0x0c000c00u | (kg >= 2 ? (uint32_t(t) << 16) | uint32_t(4 + t) : (uint32_t(4 + t) << 16) | uint32_t(t));
         }
     }
+    __device__ __forceinline__ int limit() const { return SHIFTED ? last_out : args.n_out; }
     __device__ __forceinline__ void load(Weights &dst, uint32_t at) const {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -100,11 +103,11 @@ struct MidW8 {
     __device__ __forceinline__ void factors(int col) {
         bias4 = half4_t{_Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f), _Float16(-0.0f)};
         scale4 = bias4;
-        if (col >= limit) return;
+        if (col >= limit()) return;
         if (SHIFTED) {
 #pragma unroll
             for (int t = 0; t < 4; t += 2)
-                if (col + t < limit) {  // (N is even)
+                if (col + t < limit()) {  // (N is even)
                     __builtin_memcpy(reinterpret_cast<_Float16 *>(&scale4) + t, args.scale + col + t, 4);
                     if (args.bias != nullptr) __builtin_memcpy(reinterpret_cast<_Float16 *>(&bias4) + t, args.bias + col + t, 4);
                 }
@@ -207,7 +210,7 @@ struct MidW8 {
             for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, af[q]), b.h[q][t], acc[t], 0, 0, 0);
     }
     __device__ __forceinline__ void store(int row, int col, const float (&v)[4]) const {
-        if (col >= limit) return;
+        if (col >= limit()) return;
         half4_t o;
 #pragma unroll
         for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t], float(scale4[t]), float(bias4[t]));
@@ -215,7 +218,7 @@ struct MidW8 {
         if (SHIFTED) {
 #pragma unroll
             for (int t = 0; t < 4; t += 2)
-                if (col + t < limit) __builtin_memcpy(dst + t, reinterpret_cast<const _Float16 *>(&o) + t, 4);
+                if (col + t < limit()) __builtin_memcpy(dst + t, reinterpret_cast<const _Float16 *>(&o) + t, 4);
         } else if (args.vector_out) {
             *reinterpret_cast<half4_t *>(dst) = o;
         } else {
