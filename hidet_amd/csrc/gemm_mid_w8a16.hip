@@ -1,5 +1,5 @@
 // W8A16 on gemm_mid.h: c[m, n] = (sum_k a[m, k] * w[k, n]) * scale[n] (+ bias[n]), int8 weights widened exactly to float16
-// (0x6400 | (q ^ 0x80) is 1152 + q, one packed subtract removes the 1152), float16 MFMA, fp32 sums.
+// (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25, is q / 512), float16 MFMA, fp32 sums; the results are multiplied by 512.
 #include "gemm_mid.h"
 
 namespace qmm {
@@ -39,7 +39,7 @@ struct MidW8 {
         half8_t h[kAChunks][4];
     };
     static constexpr int kMfmas = 4;      // per row block
-    static constexpr int kWidenOps = SHIFTED ? 52 : 48;  // VALU instructions of widen()
+    static constexpr int kWidenOps = SHIFTED ? 44 : 40;  // VALU instructions of widen()
     int side_;
     __amdgpu_buffer_rsrc_t rsrc;
     int w_stage;       // bytes from one stage to the next
@@ -145,11 +145,12 @@ struct MidW8 {
 #pragma unroll
         for (int p = 0; p < 4; ++p) dst.pair[p] = v[p];
     }
-    static __device__ __forceinline__ half8_t minus_1152(const uint32_t (&u)[4]) {
+    // u: two bytes q ^ 0x80 below zero bytes (the xor is done four codes at a time, where 0x6480 in front of a subtraction takes one for two)
+    static __device__ __forceinline__ half8_t over_512(const uint32_t (&u)[4]) {
         half8_t out;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const half2_t v = __builtin_bit_cast(half2_t, u[p] ^ 0x64806480u) - half2_t{_Float16(1152.0f), _Float16(1152.0f)};
+            const half2_t v = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, u[p]), half2_t{_Float16(32768.0f), _Float16(32768.0f)}, half2_t{_Float16(-0.25f), _Float16(-0.25f)});
             out[2 * p] = v[0];
             out[2 * p + 1] = v[1];
         }
@@ -163,11 +164,15 @@ struct MidW8 {
             asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]) : "n"(NEWER));
     }
     __device__ __forceinline__ void widen(const Weights &raw, Fragments &b, int) const {
+        constexpr uint32_t kFlip = 0x80808080u;
         auto dword = [&](int i, int p) { return uint32_t(p & 1 ? raw.pair[i + p / 2] >> 32 : raw.pair[i + p / 2]); };
-        uint32_t odd[4];
-        if constexpr (SHIFTED) {
+        uint32_t lo[4], hi[4];  // rows 2 p and 2 p + 1
+        if constexpr (!NK) {
 #pragma unroll
-            for (int p = 0; p < 4; ++p) odd[p] = __builtin_amdgcn_alignbyte(dword(4, p), dword(2, p), 2);
+            for (int p = 0; p < 4; ++p) {
+                lo[p] = (SHIFTED ? dword(0, p) : uint32_t(raw.pair[p])) ^ kFlip;
+                hi[p] = (SHIFTED ? __builtin_amdgcn_alignbyte(dword(4, p), dword(2, p), 2) : uint32_t(raw.pair[p] >> 32)) ^ kFlip;
+            }
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -177,16 +182,15 @@ struct MidW8 {
                 for (int q = 0; q < 2; ++q) {  // bytes 8 q .. 8 q + 7 of the lane's sixteen
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
-                        const uint32_t src = raw.u[4 * t + 2 * q + p / 2];
+                        const uint32_t src = raw.u[4 * t + 2 * q + p / 2] ^ kFlip;
                         u[p] = __builtin_amdgcn_perm(src, src, (p & 1) ? 0x0c030c02u : 0x0c010c00u);
                     }
-                    b.h[q][t] = minus_1152(u);
+                    b.h[q][t] = over_512(u);
                 }
             } else {
 #pragma unroll
-                for (int p = 0; p < 4; ++p)
-                    u[p] = SHIFTED ? __builtin_amdgcn_perm(odd[p], dword(0, p), sel[t]) : __builtin_amdgcn_perm(uint32_t(raw.pair[p] >> 32), uint32_t(raw.pair[p]), sel[t]);
-                b.h[0][t] = minus_1152(u);
+                for (int p = 0; p < 4; ++p) u[p] = __builtin_amdgcn_perm(hi[p], lo[p], sel[t]);
+                b.h[0][t] = over_512(u);
             }
         }
     }
@@ -213,7 +217,7 @@ struct MidW8 {
         if (col >= limit()) return;
         half4_t o;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t], float(scale4[t]), float(bias4[t]));
+        for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t] * 512.0f, float(scale4[t]), float(bias4[t]));
         _Float16 *dst = args.c + int64_t(row) * args.ldc + col;
         if (SHIFTED) {
 #pragma unroll
