@@ -1,5 +1,7 @@
 // W8A16 on gemm_mid.h: c[m, n] = (sum_k a[m, k] * w[k, n]) * scale[n] (+ bias[n]), int8 weights widened exactly to float16
-// (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25, is q / 512), float16 MFMA, fp32 sums; the results are multiplied by 512.
+// (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25, is q / 512), float16 MFMA, fp32 sums; the results are multiplied by 512. Powers of
+// two throughout: no bit differs from sums of q. The loop waits for its vector instructions as much as for its MFMAs, and this takes 40 for 32 codes
+// of four columns where 1152 + q (0x6400 | (q ^ 0x80)) less 1152 took 48: 128 x 4096 x 4096 14.8 -> 14.5 us, 128 x 2048 x 6144 11.4 -> 11.0.
 #include "gemm_mid.h"
 
 namespace qmm {
