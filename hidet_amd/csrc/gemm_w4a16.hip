@@ -470,31 +470,35 @@ void launch_cfg16(const void *a, const void *w, const void *scales, void *c, int
 // ---- dequantise once per workgroup --------------------------------------------------------------------------------------
 //
 // gemm_w4a16_kernel16 widens every weight once per wave and M tile; with M in the hundreds or thousands that is
-// several times per weight and the VALU, not the MFMA, sets the pace. Here a workgroup of 8 waves owns 256 rows x 128
-// columns and widens each weight of a 64-row stage ONCE: the packed rows (4 KiB) and the group's scales (256 B) come
+// several times per weight and the VALU, not the MFMA, sets the pace. Here a workgroup of 8 waves owns 256 rows x 128 (NB = 4;
+// 96 with NB = 3, narrower_tiles()) columns and widens each weight of a 64-row stage ONCE: the packed rows (4 KiB; sizes here are those of NB = 4) and the group's scales (256 B) come
 // into an LDS ring by buffer_load ... lds three stages ahead; thread (byte b, 8-row chunk c) reads its 8 bytes (two
 // columns x 8 rows), widens the 16 weights (v_bfe_i32, v_cvt_f32_i32, v_mul, v_cvt_pk) and writes two 16-byte chunks
 // into a double-buffered tile laid out like the activation tile (one 128-byte row of 64 k per output column, chunks
 // swizzled by row), from which every wave reads its B fragments. LDS row r of that tile holds output column
-// (r / 64) * 64 + (r % 16) * 4 + (r / 16) % 4: the 16 lanes of a fragment read 16 consecutive LDS rows (no bank
-// conflicts) and a lane's four MFMA column blocks are four consecutive output columns (8-byte stores).
+// (r / 64) * 64 + (r % 16) * 4 + (r / 16) % 4 (NB = 3: 48 and 3 for 64 and 4): the 16 lanes of a fragment read 16 consecutive LDS rows (no bank
+// conflicts) and a lane's NB MFMA column blocks are NB consecutive output columns (8-byte stores; 4 + 2).
 //
 // Every LDS access of the kernel is hand-placed asm: the compiler orders any LDS access of its own behind ALL
 // outstanding buffer_load ... lds (it cannot tell which bytes they write), which would serialise the ring.
 
+// NB: 16-column blocks of a wave, 4 or 3.
+template <int NB>
 struct GemmW4LdsCfg {
     static constexpr int kBM = 256;
-    static constexpr int kBN = 128;
+    static constexpr int kBN = 32 * NB;
     static constexpr int kThreads = 512;
     static constexpr int kAChunks = kBM * 8 / kThreads;
     static constexpr int kASlotBytes = kBM * 128;
     static constexpr int kBBufBytes = kBN * 128;
     static constexpr int kBBase = 3 * kASlotBytes;
     static constexpr int kRawBase = kBBase + 2 * kBBufBytes;
-    static constexpr int kRawSlotBytes = 64 * 64 + 256;  // 64 rows x 64 bytes, then 128 scales
+    static constexpr int kRawRowBytes = kBN / 2;
+    static constexpr int kRawScales = 64 * kRawRowBytes;
+    static constexpr int kRawSlotBytes = kRawScales + kBN * 2;  // 64 packed rows, then the scales
     static constexpr int kRingBytes = kRawBase + 3 * kRawSlotBytes;
     static constexpr int kLdsBytes = kRingBytes + 16;  // + the fix-up's flag; the ring must start at LDS address 0
-    };
+};
 
 template <int OFFSET>
 __device__ __forceinline__ uint32_t lds_read_u8_early(uint32_t addr) {
@@ -518,6 +522,12 @@ __device__ __forceinline__ void lds_wait_keep_newer(uint32_t (&b)[8], uint32_t &
                  : "n"(NEWER));
 }
 template <int NEWER>
+__device__ __forceinline__ void lds_wait_keep_newer(int4v_t (&f)[4], int4v_t (&g)[3]) {
+    asm volatile("s_waitcnt lgkmcnt(%7)"
+                 : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(g[0]), "+v"(g[1]), "+v"(g[2])
+                 : "n"(NEWER));
+}
+template <int NEWER>
 __device__ __forceinline__ void lds_wait_keep_newer(int4v_t (&f)[4], int4v_t (&g)[4]) {
     asm volatile("s_waitcnt lgkmcnt(%8)"
                  : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(g[0]), "+v"(g[1]), "+v"(g[2]), "+v"(g[3])
@@ -526,11 +536,11 @@ __device__ __forceinline__ void lds_wait_keep_newer(int4v_t (&f)[4], int4v_t (&g
 
 // Stages [s_begin, s_end) of output tile (tile_m, tile_n), by the whole workgroup. `split`: the tile is computed in
 // pieces and fix(acc, rows_valid) exchanges them; it returns true in the workgroup that finishes the tile.
-template <int DT, typename Fix>
+template <int DT, int NB, typename Fix>
 __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__ a, int64_t lda, const uint8_t *__restrict__ w,
                                                     const uint16_t *__restrict__ scales, uint16_t *__restrict__ c, int m, int k, int n,
                                                     int group, int tile_m, int tile_n, int s_begin, int s_end, bool split, Fix fix) {
-    using Cfg = GemmW4LdsCfg;
+    using Cfg = GemmW4LdsCfg<NB>;
     using T = W4G<DT>;
     extern __shared__ uint4 lds[];  // no static LDS in this kernel: every access addresses the ring from 0
 
@@ -539,14 +549,14 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;  // 4 x 2 waves of 64 rows x 64 columns
+    const int wm = wave >> 1, wn = wave & 1;  // 4 x 2 waves of 64 rows x 16 NB columns
     const int kg = lane >> 4, ns = lane & 15;
 
-    float4_t acc[4][4];
+    float4_t acc[4][NB];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[rb][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < NB; ++t) acc[rb][t] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     const int row_bytes = n >> 1;
     const __amdgpu_buffer_rsrc_t rsrc_w =
@@ -565,11 +575,11 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
         const int row = m0 + r;
         a_off[j] = row < m ? int((int64_t(row) * lda + ((id & 7) ^ lds_swizzle_key_step1(r)) * 8) * 2) : kOutside;
     }
-    // packed rows: lanes 0..31 of wave v bring 16 bytes each: row 8v + lane / 4 of the stage, quarter lane % 4 of the
-    // tile's 64 bytes. scales: lanes 0..7 bring one dword (two columns) each. (n % 32 == 0: whole quarters.)
-    const int wq_col = (n0 >> 1) + (lane & 3) * 16;
-    const int wq_off = wq_col < row_bytes ? (lane >> 2) * row_bytes + wq_col : kOutside;
-    const int sq_col = n0 + 2 * (wave * 8 + lane);
+    // packed rows: lanes 0 .. 8 NB - 1 of wave v bring 16 bytes each: row 8v + lane / NB of the stage, piece lane % NB of the
+    // tile's 16 NB bytes. scales: lanes 0 .. 2 NB - 1 bring one dword (two columns) each. (n % 32 == 0: whole pieces.)
+    const int wq_col = (n0 >> 1) + (lane % NB) * 16;
+    const int wq_off = wq_col < row_bytes ? (lane / NB) * row_bytes + wq_col : kOutside;
+    const int sq_col = n0 + 2 * (wave * 2 * NB + lane);
     const int sq_off = sq_col < n ? sq_col * 2 : kOutside;
 
     const int stages = k / kBK;
@@ -607,36 +617,39 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
     auto load_raw = [&](int st, int slot) {
         const int stc = st < stages ? st : stages - 1;
         char *dst = reinterpret_cast<char *>(lds) + Cfg::kRawBase + slot * Cfg::kRawSlotBytes;
-        if (lane < 32)
-            buffer_load_to_lds_b128(rsrc_w, reinterpret_cast<uint4 *>(dst + wave * 512), wq_off, (stc * kBK + wave * 8) * row_bytes);
-        if (lane < 8)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_s, (__attribute__((address_space(3))) void *)(dst + 4096 + wave * 32),
+        if (lane < 8 * NB)
+            buffer_load_to_lds_b128(rsrc_w, reinterpret_cast<uint4 *>(dst + wave * 8 * Cfg::kRawRowBytes), wq_off, (stc * kBK + wave * 8) * row_bytes);
+        if (lane < 2 * NB)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_s, (__attribute__((address_space(3))) void *)(dst + Cfg::kRawScales + wave * 8 * NB),
                                                      4, sq_off, ((stc * kBK) / group) * n * 2, 0, 0);
     };
 
-    // Dequantisation: thread (lane, wave) widens bytes `lane` (columns 2 lane, 2 lane + 1) of rows 8 wave .. 8 wave + 7.
+    // Dequantisation: thread (lane, wave) widens bytes `byte` = lane (columns 2 byte, 2 byte + 1) of rows 8 wave .. 8 wave + 7. Lanes that a
+    // narrower tile has no byte for do the work of the sixteen in front of them over, the same writes included.
     // (the upper half of a wave takes the neighbouring k-group, wave ^ 1: a wave's two 16-byte writes of a stage then land on
     // all sixteen 16-byte bank groups, four lanes each, instead of eight lanes on eight of them)
-    const int kgrp = wave ^ (lane >> 5);
-    const uint32_t raw_rd = uint32_t(Cfg::kRawBase + kgrp * 512 + lane);
-    const uint32_t sc_rd = uint32_t(Cfg::kRawBase + 4096 + lane * 4);
+    const int byte = lane < 16 * NB ? lane : lane - 16;
+    const int kgrp = wave ^ (byte >> 5);
+    const uint32_t raw_rd = uint32_t(Cfg::kRawBase + kgrp * 8 * Cfg::kRawRowBytes + byte);
+    const uint32_t sc_rd = uint32_t(Cfg::kRawBase + Cfg::kRawScales + byte * 4);
     uint32_t bw_addr[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-        const int sig = (lane >> 5) * 64 + (2 * (lane & 1) + e) * 16 + ((lane & 31) >> 1);
+        const int col = 2 * byte + e, part = col / (16 * NB), at = col % (16 * NB);
+        const int sig = part * 16 * NB + (at % NB) * 16 + at / NB;
         bw_addr[e] = uint32_t(Cfg::kBBase + (sig * 8 + (kgrp ^ lds_swizzle_key_step1(sig))) * 16);
     }
     uint32_t bytes[8], sc2;
     auto read_raw = [&](int slot) {
         const uint32_t base = raw_rd + slot * Cfg::kRawSlotBytes;
-        bytes[0] = lds_read_u8_early<0 * 64>(base);
-        bytes[1] = lds_read_u8_early<1 * 64>(base);
-        bytes[2] = lds_read_u8_early<2 * 64>(base);
-        bytes[3] = lds_read_u8_early<3 * 64>(base);
-        bytes[4] = lds_read_u8_early<4 * 64>(base);
-        bytes[5] = lds_read_u8_early<5 * 64>(base);
-        bytes[6] = lds_read_u8_early<6 * 64>(base);
-        bytes[7] = lds_read_u8_early<7 * 64>(base);
+        bytes[0] = lds_read_u8_early<0 * Cfg::kRawRowBytes>(base);
+        bytes[1] = lds_read_u8_early<1 * Cfg::kRawRowBytes>(base);
+        bytes[2] = lds_read_u8_early<2 * Cfg::kRawRowBytes>(base);
+        bytes[3] = lds_read_u8_early<3 * Cfg::kRawRowBytes>(base);
+        bytes[4] = lds_read_u8_early<4 * Cfg::kRawRowBytes>(base);
+        bytes[5] = lds_read_u8_early<5 * Cfg::kRawRowBytes>(base);
+        bytes[6] = lds_read_u8_early<6 * Cfg::kRawRowBytes>(base);
+        bytes[7] = lds_read_u8_early<7 * Cfg::kRawRowBytes>(base);
         sc2 = lds_read_b32_early(sc_rd + slot * Cfg::kRawSlotBytes);
     };
     uint4v_t chunk[2];
@@ -655,23 +668,23 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
     // LDS byte addresses of this lane's A fragment (row block 0, ring slot 0) and B fragment (column block 0, buffer 0)
     uint32_t af_addr[2], bf_addr[2];
     {
-        const int ra = wm * 64 + ns, rb_ = wn * 64 + ns;
+        const int ra = wm * 64 + ns, rb_ = wn * 16 * NB + ns;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             af_addr[q] = uint32_t((ra * 8 + ((q * 4 + kg) ^ lds_swizzle_key_step1(ra))) * 16);
             bf_addr[q] = uint32_t(Cfg::kBBase + (rb_ * 8 + ((q * 4 + kg) ^ lds_swizzle_key_step1(rb_))) * 16);
         }
     }
-    int4v_t af[2][4], bf[2][4];
-    auto read_frags = [&](int4v_t (&dst)[4], uint32_t addr) {
+    int4v_t af[2][4], bf[2][NB];
+    auto read_frags = [&](auto &dst, uint32_t addr) {
         dst[0] = lds_read_b128_early<0 * 2048>(addr);
         dst[1] = lds_read_b128_early<1 * 2048>(addr);
         dst[2] = lds_read_b128_early<2 * 2048>(addr);
-        dst[3] = lds_read_b128_early<3 * 2048>(addr);
+        if constexpr (sizeof(dst) / sizeof(dst[0]) > 3) dst[3] = lds_read_b128_early<3 * 2048>(addr);
     };
-    auto mfmas = [&](int4v_t (&fa)[4], int4v_t (&fb)[4]) {
+    auto mfmas = [&](int4v_t (&fa)[4], int4v_t (&fb)[NB]) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < NB; ++t)
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb)
                 acc[rb][t] = T::mfma(__builtin_bit_cast(uint4, fa[rb]), __builtin_bit_cast(uint4, fb[t]), acc[rb][t]);
@@ -687,9 +700,9 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
     // so every LDS read has half a stage to land and the only LDS traffic between the last MFMA of H1 and the barrier
     // is the two writes. Ring slot of stage x is (x - s_begin) % 3 for activations and packed rows, tile buffer
     // (x - s_begin) % 2.
-    auto mfmas_half = [&](int4v_t (&fa)[4], int4v_t (&fb)[4], int t0) {
+    auto mfmas_half = [&](int4v_t (&fa)[4], int4v_t (&fb)[NB], int t0) {
 #pragma unroll
-        for (int t = t0; t < t0 + 2; ++t)
+        for (int t = t0; t < (t0 + 2 < NB ? t0 + 2 : NB); ++t)
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb)
                 acc[rb][t] = T::mfma(__builtin_bit_cast(uint4, fa[rb]), __builtin_bit_cast(uint4, fb[t]), acc[rb][t]);
@@ -720,16 +733,16 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
             const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot >= 1 ? slot - 1 : 2;
             const uint32_t a_next = uint32_t(slot1 * Cfg::kASlotBytes), b_other = uint32_t((buf ^ 1) * Cfg::kBBufBytes);
             // H1
-            lds_wait_keep_newer<8>(bytes, sc2);
-            lds_wait_keep_newer<8>(af[0], bf[0]);
+            lds_wait_keep_newer<4 + NB>(bytes, sc2);
+            lds_wait_keep_newer<4 + NB>(af[0], bf[0]);
             dequant();
             mfmas(af[0], bf[0]);
             // the two waves of a SIMD run in step: widening must sit in the shadow of this wave's own MFMAs, or the
             // MFMA pipe idles while both widen
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // four VALU
+            for (int i = 0; i < 4 * NB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, NB == 4 ? 4 : 6, 0);  // its share of the VALU
             }
             __builtin_amdgcn_sched_barrier(0);
             lds_write_b128(bw_addr[0] + b_other, chunk[0]);
@@ -793,14 +806,21 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
         if (!fix(acc, rows_valid)) return;
     }
 
-    const int col = n0 + wn * 64 + ns * 4;  // first of this lane's 4 columns
+    const int col = n0 + wn * 16 * NB + ns * NB;  // first of this lane's columns
     if (col >= n) return;
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int row = m0 + wm * 64 + rb * 16 + kg * 4 + v;
-            if (row < m) {
+            if constexpr (NB == 3) {  // the even column and its neighbour as one dword, the one before or behind them alone
+                if (row >= m) continue;
+                const int odd = ns & 1;
+                const uint32_t h0 = T::from_f32(acc[rb][0][v]), h1 = T::from_f32(acc[rb][1][v]), h2 = T::from_f32(acc[rb][2][v]);
+                uint16_t *dst = c + int64_t(row) * n + col;
+                if (col + odd < n) *reinterpret_cast<uint32_t *>(dst + odd) = odd ? h1 | (h2 << 16) : h0 | (h1 << 16);
+                if (col + (odd ? 0 : 2) < n) dst[odd ? 0 : 2] = uint16_t(odd ? h0 : h2);
+            } else if (row < m) {
                 uint2 o;
                 o.x = uint32_t(T::from_f32(acc[rb][0][v])) | (uint32_t(T::from_f32(acc[rb][1][v])) << 16);
                 o.y = uint32_t(T::from_f32(acc[rb][2][v])) | (uint32_t(T::from_f32(acc[rb][3][v])) << 16);
@@ -813,19 +833,19 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
 // the grid is `concurrent` workgroups per XCD and a workgroup computes its run of (tile, stage) units of the XCD's
 // region (gemm_tiling.h: runs across the tiles), piece by piece; `tail_stride` is then the stride of the per-XCD blocks
 // of tile counters, and `partials` holds two pieces per workgroup.
-template <int DT, bool STREAM>
+template <int DT, bool STREAM, int NB = 4>
 __global__ __launch_bounds__(512, 1) void gemm_w4a16_lds_kernel(
     const uint16_t *__restrict__ a, int64_t lda, const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
     uint16_t *__restrict__ c, int m, int k, int n, int group, int tiles_m, int tiles_n, int xm, int xn, int concurrent,
     int tail_parts, int tail_stride, float *__restrict__ partials, uint32_t *__restrict__ counters) {
-    using Cfg = GemmW4LdsCfg;
+    using Cfg = GemmW4LdsCfg<NB>;
     extern __shared__ uint4 lds[];
     int *s_last = reinterpret_cast<int *>(lds + Cfg::kRingBytes / 16);
     const int stages = k / kBK;
     if constexpr (!STREAM) {
         GemmWorkItem item;
         if (!gemm_work_item(tiles_m, tiles_n, xm, xn, concurrent, tail_parts, tail_stride, &item)) return;
-        gemm_w4a16_lds_tile<DT>(a, lda, w, scales, c, m, k, n, group, item.tile_m, item.tile_n, (stages * item.part) / item.parts,
+        gemm_w4a16_lds_tile<DT, NB>(a, lda, w, scales, c, m, k, n, group, item.tile_m, item.tile_n, (stages * item.part) / item.parts,
                                 (stages * (item.part + 1)) / item.parts, item.parts > 1, [&](auto &acc, uint32_t rows_valid) {
                                     return gemm_k_split_fixup<Cfg::kThreads>(acc, item, partials, counters, s_last, rows_valid);
                                 });
@@ -840,7 +860,7 @@ __global__ __launch_bounds__(512, 1) void gemm_w4a16_lds_kernel(
             const GemmStreamPiece piece = gemm_stream_piece(units, stages, concurrent, j, local);
             int tile_m, tile_n;
             gemm_tile_of_region(reg, local, &tile_m, &tile_n);
-            gemm_w4a16_lds_tile<DT>(a, lda, w, scales, c, m, k, n, group, tile_m, tile_n, piece.s_begin, piece.s_end, piece.parts > 1,
+            gemm_w4a16_lds_tile<DT, NB>(a, lda, w, scales, c, m, k, n, group, tile_m, tile_n, piece.s_begin, piece.s_end, piece.parts > 1,
                                     [&](auto &acc, uint32_t rows_valid) {
                                         const auto piece_at = [&](int p) {
                                             const int jp = piece.first + p;
@@ -858,7 +878,7 @@ __global__ __launch_bounds__(512, 1) void gemm_w4a16_lds_kernel(
 // time is about 74 us at K = 4096 (measured: M = 512, all 172 tiles in 4 parts: 82 -> 104 us; M = 1024, 88 tail
 // tiles in 2 parts: 146 -> 121 us).
 GemmTail lds_tail_of(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
-    using Cfg = GemmW4LdsCfg;
+    using Cfg = GemmW4LdsCfg<4>;
     GemmTail tail = make_gemm_tail_by_rounds(tiling, 32, 4, 0.0007 * 4096.0 / double(k));
     while (tail.parts > 1 &&
            (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
@@ -875,22 +895,44 @@ bool whole_stages(int64_t m, int64_t k, int64_t n, int64_t lda, int group) {
 // ahead except where its tall tiles leave a second or third tile row mostly empty (3 or 5 tile rows of 128).
 bool tall_tiles(int64_t m, int64_t n) { return n % 32 == 0 && cdiv(m, 128) != 3 && cdiv(m, 128) != 5; }
 
+// Tiles of 96 columns instead of 128 where either width is one round of the chip and the wider tiles have no K ranges: a CU has one tile,
+// and three quarters of one take 0.83 of the time (a stage 0.88 against 1.06 us: loads, barrier and latencies do not shrink). bfloat16, K = 4096, 128 and 96 columns, us: 512 x
+// 11008 73.2 and 63.8, 512 x 9216 66.0 and 53.5, 1024 x 5632 73.2 and 64.8, 1280 x 4096 73.1 and 63.6, 192 x 20480 71.3 and 54.2; of K =
+// 11008, 512 x 11008 184 and 159. With K ranges the wider ones already fill the chip (512 x 5632 46.8 and 60.7), a second round
+// costs more than narrower tiles give (512 x 14336 76 and 122, 1024 x 11008 119 and 125, 4096 x 11008 409 and 492), and up to 128 rows
+// a stage costs what its widening costs (128 x 22016 55.1 and 55.7).
+bool narrower_tiles(int64_t m, int64_t n, const GemmTiling &wide, const GemmTail &wide_tail) {
+    using Cfg = GemmW4LdsCfg<3>;
+    return m > 128 && wide.region_tiles <= 32 && wide_tail.parts == 1 && make_gemm_tiling(int(cdiv(m, Cfg::kBM)), int(cdiv(n, Cfg::kBN)), 32).region_tiles <= 32;
+}
+
 template <int DT>
 void launch_lds(const void *a, const void *w, const void *scales, void *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                 int group, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
-    using Cfg = GemmW4LdsCfg;
+    using Cfg = GemmW4LdsCfg<4>;
     const int tiles_m = int(cdiv(m, Cfg::kBM)), tiles_n = int(cdiv(n, Cfg::kBN));
     constexpr int kConcurrent = 32;
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, kConcurrent);
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     const GemmTail tail = lds_tail_of(tiling, k, ws);
+    if (narrower_tiles(m, n, tiling, tail)) {
+        using Narrow = GemmW4LdsCfg<3>;
+        const int columns = int(cdiv(n, Narrow::kBN));
+        const GemmTiling narrow = make_gemm_tiling(tiles_m, columns, kConcurrent);
+        allow_dynamic_lds(reinterpret_cast<const void *>(gemm_w4a16_lds_kernel<DT, false, 3>), Narrow::kLdsBytes);
+        launch(gemm_w4a16_lds_kernel<DT, false, 3>, dim3(uint32_t(narrow.grid())), dim3(Narrow::kThreads), size_t(Narrow::kLdsBytes), stream,
+               static_cast<const uint16_t *>(a), lda, static_cast<const uint8_t *>(w), static_cast<const uint16_t *>(scales),
+               static_cast<uint16_t *>(c), int(m), int(k), int(n), group, tiles_m, columns, narrow.xm, narrow.xn, kConcurrent, 1, 0,
+               static_cast<float *>(nullptr), static_cast<uint32_t *>(nullptr));
+        return;
+    }
     const int64_t grid = gemm_grid_with_tail(tiling, kConcurrent, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
     // Runs across the tiles instead (gemm_tiling.h), one workgroup per CU, when the busiest XCD has a few tiles more than
     // a whole number of rounds: measured against the plan above at K = 4096, N = 11008, the run plan costs about a third
     // of a round whatever the size (a second prologue per workgroup and 128 KiB per piece through memory), so it wins
     // where the few tail tiles would cost half a round (M = 768, 33 tiles per XCD: 123 -> 105 us; M = 1536, 65: 194 ->
-    // 187 us) and nowhere else (M = 512, 22 tiles on 32 CUs: 80 against 78 us with a third of the CUs idle; M = 1024: 129
+    // 187 us) and nowhere else (M = 512, 22 tiles on 32 CUs: 80 against 78 us with a third of the CUs idle, 64 on narrower tiles; M = 1024: 129
     // against 127 us; M = 4096: 450 against 416 us, the workgroups of a region no longer walk K in step and share less
     // in the L2)
     const int stages = int(k / kBK);
@@ -926,7 +968,8 @@ bool gemm_w4a16_supported(const void *a, const void *w, const void *scales, cons
 
 // Estimated time in microseconds, for the choice between these kernels and the narrow tiles of gemm_mid.h: a fixed part, what a
 // 64-deep stage takes with so many rows in the last tile row, and the exchange of K ranges; 0.98 of that where they tie. From K = 4096 and 11008, N = 4096 and 11008, 33 to 1024
-// rows (4096 x 11008, 128 / 160 rows: narrow 34.7 / 51.5 us, these 36.5 / 43.3). Groups that are no whole stages (32, 96) run
+// rows (4096 x 11008, 128 / 160 rows: narrow 34.7 / 51.5 us, these 36.5 / 43.3). That of the 128-column tiles also where narrower_tiles() takes
+// less: the narrow tiles of gemm_mid.h scale their sums and do not round a weight, and keep what they have. Groups that are no whole stages (32, 96) run
 // on the kernel that takes any, at 0.077 us per k whatever the rows (4096 x 11008, 512 rows: 346 us, narrow 101).
 double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n, int64_t lda, int group, bool biased, void *workspace, int64_t workspace_bytes) {
     const double bias = biased ? 4.0 + double(m * n) * 1e-6 : 0.0;  // a pass over the result
@@ -936,7 +979,7 @@ double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n, int64_t lda, int 
         const int64_t tiles = cdiv(m, 128) * cdiv(n, 256), parts = std::max<int64_t>(1, std::min<int64_t>(4, 192 / tiles));
         return 0.98 * (8.0 + double(cdiv(tiles, 512)) * (parts > 1 ? 1.3 : 0.98) * stages / double(parts) + (parts > 1 ? 2.7 * double(parts) : 0.0) + bias);
     }
-    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, GemmW4LdsCfg::kBM)), int(cdiv(n, GemmW4LdsCfg::kBN)), 32);
+    const GemmTiling tiling = make_gemm_tiling(int(cdiv(m, GemmW4LdsCfg<4>::kBM)), int(cdiv(n, GemmW4LdsCfg<4>::kBN)), 32);
     const GemmTail tail = lds_tail_of(tiling, k, split_workspace(workspace, workspace_bytes));
     const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
     const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);

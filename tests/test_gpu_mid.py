@@ -110,6 +110,16 @@ def test_w4a16_depths_of_a_stage(m, k, n, group, dtype):
     test_w4a16_rows_of_a_batch(m, k, n, group, dtype)
 
 
+# the tall tiles of 96 columns: N = 96 i, + 32 and + 64 (a lane's three columns lie across the end), part-filled and short row tiles, one stage, fewer
+# and more of them than the rings hold
+@pytest.mark.parametrize('m,k,n,group', [(512, 64, 11040, 64), (400, 192, 11072, 64), (385, 512, 11008, 128), (490, 1024, 12288, 128), (449, 256, 10016, 256),
+                                         (250, 128, 24544, 128), (200, 320, 20000, 64)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_w4a16_tiles_of_96_columns(m, k, n, group, dtype):
+    announce('int4 tiles of 96 columns', m, k, n, group, dtype)
+    test_w4a16_rows_of_a_batch(m, k, n, group, dtype)
+
+
 def test_w4a16_infinite_and_large_activations():
     g = torch.Generator(device='cuda')
     g.manual_seed(8)
