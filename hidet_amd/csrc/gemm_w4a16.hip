@@ -723,8 +723,10 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
     __builtin_amdgcn_s_barrier();
     load_a(s_begin + 2, 2, std::false_type());
     load_raw(s_begin + 3, 0);
-    read_raw(1);
+    // The bytes of stage s_begin + 1 are read inside the branches below: from in front of a choice between loops the compiler copies the
+    // destinations to the registers of each loop, and the copies do not wait for the reads (tests/test_lds_waits.py).
     auto active_loop = [&](auto all_tag) {
+        read_raw(1);
         read_frags(af[0], af_addr[0]);
         read_frags(bf[0], bf_addr[0]);
         read_frags(af[1], af_addr[1]);
@@ -778,6 +780,8 @@ __device__ __forceinline__ void gemm_w4a16_lds_tile(const uint16_t *__restrict__
         active_loop(std::false_type());
     } else {
         // same loads, widening, writes and barriers; no fragments, no MFMAs
+        read_raw(1);
+        lds_wait_keep_newer<0>(bytes, sc2);
         for (int s = s_begin, slot = 0, buf = 0; s < s_end; ++s) {
             const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot >= 1 ? slot - 1 : 2;
             const uint32_t b_other = uint32_t((buf ^ 1) * Cfg::kBBufBytes);
