@@ -1,7 +1,9 @@
 // W8A16 on gemm_mid.h: c[m, n] = (sum_k a[m, k] * w[k, n]) * scale[n] (+ bias[n]), int8 weights widened exactly to float16
 // (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25, is q / 512), float16 MFMA, fp32 sums; the results are multiplied by 512. Powers of
 // two throughout: no bit differs from sums of q. The loop waits for its vector instructions as much as for its MFMAs, and this takes 40 for 32 codes
-// of four columns where 1152 + q (0x6400 | (q ^ 0x80)) less 1152 took 48: 128 x 4096 x 4096 14.8 -> 14.5 us, 128 x 2048 x 6144 11.4 -> 11.0.
+// of four columns where 1152 + q (0x6400 | (q ^ 0x80)) less 1152 takes 48: 96 x 4096 x 4096 13.2 -> 12.9 us, 128 x 2048 x 6144 10.7 -> 10.3, 64 x 1024 x
+// 8192 7.3 -> 7.1. Tiles of 128 rows have MFMAs enough to hide either and keep 1152 + q (160 / 256 x 4096 x 11008 31.7 / 32.2 us with that, 32.0 / 32.5
+// with q / 512; 384 x 4096 x 4096 20.8 and 21.5, 852 x 3648 x 3024 31.95 and 32.3).
 #include "gemm_mid.h"
 
 namespace qmm {
@@ -17,7 +19,8 @@ struct MidW8Args {
 // SHIFTED: row-major weights of N = 4 i + 2. Their odd rows start between two dwords, which direct-to-LDS loads cannot; they are loaded
 // from two bytes in front, so that in LDS a lane's four columns of an odd row lie across two dwords. The second of them is one more read, and the
 // last lane's is missing: a tile has 124 columns. (A copy of the weight with rows of whole dwords, for the plain form: 4100 x 4098 11 us.)
-template <bool NK, bool SHIFTED = false>
+// OFFSET: codes widened as 1152 + q less 1152 (row-major, rows of whole dwords).
+template <bool NK, bool SHIFTED = false, bool OFFSET = false>
 struct MidW8 {
     using Args = MidW8Args;
     // Row-major: a stage is 32 rows of 128 columns, so that memory is read in whole 128-byte lines (64-byte pieces reached
@@ -41,7 +44,7 @@ struct MidW8 {
         half8_t h[kAChunks][4];
     };
     static constexpr int kMfmas = 4;      // per row block
-    static constexpr int kWidenOps = SHIFTED ? 44 : 40;  // VALU instructions of widen()
+    static constexpr int kWidenOps = OFFSET ? 48 : SHIFTED ? 44 : 40;  // VALU instructions of widen()
     int side_;
     __amdgpu_buffer_rsrc_t rsrc;
     int w_stage;       // bytes from one stage to the next
@@ -158,6 +161,17 @@ struct MidW8 {
         }
         return out;
     }
+    // u: two bytes q below zero bytes
+    static __device__ __forceinline__ half8_t minus_1152(const uint32_t (&u)[4]) {
+        half8_t out;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const half2_t v = __builtin_bit_cast(half2_t, u[p] ^ 0x64806480u) - half2_t{_Float16(1152.0f), _Float16(1152.0f)};
+            out[2 * p] = v[0];
+            out[2 * p + 1] = v[1];
+        }
+        return out;
+    }
     template <int NEWER>
     static __device__ __forceinline__ void settle(Weights &raw) {
         if constexpr (SHIFTED)
@@ -166,6 +180,17 @@ struct MidW8 {
             asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(raw.pair[0]), "+v"(raw.pair[1]), "+v"(raw.pair[2]), "+v"(raw.pair[3]) : "n"(NEWER));
     }
     __device__ __forceinline__ void widen(const Weights &raw, Fragments &b, int) const {
+        if constexpr (OFFSET) {
+            static_assert(!NK && !SHIFTED, "dwords of four columns");
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                uint32_t u[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) u[p] = __builtin_amdgcn_perm(uint32_t(raw.pair[p] >> 32), uint32_t(raw.pair[p]), sel[t]);
+                b.h[0][t] = minus_1152(u);
+            }
+            return;
+        }
         constexpr uint32_t kFlip = 0x80808080u;
         auto dword = [&](int i, int p) { return uint32_t(p & 1 ? raw.pair[i + p / 2] >> 32 : raw.pair[i + p / 2]); };
         uint32_t lo[4], hi[4];  // rows 2 p and 2 p + 1
@@ -219,7 +244,7 @@ struct MidW8 {
         if (col >= limit()) return;
         half4_t o;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(v[t] * 512.0f, float(scale4[t]), float(bias4[t]));
+        for (int t = 0; t < 4; ++t) o[t] = scaled_biased_f16(OFFSET ? v[t] : v[t] * 512.0f, float(scale4[t]), float(bias4[t]));
         _Float16 *dst = args.c + int64_t(row) * args.ldc + col;
         if (SHIFTED) {
 #pragma unroll
@@ -266,18 +291,19 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
     }
     if ((k + 64) * n >= kMost) return false;
     constexpr double kFullRound = 0.62;  // 256 pieces of 16 KiB at 6.8 TB/s
-    auto run = [&](auto form) {
+    auto run = [&](auto form, auto high) {
         using Op = typename decltype(form)::type;
+        using High = typename decltype(high)::type;  // on 128 rows
         const MidChoice c2 = mid_choose<Op, 2, 6>({5.5, 0.36, 1.4, 0.4, kFullRound}, ws, m, n, k), c4 = mid_choose<Op, 4, 4>({6.0, 0.5, 1.5, 0.5, kFullRound}, ws, m, n, k),
-                        c8 = mid_choose<Op, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
+                        c8 = mid_choose<High, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
         const double us = std::min({c2.us, c4.us, c8.us});
         if ((us == c2.us ? c2 : us == c4.us ? c4 : c8).busy_us > limit_us) return false;
         if (us == c2.us) mid_launch<Op, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
         else if (us == c4.us) mid_launch<Op, 4, 4>(c4, a, w, las, n, args, m, n, k, ws, stream);
-        else mid_launch<Op, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);
+        else mid_launch<High, 8, 3>(c8, a, w, las, n, args, m, n, k, ws, stream);
         return true;
     };
-    return shifted ? run(Form<MidW8<false, true>>()) : run(Form<MidW8<false>>());
+    return shifted ? run(Form<MidW8<false, true>>(), Form<MidW8<false, true>>()) : run(Form<MidW8<false>>(), Form<MidW8<false, false, true>>());
 }
 
 }  // namespace qmm
