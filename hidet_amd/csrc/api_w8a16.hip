@@ -83,40 +83,59 @@ __global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p) {
     }
 }
 
+// Where the copies go: panels of `cols` columns and `rows` rows, at the end of the scratch memory (offsets from its beginning).
+struct PadPlan {
+    int64_t kp, rows, cols, a_bytes;
+    int64_t a_at, bias_at, scale_at, w_at;
+    bool copy_a;
+};
+// False: there is not enough scratch memory for a panel.
+bool padded_plan(bool gemm, const void *a, int64_t m, int64_t k, int64_t n, int64_t lda, const Workspace &ws, PadPlan *plan) {
+    PadPlan p{};
+    p.kp = gemm ? cdiv(k, 64) * 64 : k;
+    p.copy_a = gemm && (p.kp != k || lda % 8 != 0 || !aligned(a, 16) || (m * lda + k) * 2 >= (int64_t(1) << 31) - (1 << 20));
+    const int64_t room = ws.scratch_bytes / 4 * 3;  // a quarter stays for partial tiles
+    p.rows = p.copy_a ? std::min<int64_t>(m, room / 3 / (p.kp * 2) / 128 * 128) : m;
+    if (p.rows <= 0) return false;
+    p.a_bytes = p.copy_a ? cdiv(p.rows * p.kp * 2, 256) * 256 : 0;
+    p.cols = cdiv(n, 16) * 16;  // per panel
+    const int64_t per_col = p.kp + 4, fixed = p.a_bytes + 1024;
+    const int64_t most = std::min<int64_t>(room - fixed, int64_t(1) << 30) / per_col;
+    if (p.cols > most) p.cols = most / 256 * 256;
+    if (p.cols <= 0) return false;
+    // the bandwidth-bound kernel writes whole rows (one panel) and addresses a wave's rows with 31-bit offsets
+    if (!gemm && (p.cols < n || (k + 192) * p.cols >= (int64_t(1) << 31) - (1 << 20))) return false;
+    p.a_at = ws.scratch_bytes / 256 * 256 - p.a_bytes;
+    p.bias_at = p.a_at - cdiv(p.cols * 2, 256) * 256;
+    p.scale_at = p.bias_at - cdiv(p.cols * 2, 256) * 256;
+    p.w_at = p.scale_at - cdiv(p.kp * p.cols, 256) * 256;
+    *plan = p;
+    return p.w_at >= 0;
+}
+
 // The matmul on padded copies, in panels of columns and rows that fit the scratch memory (the GEMM; without `gemm`, for up to 16 rows,
 // the bandwidth-bound kernel, which reads activations of any alignment, on one panel): the copies lie at its end, what is before them is left to the GEMM's partial tiles. False: there
 // is not enough of it for a panel.
 bool w8a16_padded(bool gemm, const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
                   int64_t lda, const Workspace &ws, hipStream_t stream) {
-    const int64_t kp = gemm ? cdiv(k, 64) * 64 : k;
-    const bool copy_a = gemm && (kp != k || lda % 8 != 0 || !aligned(a, 16) || (m * lda + k) * 2 >= (int64_t(1) << 31) - (1 << 20));
-    const int64_t room = ws.scratch_bytes / 4 * 3;  // a quarter stays for partial tiles
-    const int64_t rows = copy_a ? std::min<int64_t>(m, room / 3 / (kp * 2) / 128 * 128) : m;
-    if (rows <= 0) return false;
-    const int64_t a_bytes = copy_a ? cdiv(rows * kp * 2, 256) * 256 : 0;
-    int64_t cols = cdiv(n, 16) * 16;  // per panel
-    const int64_t per_col = kp + 4, fixed = a_bytes + 1024;
-    const int64_t most = std::min<int64_t>(room - fixed, int64_t(1) << 30) / per_col;
-    if (cols > most) cols = most / 256 * 256;
-    if (cols <= 0) return false;
-    // the bandwidth-bound kernel writes whole rows (one panel) and addresses a wave's rows with 31-bit offsets
-    if (!gemm && (cols < n || (k + 192) * cols >= (int64_t(1) << 31) - (1 << 20))) return false;
-    char *end = ws.scratch + ws.scratch_bytes / 256 * 256;
+    PadPlan plan;
+    if (!padded_plan(gemm, a, m, k, n, lda, ws, &plan)) return false;
+    const int64_t kp = plan.kp, rows = plan.rows, cols = plan.cols;
+    const bool copy_a = plan.copy_a;
     PadArgs p{};
     p.w = static_cast<const int8_t *>(w);
     p.scale = static_cast<const _Float16 *>(scale);
     p.bias = static_cast<const _Float16 *>(bias);
-    p.ap = reinterpret_cast<_Float16 *>(end - a_bytes);
-    p.biasp = reinterpret_cast<_Float16 *>(end - a_bytes - cdiv(cols * 2, 256) * 256);
-    p.scalep = p.biasp - cdiv(cols * 2, 256) * 128;
-    p.wp = reinterpret_cast<int8_t *>(p.scalep) - cdiv(kp * cols, 256) * 256;
+    p.ap = reinterpret_cast<_Float16 *>(ws.scratch + plan.a_at);
+    p.biasp = reinterpret_cast<_Float16 *>(ws.scratch + plan.bias_at);
+    p.scalep = reinterpret_cast<_Float16 *>(ws.scratch + plan.scale_at);
+    p.wp = reinterpret_cast<int8_t *>(ws.scratch + plan.w_at);
     p.n = n;
     p.lda = lda;
     p.k = int(k);
     p.kp = int(kp);
     Workspace left = ws;
-    left.scratch_bytes = reinterpret_cast<char *>(p.wp) - ws.scratch;
-    if (left.scratch_bytes < 0) return false;
+    left.scratch_bytes = plan.w_at;
     for (int64_t n0 = 0; n0 < n; n0 += cols) {
         p.n0 = int(n0);
         p.cols = int(std::min(cols, n - n0));
@@ -142,8 +161,13 @@ bool w8a16_padded(bool gemm, const void *a, const void *w, const void *scale, co
     return true;
 }
 
-// What the copy and the prefill tiles take together (the copy: 4100 x 4098 10.9 us, 1026 x 2050 4.0).
-double padded_estimate_us(int64_t m, int64_t k, int64_t n, const Workspace &ws) {
+// What the copy and the prefill tiles take together (the copy: 4100 x 4098 10.9 us, 1026 x 2050 4.0). No limit where no copy would be made, because
+// the matrix is tiny or the scratch memory holds no panel of it, and the call would run element by element.
+double padded_estimate_us(const void *a, int64_t m, int64_t k, int64_t n, int64_t lda, const Workspace &ws) {
+    PadPlan plan;
+    if (m * k * n <= kElementWise || !((m <= 16 && padded_plan(false, a, m, k, n, lda, ws, &plan)) ||
+                                       ((m > 16 || k >= kPanelK) && padded_plan(true, a, m, k, n, lda, ws, &plan))))
+        return 1e29;
     return 3.0 + double(k) * double(n) / 2.15e6 + gemm_w8a16_estimate_us(m, cdiv(k, 64) * 64, cdiv(n, 16) * 16, ws);
 }
 
@@ -180,7 +204,7 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     // 21.3 and 11.1, 203 x 4096 x 4098 27.9 and 20.4, 600 x 4096 x 4098 45 and 37, 16 x 8192 x 8190 35 and 18; 1 x 2002 x 514 element by element 193
     // and 7.7 (0.1 us per k whatever else).
     if (n % 4 == 2 && k > 0 && m <= kMidRows && (k >= 64 || m * k * n > kElementWise) &&
-        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, padded_estimate_us(m, k, n, ws), ws, stream))
+        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, padded_estimate_us(a, m, k, n, lda, ws), ws, stream))
         return;
     // Sizes the GEMM does not take (K no multiple of 64, N of 4): up to 32 rows two passes of the bandwidth-bound kernel,
     // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the

@@ -94,6 +94,25 @@ def test_int8_decode_of_a_large_ragged_weight_costs_no_more_than_more_rows(m):
     assert fastest_ms(lambda: quant.symmetric_quant_matmul(x[:m], w, s)) < 8 * fastest_ms(lambda: quant.symmetric_quant_matmul(x, w, s))
 
 
+def test_int8_off_the_dwords_without_room_for_a_copy():
+    """N = 4 i + 2 where the prefill tiles would be estimated faster on a padded copy that the workspace has no room for: on the narrow
+    tiles as it lies (element by element a hundred times slower)."""
+    announce('ragged int8 off the dwords, no room')
+    m, k, n = 1000, 4096, 4098
+    w = torch.randint(-7, 8, (k, n), device='cuda', dtype=torch.int8)
+    x = torch.randint(-3, 4, (m, k), device='cuda').half()
+    s = torch.ones(n, device='cuda', dtype=torch.float16)
+    c = torch.empty((m, n), dtype=torch.float16, device='cuda')
+    small = torch.zeros(int(ffi.load_library().hidet_qmm_workspace_bytes_for_scratch(1 << 16)), dtype=torch.uint8, device='cuda')
+
+    def call():
+        ffi.call('hidet_symmetric_quant_matmul_f16_i8', x, w, s, c, m, k, n, k, 0, small, small.numel(), ffi.current_stream(x.device))
+
+    call()
+    assert torch.equal(c, (x.float() @ w.float()).half())
+    assert fastest_ms(call) < 8 * fastest_ms(lambda: quant.symmetric_quant_matmul(x, w, s))
+
+
 @pytest.mark.parametrize('m,k,n,group', [(1, 256, 24, 128), (16, 4096, 264, 128), (3, 1024, 1032, 32), (20, 512, 520, 64)])
 def test_int4_exact(m, k, n, group):
     announce('ragged int4', m, k, n, group)
