@@ -21,7 +21,9 @@ def operands(rng, m, k, n, e5m2):
 # e5m2 operands take these tiles from 17 rows on, e4m3 above 1024
 @pytest.mark.parametrize('m,k,n,e5m2', [(1025, 128, 128, False), (1280, 256, 384, False), (1217, 384, 256, False), (1300, 8192 + 128, 128, False),
                                         (1216, 128 * 130, 128, False), (17, 128, 128, True), (65, 8192 + 256, 128, True),
-                                        (129, 128 * 66, 256, True), (193, 640, 128, True), (256, 128 * 65, 128, True)])
+                                        (129, 128 * 66, 256, True), (193, 640, 128, True), (256, 128 * 65, 128, True),
+                                        # 129 to 192 rows of the last tile, which is computed as a full one; with K ranges and without
+                                        (1153, 128, 256, False), (1180, 128 * 9, 3072, False), (2200, 7168, 1536, False), (192, 1024, 256, True)])
 def test_block_scaled(m, k, n, e5m2):
     announce('block-scaled tiles', m, k, n, e5m2)
     rng = np.random.default_rng(m + k + n)
@@ -34,7 +36,7 @@ def test_block_scaled(m, k, n, e5m2):
     assert np.array_equal(host(got), exact.astype(np.float32))
 
 
-@pytest.mark.parametrize('m,k,n', [(1025, 128, 132), (1280, 256, 1000), (2048, 384, 1024), (1217, 8320, 260)])
+@pytest.mark.parametrize('m,k,n', [(1025, 128, 132), (1280, 256, 1000), (2048, 384, 1024), (1217, 8320, 260), (1153, 128, 260), (1200, 1152, 1000), (2190, 4096, 1536)])
 def test_per_tensor(m, k, n):
     announce('per-tensor tiles', m, k, n)
     rng = np.random.default_rng(m + k + n)
