@@ -20,7 +20,7 @@ void skinny_fp8_block_scaled_launch(const void *a, const void *b, const void *sc
 bool mid_fp8_launch(const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int out_dtype,
                     const void *scale_a, const void *scale_b, bool block_scaled, double limit_us, void *workspace, int64_t workspace_bytes,
                     hipStream_t stream);
-double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, void *workspace, int64_t workspace_bytes);
+double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, bool scaled, void *workspace, int64_t workspace_bytes);
 }  // namespace qmm
 
 using namespace qmm;
@@ -56,7 +56,7 @@ HIDET_API void hidet_matmul_f8(const void *a, const void *b, void *c, int64_t m,
     if (m <= 16 && skinny_fp8_supported(b, k, ldb))
         skinny_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, stream);
     else if (m <= kMidRows && k > 0 && k % 16 == 0 && lda % 16 == 0 && ldb % 16 == 0 && n % 4 == 0 && aligned(a, 16) && aligned(b, 16) && aligned(c, 16) &&
-             mid_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, false, gemm_fp8_estimate_us(m, n, k, workspace, workspace_bytes), workspace, workspace_bytes, stream))
+             mid_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, false, gemm_fp8_estimate_us(m, n, k, false, workspace, workspace_bytes), workspace, workspace_bytes, stream))
         return;
     else
         gemm_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, workspace, workspace_bytes, stream);
@@ -101,7 +101,7 @@ static void f8_scaled_dispatch(const void *a, const void *b, const void *scale_a
     if (m <= 16)  // decode: the bandwidth-bound kernel, one pass over b
         skinny_fp8_block_scaled_launch(a, b, scale_a, scale_b, c, m, n, k, out_dtype, e5m2, stream);
     else if (!e5m2 && m <= kMidRows &&
-             mid_fp8_launch(a, b, c, m, n, k, k, k, out_dtype, scale_a, scale_b, true, gemm_fp8_estimate_us(m, n, k, workspace, workspace_bytes), workspace, workspace_bytes, stream))
+             mid_fp8_launch(a, b, c, m, n, k, k, k, out_dtype, scale_a, scale_b, true, gemm_fp8_estimate_us(m, n, k, true, workspace, workspace_bytes), workspace, workspace_bytes, stream))
         return;
     else
         gemm_fp8_scaled_launch(a, b, scale_a, scale_b, c, m, n, k, out_dtype, e5m2, workspace, workspace_bytes, stream);

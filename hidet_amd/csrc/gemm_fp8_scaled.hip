@@ -18,6 +18,7 @@
 // MFMAs (on zeros 139, on real operands 180; without scales 149), raised priority during the MFMAs (180; 150).
 // gemm_fp8_scaled_kernel (128 x 128 tile, register-staged double-buffered LDS) takes the rest.
 #include "common.h"
+#include "gemm_fp8_plan.h"
 #include "gemm_tiling.h"
 #include "numeric.h"
 
@@ -164,7 +165,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_scaled_kernel(const uint
 
 // ---- fast path ---------------------------------------------------------------------------------------------------------
 
-constexpr int kM8 = 256, kN8 = 128;           // workgroup tile
 constexpr int kThreads8 = 512;
 constexpr int kOperandChunks8 = (kM8 + kN8) * 8;       // 16-byte chunks of one k block: A rows then B rows
 constexpr int kSlotChunks8 = kOperandChunks8 + kM8 / 4;  // + the block's scales of the rows
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
     extern __shared__ uint4 lds[];  // [3][kSlotChunks8]; no static LDS: fragment reads address the ring from 0
     int &s_last = *reinterpret_cast<int *>(lds + kRingBytes8 / 16);
     GemmWorkItem item;
-    if (!gemm_work_item(tiles_m, tiles_n, xm, xn, 32, tail_parts, tail_stride, &item, panel)) return;
+    if (!gemm_work_item(tiles_m, tiles_n, xm, xn, kConcurrent8, tail_parts, tail_stride, &item, panel)) return;
     const int tile_m = item.tile_m, tile_n = item.tile_n;
     const int m0 = tile_m * kM8, n0 = tile_n * kN8;
     const int kblocks = k / 128;
@@ -535,28 +535,13 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
 
 }  // namespace
 
-// Tail split (tiles that do not fill a round of one workgroup per CU are computed in K ranges and summed in range
-// order by the last workgroup to arrive): at most 4 ranges of at least 4 k blocks, and only with a workspace that
-// holds the partial tiles (8 XCDs x their tail tiles x parts) in its scratch part.
-static GemmTail tail8_of(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
-    GemmTail tail = make_gemm_tail(tiling, 32, 32, 4);
-    if (ws.scratch == nullptr) tail.parts = 1;
-    while (tail.parts > 1 &&
-           (k / 128 < 4 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * kM8 * kN8 * 4))
-        --tail.parts;
-    return tail;
-}
-
-// Estimated time in microseconds of the tiled kernels, for the choice between them and the narrow tiles of gemm_mid.h: a fixed
-// part, 1.0 us per k block and round of 256 x 128 tiles and what an exchange of K ranges costs; where K is no multiple of 128
-// (the register-staged 256 x 256 kernel) 3.5 us per k block and round.
-double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, void *workspace, int64_t workspace_bytes) {
+// Estimated time in microseconds of the tiled kernels, for the choice between them and the narrow tiles of gemm_mid.h: the plan's time and a fixed part
+// with which that choice is right (8 us are spent; the narrow tiles' estimates are too low by the rest with block scales and too high without: of 242
+// shapes of 64 to 1024 rows each, a kernel that is more than 3 % slower is taken for none and for 9); where K is no multiple of 128 (the
+// register-staged 256 x 256 kernel) 3.5 us per k block and round.
+double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, bool scaled, void *workspace, int64_t workspace_bytes) {
     if (k % 128 != 0) return 8.0 + double(cdiv(cdiv(m, 256) * cdiv(n, 256), 256)) * 3.5 * double(cdiv(k, 128));
-    const GemmTiling tiling = make_gemm_tiling_weighted(int(cdiv(m, kM8)), int(cdiv(n, kN8)), 32, kM8, kN8);
-    const GemmTail tail = tail8_of(tiling, k, split_workspace(workspace, workspace_bytes));
-    const int whole = tiling.region_tiles / 32, rest = tiling.region_tiles % 32;
-    const double rounds = whole + (rest > 0 ? double((rest * tail.parts + 31) / 32) / tail.parts : 0.0);
-    return 7.0 + rounds * double(k) / 128.0 + (tail.parts > 1 ? 5.0 + 0.4 * tail.parts : 0.0);
+    return (scaled ? 6.3 : 11.3) + make_fp8_plan(m, n, k, scaled, split_workspace(workspace, workspace_bytes)).us;
 }
 
 // Launch of the 8-wave kernel; SCALED selects block scales (scale_a [K/128, M], scale_b [N/128, K/128]) or optional
@@ -566,10 +551,11 @@ static void launch_kernel8(const void *a, int64_t lda, const void *b, int64_t ld
                            void *c, int64_t m, int64_t n, int64_t k, int out_dtype, void *workspace, int64_t workspace_bytes,
                            hipStream_t stream) {
     const int tiles_m = int(cdiv(m, kM8)), tiles_n = int(cdiv(n, kN8));
-    const GemmTiling tiling = make_gemm_tiling_weighted(tiles_m, tiles_n, 32, kM8, kN8);
     const Workspace ws = split_workspace(workspace, workspace_bytes);
-    const GemmTail tail = tail8_of(tiling, k, ws);
-    const int64_t grid = gemm_grid_with_tail(tiling, 32, tail);
+    const Fp8Plan plan = make_fp8_plan(m, n, k, SCALED, ws);
+    const GemmTiling &tiling = plan.tiling;
+    const GemmTail &tail = plan.tail;
+    const int64_t grid = gemm_grid_with_tail(tiling, kConcurrent8, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
     auto go = [&](auto kern) {
         allow_dynamic_lds(reinterpret_cast<const void *>(kern), kLdsBytes8);

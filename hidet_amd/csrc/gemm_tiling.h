@@ -62,17 +62,16 @@ inline GemmTiling make_gemm_tiling(int tiles_m, int tiles_n, int concurrent) {
     return best;
 }
 
-// The same for tiles whose two operand slices differ in size (`row_bytes` and `col_bytes` of a tile's slices per step of K, in any
-// common unit): regions and panels so that the workgroups an XCD runs together pull the fewest bytes into its L2, `panel` columns x
-// concurrent / panel rows at a time. (FP8 tiles of 256 x 128: 8192 x 2048 x 1024 29.0 -> 23.3 us, 16384 x 7168 x 1536 190 -> 187 against
-// make_gemm_tiling; what an L2 misses comes from the last-level cache at about the rate that a copy has.)
-inline GemmTiling make_gemm_tiling_weighted(int tiles_m, int tiles_n, int concurrent, int row_bytes, int col_bytes) {
-    GemmTiling best{tiles_m, tiles_n, 1, 8, 0, kPanelCols};
-    int64_t best_rounds = 0, best_bytes = -1;
+// Layouts for tiles whose two operand slices differ in size (`row_bytes` and `col_bytes` of a tile's slices per step of K, in any common
+// unit): calls visit(tiling, bytes) for every grid of regions, with the panel width whose workgroups, `panel` columns x concurrent / panel rows
+// at a time, pull the fewest bytes into their XCD's L2 (what an L2 misses comes from the last-level cache at about the rate that a copy has).
+template <typename Visit>
+inline void for_each_gemm_tiling(int tiles_m, int tiles_n, int concurrent, int row_bytes, int col_bytes, Visit visit) {
     for (int xm = 1; xm <= 8; xm *= 2) {
         const int xn = 8 / xm;
         const int rr = (tiles_m + xm - 1) / xm, rc = (tiles_n + xn - 1) / xn;
-        const int64_t rounds = (int64_t(rr) * rc + concurrent - 1) / concurrent;
+        int64_t fewest = -1;
+        int best = 1;
         for (int panel = 1; panel <= concurrent; panel *= 2) {
             const int width = panel < rc ? panel : rc, full = rc / width;  // panels of `width` columns and a last narrower one
             auto bytes_of = [&](int w) {  // of one panel: its rows in batches, each with the panel's columns
@@ -81,13 +80,14 @@ inline GemmTiling make_gemm_tiling_weighted(int tiles_m, int tiles_n, int concur
                 return int64_t(rr) * row_bytes + int64_t((rr + batch - 1) / batch) * w * col_bytes;
             };
             const int64_t bytes = full * bytes_of(width) + bytes_of(rc - full * width);
-            if (best_bytes >= 0 && (rounds > best_rounds || (rounds == best_rounds && bytes >= best_bytes))) continue;
-            best_rounds = rounds;
-            best_bytes = bytes;
-            best = GemmTiling{tiles_m, tiles_n, xm, xn, rr * rc, panel};
+            if (fewest < 0 || bytes < fewest) {
+                fewest = bytes;
+                best = panel;
+            }
+            if (panel >= rc) break;  // wider ones are the same
         }
+        visit(GemmTiling{tiles_m, tiles_n, xm, xn, rr * rc, best}, fewest);
     }
-    return best;
 }
 
 struct GemmRegion {
