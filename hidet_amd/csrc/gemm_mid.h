@@ -416,9 +416,9 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 // the groups and, where K is cut, the exchange of `parts` partial tiles. The coefficients come from K = 4096 and 11008, N = 4096
 // and 11008, 17 to 400 rows, 1 to 8 pieces, and give those times to about 15 %.
 // `full_round` (0: not known) is the least a round takes with every CU at work: the weights of a round then come at the
-// rate of the memory.
+// rate of the memory. `exchange_piece` (0: in the others): what every piece of the launch adds to an exchange, all of them meeting at the same time.
 struct MidCost {
-    double fixed, round, exchange, exchange_part, full_round;
+    double fixed, round, exchange, exchange_part, full_round, exchange_piece;
 };
 
 struct MidChoice {
@@ -437,7 +437,7 @@ MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_
     MidChoice best;
     for (int64_t p = 1; p <= std::max<int64_t>(1, most); ++p) {
         const int64_t rounds = cdiv(cdiv(stages, p), Cfg::kGroups), share = rounds * Cfg::kGroups, parts = cdiv(stages, share);
-        const double rest = cost.fixed + (parts > 1 ? cost.exchange + double(parts) * cost.exchange_part : 0.0);
+        const double rest = cost.fixed + (parts > 1 ? cost.exchange + double(parts) * (cost.exchange_part + double(tiles) * cost.exchange_piece) : 0.0);
         const double us = double(cdiv(tiles * parts, cus)) * (rest + double(rounds) * cost.round);
         if (us >= best.us) continue;
         const auto batch = [&](int64_t active) {  // workgroups side by side

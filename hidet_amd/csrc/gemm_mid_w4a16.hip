@@ -10,7 +10,7 @@
 // What bounds it is the vector ALU, widening and scaling: 112 instructions for 64 k of a wave's 64 columns and 64 more per stage to scale 64 rows,
 // beside 32 MFMAs of four times the length of an instruction. So a stage is as deep as groups of 64 and 128 and the registers allow: 64 k, scaled once, with
 // half the barriers (32 before: 4096 x 4096, 128 / 256 / 512 rows 18.6 / 27.4 / 35.6 us; 11008 x 4096, 64 / 256 rows 23.9 / 48.9, 128 rows on the tall
-// tiles 38.7 -> 27.2), and the codes of two rows are gathered in one byte permutation. Groups of an odd number of 32 keep stages of 32.
+// tiles 38.7 -> 27.2), and the codes of two rows are gathered in one byte permutation. Groups of an odd number of 32 keep stages of 32, and so do small launches (launch_w4).
 #include "gemm_mid.h"
 #include "w4_traits.h"
 
@@ -173,17 +173,33 @@ struct MidW4 {
     }
 };
 
-template <int DT, int STEPS>
-bool launch_w4(const void *a, const void *w, const MidW4Args &args, int64_t m, int64_t n, int64_t k, int64_t lda, double limit_us, const Workspace &ws,
+// `args_of`: the arguments for stages of so many MFMA steps. Tiles of 32 rows have stages of 32 k also where groups allow 64, if a workgroup has few rounds:
+// more pieces of K divide the rest better and each costs less. us, stages of 32 and 64 k: 26 rows, 1408 x 2240 8.1 and 8.5, 1920 x 1096 7.8 and
+// 8.2, 6528 x 1448 12.0 and 12.2, 128 rows, 1920 x 1096 9.0 and 9.3; 2560 x 4096 13.4 and 12.9, 3072 x 2048 11.3 and 11.1. The second pair of costs is a
+// fit to such times alone (3 %), the first one is comparable with `limit_us`.
+template <int DT, int STEPS, typename ArgsOf>
+bool launch_w4(const void *a, const void *w, ArgsOf args_of, int64_t m, int64_t n, int64_t k, int64_t lda, double limit_us, const Workspace &ws,
                hipStream_t stream) {
     using Low = MidW4<DT, 2, STEPS>;
     using High = MidW4<DT, 4, STEPS>;
     constexpr int kLow = STEPS == 1 ? 6 : 4, kHigh = STEPS == 1 ? 5 : 3;  // stages in the ring
     const MidCost low = {5.5, STEPS == 1 ? 0.5 : 0.9, 1.4, 0.4}, high = {6.0, STEPS == 1 ? 0.9 : 1.5, 1.5, 0.5};
-    const MidChoice c2 = mid_choose<Low, 2, kLow>(low, ws, m, n, k), c4 = mid_choose<High, 4, kHigh>(high, ws, m, n, k);
+    MidChoice c2 = mid_choose<Low, 2, kLow>(low, ws, m, n, k), c4 = mid_choose<High, 4, kHigh>(high, ws, m, n, k);
     if (std::min(c2.us, c4.us) > limit_us) return false;
-    if (c2.us < c4.us) mid_launch<Low, 2, kLow>(c2, a, w, lda * 2, n / 2, args, m, n, k, ws, stream);
-    else mid_launch<High, 4, kHigh>(c4, a, w, lda * 2, n / 2, args, m, n, k, ws, stream);
+    if (c2.us >= c4.us) {
+        mid_launch<High, 4, kHigh>(c4, a, w, lda * 2, n / 2, args_of(STEPS), m, n, k, ws, stream);
+        return true;
+    }
+    if constexpr (STEPS == 2) {
+        using Shallow = MidW4<DT, 2, 1>;
+        const MidChoice shallow = mid_choose<Shallow, 2, 6>({3.38, 0.612, 1.95, 0.17, 0.0, 0.004}, ws, m, n, k);
+        c2 = mid_choose<Low, 2, kLow>({3.61, 1.044, 1.96, 0.21, 0.0, 0.004}, ws, m, n, k);
+        if (shallow.us < c2.us) {
+            mid_launch<Shallow, 2, 6>(shallow, a, w, lda * 2, n / 2, args_of(1), m, n, k, ws, stream);
+            return true;
+        }
+    }
+    mid_launch<Low, 2, kLow>(c2, a, w, lda * 2, n / 2, args_of(STEPS), m, n, k, ws, stream);
     return true;
 }
 
@@ -197,13 +213,15 @@ bool mid_w4a16_launch(const void *a, const void *w, const void *scales, const vo
         lda * 256 + k * 2 >= kMost || (k + 64) * (n / 2) >= kMost || (k / group) * n * 2 >= kMost)
         return false;
     const Workspace ws = split_workspace(workspace, workspace_bytes);
+    auto args_of = [&](int steps) {
+        const int group_stages = group / (32 * steps);
+        return MidW4Args{static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(c), group_stages, mid_magic(group_stages),
+                         int((k / group) * n * 2), aligned(c, 8)};
+    };
     auto run = [&](auto steps) {
         constexpr int STEPS = decltype(steps)::value;
-        const int group_stages = group / (32 * STEPS);
-        const MidW4Args args{static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(c), group_stages, mid_magic(group_stages),
-                             int((k / group) * n * 2), aligned(c, 8)};
-        return dtype == HIDET_QMM_F16 ? launch_w4<HIDET_QMM_F16, STEPS>(a, w, args, m, n, k, lda, limit_us, ws, stream)
-                                      : launch_w4<HIDET_QMM_BF16, STEPS>(a, w, args, m, n, k, lda, limit_us, ws, stream);
+        return dtype == HIDET_QMM_F16 ? launch_w4<HIDET_QMM_F16, STEPS>(a, w, args_of, m, n, k, lda, limit_us, ws, stream)
+                                      : launch_w4<HIDET_QMM_BF16, STEPS>(a, w, args_of, m, n, k, lda, limit_us, ws, stream);
     };
     return group % 64 == 0 ? run(std::integral_constant<int, 2>()) : run(std::integral_constant<int, 1>());
 }

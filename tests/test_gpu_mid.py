@@ -103,7 +103,9 @@ def test_w4a16_rows_of_a_batch(m, k, n, group, dtype):
 # 64-deep stages (groups of 64 and its multiples): one, two and an odd number of stages, fewer and more of them than the ring holds, a group a stage
 # and several, pieces of K that begin inside a group; one chunk of columns. Groups of an odd number of 32 beside them.
 @pytest.mark.parametrize('m,k,n,group', [(17, 64, 8, 64), (33, 128, 136, 64), (64, 128, 8, 128), (40, 960, 264, 192), (65, 8256, 120, 64), (100, 11008, 1032, 256),
-                                         (128, 1152, 2056, 128), (40, 1248, 264, 96), (65, 160, 8, 160)])
+                                         (128, 1152, 2056, 128), (40, 1248, 264, 96), (65, 160, 8, 160),
+                                         # 32 rows a tile, groups of 64 and more: 32-deep stages by their estimate (one to eight pieces of K), 64-deep ones
+                                         (17, 64, 1032, 64), (26, 1408, 2240, 128), (20, 1984, 136, 64), (31, 6528, 1448, 192), (96, 1024, 4096, 128), (128, 2560, 4096, 128)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_w4a16_depths_of_a_stage(m, k, n, group, dtype):
     announce('int4 stages', m, k, n, group, dtype)
