@@ -75,7 +75,7 @@ void w4a16_dispatch(const void *a, const void *w, const void *scales, const void
     QMM_CHECK(a && c && (k == 0 || (w && scales)), "null tensor pointer");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     // Beyond one 16-row pass of the bandwidth-bound kernel the narrow tiles (gemm_mid.h) or, where those are estimated to take
-    // longer, the MFMA GEMM on tall ones (K = 4096, N = 11008: 128 / 256 / 512 rows narrow 34.7 / 67 / 101 us, tall 36.9 / 48.5 / 64). What
+    // longer, the MFMA GEMM on tall ones (K = 4096, N = 11008: 128 / 160 / 192 / 512 rows narrow 27.6 / 39.8 / 59.8 / 80.2 us, tall 35.5 / 42.9 / 44.9 / 64.4). What
     // neither takes is done in passes of 16 rows.
     const bool gemm = m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size);
     if (m > 16 && m <= 1024 &&

@@ -975,9 +975,9 @@ bool gemm_w4a16_supported(const void *a, const void *w, const void *scales, cons
 
 // Estimated time in microseconds, for the choice between these kernels and the narrow tiles of gemm_mid.h: a fixed part, what a
 // 64-deep stage takes with so many rows in the last tile row, and the exchange of K ranges; 0.98 of that where they tie. From K = 4096 and 11008, N = 4096 and 11008, 33 to 1024
-// rows (4096 x 11008, 128 / 160 rows: narrow 34.7 / 51.5 us, these 36.5 / 43.3). That of the 128-column tiles also where narrower_tiles() takes
+// rows (4096 x 11008, 160 / 192 rows: narrow 39.8 / 59.8 us, these 42.9 / 44.9). That of the 128-column tiles also where narrower_tiles() takes
 // less: the narrow tiles of gemm_mid.h scale their sums and do not round a weight, and keep what they have. Groups that are no whole stages (32, 96) run
-// on the kernel that takes any, at 0.077 us per k whatever the rows (4096 x 11008, 512 rows: 346 us, narrow 101).
+// on the kernel that takes any, at 0.077 us per k whatever the rows (4096 x 11008, 512 rows: 346 us, narrow tiles of 32-deep stages 101).
 double gemm_w4a16_estimate_us(int64_t m, int64_t k, int64_t n, int64_t lda, int group, bool biased, void *workspace, int64_t workspace_bytes) {
     const double bias = biased ? 4.0 + double(m * n) * 1e-6 : 0.0;  // a pass over the result
     if (!whole_stages(m, k, n, lda, group)) return 0.98 * (5.0 + 0.077 * double(k) * double(cdiv(cdiv(m, 64) * cdiv(n, 256), 512)) + bias);

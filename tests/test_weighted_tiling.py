@@ -1,5 +1,6 @@
-"""Launch plans whose panels follow the size of the operand slices: a small host program enumerates every workgroup of many
-launches and checks that each output tile, and each K range of it, is computed exactly once."""
+"""Launch plans chosen by an estimate over every layout: a small host program enumerates every workgroup of many
+launches and checks that each output tile, and each K range of it, is computed exactly once, and which
+plans are chosen."""
 import os
 import shutil
 import subprocess
