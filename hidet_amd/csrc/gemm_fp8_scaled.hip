@@ -11,7 +11,7 @@
 // (buffer_load ... lds) three k blocks ahead, one barrier per k block in the middle of its MFMAs, fragments fetched half a block
 // ahead, the scratch accumulator double-buffered per row block so that the fold of row block i - 1 runs behind the MFMAs of row
 // block i. The running sums live in VGPRs (the VALU cannot read accumulation registers). What bounds it: on real operands the
-// power limit (16384 x 7168 x 1536 179 us, on zeros 150, all of these in one session, in others 195 to 204 in a graph of calls: before the
+// power limit (16384 x 7168 x 1536 179 us, on zeros 150, all of these in one session, in others 192 to 204 in a graph of calls: before the
 // scales came through the LDS, the barrier moved and the layout weighed bytes 188 and 163; 2048 x 7168 x 4096 62.0 -> 58.6, 8192 x 2048 x 1024
 // 28.4 -> 23.3; without scales 16384 x 7168 x 1536 151 -> 142, 1536 x 4096 x 4096 28.6 -> 27.2, 8192 x 2048 x 1024 27.0 -> 19.9). Matrix and vector instructions of a SIMD hardly overlap, also between its two
 // waves. Measured and dropped: single MFMAs alternating with their folds (fewer cycles but 226 us: the clock falls), 32 x 32 x 64
