@@ -4,6 +4,7 @@
 // Codes and scales match the CPU definition (IEEE division, then rounding) bit for bit. A product with the reciprocal stands in
 // for a division only where it provably rounds alike (round_quotients_f32, round_quotients_16, e4m3_codes4).
 #include "common.h"
+#include "gemm_tiling.h"
 #include "numeric.h"
 
 namespace qmm {
@@ -376,6 +377,262 @@ __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const v
             store_codes_upto4<QT>(q, (o * R + r + kQuantLanes * j) * inner + col, count, code);
         }
         if constexpr (TRIPS == 1) break;
+    }
+}
+
+// ---- maxima and codes in one pass over the weight ----------------------------------------------
+//
+// The two kernels above read the weight twice and are two launches. The ones here keep what they have read in registers: a workgroup of
+// kStripThreads holds NV quads of columns per thread (and NL in LDS) between the maxima and the codes, rows beyond that are read again.
+
+// A quad of columns as it lies in memory, at the alignment of one element; zeros past the end of the buffer, without a trip to memory.
+template <int DT>
+struct Quad {
+    typedef uint4v_t type;
+};
+typedef uint32_t uint2v_t __attribute__((ext_vector_type(2)));
+template <>
+struct Quad<HIDET_QMM_F16> {
+    typedef uint2v_t type;
+};
+template <>
+struct Quad<HIDET_QMM_BF16> {
+    typedef uint2v_t type;
+};
+template <int DT>
+__device__ __forceinline__ typename Quad<DT>::type load_quad(const __amdgpu_buffer_rsrc_t &from, int offset) {
+    if constexpr (DT == HIDET_QMM_F32) return __builtin_bit_cast(uint4v_t, __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, 0));
+    else return __builtin_bit_cast(uint2v_t, __builtin_amdgcn_raw_buffer_load_b64(from, offset, 0, 0));
+}
+template <int DT>
+__device__ __forceinline__ void quad_to_f32(const typename Quad<DT>::type &v, float (&x)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (DT == HIDET_QMM_F32) x[e] = __uint_as_float(v[e]);
+        else {
+            const uint16_t h = uint16_t(v[e >> 1] >> (16 * (e & 1)));
+            x[e] = DT == HIDET_QMM_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+        }
+    }
+}
+template <int DT>
+__device__ __forceinline__ void quad_max(float (&m)[4], const typename Quad<DT>::type &v) {
+    float t[4];
+    quad_to_f32<DT>(v, t);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(t[e]));
+}
+template <int DT, int QT>
+__device__ __forceinline__ void store_quad_codes(const typename Quad<DT>::type &v, const float (&s)[4], const float (&inv)[4], bool fast, void *q) {
+    float t[4];
+    uint32_t code[4];
+    quad_to_f32<DT>(v, t);
+    codes4<DT, QT>(t, s, inv, fast, code);
+    store_codes_upto4<QT>(q, 0, 4, code);
+}
+// The quads stay as they are in memory: the compiler would keep the unpacked values of the maxima for the codes.
+template <int N, typename V>
+__device__ __forceinline__ void keep_packed(V (&x)[N]) {
+#pragma unroll
+    for (int v = 0; v < N; ++v)
+#pragma unroll
+        for (int i = 0; i < int(sizeof(V) / 4); ++i) asm volatile("" : "+v"(x[v][i]));
+}
+
+// A strip of 4 CL columns over all rows of [R, inner] per workgroup, kStripThreads / CL rows at a time. Neighbouring strips share the cache
+// lines of the codes, so an XCD has a run of them. The last quad of a row that is no multiple of four is moved back into the row: its lane and
+// the one before store the same codes twice.
+constexpr int kStripThreads = 512;
+template <int DT, int QT, int CL, int NV, int WAVES>
+__global__ __launch_bounds__(kStripThreads, WAVES) void quantize_strip_kernel(const char *__restrict__ w, char *__restrict__ q, void *__restrict__ scale, int R, int inner,
+                                                                              int strips, int items, int per_xcd) {
+    constexpr int kElement = DT == HIDET_QMM_F32 ? 4 : 2, kCode = QT == HIDET_QMM_I8 ? 1 : 2;
+    constexpr int kLanes = kStripThreads / CL, kWaves = kStripThreads / 64, kBatch = DT == HIDET_QMM_F32 ? 4 : 8;
+    typedef typename Quad<DT>::type V;
+    __shared__ float4_t red[kWaves][CL];
+    const int tid = threadIdx.x, tx = tid % CL, ty = tid / CL, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int item = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
+    if (item >= items || int(blockIdx.x >> 3) >= per_xcd) return;
+    const int o = item / strips, place = ((item - o * strips) * CL + tx) * 4, col = min(place, inner - 4);
+    const int row_bytes = inner * kElement, offset = ty * row_bytes + col * kElement;
+    const int64_t step = int64_t(kLanes) * row_bytes, bytes = int64_t(R) * row_bytes;
+    w += o * bytes;
+    q += o * bytes / kElement * kCode;
+    auto trip = [&](int v) {  // rows v kLanes and on
+        const int64_t left = bytes - v * step;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(w) + v * step, 0, left > 0 ? int(left) : 0, 0x00020000);
+    };
+    V x[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) x[v] = load_quad<DT>(trip(v), offset);
+    __builtin_amdgcn_sched_barrier(0);
+    float m[4] = {0.f, 0.f, 0.f, 0.f};
+    const int trips = (R + kLanes - 1) / kLanes;
+    for (int v = NV; v < trips; v += kBatch) {
+        V y[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) y[j] = load_quad<DT>(trip(v + j), offset);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) quad_max<DT>(m, y[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) quad_max<DT>(m, x[v]);
+    keep_packed(x);
+#pragma unroll
+    for (int d = CL; d < 64; d <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], __shfl_xor(m[e], d));
+    if ((tid & 63) < CL) red[wave][tx] = float4_t{m[0], m[1], m[2], m[3]};
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kWaves; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t][tx][e]);
+    if (place >= inner) return;
+    float s[4], inv[4];
+    const bool fast = scales4<DT, QT>(m, s, inv);
+    if (ty == 0) store_upto4<DT>(scale, int64_t(o) * inner + col, 4, s);
+    char *out = q + (int64_t(ty) * inner + col) * kCode;
+    const int64_t out_step = int64_t(kLanes) * inner * kCode;
+    auto emit = [&](int v, const V &quad) {
+        if (v * kLanes + ty < R) store_quad_codes<DT, QT>(quad, s, inv, fast, out + v * out_step);
+    };
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        emit(v, x[v]);
+        __builtin_amdgcn_sched_barrier(0);  // (one quad's values at a time in registers)
+    }
+    for (int v = NV; v < trips; v += kBatch) {
+        V y[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) y[j] = load_quad<DT>(trip(v + j), offset);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) emit(v + j, y[j]);
+    }
+}
+
+// 256 columns x `share` rows per workgroup, all workgroups resident at once: the `ranges` workgroups of a column block (a group) leave their maxima in
+// memory, count themselves in, and go on when all have. What a workgroup waits for is bounded: one that gives up reads its columns itself,
+// so a launch ends with the right codes whatever else keeps workgroups of it from starting. Counters of a group lie on cache lines of their own (next to each other the atomics of all
+// groups queue up: 2048 x 4096 float32 35 us instead of 16); the last to leave returns them to zero.
+constexpr int kMeetCounterWords = 64, kMeetGroups = kExchangeLostWord / (2 * kMeetCounterWords), kMeetSpins = 512;
+template <int DT, int QT, int NV, int NL>
+__global__ __launch_bounds__(kStripThreads, 4) void quantize_meet_kernel(const char *__restrict__ w, char *__restrict__ q, void *__restrict__ scale, float *partials,
+                                                                         uint32_t *counters, int R, int inner, int col_blocks, int groups, int ranges, int share, int spins) {
+    constexpr int kElement = DT == HIDET_QMM_F32 ? 4 : 2, kCode = QT == HIDET_QMM_I8 ? 1 : 2, kAgentScope = 1 << 4;  // sc1
+    constexpr int kWaves = kStripThreads / 64, kBatch = 4, kHeld = kWaves * (NV + NL);
+    typedef typename Quad<DT>::type V;
+    static_assert(NL == 0 || sizeof(V) == 16, "16 bytes per lane go to LDS");
+    extern __shared__ uint4 lds[];
+    float4_t *red = reinterpret_cast<float4_t *>(lds + NL * kStripThreads);  // [kWaves][64], then the flag
+    int *all_here = reinterpret_cast<int *>(red + kWaves * 64);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int range = int(blockIdx.x) / groups, group = int(blockIdx.x) - range * groups, o = group / col_blocks;
+    const int place = (group - o * col_blocks) * 256 + 4 * lane, col = min(place, inner - 4), offset = col * kElement;
+    const int first = range * share + wave, end = min(R, (range + 1) * share);
+    const int64_t row_bytes = int64_t(inner) * kElement;
+    w += int64_t(o) * R * row_bytes;
+    q += int64_t(o) * R * inner * kCode;
+    auto row = [&](int r, int past) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(w) + r * row_bytes, 0, r < past ? int(row_bytes) : 0, 0x00020000); };
+    V x[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) x[v] = load_quad<DT>(row(first + kWaves * v, end), offset);
+    if constexpr (NL > 0) {
+#pragma unroll
+        for (int l = 0; l < NL; ++l) buffer_load_to_lds_b128(row(first + kWaves * (NV + l), end), lds + l * kStripThreads + wave * 64, offset, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float m[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int r = first + kHeld; r < end; r += kWaves * kBatch) {
+        V y[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) y[j] = load_quad<DT>(row(r + kWaves * j, end), offset);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) quad_max<DT>(m, y[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) quad_max<DT>(m, x[v]);
+    keep_packed(x);
+    const V *held = reinterpret_cast<const V *>(lds) + tid;  // what this lane's own loads put there
+    if constexpr (NL > 0) {
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int l = 0; l < NL; ++l) quad_max<DT>(m, held[l * kStripThreads]);
+    }
+    auto waves_max = [&] {
+#pragma unroll
+        for (int t = 0; t < kWaves; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[t * 64 + lane][e]);
+    };
+    red[wave * 64 + lane] = float4_t{m[0], m[1], m[2], m[3]};
+    __syncthreads();
+    uint32_t *arrived = counters + 2 * kMeetCounterWords * group, *left = arrived + kMeetCounterWords;
+    const __amdgpu_buffer_rsrc_t maxima = __builtin_amdgcn_make_buffer_rsrc(partials + int64_t(group) * ranges * 256, 0, ranges * 1024, 0x00020000);
+    if (wave == 0) {
+        waves_max();
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v_t, float4_t{m[0], m[1], m[2], m[3]}), maxima, (range * 64 + lane) * 16, 0, kAgentScope);
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // acknowledged: they write through
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0) {
+            uint32_t n = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+            for (int i = 0; i < spins && n < uint32_t(ranges); ++i) {
+                __builtin_amdgcn_s_sleep(1);
+                n = __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            *all_here = n >= uint32_t(ranges);
+        }
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    m[0] = m[1] = m[2] = m[3] = 0.0f;
+    if (*all_here) {
+        for (int i = wave; i < ranges; i += kWaves) {
+            const float4_t v = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(maxima, (i * 64 + lane) * 16, 0, kAgentScope));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], v[e]);
+        }
+    } else {
+        for (int r = wave; r < R; r += kWaves) quad_max<DT>(m, load_quad<DT>(row(r, R), offset));
+    }
+    __syncthreads();  // (wave 0 may still be reading the workgroup's own maxima)
+    red[wave * 64 + lane] = float4_t{m[0], m[1], m[2], m[3]};
+    __syncthreads();
+    waves_max();
+    if (tid == 0 && __hip_atomic_fetch_add(left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == uint32_t(ranges)) {
+        __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(left, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (place >= inner) return;
+    float s[4], inv[4];
+    const bool fast = scales4<DT, QT>(m, s, inv);
+    if (range == 0 && wave == 0) store_upto4<DT>(scale, int64_t(o) * inner + col, 4, s);
+    auto emit = [&](int r, const V &quad) {
+        if (r < end) store_quad_codes<DT, QT>(quad, s, inv, fast, q + (int64_t(r) * inner + col) * kCode);
+    };
+    V y[kBatch];
+    auto load_rest = [&](int r) {
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) y[j] = load_quad<DT>(row(r + kWaves * j, end), offset);
+    };
+    load_rest(first + kHeld);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        emit(first + kWaves * v, x[v]);
+        __builtin_amdgcn_sched_barrier(0);  // (one quad's values at a time in registers)
+    }
+    if constexpr (NL > 0) {
+#pragma unroll
+        for (int l = 0; l < NL; ++l) emit(first + kWaves * (NV + l), held[l * kStripThreads]);
+    }
+    for (int r = first + kHeld; r < end; r += kWaves * kBatch) {
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) emit(r + kWaves * j, y[j]);
+        load_rest(r + kWaves * kBatch);
     }
 }
 
@@ -847,16 +1104,76 @@ constexpr int64_t kNarrowGroups = 1024;
 // together (float32, kMaxRanges -> more: 16384 x 128, 32768 elements, 12.0 -> 13.2 us; 65536 x 128, 131072 elements, 30.4 -> 20.6).
 constexpr int64_t kCombineFrom = 65536;
 
+// One pass over the weight where the matrix is of a size for it; false: nothing was launched.
+//
+// Strips where a CU's strip is short: 8, 16 or 32 columns, the fewest that one round of the chip covers the matrix with, up to the rows from which
+// the other kernel is as fast (a thread holds 32 registers of quads; rows beyond those it holds are read twice). Two launches -> strips, us: float32 600 x 800
+// 6.9 -> 4.0, 1024 x 1024 7.3 -> 5.0, 1024 x 4096 12.3 -> 8.7, 512 x 8192 11.5 -> 7.8; bfloat16 512 x 8192 10.5 -> 6.7, 1448 x 4096 12.9 -> 9.9, 1500 x 2501 12.9 -> 9.5.
+// At their limits, strips and the other kernel: float32 1448 x 1024 8.5 and 8.5, 2048 x 4096 16.1 and 15.7, 1024 x 8192 14.1 and 14.4, 512 / 724 x 11008 10.9 / 15.6 and
+// 12.1 / 14.7; bfloat16 2048 x 2048 11.5 and 9.5, 1448 x 8192 14.3 and 14.5, 1024 / 1448 x 11008 15.0 / 21.6 and 15.2 / 18.3.
+//
+// Above, workgroups that meet, all resident: two per CU, of 64 or 128 rows at least (more workgroups cost more in the meeting than they save: float32 2048 x 2048 with
+// 16 / 32 / 64 rows 14.3 / 14.3 / 11.3), 64 to a column block at most, with as few quads held as the rows need (code that is not needed comes from memory all the
+// same: bfloat16 2048 x 2048, 16 / 32 quads 9.5 / 11.1). Two launches -> these, us: float32 4096 x 11008 74 -> 58, 3000 x 6400 35 -> 27, 2048 x 11008 40.5 -> 31, 4096 x 4096 31 -> 26.6;
+// bfloat16 4096 x 11008 50 -> 38, 4096 x 2048 15.6 -> 13.0. float32 of up to 1024 columns and less than 12 MB stays with two launches (2048 x 1024 9.5 and
+// 10.1, 4096 x 512 10.3 and 11.0), and so do matrices of which the workgroups would hold less than a quarter or that are too narrow to fill the chip
+// (bfloat16 65536 x 512 40 and 57).
+template <int DT, typename F>
+bool quantize_in_one_pass(F &&go, const void *w, void *wq, void *scale, int64_t outer, int64_t reduce, int64_t inner, const Workspace &ws) {
+    using std::integral_constant;
+    constexpr int kElement = DT == HIDET_QMM_F32 ? 4 : 2, kWide = 4 / kElement;  // kWide: quads of a register quad
+    const int64_t cus = std::max(1, device_cus()), row_bytes = inner * kElement;
+    if (reduce * row_bytes >= (int64_t(1) << 31) || row_bytes >= (int64_t(1) << 23) || outer > cus) return false;
+    const char *from = static_cast<const char *>(w);
+    char *to = static_cast<char *>(wq);
+    auto strips = [&](auto cl, auto nv, auto waves) {
+        constexpr int CL = decltype(cl)::value, NV = decltype(nv)::value, WAVES = decltype(waves)::value;
+        const int64_t per_slice = cdiv(inner, 4 * CL), items = outer * per_slice, per_xcd = cdiv(items, 8);
+        go(quantize_strip_kernel<DT, HIDET_QMM_I8, CL, NV, WAVES>, quantize_strip_kernel<DT, HIDET_QMM_I16, CL, NV, WAVES>, dim3(uint32_t(8 * per_xcd)), kStripThreads, 0,
+           from, to, scale, int(reduce), int(inner), int(per_slice), int(items), int(per_xcd));
+        return true;
+    };
+    auto one_round = [&](int columns) { return outer * cdiv(inner, columns) <= cus; };
+    const bool f32 = DT == HIDET_QMM_F32;
+    if (one_round(8)) {
+        if (reduce <= (!f32 && inner <= 1024 ? 2048 : 1536)) return strips(integral_constant<int, 2>(), integral_constant<int, 4 * kWide>(), integral_constant<int, 8>());
+    } else if (one_round(16)) {
+        if (reduce <= (f32 ? 2048 : 1536)) return strips(integral_constant<int, 4>(), integral_constant<int, 8 * kWide>(), integral_constant<int, 6>());
+    } else if (outer * cdiv(inner, 32) <= 2 * cus) {
+        if (reduce <= (one_round(32) ? (f32 ? 1024 : 1536) : (f32 ? 640 : 1024))) return strips(integral_constant<int, 8>(), integral_constant<int, 8 * kWide>(), integral_constant<int, 6>());
+    }
+    const int64_t col_blocks = cdiv(inner, 256), groups = outer * col_blocks;
+    if (ws.counters == nullptr || groups > kMeetGroups || (f32 && inner <= 1024 && outer * reduce * row_bytes < (12 << 20))) return false;
+    const int64_t ranges_most = std::min<int64_t>(64, 2 * cus / groups);
+    if (ranges_most < 2) return false;
+    const int64_t least = f32 && reduce <= 2048 ? 64 : 128, share = cdiv(std::max(least, cdiv(reduce, ranges_most)), 8) * 8, ranges = cdiv(reduce, share);
+    if (ws.scratch_bytes < groups * ranges * 1024 || (share > 256 && groups * ranges < cus)) return false;
+    auto meet = [&](auto nv, auto nl) {
+        constexpr int NV = decltype(nv)::value, NL = decltype(nl)::value, kLds = NL * kStripThreads * 16 + kStripThreads * 16 + 16;
+        if (share > 4 * 8 * (NV + NL)) return false;
+        allow_dynamic_lds(reinterpret_cast<const void *>(quantize_meet_kernel<DT, HIDET_QMM_I8, NV, NL>), kLds);
+        allow_dynamic_lds(reinterpret_cast<const void *>(quantize_meet_kernel<DT, HIDET_QMM_I16, NV, NL>), kLds);
+        go(quantize_meet_kernel<DT, HIDET_QMM_I8, NV, NL>, quantize_meet_kernel<DT, HIDET_QMM_I16, NV, NL>, dim3(uint32_t(groups * ranges)), kStripThreads, kLds, from, to, scale,
+           reinterpret_cast<float *>(ws.scratch), ws.counters, int(reduce), int(inner), int(col_blocks), int(groups), int(ranges), int(share),
+           std::min(kMeetSpins, exchange_spin_limit().load(std::memory_order_relaxed)));
+        return true;
+    };
+    if (share <= 64 * kWide) return meet(integral_constant<int, 8 * kWide>(), integral_constant<int, 0>());
+    if (share <= 128 * kWide) return meet(integral_constant<int, 16 * kWide>(), integral_constant<int, 0>());
+    return meet(integral_constant<int, 20 * kWide>(), integral_constant<int, f32 ? 8 : 0>());
+}
+
 // The quantizer's launches for [outer, reduce, inner], no extent zero, outer at most quantize_slices_most(reduce, inner).
 template <int DT>
-void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_t reduce, int64_t inner, int q_dtype, float *amax, int64_t scratch_bytes,
-                     hipStream_t stream) {
+void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_t reduce, int64_t inner, int q_dtype, const Workspace &ws, hipStream_t stream) {
+    float *amax = reinterpret_cast<float *>(ws.scratch);
     const int64_t total = outer * reduce * inner, nscale = outer * inner;
     const int esize = DT == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
-    auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) {
-        if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), 0, stream, args...);
-        else launch(i16, grid, dim3(threads), 0, stream, args...);
+    auto go_lds = [&](auto i8, auto i16, dim3 grid, int threads, size_t lds, auto... args) {
+        if (q_dtype == HIDET_QMM_I8) launch(i8, grid, dim3(threads), lds, stream, args...);
+        else launch(i16, grid, dim3(threads), lds, stream, args...);
     };
+    auto go = [&](auto i8, auto i16, dim3 grid, int threads, auto... args) { go_lds(i8, i16, grid, threads, 0, args...); };
     if (inner == 1) {
         // rows that fit a workgroup's registers: one pass
         if (reduce % 4 == 0 && reduce <= 4 * 4 * 1024 && aligned(w, 4 * esize) && aligned(wq, 4 * qsize)) {
@@ -881,7 +1198,7 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
     }
     const int64_t col_blocks = cdiv(inner, 256), row_blocks = cdiv(reduce, kQuantRows);
     QMM_CHECK(col_blocks * row_blocks < (int64_t(1) << 31), "tensor too large for one launch");
-    const int64_t spare = scratch_bytes / (nscale * 4) - 1;  // rows of maxima the scratch memory holds beside the final ones
+    const int64_t spare = ws.scratch_bytes / (nscale * 4) - 1;  // rows of maxima the scratch memory holds beside the final ones
     float *partials = amax + nscale;
     auto quantize = [&](int ranges) {
         auto run = [&](auto i8, auto i16, int64_t rows) {
@@ -912,6 +1229,7 @@ void quantize_slices(const void *w, void *wq, void *scale, int64_t outer, int64_
         quantize(1);
         return;
     }
+    if (quantize_in_one_pass<DT>(go_lds, w, wq, scale, outer, reduce, inner, ws)) return;
     // Workgroups of 256 columns where 16 row ranges of them are two workgroups per CU, else of 64, which need a quarter of the
     // ranges (float32, 256 -> 64: 4096 x 4096 35.3 -> 29.4 us, 16384 x 1024 42.8 -> 34.8, 65536 x 1024 150 -> 122, 65536 x 512 103 -> 56, but 16384 x 4096 106 -> 110;
     // bfloat16 65536 x 1024 120 -> 82). Ranges of 64 (128) rows at least, as many as two workgroups per CU take and the scratch memory
@@ -969,7 +1287,6 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
     QMM_CHECK(ws.scratch_bytes >= nscale * 4, "workspace too small: its scratch part (three quarters of what follows the first 64 KiB) must hold "
                                                   << nscale * 4 << " bytes, got a workspace of " << workspace_bytes);
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    float *amax = reinterpret_cast<float *>(ws.scratch);
     dispatch_float(w_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
         const int esize = DT == HIDET_QMM_F32 ? 4 : 2, qsize = q_dtype == HIDET_QMM_I8 ? 1 : 2;
@@ -982,7 +1299,7 @@ HIDET_API void hidet_symmetric_quantize(const void *w, void *wq, void *scale, in
         const int64_t step = quantize_slices_most(reduce, inner);
         for (int64_t o = 0; o < outer; o += step)  // (one launch after the other: they share the scratch memory)
             quantize_slices<DT>(static_cast<const char *>(w) + o * reduce * inner * esize, static_cast<char *>(wq) + o * reduce * inner * qsize,
-                                static_cast<char *>(scale) + o * inner * esize, std::min(step, outer - o), reduce, inner, q_dtype, amax, ws.scratch_bytes, stream);
+                                static_cast<char *>(scale) + o * inner * esize, std::min(step, outer - o), reduce, inner, q_dtype, ws, stream);
     });
     QMM_ENTRY_END
 }
