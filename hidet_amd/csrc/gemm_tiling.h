@@ -154,8 +154,9 @@ __device__ __forceinline__ void lds_wait_keep_newer(int4v_t &lo, int4v_t &hi) {
 
 // 16 bytes per lane from a buffer straight into LDS: lane i of the wave writes lds_dst + 16 * i (lds_dst must be
 // wave-uniform), reading buffer offset voff (per lane) + soff (scalar).
+template <int AUX = 0>  // (2: non-temporal)
 __device__ __forceinline__ void buffer_load_to_lds_b128(__amdgpu_buffer_rsrc_t rsrc, uint4 *lds_dst, int voff, int soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)lds_dst, 16, voff, soff, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)lds_dst, 16, voff, soff, 0, AUX);
 }
 
 // Work item of this workgroup. The items of an XCD, in launch order: the tiles of its region that fill whole rounds
