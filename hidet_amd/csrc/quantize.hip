@@ -835,7 +835,8 @@ __global__ __launch_bounds__(256) void dequantize_long_row_kernel(const void *__
 // workgroups share a CU and one's loads run under another's codes (16 rows, two workgroups: 42.8 us).
 // ROWS = 0, groups beyond that: the rows are read twice. K = 4096, N = 11008, groups of 128: 82 - 87 us with the group
 // read twice in 8-byte loads, a division per weight and one-byte stores -> 38.3 us = 5.3 TB/s.
-template <int ST, int CL, int ROWS>
+// ONCE (kReadOnceFrom): non-temporal loads, us: 4096 x 11008 40.4 -> 36.1 = 5.6 TB/s, 4096 x 4096 16.7 -> 15.2, 2048 x 2048 6.8 -> 6.5.
+template <int ST, int CL, int ROWS, bool ONCE = false>
 __global__ __launch_bounds__(512, 6) void group_quantize_int4_kernel(const float *__restrict__ w, uint8_t *__restrict__ packed,
                                                                      void *__restrict__ scales, int64_t n, int group) {
     constexpr int LANES = 512 / CL;
@@ -853,7 +854,8 @@ __global__ __launch_bounds__(512, 6) void group_quantize_int4_kernel(const float
         const float *row = base + int64_t(i * LANES + ty0) * n;
         if (i * LANES + ty < group) {
             if (cols == 4) {
-                v = *reinterpret_cast<const float4_at4_t *>(row + lane_off);
+                const float4_at4_t *from = reinterpret_cast<const float4_at4_t *>(row + lane_off);
+                v = ONCE ? __builtin_nontemporal_load(from) : *from;
             } else if (cols == 2) {
                 v[0] = row[lane_off];
                 v[1] = row[lane_off + 1];
@@ -1381,8 +1383,11 @@ HIDET_API void hidet_group_quantize_int4(const void *w, void *packed, void *scal
             launch(kern, dim3(cdiv(n, 4 * cl), k / group_size), dim3(512), 0, stream, static_cast<const float *>(w),
                    static_cast<uint8_t *>(packed), scales, n, group_size);
         };
+        const bool once = k * n * 4 >= 2 * kReadOnceFrom && n % 32 == 0;  // rows of whole cache lines (1024 x 1600 6.5 us, non-temporal 7.1; 2048 x 5002 15.4 and 16.3)
         if (group_size <= 32) go(group_quantize_int4_kernel<ST, 64, 4>, 64);
+        else if (group_size <= 64 && once) go(group_quantize_int4_kernel<ST, 64, 8, true>, 64);
         else if (group_size <= 64) go(group_quantize_int4_kernel<ST, 64, 8>, 64);
+        else if (group_size <= 128 && once) go(group_quantize_int4_kernel<ST, 32, 8, true>, 32);
         else if (group_size <= 128) go(group_quantize_int4_kernel<ST, 32, 8>, 32);
         else if (group_size <= 256) go(group_quantize_int4_kernel<ST, 16, 8>, 16);
         else go(group_quantize_int4_kernel<ST, 64, 0>, 64);
