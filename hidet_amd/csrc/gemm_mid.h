@@ -359,7 +359,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // every store of this lane has been acknowledged (they write through)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();
-        uint32_t *counter = counters + item.tile;
+        uint32_t *counter = counters + item.tile * kCounterWords;
         if (tid == 0) {
             const uint32_t old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             *flag = (old == uint32_t(parts - 1));
@@ -454,7 +454,7 @@ void mid_launch(const MidChoice &choice, const void *a, const void *w, int64_t a
     using Cfg = MidCfg<Op, RB, DEPTH>;
     const int64_t tiles_m = cdiv(m, RB * 16), tiles_n = cdiv(n, Cfg::kPitch), items = tiles_m * tiles_n * choice.parts;
     QMM_CHECK(items < (int64_t(1) << 28), "problem too large for one launch");
-    static_assert(256 * 4 * 4 <= kCounterBytes / 2, "one counter per tile that is cut");
+    static_assert(256 * kCounterWords <= kExchangeLostWord, "one counter per tile that is cut");
     allow_dynamic_lds(reinterpret_cast<const void *>(gemm_mid_kernel<Op, RB, DEPTH>), Cfg::kLdsBytes);
     launch(gemm_mid_kernel<Op, RB, DEPTH>, dim3(uint32_t(8 * cdiv(items, 8))), dim3(kMidThreads), size_t(Cfg::kLdsBytes), stream,
            static_cast<const char *>(a), static_cast<const char *>(w), int(a_stride), int(w_stride), int(k), int(m), int(n), int(tiles_m),
