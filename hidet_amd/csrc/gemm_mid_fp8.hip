@@ -162,7 +162,10 @@ struct MidF8 {
 template <bool SCALED>
 bool launch_f8(const void *a, const void *b, const MidF8Args &args, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
                double limit_us, const Workspace &ws, hipStream_t stream) {
-    const MidChoice c2 = mid_choose<MidF8<SCALED, 2>, 2, 3>({5.0, 0.6, 1.0, 0.25}, ws, m, n, k), c4 = mid_choose<MidF8<SCALED, 4>, 4, 3>({5.5, 0.9, 1.2, 0.4}, ws, m, n, k);
+    // (fits to the mean of what a split takes on weights from memory and from the last-level cache: more workgroups pay where the weights come from memory)
+    const MidCost low = SCALED ? MidCost{3.01, 0.798, 1.78, 0.0955, 0.0, 0.0066} : MidCost{3.43, 0.578, 1.81, 0.0854, 0.0, 0.0053};
+    const MidCost high = SCALED ? MidCost{3.81, 1.057, 1.59, 0.295, 0.0, 0.0109} : MidCost{4.69, 0.722, 1.34, 0.25, 0.0, 0.0091};
+    const MidChoice c2 = mid_choose<MidF8<SCALED, 2>, 2, 3>(low, ws, m, n, k), c4 = mid_choose<MidF8<SCALED, 4>, 4, 3>(high, ws, m, n, k);
     if (std::min(c2.us, c4.us) > limit_us) return false;
     if (c2.us < c4.us) mid_launch<MidF8<SCALED, 2>, 2, 3>(c2, a, b, lda, ldb, args, m, n, k, ws, stream);
     else mid_launch<MidF8<SCALED, 4>, 4, 3>(c4, a, b, lda, ldb, args, m, n, k, ws, stream);

@@ -175,27 +175,27 @@ struct MidW4 {
 
 // `args_of`: the arguments for stages of so many MFMA steps. Tiles of 32 rows have stages of 32 k also where groups allow 64, if a workgroup has few rounds:
 // more pieces of K divide the rest better and each costs less. us, stages of 32 and 64 k: 26 rows, 1408 x 2240 8.1 and 8.5, 1920 x 1096 7.8 and
-// 8.2, 6528 x 1448 12.0 and 12.2, 128 rows, 1920 x 1096 9.0 and 9.3; 2560 x 4096 13.4 and 12.9, 3072 x 2048 11.3 and 11.1. The second pair of costs is a
-// fit to such times alone (3 %), the first one is comparable with `limit_us`.
+// 8.2, 6528 x 1448 12.0 and 12.2, 128 rows, 1920 x 1096 9.0 and 9.3; 2560 x 4096 13.4 and 12.9, 3072 x 2048 11.3 and 11.1.
 template <int DT, int STEPS, typename ArgsOf>
 bool launch_w4(const void *a, const void *w, ArgsOf args_of, int64_t m, int64_t n, int64_t k, int64_t lda, double limit_us, const Workspace &ws,
                hipStream_t stream) {
     using Low = MidW4<DT, 2, STEPS>;
     using High = MidW4<DT, 4, STEPS>;
     constexpr int kLow = STEPS == 1 ? 6 : 4, kHigh = STEPS == 1 ? 5 : 3;  // stages in the ring
-    const MidCost low = {5.5, STEPS == 1 ? 0.5 : 0.9, 1.4, 0.4}, high = {6.0, STEPS == 1 ? 0.9 : 1.5, 1.5, 0.5};
-    MidChoice c2 = mid_choose<Low, 2, kLow>(low, ws, m, n, k), c4 = mid_choose<High, 4, kHigh>(high, ws, m, n, k);
-    if (std::min(c2.us, c4.us) > limit_us) return false;
-    if (c2.us >= c4.us) {
+    const MidCost low = STEPS == 1 ? MidCost{5.5, 0.5, 1.4, 0.4} : MidCost{4.21, 1.019, 1.75, 0.086, 0.0, 0.0058};
+    const MidCost high = STEPS == 1 ? MidCost{6.0, 0.9, 1.5, 0.5} : MidCost{5.1, 1.38, 1.51, 0.241, 0.0, 0.009};
+    const MidChoice c2 = mid_choose<Low, 2, kLow>(low, ws, m, n, k), c4 = mid_choose<High, 4, kHigh>(high, ws, m, n, k);
+    MidChoice shallow;
+    if constexpr (STEPS == 2) shallow = mid_choose<MidW4<DT, 2, 1>, 2, 6>({3.91, 0.602, 1.71, 0.0625, 0.0, 0.0049}, ws, m, n, k);
+    const double us = std::min({c2.us, c4.us, shallow.us});
+    if (us > limit_us) return false;
+    if (us == c4.us) {
         mid_launch<High, 4, kHigh>(c4, a, w, lda * 2, n / 2, args_of(STEPS), m, n, k, ws, stream);
         return true;
     }
     if constexpr (STEPS == 2) {
-        using Shallow = MidW4<DT, 2, 1>;
-        const MidChoice shallow = mid_choose<Shallow, 2, 6>({3.38, 0.612, 1.95, 0.17, 0.0, 0.004}, ws, m, n, k);
-        c2 = mid_choose<Low, 2, kLow>({3.61, 1.044, 1.96, 0.21, 0.0, 0.004}, ws, m, n, k);
-        if (shallow.us < c2.us) {
-            mid_launch<Shallow, 2, 6>(shallow, a, w, lda * 2, n / 2, args_of(1), m, n, k, ws, stream);
+        if (us == shallow.us) {
+            mid_launch<MidW4<DT, 2, 1>, 2, 6>(shallow, a, w, lda * 2, n / 2, args_of(1), m, n, k, ws, stream);
             return true;
         }
     }

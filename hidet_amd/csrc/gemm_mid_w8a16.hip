@@ -294,8 +294,9 @@ bool mid_w8a16_launch(const void *a, const void *w, bool nk, const void *scale, 
     auto run = [&](auto form, auto high) {
         using Op = typename decltype(form)::type;
         using High = typename decltype(high)::type;  // on 128 rows
-        const MidChoice c2 = mid_choose<Op, 2, 6>({5.5, 0.36, 1.4, 0.4, kFullRound}, ws, m, n, k), c4 = mid_choose<Op, 4, 4>({6.0, 0.5, 1.5, 0.5, kFullRound}, ws, m, n, k),
-                        c8 = mid_choose<High, 8, 3>({6.5, 0.8, 1.8, 1.0, kFullRound}, ws, m, n, k);
+        const MidChoice c2 = mid_choose<Op, 2, 6>({4.07, 0.37, 1.55, 0.077, kFullRound, 0.006}, ws, m, n, k),
+                        c4 = mid_choose<Op, 4, 4>({4.85, 0.485, 1.2, 0.252, kFullRound, 0.0089}, ws, m, n, k),
+                        c8 = mid_choose<High, 8, 3>({6.96, 0.765, 1.42, 0.426, kFullRound, 0.0142}, ws, m, n, k);
         const double us = std::min({c2.us, c4.us, c8.us});
         if ((us == c2.us ? c2 : us == c4.us ? c4 : c8).busy_us > limit_us) return false;
         if (us == c2.us) mid_launch<Op, 2, 6>(c2, a, w, las, n, args, m, n, k, ws, stream);
