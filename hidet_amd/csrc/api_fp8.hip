@@ -1,5 +1,6 @@
 // Entry points of the FP8 matmuls: argument checks and the choice of kernel family.
 #include "common.h"
+#include "skinny_fp8_tall.h"
 
 namespace qmm {
 bool skinny_fp8_supported(const void *b, int64_t k, int64_t ldb);
@@ -41,6 +42,17 @@ static void check_out_dtype(int out_dtype) {
               "output dtype must be float32, float16, bfloat16 or float8_e4m3, got code " << out_dtype);
 }
 
+// 17 to kMidRows rows: the kernel without an exchange, the narrow tiles or the tiled GEMM (false: nothing was launched), by their estimates.
+static bool small_fp8_launch(const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int out_dtype, const void *scale_a,
+                             const void *scale_b, bool block_scaled, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+    const double gemm_us = gemm_fp8_estimate_us(m, n, k, block_scaled, workspace, workspace_bytes);
+    const SkinnyFp8TallPlan tall = skinny_fp8_tall_plan(block_scaled, m, n, k);
+    if (mid_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, block_scaled, std::min(gemm_us, 1.15 * tall.us), workspace, workspace_bytes, stream)) return true;
+    if (1.15 * tall.us > gemm_us) return false;
+    skinny_fp8_tall_launch(tall, block_scaled, a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, stream);
+    return true;
+}
+
 HIDET_API void hidet_matmul_f8(const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda,
                                int64_t ldb, int out_dtype, const void *scale_a, const void *scale_b, void *workspace,
                                int64_t workspace_bytes, void *stream_) {
@@ -56,7 +68,7 @@ HIDET_API void hidet_matmul_f8(const void *a, const void *b, void *c, int64_t m,
     if (m <= 16 && skinny_fp8_supported(b, k, ldb))
         skinny_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, stream);
     else if (m <= kMidRows && k > 0 && k % 16 == 0 && lda % 16 == 0 && ldb % 16 == 0 && n % 4 == 0 && aligned(a, 16) && aligned(b, 16) && aligned(c, 16) &&
-             mid_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, false, gemm_fp8_estimate_us(m, n, k, false, workspace, workspace_bytes), workspace, workspace_bytes, stream))
+             small_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, false, workspace, workspace_bytes, stream))
         return;
     else
         gemm_fp8_launch(a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, workspace, workspace_bytes, stream);
@@ -100,8 +112,7 @@ static void f8_scaled_dispatch(const void *a, const void *b, const void *scale_a
     check_workspace(workspace, workspace_bytes);
     if (m <= 16)  // decode: the bandwidth-bound kernel, one pass over b
         skinny_fp8_block_scaled_launch(a, b, scale_a, scale_b, c, m, n, k, out_dtype, e5m2, stream);
-    else if (!e5m2 && m <= kMidRows &&
-             mid_fp8_launch(a, b, c, m, n, k, k, k, out_dtype, scale_a, scale_b, true, gemm_fp8_estimate_us(m, n, k, true, workspace, workspace_bytes), workspace, workspace_bytes, stream))
+    else if (!e5m2 && m <= kMidRows && small_fp8_launch(a, b, c, m, n, k, k, k, out_dtype, scale_a, scale_b, true, workspace, workspace_bytes, stream))
         return;
     else
         gemm_fp8_scaled_launch(a, b, scale_a, scale_b, c, m, n, k, out_dtype, e5m2, workspace, workspace_bytes, stream);

@@ -8,6 +8,9 @@
 // meet in LDS; a workgroup owns 16 output columns, so N / 16 workgroups stream b exactly once.
 #include "common.h"
 #include "numeric.h"
+#include "skinny_fp8_tall.h"
+
+#include <cmath>
 
 namespace qmm {
 namespace {
@@ -195,6 +198,146 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_fp8_staged_kernel(const uin
     }
 }
 
+// 17 rows and more, K a multiple of 16 (block-scaled 128), aligned activations: the kernel above for 16 RB rows x 16 CG columns per workgroup. A weight of a few megabytes is
+// read in less time than the narrow tiles (gemm_mid.h) take to fill their rings and to bring the pieces of K together: nothing is shared between waves here before the end, so
+// there is no barrier and no exchange, and a launch costs 2.5 us beside its loads. Those bound it, about 70 KB per us and CU from the L2: every workgroup reads its
+// rows' activations for 16 or 32 columns only, so wide and deep matrices stay with the narrow tiles. Per-tensor scales, narrow tiles -> here, us, weights from
+// the last-level cache: 24 x 1024 x 1024 5.5 -> 2.9, 32 x 2048 x 2048 7.1 -> 3.6, 32 x 4096 x 4096 9.2 -> 5.8, 64 x 4096 x 4096 9.4 -> 7.4, 128 x 4096 x 1024 7.5 -> 5.2, 256 x
+// 2048 x 2048 7.4 -> 6.8; block-scaled 24 x 7168 x 1536 9.5 -> 7.0. One step of a wave in flight: with the next one's loads (two) in front of the multiplication
+// 32 x 4096 x 4096 takes 6.3 (7.2); sixteen waves of half the steps are as fast.
+constexpr int kTallWaves = 8;
+template <int RB, int CG>
+constexpr int tall_lds_bytes(bool scaled) {
+    const int stage = kTallWaves * RB * 16 * 9 * 16, sums = kTallWaves * RB * CG * 16 * 17 * 4;
+    return (stage > sums ? stage : sums) + (scaled ? kTallWaves * RB * 64 : 0);
+}
+// TAIL: K is no multiple of 128 (a kernel of its own: the branch in the loop costs the others up to 12 %).
+template <bool SCALED, bool TAIL, int RB, int CG>
+__global__ __launch_bounds__(64 * kTallWaves) void skinny_fp8_tall_kernel(const uint8_t *a, const uint8_t *b, int64_t lda, int64_t ldb, int m, int n, int k, int tiles_m, int tiles_n,
+                                                              const float *__restrict__ scale_a, const float *__restrict__ scale_b, void *__restrict__ c, int out_dtype) {
+    constexpr int kTile = RB * 16 * 9;  // a wave's activations of a step, 16-byte pieces: rows of 128 + 16 bytes
+    extern __shared__ uint4v_t memory[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = lane >> 4, ls = lane & 15;
+    // the row tiles of a column tile are neighbours on one XCD: they read the same weights
+    const int local = int(blockIdx.x >> 3), tile_n = local / tiles_m * 8 + int(blockIdx.x & 7), m0 = local % tiles_m * (16 * RB), n0 = tile_n * (16 * CG);
+    if (tile_n >= tiles_n) return;
+    const int steps = (k + 127) >> 7;
+    const int steps_per_wave = (steps + kTallWaves - 1) / kTallWaves;
+    const int s_begin = wave * steps_per_wave, s_end = min(steps, s_begin + steps_per_wave);
+
+    float4_t acc[RB][CG];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int g = 0; g < CG; ++g) acc[r][g] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const float *sa_col[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) sa_col[r] = SCALED ? scale_a + min(m0 + 16 * r + ls, m - 1) : nullptr;
+    const float *sb_row = SCALED ? scale_b + int64_t(n0 >> 7) * steps : nullptr;  // the columns lie in one 128-column block
+    const uint8_t *bp[CG], *ap[2 * RB];
+#pragma unroll
+    for (int g = 0; g < CG; ++g) bp[g] = b + int64_t(min(n0 + 16 * g + ls, n - 1)) * ldb + 32 * kg;
+#pragma unroll
+    for (int i = 0; i < 2 * RB; ++i) ap[i] = a + int64_t(min(m0 + 8 * i + (lane >> 3), m - 1)) * lda + 16 * (lane & 7);  // 8 rows each
+
+    uint4v_t *const tile = memory + wave * kTile;
+    float *const factors = reinterpret_cast<float *>(memory) + (tall_lds_bytes<RB, CG>(false) + wave * RB * 64) / 4;  // SCALED: of a step's rows
+    for (int st = s_begin; st < s_end; ++st) {
+        uint4v_t w[CG][2], x[2 * RB];
+        float f[RB];
+        const int left = k - st * 128;
+        if (!TAIL || left >= 128) {
+#pragma unroll
+            for (int g = 0; g < CG; ++g) {
+                w[g][0] = *reinterpret_cast<const uint4v_t *>(bp[g] + int64_t(st) * 128);
+                w[g][1] = *reinterpret_cast<const uint4v_t *>(bp[g] + int64_t(st) * 128 + 16);
+            }
+#pragma unroll
+            for (int i = 0; i < 2 * RB; ++i) x[i] = *reinterpret_cast<const uint4v_t *>(ap[i] + int64_t(st) * 128);
+        } else {  // the step that K ends in, with a whole 16-byte piece
+#pragma unroll
+            for (int g = 0; g < CG; ++g)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    w[g][h] = uint4v_t{0, 0, 0, 0};
+                    if (32 * kg + 16 * h < left) w[g][h] = *reinterpret_cast<const uint4v_t *>(bp[g] + int64_t(st) * 128 + 16 * h);
+                }
+#pragma unroll
+            for (int i = 0; i < 2 * RB; ++i) {
+                x[i] = uint4v_t{0, 0, 0, 0};
+                if (16 * (lane & 7) < left) x[i] = *reinterpret_cast<const uint4v_t *>(ap[i] + int64_t(st) * 128);
+            }
+        }
+        if (SCALED) {
+            const float sb = sb_row[st];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) f[r] = sa_col[r][int64_t(st) * m] * sb;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all of the step's loads are under way
+#pragma unroll
+        for (int i = 0; i < 2 * RB; ++i) tile[(8 * i + (lane >> 3)) * 9 + (lane & 7)] = x[i];
+        if (SCALED)
+#pragma unroll
+            for (int r = 0; r < RB; ++r) factors[16 * r + ls] = f[r];  // the four lane groups store the same 16 values
+        __builtin_amdgcn_wave_barrier();
+        int8v_t cv[CG];
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) cv[g][e] = int(w[g][e >> 2][e & 3]);
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const uint4v_t x0 = tile[(16 * r + ls) * 9 + 2 * kg], x1 = tile[(16 * r + ls) * 9 + 2 * kg + 1];
+            int8v_t rv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rv[e] = int(x0[e]), rv[4 + e] = int(x1[e]);
+#pragma unroll
+            for (int g = 0; g < CG; ++g) {
+                if (SCALED) {
+                    const float4_t f4 = reinterpret_cast<const float4_t *>(factors)[4 * r + kg];
+                    const float4_t part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rv, cv[g], zero, 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[r][g][v] = fmaf(part[v], f4[v], acc[r][g][v]);
+                } else {
+                    acc[r][g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rv, cv[g], acc[r][g], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the sums take the place of the activations
+    float *red = reinterpret_cast<float *>(memory);  // [wave][RB][CG][16][17]
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int g = 0; g < CG; ++g)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) red[(((wave * RB + r) * CG + g) * 16 + 4 * kg + v) * 17 + ls] = acc[r][g][v];
+    float alpha = 1.0f;
+    if (!SCALED && scale_a != nullptr) alpha = *scale_a;
+    if (!SCALED && scale_b != nullptr) alpha *= *scale_b;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (RB * CG + 1) / 2; ++i) {
+        const int at = i * 512 + tid, cn = at & 15, row = (at >> 4) % (16 * RB), g = at / (256 * RB);
+        const int col = n0 + 16 * g + cn;
+        if (g < CG && m0 + row < m && col < n) {
+            float v = 0.f;
+#pragma unroll
+            for (int p = 0; p < kTallWaves; ++p) v += red[(((p * RB + (row >> 4)) * CG + g) * 16 + (row & 15)) * 17 + cn];
+            v *= alpha;
+            const int64_t o = int64_t(m0 + row) * n + col;
+            if (out_dtype == HIDET_QMM_F32) static_cast<float *>(c)[o] = v;
+            else if (out_dtype == HIDET_QMM_BF16) static_cast<uint16_t *>(c)[o] = f32_to_bf16_bits(v);
+            else if (out_dtype == HIDET_QMM_F16) static_cast<uint16_t *>(c)[o] = f32_to_f16_bits(v);
+            else static_cast<uint8_t *>(c)[o] = f32_to_e4m3(v);
+        }
+    }
+}
+
 }  // namespace
 
 bool skinny_fp8_supported(const void *b, int64_t k, int64_t ldb) { return (ldb % 16 == 0) && (k % 16 == 0) && aligned(b, 16) && k > 0; }
@@ -224,6 +367,52 @@ void skinny_fp8_launch(const void *a, const void *b, void *c, int64_t m, int64_t
         default: QMM_FAIL("unsupported output dtype code " << out_dtype);
     }
 #undef QMM_FP8_SKINNY
+}
+
+// Row blocks and column groups per workgroup of the smallest estimated time: fits (7 %) to 1550 to 1790 launches on 270 to 310 shapes of 17 to 1024 rows, K and N of 512
+// to 8192, in the mean of weights from memory and from the last-level cache. The caller takes this kernel where it is ahead of the other estimates by 15 %: over the
+// fastest kernel that costs 0.8 % in the mean (block-scaled 1.0 to 1.3), at an even chance 0.6 to 1.1 (0.7 to 0.9), but then 39 of 1158 calls would be more than 3 % slower
+// than on the others, now 3.
+SkinnyFp8TallPlan skinny_fp8_tall_plan(bool scaled, int64_t m, int64_t n, int64_t k) {
+    SkinnyFp8TallPlan best;
+    const double cus = std::max(1, device_cus()), steps = double(cdiv(cdiv(k, 128), kTallWaves));  // steps of a wave
+    for (int most = 1; most <= 4; ++most) {
+        const int64_t tiles_m = cdiv(m, 16 * most);
+        const int rb = int(cdiv(cdiv(m, tiles_m), 16));
+        for (int cg = 1; cg <= 2; ++cg) {
+            const double groups = double(tiles_m) * double(cdiv(n, 16 * cg)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
+            const double us = scaled ? 2.33 + 0.151 * share * rb * cg + rounds * steps * (0.1885 * rb + 0.363 * cg + 0.024 * rb * cg)
+                                     : 2.33 + 0.125 * share * rb * cg + rounds * steps * (0.145 * rb + 0.391 * cg + 0.026 * rb * cg);
+            if (us < best.us) best = SkinnyFp8TallPlan{us, rb, cg};
+        }
+    }
+    return best;
+}
+
+void skinny_fp8_tall_launch(const SkinnyFp8TallPlan &plan, bool scaled, const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                            int out_dtype, const void *scale_a, const void *scale_b, hipStream_t stream) {
+    const int64_t tiles_m = cdiv(m, 16 * plan.rb), tiles_n = cdiv(n, 16 * plan.cg), grid = tiles_m * cdiv(tiles_n, 8) * 8;
+    QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
+    auto go = [&](auto kern, int lds) {
+        allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+        launch(kern, dim3(uint32_t(grid)), dim3(64 * kTallWaves), size_t(lds), stream, static_cast<const uint8_t *>(a), static_cast<const uint8_t *>(b), lda, ldb, int(m), int(n), int(k),
+               int(tiles_m), int(tiles_n), static_cast<const float *>(scale_a), static_cast<const float *>(scale_b), c, out_dtype);
+    };
+    auto of = [&](auto rb, auto cg) {
+        constexpr int RB = decltype(rb)::value, CG = decltype(cg)::value;
+        if (scaled) go(skinny_fp8_tall_kernel<true, false, RB, CG>, tall_lds_bytes<RB, CG>(true));
+        else if (k % 128 == 0) go(skinny_fp8_tall_kernel<false, false, RB, CG>, tall_lds_bytes<RB, CG>(false));
+        else go(skinny_fp8_tall_kernel<false, true, RB, CG>, tall_lds_bytes<RB, CG>(false));
+    };
+    auto rows = [&](auto cg) {
+        using std::integral_constant;
+        if (plan.rb == 1) of(integral_constant<int, 1>(), cg);
+        else if (plan.rb == 2) of(integral_constant<int, 2>(), cg);
+        else if (plan.rb == 3) of(integral_constant<int, 3>(), cg);
+        else of(integral_constant<int, 4>(), cg);
+    };
+    if (plan.cg == 1) rows(std::integral_constant<int, 1>());
+    else rows(std::integral_constant<int, 2>());
 }
 
 // float8_e5m2 operands, up to 16 rows: the plain kernel with the MFMA's bf8 format
