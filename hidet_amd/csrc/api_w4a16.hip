@@ -1,5 +1,6 @@
 // Entry point of the group-wise W4A16 matmul: argument checks and the choice of kernel family.
 #include "common.h"
+#include "skinny_common.h"
 
 namespace qmm {
 void skinny_w4a16_launch(const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k,
@@ -75,9 +76,12 @@ void w4a16_dispatch(const void *a, const void *w, const void *scales, const void
     QMM_CHECK(a && c && (k == 0 || (w && scales)), "null tensor pointer");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     // Beyond one 16-row pass of the bandwidth-bound kernel the narrow tiles (gemm_mid.h) or, where those are estimated to take
-    // longer, the MFMA GEMM on tall ones (K = 4096, N = 11008: 128 / 160 / 192 / 512 rows narrow 27.6 / 39.8 / 59.8 / 80.2 us, tall 35.5 / 42.9 / 44.9 / 64.4). What
+    // longer, the MFMA GEMM on tall ones, and up to 16 rows the narrow tiles too where they are estimated to be ahead by 2 % (K = 4096, N = 11008: 128 / 160 / 192 / 512 rows narrow 27.6 / 39.8 / 59.8 / 80.2 us, tall 35.5 / 42.9 / 44.9 / 64.4). What
     // neither takes is done in passes of 16 rows.
     const bool gemm = m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size);
+    if (m <= 16 && parallel_k_parts == 0 && k >= kSkinnyEstimateK &&
+        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype, skinny_estimate_us(false, m, k, n) / 1.02, workspace, workspace_bytes, stream))
+        return;
     if (m > 16 && m <= 1024 &&
         mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype,
                          gemm ? gemm_w4a16_estimate_us(m, k, n, lda, group_size, bias != nullptr, workspace, workspace_bytes) : 1e29, workspace, workspace_bytes, stream))

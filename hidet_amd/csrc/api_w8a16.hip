@@ -1,5 +1,6 @@
 // Entry point of the W8A16 matmul: argument checks and the choice of kernel family.
 #include "common.h"
+#include "skinny_common.h"
 
 namespace qmm {
 bool skinny_w8a16_supported(const void *w, const void *scale, const void *bias, int64_t k, int64_t n);
@@ -188,8 +189,8 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     // over the weights, and the GEMMs take over: narrow tiles (gemm_mid.h) or the prefill tiles, whichever is estimated to be
     // the faster (K=4096, N=11008, weights from HBM: narrow 14.6 / 18.3 / 24.1 / 34.6 us at M=17 / 64 / 128 / 256, prefill tiles 17.0 /
     // 20.6 / 29.2 / 39.1; at M=512 64 against 57; a wide weight, 4096 x 57344: narrow 54 / 65 us at M=17 / 64, prefill tiles 46 / 52). For 9 to 16 rows the bandwidth-bound kernel is
-    // ahead of the GEMM on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
-    // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49).
+    // ahead of the prefill tiles on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
+    // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49), but not of the narrow ones (below).
     if (m > 16 && k > 0 && n % 4 != 2) {
         const bool gemm = gemm_w8a16_supported(a, w, c, m, k, n, lda);
         const double limit = gemm ? gemm_w8a16_estimate_us(m, k, n, ws) : 1e29;
@@ -199,6 +200,11 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
             return;
         }
     }
+    // A decode batch that the narrow tiles serve sooner: ahead by 3 % (of 512 shapes 246 go there, 17 % faster in the mean, 13 on weights from memory; 5 and 20 of them
+    // are more than 3 % slower).
+    if (m <= 16 && parallel_k_parts == 0 && k >= kSkinnyEstimateK && n % 4 == 0 && skinny_w8a16_supported(w, scale, bias, k, n) &&
+        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, skinny_estimate_us(true, m, k, n) / 1.03, ws, stream))
+        return;
     // N = 4 i + 2 on the narrow tiles as it lies, also for one pass of 16 rows (which the bandwidth-bound kernel takes on a copy only),
     // unless the copy and the prefill tiles are estimated to take less. us, on copies against that: 1 x 1026 x 2050 14.0 and 7.6, 16 x 4096 x 4098
     // 21.3 and 11.1, 203 x 4096 x 4098 27.9 and 20.4, 600 x 4096 x 4098 45 and 37, 16 x 8192 x 8190 35 and 18; 1 x 2002 x 514 element by element 193
