@@ -1,6 +1,7 @@
 // Entry point of the W8A16 matmul: argument checks and the choice of kernel family.
 #include "common.h"
 #include "skinny_common.h"
+#include "skinny_w8a16_nk_tall.h"
 
 namespace qmm {
 bool skinny_w8a16_supported(const void *w, const void *scale, const void *bias, int64_t k, int64_t n);
@@ -239,14 +240,20 @@ void w8a16_nk_dispatch(const void *a, const void *w_nk, const void *scale, const
     QMM_CHECK(skinny_w8a16_nk_supported(w_nk, k, ldw),
               "K-contiguous weights need K and the row stride to be multiples of 16 and a 16-byte aligned pointer, got K=" << k
                                                                                                                          << " ldw=" << ldw);
-    // More than one pass of 16 rows: up to 64 the narrow tiles reading the same layout (4096 x 4096, 49 rows: 12.3 us, the prefill
+    // More than one pass of 16 rows: up to 64 the kernel without an exchange for small weights or the narrow tiles reading the same layout (4096 x 4096, 49 rows: 12.3 us, the prefill
     // tiles 19.9) unless they are estimated to take longer, which they do on very wide weights (1024 x 131072, 33 rows: 61 us
     // against 47; 4096 x 57344, 64 rows: 84 against 78); else the prefill tiles, where their conditions hold.
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     const bool gemm = m > 16 && gemm_w8a16_nk_supported(a, w_nk, c, m, k, n, lda, ldw);
-    if (m > 16 && m <= 64 && k > 0 &&
-        mid_w8a16_launch(a, w_nk, true, scale, bias, c, m, k, n, lda, ldw, n, n, gemm ? gemm_w8a16_nk_estimate_us(m, k, n, ws) : 1e29, ws, stream))
-        return;
+    if (m > 16 && m <= 64 && k > 0) {
+        const double gemm_us = gemm ? gemm_w8a16_nk_estimate_us(m, k, n, ws) : 1e29;
+        const SkinnyNkTallPlan tall = skinny_w8a16_nk_tall_plan(a, m, n, k, lda);
+        if (mid_w8a16_launch(a, w_nk, true, scale, bias, c, m, k, n, lda, ldw, n, n, std::min(gemm_us, 1.2 * tall.us), ws, stream)) return;
+        if (1.2 * tall.us <= gemm_us) {
+            skinny_w8a16_nk_tall_launch(tall, a, w_nk, scale, bias, c, m, k, n, lda, ldw, stream);
+            return;
+        }
+    }
     if (gemm) gemm_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, ws, stream);
     else
         skinny_w8a16_nk_launch(a, w_nk, scale, bias, c, m, k, n, lda, ldw, stream);

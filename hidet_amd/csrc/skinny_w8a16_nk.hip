@@ -18,6 +18,9 @@
 // flight at a time and the 8 to 11 waves per CU hide the latency (the FP8 kernel of the same shape was measured a third
 // slower with all of a trip's loads really issued up front).
 #include "common.h"
+#include "skinny_w8a16_nk_tall.h"
+
+#include <cmath>
 
 namespace qmm {
 namespace {
@@ -248,7 +251,166 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_nk_wide_kernel(const 
     }
 }
 
+// 17 rows and more of small weights, aligned activations: 16 RB rows x 16 CG columns per workgroup, eight waves that split K and meet once, in LDS. The narrow tiles (gemm_mid.h)
+// take 7 us for what this reads in 1 to 2: no ring, no barrier before the end, no exchange. What bounds it is what a CU gets from the L2 (every workgroup reads its rows' activations
+// for 16 or 32 columns only), so wide and deep matrices stay with the narrow tiles. A wave has one step in flight, its activations turned into fragments through
+// an LDS tile of its own as above; codes are widened exactly, to q / 512 (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25), once for all rows.
+// us, narrow tiles -> here, weights from the last-level cache: 17 x 1024 x 1024 6.9 -> 3.0, 32 x 2048 x 1024 7.7 -> 3.6, 32 x 4096 x 4096 10.2 -> 7.5, 48 x 1536 x 3072 8.3 -> 4.8, 64 x
+// 2048 x 2048 8.0 -> 4.5, 64 x 3072 x 4096 11.3 -> 8.0. TAIL: K is no multiple of 128 (but of 16).
+constexpr int kTallWaves = 8;
+template <int RB, int CG>
+constexpr int tall_lds_bytes() {
+    const int stage = kTallWaves * RB * 16 * 17 * 16, sums = kTallWaves * RB * CG * 16 * 17 * 4;
+    return stage > sums ? stage : sums;
+}
+template <bool TAIL, int RB, int CG>
+__global__ __launch_bounds__(64 * kTallWaves) void skinny_w8a16_nk_tall_kernel(const _Float16 *a, const int8_t *w, int64_t lda, int64_t ldw, int m, int n, int k, int tiles_m,
+                                                                               int tiles_n, const _Float16 *__restrict__ scale, const _Float16 *__restrict__ bias,
+                                                                               _Float16 *__restrict__ c) {
+    constexpr int kTile = RB * 16 * 17;  // a wave's activations of a step, 16-byte pieces: rows of 256 + 16 bytes
+    extern __shared__ uint4v_t memory[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = lane >> 4, ls = lane & 15;
+    // the row tiles of a column tile are neighbours on one XCD: they read the same weights
+    const int local = int(blockIdx.x >> 3), tile_n = local / tiles_m * 8 + int(blockIdx.x & 7), m0 = local % tiles_m * (16 * RB), n0 = tile_n * (16 * CG);
+    if (tile_n >= tiles_n) return;
+    const int steps = (k + 127) >> 7;
+    const int steps_per_wave = (steps + kTallWaves - 1) / kTallWaves;
+    const int s_begin = wave * steps_per_wave, s_end = min(steps, s_begin + steps_per_wave);
+
+    float4_t acc[RB][CG];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int g = 0; g < CG; ++g) acc[r][g] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const int8_t *wp[CG];
+    const _Float16 *ap[4 * RB];
+#pragma unroll
+    for (int g = 0; g < CG; ++g) wp[g] = w + int64_t(min(n0 + 16 * g + ls, n - 1)) * ldw + 32 * kg;
+#pragma unroll
+    for (int i = 0; i < 4 * RB; ++i) ap[i] = a + int64_t(min(m0 + 4 * i + kg, m - 1)) * lda + 8 * ls;  // 4 rows each
+    uint4v_t *const tile = memory + wave * kTile;
+    for (int st = s_begin; st < s_end; ++st) {
+        uint4v_t raw[CG][2], x[4 * RB];
+        const int left = k - st * 128;
+        if (!TAIL || left >= 128) {
+#pragma unroll
+            for (int g = 0; g < CG; ++g) {
+                raw[g][0] = *reinterpret_cast<const uint4v_t *>(wp[g] + int64_t(st) * 128);
+                raw[g][1] = *reinterpret_cast<const uint4v_t *>(wp[g] + int64_t(st) * 128 + 16);
+            }
+#pragma unroll
+            for (int i = 0; i < 4 * RB; ++i) x[i] = *reinterpret_cast<const uint4v_t *>(ap[i] + int64_t(st) * 128);
+        } else {  // the step that K ends in: activations past it are zeros, whatever the codes
+#pragma unroll
+            for (int g = 0; g < CG; ++g)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    raw[g][h] = uint4v_t{0, 0, 0, 0};
+                    if (32 * kg + 16 * h < left) raw[g][h] = *reinterpret_cast<const uint4v_t *>(wp[g] + int64_t(st) * 128 + 16 * h);
+                }
+#pragma unroll
+            for (int i = 0; i < 4 * RB; ++i) {
+                x[i] = uint4v_t{0, 0, 0, 0};
+                if (8 * ls < left) x[i] = *reinterpret_cast<const uint4v_t *>(ap[i] + int64_t(st) * 128);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all of the step's loads are under way
+#pragma unroll
+        for (int i = 0; i < 4 * RB; ++i) tile[(4 * i + kg) * 17 + ls] = x[i];
+        __builtin_amdgcn_wave_barrier();
+        half8_t q[CG][4];
+#pragma unroll
+        for (int g = 0; g < CG; ++g)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t u[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const uint32_t src = raw[g][j >> 1][2 * (j & 1) + (p >> 1)] ^ 0x80808080u;
+                    u[p] = __builtin_amdgcn_perm(src, src, (p & 1) ? 0x0c030c02u : 0x0c010c00u);
+                    const half2_t v = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, u[p]), half2_t{_Float16(32768.0f), _Float16(32768.0f)}, half2_t{_Float16(-0.25f), _Float16(-0.25f)});
+                    q[g][j][2 * p] = v[0];
+                    q[g][j][2 * p + 1] = v[1];
+                }
+            }
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const half8_t xa = __builtin_bit_cast(half8_t, tile[(16 * r + ls) * 17 + 4 * kg + j]);
+#pragma unroll
+                for (int g = 0; g < CG; ++g) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, q[g][j], acc[r][g], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the sums take the place of the activations
+    float *red = reinterpret_cast<float *>(memory);  // [wave][RB][CG][16][17]
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int g = 0; g < CG; ++g)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) red[(((wave * RB + r) * CG + g) * 16 + 4 * kg + v) * 17 + ls] = acc[r][g][v];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (RB * CG + 1) / 2; ++i) {
+        const int at = i * 512 + tid, cn = at & 15, row = (at >> 4) % (16 * RB), g = at / (256 * RB);
+        const int col = n0 + 16 * g + cn;
+        if (g < CG && m0 + row < m && col < n) {
+            float v = 0.f;
+#pragma unroll
+            for (int p = 0; p < kTallWaves; ++p) v += red[(((p * RB + (row >> 4)) * CG + g) * 16 + (row & 15)) * 17 + cn];
+            c[int64_t(m0 + row) * n + col] = scaled_biased_f16(v * 512.0f, float(scale[col]), bias != nullptr ? float(bias[col]) : -0.0f);
+        }
+    }
+}
+
 }  // namespace
+
+// Row blocks and column groups per workgroup of the smallest estimated time: a fit (9 %) to 2224 launches on 390 shapes of 17 to 64 rows, K and N of 1024 to 11008, in the mean of
+// weights from memory and from the last-level cache. The caller takes this kernel where it is ahead of the narrow tiles' estimate, which is about 17 % too high, by 20 %: of those
+// shapes 1 to 2 % over the faster kernel in the mean, and none more than 3 % slower than on the tiles alone at 25 %, eight of 780 at 15.
+SkinnyNkTallPlan skinny_w8a16_nk_tall_plan(const void *a, int64_t m, int64_t n, int64_t k, int64_t lda) {
+    SkinnyNkTallPlan best;
+    if (lda % 8 != 0 || !aligned(a, 16)) return best;
+    const double cus = std::max(1, device_cus()), steps = double(cdiv(cdiv(k, 128), kTallWaves));  // steps of a wave
+    for (int most = 1; most <= 4; ++most) {
+        const int64_t tiles_m = cdiv(m, 16 * most);
+        const int rb = int(cdiv(cdiv(m, tiles_m), 16));
+        for (int cg = 1; cg <= 2; ++cg) {
+            const double groups = double(tiles_m) * double(cdiv(n, 16 * cg)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
+            const double us = 2.07 + 0.122 * share * rb * cg + rounds * steps * (0.319 * rb + 0.343 * cg + 0.086 * rb * cg);
+            if (us < best.us) best = SkinnyNkTallPlan{us, rb, cg};
+        }
+    }
+    return best;
+}
+
+void skinny_w8a16_nk_tall_launch(const SkinnyNkTallPlan &plan, const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
+                                 int64_t lda, int64_t ldw, hipStream_t stream) {
+    const int64_t tiles_m = cdiv(m, 16 * plan.rb), tiles_n = cdiv(n, 16 * plan.cg), grid = tiles_m * cdiv(tiles_n, 8) * 8;
+    QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
+    auto go = [&](auto kern, int lds) {
+        allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+        launch(kern, dim3(uint32_t(grid)), dim3(64 * kTallWaves), size_t(lds), stream, static_cast<const _Float16 *>(a), static_cast<const int8_t *>(w), lda, ldw, int(m), int(n), int(k),
+               int(tiles_m), int(tiles_n), static_cast<const _Float16 *>(scale), static_cast<const _Float16 *>(bias), static_cast<_Float16 *>(c));
+    };
+    auto of = [&](auto rb, auto cg) {
+        constexpr int RB = decltype(rb)::value, CG = decltype(cg)::value;
+        if (k % 128 == 0) go(skinny_w8a16_nk_tall_kernel<false, RB, CG>, tall_lds_bytes<RB, CG>());
+        else go(skinny_w8a16_nk_tall_kernel<true, RB, CG>, tall_lds_bytes<RB, CG>());
+    };
+    auto rows = [&](auto cg) {
+        using std::integral_constant;
+        if (plan.rb == 1) of(integral_constant<int, 1>(), cg);
+        else if (plan.rb == 2) of(integral_constant<int, 2>(), cg);
+        else if (plan.rb == 3) of(integral_constant<int, 3>(), cg);
+        else of(integral_constant<int, 4>(), cg);
+    };
+    if (plan.cg == 1) rows(std::integral_constant<int, 1>());
+    else rows(std::integral_constant<int, 2>());
+}
 
 bool skinny_w8a16_nk_supported(const void *w, int64_t k, int64_t ldw) {
     return (ldw % 16 == 0) && (k % 16 == 0) && aligned(w, 16) && k > 0;
