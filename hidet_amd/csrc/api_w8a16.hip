@@ -2,6 +2,7 @@
 #include "common.h"
 #include "skinny_common.h"
 #include "skinny_w8a16_nk_tall.h"
+#include "skinny_w8a16_small.h"
 
 namespace qmm {
 bool skinny_w8a16_supported(const void *w, const void *scale, const void *bias, int64_t k, int64_t n);
@@ -192,10 +193,19 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     // 20.6 / 29.2 / 39.1; at M=512 64 against 57; a wide weight, 4096 x 57344: narrow 54 / 65 us at M=17 / 64, prefill tiles 46 / 52). For 9 to 16 rows the bandwidth-bound kernel is
     // ahead of the prefill tiles on every shape measured (4096 x 11008: 13.5 - 14.1 against 16.5 us; 8192 x 8192: 16.9 - 18.2
     // against 22.4; 8192 x 28672: 42.6 - 43.8 against 49), but not of the narrow ones (below).
+    // Small weights take a kernel without an exchange where it is ahead of the others by 8 % (skinny_w8a16_small.hip).
+    const SkinnySmallPlan small = m <= kMidRows && parallel_k_parts == 0 ? skinny_w8a16_small_plan(a, m, n, k, lda) : SkinnySmallPlan();
+    const double small_us = 1.08 * small.us;
+    const auto small_launch = [&](double limit) {
+        if (small_us > limit) return false;
+        skinny_w8a16_small_launch(small, a, w, scale, bias, c, m, k, n, lda, stream);
+        return true;
+    };
     if (m > 16 && k > 0 && n % 4 != 2) {
         const bool gemm = gemm_w8a16_supported(a, w, c, m, k, n, lda);
         const double limit = gemm ? gemm_w8a16_estimate_us(m, k, n, ws) : 1e29;
-        if (m <= kMidRows && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, limit, ws, stream)) return;
+        if (m <= kMidRows && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, std::min(limit, small_us), ws, stream)) return;
+        if (small_launch(limit)) return;
         if (gemm) {
             gemm_w8a16_launch(a, w, scale, bias, c, m, k, n, lda, n, n, ws, stream);
             return;
@@ -203,16 +213,20 @@ void w8a16_dispatch(const void *a, const void *w, const void *scale, const void 
     }
     // A decode batch that the narrow tiles serve sooner: ahead by 3 % (of 512 shapes 246 go there, 17 % faster in the mean, 13 on weights from memory; 5 and 20 of them
     // are more than 3 % slower).
-    if (m <= 16 && parallel_k_parts == 0 && k >= kSkinnyEstimateK && n % 4 == 0 && skinny_w8a16_supported(w, scale, bias, k, n) &&
-        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, skinny_estimate_us(true, m, k, n) / 1.03, ws, stream))
-        return;
+    if (m <= 16 && parallel_k_parts == 0 && k > 0 && n % 4 == 0 && skinny_w8a16_supported(w, scale, bias, k, n)) {
+        const double limit = skinny_estimate_us(true, m, k, n) / 1.03;
+        if (k >= kSkinnyEstimateK && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, std::min(limit, small_us), ws, stream)) return;
+        if (small_launch(limit)) return;
+    }
     // N = 4 i + 2 on the narrow tiles as it lies, also for one pass of 16 rows (which the bandwidth-bound kernel takes on a copy only),
     // unless the copy and the prefill tiles are estimated to take less. us, on copies against that: 1 x 1026 x 2050 14.0 and 7.6, 16 x 4096 x 4098
     // 21.3 and 11.1, 203 x 4096 x 4098 27.9 and 20.4, 600 x 4096 x 4098 45 and 37, 16 x 8192 x 8190 35 and 18; 1 x 2002 x 514 element by element 193
     // and 7.7 (0.1 us per k whatever else).
-    if (n % 4 == 2 && k > 0 && m <= kMidRows && (k >= 64 || m * k * n > kElementWise) &&
-        mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, padded_estimate_us(a, m, k, n, lda, ws), ws, stream))
-        return;
+    if (n % 4 != 0 && k > 0 && m <= kMidRows && (k >= 64 || m * k * n > kElementWise)) {
+        const double limit = padded_estimate_us(a, m, k, n, lda, ws);
+        if (n % 4 == 2 && mid_w8a16_launch(a, w, false, scale, bias, c, m, k, n, lda, n, n, n, std::min(limit, small_us), ws, stream)) return;
+        if (small_launch(limit)) return;
+    }
     // Sizes the GEMM does not take (K no multiple of 64, N of 4): up to 32 rows two passes of the bandwidth-bound kernel,
     // which takes any K and N a multiple of 4, cost less than a copy of the weight and a GEMM; more rows and other N take the
     // copy. Tiny matrices are left to the element-wise kernel.

@@ -380,7 +380,8 @@ SkinnyFp8TallPlan skinny_fp8_tall_plan(bool scaled, int64_t m, int64_t n, int64_
         const int64_t tiles_m = cdiv(m, 16 * most);
         const int rb = int(cdiv(cdiv(m, tiles_m), 16));
         for (int cg = 1; cg <= 2; ++cg) {
-            const double groups = double(tiles_m) * double(cdiv(n, 16 * cg)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
+            // (of the XCD with the most column tiles, times eight)
+            const double groups = double(tiles_m) * double(8 * cdiv(cdiv(n, 16 * cg), 8)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
             const double us = scaled ? 2.33 + 0.151 * share * rb * cg + rounds * steps * (0.1885 * rb + 0.363 * cg + 0.024 * rb * cg)
                                      : 2.33 + 0.125 * share * rb * cg + rounds * steps * (0.145 * rb + 0.391 * cg + 0.026 * rb * cg);
             if (us < best.us) best = SkinnyFp8TallPlan{us, rb, cg};

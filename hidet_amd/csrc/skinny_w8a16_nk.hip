@@ -379,7 +379,8 @@ SkinnyNkTallPlan skinny_w8a16_nk_tall_plan(const void *a, int64_t m, int64_t n, 
         const int64_t tiles_m = cdiv(m, 16 * most);
         const int rb = int(cdiv(cdiv(m, tiles_m), 16));
         for (int cg = 1; cg <= 2; ++cg) {
-            const double groups = double(tiles_m) * double(cdiv(n, 16 * cg)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
+            // (of the XCD with the most column tiles, times eight)
+            const double groups = double(tiles_m) * double(8 * cdiv(cdiv(n, 16 * cg), 8)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
             const double us = 2.07 + 0.122 * share * rb * cg + rounds * steps * (0.319 * rb + 0.343 * cg + 0.086 * rb * cg);
             if (us < best.us) best = SkinnyNkTallPlan{us, rb, cg};
         }
