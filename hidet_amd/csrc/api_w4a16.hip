@@ -1,6 +1,7 @@
 // Entry point of the group-wise W4A16 matmul: argument checks and the choice of kernel family.
 #include "common.h"
 #include "skinny_common.h"
+#include "skinny_w4a16_small.h"
 
 namespace qmm {
 void skinny_w4a16_launch(const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k,
@@ -79,13 +80,20 @@ void w4a16_dispatch(const void *a, const void *w, const void *scales, const void
     // longer, the MFMA GEMM on tall ones, and up to 16 rows the narrow tiles too where they are estimated to be ahead by 2 % (K = 4096, N = 11008: 128 / 160 / 192 / 512 rows narrow 27.6 / 39.8 / 59.8 / 80.2 us, tall 35.5 / 42.9 / 44.9 / 64.4). What
     // neither takes is done in passes of 16 rows.
     const bool gemm = m > 32 && k > 0 && gemm_w4a16_supported(a, w, scales, c, k, n, lda, group_size);
-    if (m <= 16 && parallel_k_parts == 0 && k >= kSkinnyEstimateK &&
-        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype, skinny_estimate_us(false, m, k, n) / 1.02, workspace, workspace_bytes, stream))
-        return;
-    if (m > 16 && m <= 1024 &&
-        mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype,
-                         gemm ? gemm_w4a16_estimate_us(m, k, n, lda, group_size, bias != nullptr, workspace, workspace_bytes) : 1e29, workspace, workspace_bytes, stream))
-        return;
+    // Small weights take a kernel without an exchange where it is ahead of all of these by 5 % (skinny_w4a16_small.hip).
+    if (m <= 1024 && (m > 16 || parallel_k_parts == 0) && k > 0) {
+        const SkinnyW4SmallPlan small = parallel_k_parts == 0 ? skinny_w4a16_small_plan(a, scales, m, n, k, lda, group_size) : SkinnyW4SmallPlan();
+        const double limit = m <= 16 ? skinny_estimate_us(false, m, k, n) / 1.02
+                             : gemm ? gemm_w4a16_estimate_us(m, k, n, lda, group_size, bias != nullptr, workspace, workspace_bytes)
+                                    : 1e29;
+        if ((m > 16 || k >= kSkinnyEstimateK) &&
+            mid_w4a16_launch(a, w, scales, bias, c, m, k, n, lda, group_size, dtype, std::min(limit, 1.05 * small.us), workspace, workspace_bytes, stream))
+            return;
+        if (1.05 * small.us <= limit) {
+            skinny_w4a16_small_launch(small, a, w, scales, bias, c, m, k, n, lda, group_size, dtype, stream);
+            return;
+        }
+    }
     if (gemm) {
         gemm_w4a16_launch(a, w, scales, c, m, k, n, lda, group_size, dtype, workspace, workspace_bytes, stream);
         if (bias != nullptr) {

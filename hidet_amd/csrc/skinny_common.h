@@ -638,11 +638,11 @@ constexpr int kSkinnyFlatRows = 2, kSkinnyFlatSharers = 8;
 // of 128-column tiles is cheaper than this kernel's of up to 16 rows x 256 columns: from 4 to 8 rows on for weights of up to about 16 MB. us, this
 // kernel -> narrow tiles: int8 8 x 1024 x 4096 8.9 -> 6.8, 16 x 2048 x 2048 9.5 -> 7.0, 16 x 4096 x 4096 11.1 -> 9.2, 16 x 11008 x 4096 16.3 -> 13.8; int4 8 x 2048 x 2048
 // 8.9 -> 7.3, 16 x 4096 x 4096 10.4 -> 9.9. Below kSkinnyEstimateK the two are within 0.5 us of each other and the
-// int8 estimate is one of launches that hardly exchange anything.
+// estimates are those of launches that hardly exchange anything.
 constexpr int64_t kSkinnyEstimateK = 768;
 inline double skinny_estimate_us(bool int8, int64_t m, int64_t k, int64_t n) {
     const double kk = double(k) / 1024.0, nn = double(n) / 1024.0, rows = std::log2(double(m)), above = double(std::max<int64_t>(m - 8, 0)) * kk;
-    if (int8 && k < kSkinnyEstimateK) return 3.4 + 0.0032 * double(k) + 0.25 * rows;
+    if (k < kSkinnyEstimateK) return int8 ? 3.4 + 0.0032 * double(k) + 0.25 * rows : 4.2 + 0.0024 * double(k) + 0.2 * rows;
     return int8 ? 6.03 + 0.124 * kk * nn + 0.105 * kk + 0.59 * rows + 0.029 * above : 5.86 + 0.078 * kk * nn + 0.157 * kk + 0.57 * rows + 0.031 * above;
 }
 

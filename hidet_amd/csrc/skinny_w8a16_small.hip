@@ -18,7 +18,7 @@ namespace qmm {
 namespace {
 
 constexpr int kSmallWaves = 8;
-constexpr int64_t kSmallLeastK = 32, kSmallMostK = 2048, kSmallMostBytes = 8500000;
+constexpr int64_t kSmallMostRows = 512, kSmallLeastK = 32, kSmallMostK = 2048, kSmallMostBytes = 8500000;
 template <int RB, int CB>
 constexpr int small_lds_bytes() {
     const int stage = kSmallWaves * RB * 16 * 17 * 16, sums = kSmallWaves * RB * CB * 16 * 17 * 4;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w8a16_small_kernel(co
 SkinnySmallPlan skinny_w8a16_small_plan(const void *a, int64_t m, int64_t n, int64_t k, int64_t lda) {
     SkinnySmallPlan best;
     constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
-    if (k % 2 != 0 || k < kSmallLeastK || k > kSmallMostK || k * n > kSmallMostBytes || n < 4 || lda % 2 != 0 || !aligned(a, 4) || (k + 128) * n >= kMost || lda * 128 + k * 2 >= kMost) return best;
+    if (m > kSmallMostRows || k % 2 != 0 || k < kSmallLeastK || k > kSmallMostK || k * n > kSmallMostBytes || n < 4 || lda % 2 != 0 || !aligned(a, 4) || (k + 128) * n >= kMost || lda * 128 + k * 2 >= kMost) return best;
     const double cus = std::max(1, device_cus()), steps = double(cdiv(cdiv(k, 128), kSmallWaves));  // steps of a wave
     for (int most = 1; most <= 4; ++most) {
         const int64_t tiles_m = cdiv(m, 16 * most);
