@@ -32,6 +32,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_nk_kernel(const _Floa
                                                               _Float16 *__restrict__ c, int m, int k, int n) {
     __shared__ float red[WAVES][16][17];
     constexpr int kNkDepth = FULL ? 8 : 4;  // 128-deep steps per trip of the outer loop
+    static_assert(FULL || !ALIGNED_A, "aligned activations with a K off the steps go to the tall kernel");
     // STAGE (FULL with aligned activations, more than two rows): a wave fetches its 16 x 128 activation block of a step
     // with four fully coalesced loads (4 rows x 256 bytes each) and turns it into MFMA fragments through a private LDS
     // tile of 16 rows x (256 + 16) bytes, two slots.  Fetching the fragments straight from memory touches every cache
@@ -99,12 +100,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_nk_kernel(const _Floa
 #pragma unroll
                     for (int e = 0; e < 8; ++e) xa[d][j][e] = _Float16(0.0f);
                     if (m_ok && s0 + d < s_end && kb + 8 * j < k) {  // K % 8 == 0 on this path
-                        if (ALIGNED_A) {
-                            xa[d][j] = *reinterpret_cast<const half8_t *>(ap + int64_t(s0 + d) * 128 + 8 * j);
-                        } else {
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) xa[d][j][e] = ap[int64_t(s0 + d) * 128 + 8 * j + e];
-                        }
+                        for (int e = 0; e < 8; ++e) xa[d][j][e] = ap[int64_t(s0 + d) * 128 + 8 * j + e];
                     }
                 }
             }
@@ -251,7 +248,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w8a16_nk_wide_kernel(const 
     }
 }
 
-// 17 rows and more of small weights, aligned activations: 16 RB rows x 16 CG columns per workgroup, eight waves that split K and meet once, in LDS. The narrow tiles (gemm_mid.h)
+// 17 rows and more of small weights, or any number where K is no multiple of 128, aligned activations: 16 RB rows x 16 CG columns per workgroup, eight waves that split K and meet once, in LDS. The narrow tiles (gemm_mid.h)
 // take 7 us for what this reads in 1 to 2: no ring, no barrier before the end, no exchange. What bounds it is what a CU gets from the L2 (every workgroup reads its rows' activations
 // for 16 or 32 columns only), so wide and deep matrices stay with the narrow tiles. A wave has one step in flight, its activations turned into fragments through
 // an LDS tile of its own as above; codes are widened exactly, to q / 512 (a byte q ^ 0x80 as a subnormal number, times 2^15 less 0.25), once for all rows.
@@ -422,6 +419,12 @@ bool skinny_w8a16_nk_supported(const void *w, int64_t k, int64_t ldw) {
 void skinny_w8a16_nk_launch(const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
                             int64_t n, int64_t lda, int64_t ldw, hipStream_t stream) {
     const bool aligned_a = (lda % 8 == 0) && aligned(a, 16);
+    // K off the steps: the kernel below, with conditions in all of its loop, only where the activations are not aligned. us, that one and the tall one: 1 x 4032 x 4096 6.8 and
+    // 6.3, 16 x 4032 x 4096 9.4 and 6.3, 16 x 2112 x 11008 12.5 and 8.2, 16 x 9024 x 4096 17.7 and 10.0.
+    if (k % 128 != 0 && aligned_a) {
+        skinny_w8a16_nk_tall_launch(skinny_w8a16_nk_tall_plan(a, m, n, k, lda), a, w, scale, bias, c, m, k, n, lda, ldw, stream);
+        return;
+    }
     const dim3 grid(uint32_t(cdiv(n, 16)));
     for (int64_t m0 = 0; m0 < m; m0 += 16) {
         const int mt = int(std::min<int64_t>(16, m - m0));
@@ -445,7 +448,7 @@ void skinny_w8a16_nk_launch(const void *a, const void *w, const void *scale, con
         if (eight && stage) go(skinny_w8a16_nk_kernel<true, true, 8, true>, 8);
         else if (eight) aligned_a ? go(skinny_w8a16_nk_kernel<true, true, 8>, 8) : go(skinny_w8a16_nk_kernel<false, true, 8>, 8);
         else if (stage) go(skinny_w8a16_nk_kernel<true, true, 4, true>, 4);
-        else if (aligned_a) full ? go(skinny_w8a16_nk_kernel<true, true, 4>, 4) : go(skinny_w8a16_nk_kernel<true, false, 4>, 4);
+        else if (aligned_a) go(skinny_w8a16_nk_kernel<true, true, 4>, 4);  // (full)
         else full ? go(skinny_w8a16_nk_kernel<false, true, 4>, 4) : go(skinny_w8a16_nk_kernel<false, false, 4>, 4);
     }
 }

@@ -1,4 +1,4 @@
-"""int8 matmuls of 17 to 64 rows on small K-contiguous weights, which one workgroup per column strip computes over all of K: every number of row blocks and column groups, waves
+"""int8 matmuls of 17 to 64 rows on small K-contiguous weights, and of up to 16 where K is no multiple of 128, which one workgroup per column strip computes over all of K: every number of row blocks and column groups, waves
 without a step of K, K that ends inside a step, rows and columns past the end, a bias, strided activations; and shapes that stay with the narrow tiles. Small
 integers whose sums float16 holds: the results must be equal."""
 import numpy as np
@@ -21,7 +21,7 @@ def _case(m, k, n):
     return dev(a), quant.to_decode_layout(dev(q)), torch.from_numpy(exact)
 
 
-@pytest.mark.parametrize('m', [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize('m', [1, 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize('k,n', [(16, 8), (128, 20), (1024, 1024), (1040, 2052), (1088, 4096), (2048, 6144), (4096, 1000), (4096, 4096), (3008, 11008)])
 def test_exact(m, k, n):
     announce('int8 K-contiguous', m, k, n)
