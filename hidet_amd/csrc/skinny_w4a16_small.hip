@@ -13,16 +13,16 @@
 namespace qmm {
 namespace {
 
-constexpr int kSmallWaves = 8;
-constexpr int64_t kSmallMostRows = 512, kSmallMostK = 2048, kSmallMostBytes = 6300000;
-template <int RB, int CB>
+constexpr int64_t kSmallMostRows = 512, kSmallMostK = 3072, kSmallMostBytes = 6300000, kFewRowsMostK = 2048;  // (kFewRows...: up to 16 rows)
+constexpr int kWideSteps = 16;  // 128-deep steps of K from which on workgroups have sixteen waves
+template <int WAVES, int RB, int CB>
 constexpr int small_lds_bytes() {
-    const int stage = kSmallWaves * RB * 16 * 17 * 16, sums = kSmallWaves * RB * CB * 16 * 17 * 4;
+    const int stage = WAVES * RB * 16 * 17 * 16, sums = WAVES * RB * CB * 16 * 17 * 4;
     return stage > sums ? stage : sums;
 }
 
-template <int DT, int G, int RB, int CB>
-__global__ __launch_bounds__(64 * kSmallWaves) void skinny_w4a16_small_kernel(const char *a, const char *w, int lda, int m, int n, int k, int tiles_m, int tiles_n, uint32_t group_magic,
+template <int DT, int G, int WAVES, int RB, int CB>
+__global__ __launch_bounds__(64 * WAVES) void skinny_w4a16_small_kernel(const char *a, const char *w, int lda, int m, int n, int k, int tiles_m, int tiles_n, uint32_t group_magic,
                                                                               const uint16_t *scales, const uint16_t *__restrict__ bias, uint16_t *__restrict__ c) {
     using T = W4Traits<DT>;
     constexpr int kTile = RB * 16 * 17;  // a wave's activations of a step, 16-byte pieces: rows of 256 + 16 bytes
@@ -34,7 +34,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w4a16_small_kernel(co
     if (tile_n >= tiles_n * (xcd + 1) / 8) return;
     const int m0 = local % tiles_m * (16 * RB), n0 = tile_n * (16 * CB);
     const int steps = k >> 7;
-    const int steps_per_wave = (steps + kSmallWaves - 1) / kSmallWaves;
+    const int steps_per_wave = (steps + WAVES - 1) / WAVES;
     const int s_begin = wave * steps_per_wave, s_end = min(steps, s_begin + steps_per_wave);
     const int rows = min(m - m0, 16 * RB), col = min(n0 + CB * ls, n - CB);
 
@@ -132,12 +132,12 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w4a16_small_kernel(co
             for (int v = 0; v < 4; ++v) red[(((wave * RB + r) * CB + t) * 16 + 4 * kg + v) * 17 + ls] = acc[r][t][v];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < (RB * CB + 1) / 2; ++i) {
-        const int at = i * 512 + tid, in_row = at % (16 * CB), row = at / (16 * CB), ns = in_row / CB, t = in_row % CB, out = n0 + in_row;
+    for (int i = 0; i < (RB * CB * 256 + 64 * WAVES - 1) / (64 * WAVES); ++i) {
+        const int at = i * 64 * WAVES + tid, in_row = at % (16 * CB), row = at / (16 * CB), ns = in_row / CB, t = in_row % CB, out = n0 + in_row;
         if (row < rows && out < n) {
             float v = 0.f;
 #pragma unroll
-            for (int p = 0; p < kSmallWaves; ++p) v += red[(((p * RB + (row >> 4)) * CB + t) * 16 + (row & 15)) * 17 + ns];
+            for (int p = 0; p < WAVES; ++p) v += red[(((p * RB + (row >> 4)) * CB + t) * 16 + (row & 15)) * 17 + ns];
             const float add = bias != nullptr ? T::to_f32(bias[out]) : -0.0f;
             c[int64_t(m0 + row) * n + out] = DT == HIDET_QMM_BF16 ? biased_bf16_bits(v, add) : __builtin_bit_cast(uint16_t, scaled_biased_f16(v, 1.0f, add));
         }
@@ -148,22 +148,26 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w4a16_small_kernel(co
 
 // Row blocks and columns per lane of the smallest estimated time: a fit (13 %) to 2132 launches on 478 shapes of 1 to 256 rows, K of 256 to 2048 and N of 256 to 6144, in the mean of
 // weights from memory and from the last-level cache. Where it is ahead of the other kernels' estimates by 5 % those calls take 37 % less time in the mean (34 on weights
-// from memory) and none takes 3 % more; to K = 3072 it would be 15 of 560 on weights from memory, to 4096 30 of 636. (796 x 1024 x 3776, outside the fit, 23 us and
-// 29 here: no more than 512 rows.)
+// from memory) and none takes 3 % more. K from 2049 to 3072 against the other kernels, weights from the cache (from memory): 17 rows and more 15 to 24 % less time (2 to 12 % less, but 32 x
+// 3072 x 2048 7 % more), up to 16 rows 17 to 22 % less but up to 20 % more from memory, hence not there; K = 4096 6 % less and up to 30 % more. (796 x 1024 x 3776, outside the
+// fit, 23 us and 29 here: no more than 512 rows.)
+// The smallest strips (one row block, two columns per lane) of at most one workgroup per CU take sixteen waves where each then has a step: 3 to 7 % off at K = 2048 and 2 to 7 at 3072
+// (weights from memory: 2), but 1 % more at 1536, 5 at 1024, 16 to 26 where a CU gets two workgroups (of eight waves it holds them at once) and 2 to 5 on larger strips.
 SkinnyW4SmallPlan skinny_w4a16_small_plan(const void *a, const void *scales, int64_t m, int64_t n, int64_t k, int64_t lda, int group) {
     SkinnyW4SmallPlan best;
-    if (m > kSmallMostRows || k % 128 != 0 || k == 0 || k > kSmallMostK || group % 64 != 0 || n % 8 != 0 || k * n / 2 > kSmallMostBytes || lda % 2 != 0 || !aligned(a, 4) || !aligned(scales, 4) ||
+    if (m > kSmallMostRows || k % 128 != 0 || k == 0 || k > (m <= 16 ? kFewRowsMostK : kSmallMostK) || group % 64 != 0 || n % 8 != 0 || k * n / 2 > kSmallMostBytes || lda % 2 != 0 || !aligned(a, 4) || !aligned(scales, 4) ||
         lda * 128 + k * 2 >= (int64_t(1) << 31) - (1 << 20))
         return best;
-    const double cus = std::max(1, device_cus()), steps = double(cdiv(k / 128, kSmallWaves));  // steps of a wave
+    const double cus = std::max(1, device_cus()), steps = double(cdiv(k / 128, 8));  // steps of a wave, of eight
     for (int most = 1; most <= 4; ++most) {
         const int64_t tiles_m = cdiv(m, 16 * most);
         const int rb = int(cdiv(cdiv(m, tiles_m), 16));
         for (int cb = 2; cb <= 4; cb += 2) {
             // (of the XCD with the most column tiles, times eight)
             const double groups = double(tiles_m) * double(8 * cdiv(cdiv(n, 16 * cb), 8)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
-            const double us = 1.915 + 0.0134 * share * rb * cb + rounds * steps * (0.545 + 0.342 * rb + 0.154 * cb + 0.114 * rb * cb);
-            if (us < best.us) best = SkinnyW4SmallPlan{us, rb, cb};
+            const int waves = rb == 1 && cb == 2 && groups <= cus && k >= 128 * kWideSteps ? 16 : 8;
+            const double us = (waves == 16 ? 0.95 : 1.0) * (1.915 + 0.0134 * share * rb * cb + rounds * steps * (0.545 + 0.342 * rb + 0.154 * cb + 0.114 * rb * cb));
+            if (us < best.us) best = SkinnyW4SmallPlan{us, rb, cb, waves};
         }
     }
     return best;
@@ -178,13 +182,20 @@ void skinny_w4a16_small_launch(const SkinnyW4SmallPlan &plan, const void *a, con
     const uint32_t magic = uint32_t(((uint64_t(1) << 32) + uint32_t(group / (32 * fold)) - 1) / uint32_t(group / (32 * fold)));  // (0 for a divisor of 1)
     auto go = [&](auto kern, int lds) {
         allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
-        launch(kern, dim3(uint32_t(grid)), dim3(64 * kSmallWaves), size_t(lds), stream, static_cast<const char *>(a), static_cast<const char *>(w), int(lda), int(m), int(n), int(k),
+        launch(kern, dim3(uint32_t(grid)), dim3(uint32_t(64 * plan.waves)), size_t(lds), stream, static_cast<const char *>(a), static_cast<const char *>(w), int(lda), int(m), int(n), int(k),
                int(tiles_m), int(tiles_n), magic, static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(c));
     };
     auto of = [&](auto rb, auto cb) {
-        constexpr int RB = decltype(rb)::value, CB = decltype(cb)::value, kLds = small_lds_bytes<RB, CB>();
-        if (dtype == HIDET_QMM_BF16) fold == 4 ? go(skinny_w4a16_small_kernel<HIDET_QMM_BF16, 4, RB, CB>, kLds) : go(skinny_w4a16_small_kernel<HIDET_QMM_BF16, 2, RB, CB>, kLds);
-        else fold == 4 ? go(skinny_w4a16_small_kernel<HIDET_QMM_F16, 4, RB, CB>, kLds) : go(skinny_w4a16_small_kernel<HIDET_QMM_F16, 2, RB, CB>, kLds);
+        constexpr int RB = decltype(rb)::value, CB = decltype(cb)::value;
+        auto by = [&](auto waves) {
+            constexpr int W = decltype(waves)::value, kLds = small_lds_bytes<W, RB, CB>();
+            if (dtype == HIDET_QMM_BF16) fold == 4 ? go(skinny_w4a16_small_kernel<HIDET_QMM_BF16, 4, W, RB, CB>, kLds) : go(skinny_w4a16_small_kernel<HIDET_QMM_BF16, 2, W, RB, CB>, kLds);
+            else fold == 4 ? go(skinny_w4a16_small_kernel<HIDET_QMM_F16, 4, W, RB, CB>, kLds) : go(skinny_w4a16_small_kernel<HIDET_QMM_F16, 2, W, RB, CB>, kLds);
+        };
+        if constexpr (RB == 1 && CB == 2) {
+            if (plan.waves == 16) return by(integral_constant<int, 16>());
+        }
+        by(integral_constant<int, 8>());
     };
     auto rows = [&](auto cb) {
         if (plan.rb == 1) of(integral_constant<int, 1>(), cb);
