@@ -13,7 +13,7 @@
 namespace qmm {
 namespace {
 
-constexpr int64_t kSmallMostRows = 512, kSmallMostK = 3072, kSmallMostBytes = 6300000, kFewRowsMostK = 2048;  // (kFewRows...: up to 16 rows)
+constexpr int64_t kSmallMostRows = 512, kSmallMostK = 4096, kSmallMostBytes = 6300000, kFewRowsMostK = 2944;  // (kFewRows...: up to 16 rows)
 constexpr int kWideSteps = 16;  // 128-deep steps of K from which on workgroups have sixteen waves
 template <int WAVES, int RB, int CB>
 constexpr int small_lds_bytes() {
@@ -148,9 +148,9 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w4a16_small_kernel(const ch
 
 // Row blocks and columns per lane of the smallest estimated time: a fit (13 %) to 2132 launches on 478 shapes of 1 to 256 rows, K of 256 to 2048 and N of 256 to 6144, in the mean of
 // weights from memory and from the last-level cache. Where it is ahead of the other kernels' estimates by 5 % those calls take 37 % less time in the mean (34 on weights
-// from memory) and none takes 3 % more. K from 2049 to 3072 against the other kernels, weights from the cache (from memory): 17 rows and more 15 to 24 % less time (2 to 12 % less, but 32 x
-// 3072 x 2048 7 % more), up to 16 rows 17 to 22 % less but up to 20 % more from memory, hence not there; K = 4096 6 % less and up to 30 % more. (796 x 1024 x 3776, outside the
-// fit, 23 us and 29 here: no more than 512 rows.)
+// from memory) and none takes 3 % more. Beyond, 180 shapes of K 2176 to 4096, weights from the cache (from memory): 17 rows and more 15 to 25 % less time to K = 3328 (10 to 20), 5
+// to 9 to 4096 (4 to 6), none 3 % more; up to 16 rows 26 to 38 % less to 2944 (18 to 37), but at 3072 x 2048 and 4096 x 2872 20 % more from memory, hence not there; K = 6144 11 % more (29).
+// (796 x 1024 x 3776, outside the fit, 23 us and 29 here: no more than 512 rows.)
 // The smallest strips (one row block, two columns per lane) of at most one workgroup per CU take sixteen waves where each then has a step: 3 to 7 % off at K = 2048 and 2 to 7 at 3072
 // (weights from memory: 2), but 1 % more at 1536, 5 at 1024, 16 to 26 where a CU gets two workgroups (of eight waves it holds them at once) and 2 to 5 on larger strips.
 SkinnyW4SmallPlan skinny_w4a16_small_plan(const void *a, const void *scales, int64_t m, int64_t n, int64_t k, int64_t lda, int group) {

@@ -18,7 +18,7 @@ namespace qmm {
 namespace {
 
 constexpr int kSmallWaves = 8;
-constexpr int64_t kSmallMostRows = 512, kSmallLeastK = 32, kSmallMostK = 2048, kSmallMostBytes = 8500000;
+constexpr int64_t kSmallMostRows = 512, kSmallLeastK = 32, kSmallMostK = 2560, kSmallMostBytes = 8500000;
 template <int RB, int CB>
 constexpr int small_lds_bytes() {
     const int stage = kSmallWaves * RB * 16 * 17 * 16, sums = kSmallWaves * RB * CB * 16 * 17 * 4;
@@ -135,9 +135,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w8a16_small_kernel(co
 }  // namespace
 
 // Row blocks and columns per lane of the smallest estimated time: a fit (14 %) to 2040 launches on 456 shapes of 1 to 256 rows, K of 256 to 2048 and N of 256 to 6144, in the mean of
-// weights from memory and from the last-level cache. Weights of more than 8.5 MB or 2048 rows stay with the others: there the strips of rows that a workgroup reads of a weight
-// in memory cost more than the exchange that they save (1 x 2048 x 6144 8.2 us and 11.2 here, 16 x 3072 x 1024 7.1 and 8.5, 16 x 3072 x 3072 9.0 and 13.3).
-// Within, where this is ahead of the other kernels' estimates by 8 %, those 456 calls take 36 % less time in the mean (30 on weights from memory), and one of them in the former case and two in the latter take 3 to 4 % more.
+// weights from memory and from the last-level cache. Weights of more than 8.5 MB or 2560 rows stay with the others: there the strips of rows that a workgroup reads of a weight
+// in memory cost more than the exchange that they save (1 x 2048 x 6144 8.2 us and 11.2 here, 16 x 3072 x 1024 7.1 and 8.5, 16 x 3072 x 3072 9.0 and 13.3; 64 x 3072 x 2260 27 % more, 16 x 2772
+// x 2572 18; K of 2601 to 2944 4 to 12 % less time from the cache and the same from memory). K of 1900 to 2600, 64 shapes: 14 to 27 % less time, 7 to 17 % from memory, there six of 64 more than 3 %
+// slower (4 to 7 %, 64 x 2296 x 2476 15).
+// Within K = 2048, where this is ahead of the other kernels' estimates by 8 %, those 456 calls take 36 % less time in the mean (30 on weights from memory), and one of them in the former case and two in the latter take 3 to 4 % more.
 SkinnySmallPlan skinny_w8a16_small_plan(const void *a, int64_t m, int64_t n, int64_t k, int64_t lda) {
     SkinnySmallPlan best;
     constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);

@@ -23,7 +23,7 @@ def _case(m, k, n, group, dtype):
 
 @pytest.mark.parametrize('dtype', ['bfloat16', 'float16'])
 @pytest.mark.parametrize('m', [1, 16, 17, 33, 49, 64, 65, 130, 300])
-@pytest.mark.parametrize('k,n,group', [(128, 8, 128), (128, 40, 64), (384, 264, 128), (1024, 64, 256), (1024, 3000, 128), (1152, 2056, 64), (2048, 2048, 128), (2048, 6144, 128), (2176, 1024, 64), (2944, 136, 128), (3072, 2048, 64), (3200, 520, 128)])
+@pytest.mark.parametrize('k,n,group', [(128, 8, 128), (128, 40, 64), (384, 264, 128), (1024, 64, 256), (1024, 3000, 128), (1152, 2056, 64), (2048, 2048, 128), (2048, 6144, 128), (2176, 1024, 64), (2944, 136, 128), (3072, 2048, 64), (3200, 520, 128), (4096, 520, 256), (4224, 264, 128)])
 def test_exact(m, k, n, group, dtype):
     announce('int4 small weight', m, k, n, group, dtype)
     ty = getattr(torch, dtype)

@@ -23,7 +23,7 @@ def _case(m, k, n):
 
 
 @pytest.mark.parametrize('m', [1, 3, 16, 17, 33, 49, 64, 65, 130, 300])
-@pytest.mark.parametrize('k,n', [(32, 4), (64, 6), (130, 34), (256, 256), (510, 1026), (1024, 64), (1024, 3000), (1118, 2050), (1500, 1006), (2048, 2048), (2046, 4102), (2050, 1024)])
+@pytest.mark.parametrize('k,n', [(32, 4), (64, 6), (130, 34), (256, 256), (510, 1026), (1024, 64), (1024, 3000), (1118, 2050), (1500, 1006), (2048, 2048), (2046, 4102), (2050, 1024), (2514, 1030), (2560, 516), (2562, 520)])
 def test_exact(m, k, n):
     announce('int8 small weight', m, k, n)
     a, q, exact = _case(m, k, n)
