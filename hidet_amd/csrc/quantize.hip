@@ -383,12 +383,14 @@ __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const v
     }
 }
 
-// A weight of which whole cache lines are read, and read once, passes the last-level cache by, which then keeps what the next kernel reads and writes. Quantize and
-// dequantize, us: float32 4096 x 11008 114 -> 105 (along rows 90.0 -> 74.3), 4096 x 4096 45.1 -> 39.9, 1024 x 4096 15.0 -> 14.0, 512 x 3000 8.8 -> 8.5, bfloat16 4096 x 11008
-// 62.4 -> 59.7, along rows 2048 x 2048 9.1 -> 8.7. Smaller weights may be in that cache already (float32 512 x 2200 7.5 -> 7.9, along rows float16 700 x 1600 5.5 -> 5.8),
-// and of a line read in parts the others pay for it (float16 700 x 1600 in strips of 8 columns 7.0 -> 7.8).
+// A weight of half of the last-level cache and more of which whole cache lines are read, and read once, passes that cache by, which then keeps what the next kernel reads and
+// writes (4096 x 11008 float32, quantized and dequantized along rows 90.0 -> 74.3 us; int4 groups 40.4 -> 36.1). Smaller weights may lie in it. us, plain and non-temporal, three weights in
+// turn (and weights from memory): along rows bfloat16 902 x 3712 4.5 and 5.3 (4.6 and 5.5), float16 1632 x 10624 14.4 and 17.6 (16.8 and 17.1), float32 1086 x 8640 9.4 and 10.6
+// (10.7 and 10.6), 2032 x 10496 18.2 and 20.1 (19.8 and 20.1), but 1408 x 3648 6.5 and 6.2; in strips bfloat16 1297 x 6720 10.6 and 11.8 (11.9 and 11.3). int4, groups of 64: 3712 x
+// 5760 18.7 and 20.8 (21.6 and 20.9), 896 x 4288 7.9 and 8.7 (8.9 and 8.9), 3840 x 8896 31.8 and 30.1 (32.7 and 30.3). Of a line read in parts the others pay for it
+// (float16 700 x 1600 in strips of 8 columns 7.0 -> 7.8).
 constexpr int kNonTemporal = 2;
-constexpr int64_t kReadOnceFrom = 6000000;  // bytes
+constexpr int64_t kReadOnceFrom = int64_t(128) << 20;  // bytes
 
 // ---- maxima and codes in one pass over the weight ----------------------------------------------
 //
@@ -835,7 +837,7 @@ __global__ __launch_bounds__(256) void dequantize_long_row_kernel(const void *__
 // workgroups share a CU and one's loads run under another's codes (16 rows, two workgroups: 42.8 us).
 // ROWS = 0, groups beyond that: the rows are read twice. K = 4096, N = 11008, groups of 128: 82 - 87 us with the group
 // read twice in 8-byte loads, a division per weight and one-byte stores -> 38.3 us = 5.3 TB/s.
-// ONCE (kReadOnceFrom): non-temporal loads, us: 4096 x 11008 40.4 -> 36.1 = 5.6 TB/s, 4096 x 4096 16.7 -> 15.2, 2048 x 2048 6.8 -> 6.5.
+// ONCE (kReadOnceFrom): non-temporal loads, 4096 x 11008 40.4 -> 36.1 us = 5.6 TB/s.
 template <int ST, int CL, int ROWS, bool ONCE = false>
 __global__ __launch_bounds__(512, 6) void group_quantize_int4_kernel(const float *__restrict__ w, uint8_t *__restrict__ packed,
                                                                      void *__restrict__ scales, int64_t n, int group) {
@@ -1383,7 +1385,7 @@ HIDET_API void hidet_group_quantize_int4(const void *w, void *packed, void *scal
             launch(kern, dim3(cdiv(n, 4 * cl), k / group_size), dim3(512), 0, stream, static_cast<const float *>(w),
                    static_cast<uint8_t *>(packed), scales, n, group_size);
         };
-        const bool once = k * n * 4 >= 2 * kReadOnceFrom && n % 32 == 0;  // rows of whole cache lines (1024 x 1600 6.5 us, non-temporal 7.1; 2048 x 5002 15.4 and 16.3)
+        const bool once = k * n * 4 >= kReadOnceFrom && n % 32 == 0;  // (rows of whole cache lines)
         if (group_size <= 32) go(group_quantize_int4_kernel<ST, 64, 4>, 64);
         else if (group_size <= 64 && once) go(group_quantize_int4_kernel<ST, 64, 8, true>, 64);
         else if (group_size <= 64) go(group_quantize_int4_kernel<ST, 64, 8>, 64);
