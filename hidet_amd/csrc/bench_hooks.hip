@@ -1,6 +1,10 @@
 // Measurement and test hooks of libhidet_qmm.so (include/hidet_qmm_bench.h): events and the per-launch timing hook,
 // kernels that only read, and the host-side switch of the exchange's give-up limit. Nothing an operator call needs.
 #include "common.h"
+#include "skinny_fp8_tall.h"
+#include "skinny_w4a16_small.h"
+#include "skinny_w8a16_nk_tall.h"
+#include "skinny_w8a16_small.h"
 #include "../../include/hidet_qmm_bench.h"
 
 HIDET_API void *hidet_qmm_event_create(void) {
@@ -64,6 +68,77 @@ HIDET_API void hidet_qmm_gemv_ring_timed(const void *a, const void *const *weigh
 
 HIDET_API void hidet_qmm_set_exchange_spin_limit(int limit) {
     qmm::exchange_spin_limit().store(limit < 0 ? qmm::kExchangeSpinLimit : limit, std::memory_order_relaxed);
+}
+
+// ---- which kernel a call took, and the kernels of strips by their variant ---------------------------------------------
+HIDET_API const char *hidet_qmm_last_launch(int64_t *workgroups, int64_t *threads) {
+    const qmm::TimingSlot &ts = qmm::timing_slot();
+    if (workgroups != nullptr) *workgroups = ts.workgroups;
+    if (threads != nullptr) *threads = ts.threads;
+    const char *name = ts.kernel != nullptr ? hipKernelNameRefByPtr(ts.kernel, nullptr) : nullptr;
+    return name != nullptr ? name : "";
+}
+
+namespace {
+void check_strip(int row_blocks, bool columns, int64_t m, int64_t k, int64_t n) {
+    QMM_CHECK(row_blocks >= 1 && row_blocks <= 4 && columns, "there is no such variant of the kernel");
+    QMM_CHECK(m > 0 && k > 0 && n > 0 && m < (int64_t(1) << 24) && k < (int64_t(1) << 24) && n < (int64_t(1) << 24), "extents out of range");
+}
+}  // namespace
+
+HIDET_API void hidet_qmm_strips_f16_i8(int row_blocks, int columns, const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
+                                       int64_t n, int64_t lda, void *stream) {
+    QMM_ENTRY_BEGIN
+    check_strip(row_blocks, columns == 2 || columns == 4, m, k, n);
+    QMM_CHECK(a && w && scale && c && lda >= k && qmm::skinny_w8a16_small_supported(a, n, k, lda), "not a form that the kernel takes");
+    qmm::SkinnySmallPlan plan;
+    plan.rb = row_blocks;
+    plan.cb = columns;
+    qmm::skinny_w8a16_small_launch(plan, a, w, scale, bias, c, m, k, n, lda, static_cast<hipStream_t>(stream));
+    QMM_ENTRY_END
+}
+
+HIDET_API void hidet_qmm_strips_f16_i8_nk(int row_blocks, int groups, const void *a, const void *w_nk, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
+                                          int64_t n, int64_t lda, int64_t ldw, void *stream) {
+    QMM_ENTRY_BEGIN
+    check_strip(row_blocks, groups == 1 || groups == 2, m, k, n);
+    QMM_CHECK(a && w_nk && scale && c && lda >= k && ldw >= k && k % 16 == 0 && ldw % 16 == 0 && lda % 8 == 0 && qmm::aligned(a, 16) && qmm::aligned(w_nk, 16),
+              "not a form that the kernel takes");
+    qmm::SkinnyNkTallPlan plan;
+    plan.rb = row_blocks;
+    plan.cg = groups;
+    qmm::skinny_w8a16_nk_tall_launch(plan, a, w_nk, scale, bias, c, m, k, n, lda, ldw, static_cast<hipStream_t>(stream));
+    QMM_ENTRY_END
+}
+
+HIDET_API void hidet_qmm_strips_w4a16(int row_blocks, int columns, int waves, const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m,
+                                      int64_t k, int64_t n, int64_t lda, int group_size, int dtype, void *stream) {
+    QMM_ENTRY_BEGIN
+    check_strip(row_blocks, (columns == 2 || columns == 4) && (waves == 8 || (waves == 16 && row_blocks == 1 && columns == 2)), m, k, n);
+    QMM_CHECK(a && w && scales && c && lda >= k && (dtype == HIDET_QMM_BF16 || dtype == HIDET_QMM_F16) && group_size > 0 && k % group_size == 0 &&
+                  qmm::skinny_w4a16_small_supported(a, scales, n, k, lda, group_size),
+              "not a form that the kernel takes");
+    qmm::SkinnyW4SmallPlan plan;
+    plan.rb = row_blocks;
+    plan.cb = columns;
+    plan.waves = waves;
+    qmm::skinny_w4a16_small_launch(plan, a, w, scales, bias, c, m, k, n, lda, group_size, dtype, static_cast<hipStream_t>(stream));
+    QMM_ENTRY_END
+}
+
+HIDET_API void hidet_qmm_strips_f8(int row_blocks, int groups, int block_scaled, const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda,
+                                   int64_t ldb, int out_dtype, const void *scale_a, const void *scale_b, void *stream) {
+    QMM_ENTRY_BEGIN
+    check_strip(row_blocks, groups == 1 || groups == 2, m, k, n);
+    QMM_CHECK(a && b && c && lda >= k && ldb >= k && k % 16 == 0 && lda % 16 == 0 && ldb % 16 == 0 && qmm::aligned(a, 16) && qmm::aligned(b, 16) &&
+                  (out_dtype == HIDET_QMM_F32 || out_dtype == HIDET_QMM_F16 || out_dtype == HIDET_QMM_BF16 || out_dtype == HIDET_QMM_E4M3) &&
+                  (!block_scaled || (scale_a && scale_b && k % 128 == 0 && n % 128 == 0)),
+              "not a form that the kernel takes");
+    qmm::SkinnyFp8TallPlan plan;
+    plan.rb = row_blocks;
+    plan.cg = groups;
+    qmm::skinny_fp8_tall_launch(plan, block_scaled != 0, a, b, c, m, n, k, lda, ldb, out_dtype, scale_a, scale_b, static_cast<hipStream_t>(stream));
+    QMM_ENTRY_END
 }
 
 // ---- what a kernel that only reads can get out of the memory system ------------------------------------------------

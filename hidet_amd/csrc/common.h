@@ -81,8 +81,11 @@ inline size_t dtype_bytes(int dt) {
 
 // One-shot timing hook: when a (start, stop) event pair is armed on this thread, the next main
 // kernel launch records its own begin/end timestamps into them (hipExtLaunchKernelGGL).
+// The rest says what this thread's latest main launch was (hidet_qmm_last_launch).
 struct TimingSlot {
     hipEvent_t start = nullptr, stop = nullptr;
+    const void *kernel = nullptr;
+    uint32_t workgroups = 0, threads = 0;
 };
 TimingSlot &timing_slot();
 // true while this thread's last-error string has not been read (it stays set)
@@ -98,6 +101,9 @@ template <typename... KArgs, typename... Args>
 inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t shmem, hipStream_t stream, Args... args) {
     check_grid(grid, block);
     TimingSlot &ts = timing_slot();
+    ts.kernel = reinterpret_cast<const void *>(kernel);
+    ts.workgroups = grid.x * grid.y * grid.z;
+    ts.threads = block.x;
     if (ts.start != nullptr) {
         hipEvent_t s = ts.start, e = ts.stop;
         ts.start = ts.stop = nullptr;

@@ -146,6 +146,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w4a16_small_kernel(const ch
 
 }  // namespace
 
+bool skinny_w4a16_small_supported(const void *a, const void *scales, int64_t n, int64_t k, int64_t lda, int group) {
+    constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
+    return k > 0 && k % 128 == 0 && group > 0 && group % 64 == 0 && n % 8 == 0 && lda % 2 == 0 && aligned(a, 4) && aligned(scales, 4) && (k + 128) * n / 2 < kMost && lda * 128 + k * 2 < kMost;
+}
+
 // Row blocks and columns per lane of the smallest estimated time: a fit (13 %) to 2132 launches on 478 shapes of 1 to 256 rows, K of 256 to 2048 and N of 256 to 6144, in the mean of
 // weights from memory and from the last-level cache. Where it is ahead of the other kernels' estimates by 5 % those calls take 37 % less time in the mean (34 on weights
 // from memory) and none takes 3 % more. Beyond, 180 shapes of K 2176 to 4096, weights from the cache (from memory): 17 rows and more 15 to 25 % less time to K = 3328 (10 to 20), 5
@@ -155,9 +160,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_w4a16_small_kernel(const ch
 // (weights from memory: 2), but 1 % more at 1536, 5 at 1024, 16 to 26 where a CU gets two workgroups (of eight waves it holds them at once) and 2 to 5 on larger strips.
 SkinnyW4SmallPlan skinny_w4a16_small_plan(const void *a, const void *scales, int64_t m, int64_t n, int64_t k, int64_t lda, int group) {
     SkinnyW4SmallPlan best;
-    if (m > kSmallMostRows || k % 128 != 0 || k == 0 || k > (m <= 16 ? kFewRowsMostK : kSmallMostK) || group % 64 != 0 || n % 8 != 0 || k * n / 2 > kSmallMostBytes || lda % 2 != 0 || !aligned(a, 4) || !aligned(scales, 4) ||
-        lda * 128 + k * 2 >= (int64_t(1) << 31) - (1 << 20))
-        return best;
+    if (m > kSmallMostRows || k > (m <= 16 ? kFewRowsMostK : kSmallMostK) || k * n / 2 > kSmallMostBytes || !skinny_w4a16_small_supported(a, scales, n, k, lda, group)) return best;
     const double cus = std::max(1, device_cus()), steps = double(cdiv(k / 128, 8));  // steps of a wave, of eight
     for (int most = 1; most <= 4; ++most) {
         const int64_t tiles_m = cdiv(m, 16 * most);

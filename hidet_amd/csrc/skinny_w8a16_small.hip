@@ -134,6 +134,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w8a16_small_kernel(co
 
 }  // namespace
 
+bool skinny_w8a16_small_supported(const void *a, int64_t n, int64_t k, int64_t lda) {
+    constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
+    return k > 0 && k % 2 == 0 && n >= 4 && lda % 2 == 0 && aligned(a, 4) && (k + 128) * n < kMost && lda * 128 + k * 2 < kMost;
+}
+
 // Row blocks and columns per lane of the smallest estimated time: a fit (14 %) to 2040 launches on 456 shapes of 1 to 256 rows, K of 256 to 2048 and N of 256 to 6144, in the mean of
 // weights from memory and from the last-level cache. Weights of more than 8.5 MB or 2560 rows stay with the others: there the strips of rows that a workgroup reads of a weight
 // in memory cost more than the exchange that they save (1 x 2048 x 6144 8.2 us and 11.2 here, 16 x 3072 x 1024 7.1 and 8.5, 16 x 3072 x 3072 9.0 and 13.3; 64 x 3072 x 2260 27 % more, 16 x 2772
@@ -142,8 +147,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void skinny_w8a16_small_kernel(co
 // Within K = 2048, where this is ahead of the other kernels' estimates by 8 %, those 456 calls take 36 % less time in the mean (30 on weights from memory), and one of them in the former case and two in the latter take 3 to 4 % more.
 SkinnySmallPlan skinny_w8a16_small_plan(const void *a, int64_t m, int64_t n, int64_t k, int64_t lda) {
     SkinnySmallPlan best;
-    constexpr int64_t kMost = (int64_t(1) << 31) - (1 << 20);
-    if (m > kSmallMostRows || k % 2 != 0 || k < kSmallLeastK || k > kSmallMostK || k * n > kSmallMostBytes || n < 4 || lda % 2 != 0 || !aligned(a, 4) || (k + 128) * n >= kMost || lda * 128 + k * 2 >= kMost) return best;
+    if (m > kSmallMostRows || k < kSmallLeastK || k > kSmallMostK || k * n > kSmallMostBytes || !skinny_w8a16_small_supported(a, n, k, lda)) return best;
     const double cus = std::max(1, device_cus()), steps = double(cdiv(cdiv(k, 128), kSmallWaves));  // steps of a wave
     for (int most = 1; most <= 4; ++most) {
         const int64_t tiles_m = cdiv(m, 16 * most);

@@ -50,6 +50,11 @@ SIGNATURES = {
     'hidet_qmm_read_probe': (None, [_vp, _i64, _vp, _vp]),
     'hidet_qmm_pattern_probe': (None, [_vp, _i64, _i64, _i32, _i32, _vp, _vp]),
     'hidet_qmm_set_exchange_spin_limit': (None, [_i32]),
+    'hidet_qmm_last_launch': (ctypes.c_char_p, [_vp, _vp]),
+    'hidet_qmm_strips_f16_i8': (None, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
+    'hidet_qmm_strips_f16_i8_nk': (None, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp]),
+    'hidet_qmm_strips_w4a16': (None, [_i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp]),
+    'hidet_qmm_strips_f8': (None, [_i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     'hidet_symmetric_quantize': (None, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _vp, _i64, _vp]),
     'hidet_symmetric_dequantize': (None, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
     'hidet_symmetric_quant_matmul_f16_i8': (None, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _i64, _vp]),

@@ -46,6 +46,25 @@ void hidet_qmm_read_probe(const void *src, int64_t bytes, void *sink, void *stre
  * pattern; the difference to hidet_qmm_read_probe is the price of the [K, N] layout. */
 void hidet_qmm_pattern_probe(const void *w, int64_t k, int64_t n, int workgroups, int contiguous, void *sink, void *stream);
 
+/* ---- which kernel a call took ------------------------------------------------------------------------
+ * The name (mangled, so with its template arguments), workgroups and threads per workgroup of the latest compute-kernel launch that
+ * this thread made; "" before the first.  Tests that are meant for one kernel say so with it, where the choice is made from
+ * estimated times. */
+const char *hidet_qmm_last_launch(int64_t *workgroups, int64_t *threads);
+
+/* ---- the kernels of strips of columns over all of K, by their variant ------------------------------------
+ * The operators pick a variant by its estimated time, so some are not reached by sizes that a test can enumerate.  These launch the one that is named:
+ * row_blocks 1 to 4 (16 rows each), columns 2 or 4 per lane (row-major weights) or groups 1 or 2 of 16 columns (K-contiguous), waves 8, or 16
+ * with one row block and two columns.  The other arguments are those of the operators of the same name. */
+void hidet_qmm_strips_f16_i8(int row_blocks, int columns, const void *a, const void *w, const void *scale, const void *bias, void *c, int64_t m, int64_t k, int64_t n,
+                             int64_t lda, void *stream);
+void hidet_qmm_strips_f16_i8_nk(int row_blocks, int groups, const void *a, const void *w_nk, const void *scale, const void *bias, void *c, int64_t m, int64_t k,
+                                int64_t n, int64_t lda, int64_t ldw, void *stream);
+void hidet_qmm_strips_w4a16(int row_blocks, int columns, int waves, const void *a, const void *w, const void *scales, const void *bias, void *c, int64_t m, int64_t k,
+                            int64_t n, int64_t lda, int group_size, int dtype, void *stream);
+void hidet_qmm_strips_f8(int row_blocks, int groups, int block_scaled, const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                         int out_dtype, const void *scale_a, const void *scale_b, void *stream);
+
 /* ---- test hook -------------------------------------------------------------------------------------
  * Re-reads of the mailbox after which a collector of the split-K exchange gives up (process-wide, applies to launches
  * made afterwards; negative restores the default of about a second of polling).  Tests set 0 to reach the give-up path

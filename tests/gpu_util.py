@@ -36,3 +36,19 @@ def fastest_ms(call, tries=5):
         end.synchronize()
         best = min(best, begin.elapsed_time(end))
     return best
+
+
+def last_launch():
+    """(mangled kernel name, workgroups, threads per workgroup) of this thread's latest launch by the library."""
+    import ctypes
+
+    from hidet_amd import ffi
+
+    grid, threads = ctypes.c_int64(), ctypes.c_int64()
+    name = ffi.load_library().hidet_qmm_last_launch(ctypes.byref(grid), ctypes.byref(threads)).decode()
+    return name, grid.value, threads.value
+
+
+def variant(kernel, *arguments):
+    """What the mangled name of a kernel holds for these template arguments (truth values and integers)."""
+    return kernel + 'I' + ''.join('L{}{:d}E'.format('b' if isinstance(a, bool) else 'i', a) for a in arguments) + 'E'
