@@ -536,11 +536,11 @@ __global__ __launch_bounds__(kThreads8, 1) void gemm_fp8_kernel8(const uint8_t *
 }  // namespace
 
 // Estimated time in microseconds of the tiled kernels, for the choice between them and the narrow tiles of gemm_mid.h: the plan's time and a fixed part
-// with which that choice is right (of 110 shapes each, 40 to 1024 rows, it costs 0.2 % over the faster kernel in the mean, 0.9 and 0.6 on weights from memory); where K is no
-// multiple of 128 (the register-staged 256 x 256 kernel) 3.5 us per k block and round.
+// with which that choice is right (one microsecond more or less changes it for 3 of 427 shapes of 17 to 1100 rows); where K is no multiple of 128 (the register-staged 256 x 256
+// kernel) 3.5 us per k block and round.
 double gemm_fp8_estimate_us(int64_t m, int64_t n, int64_t k, bool scaled, void *workspace, int64_t workspace_bytes) {
     if (k % 128 != 0) return 8.0 + double(cdiv(cdiv(m, 256) * cdiv(n, 256), 256)) * 3.5 * double(cdiv(k, 128));
-    return (scaled ? 6.3 : 8.1) + make_fp8_plan(m, n, k, scaled, split_workspace(workspace, workspace_bytes)).us;
+    return (scaled ? 7.3 : 9.1) + make_fp8_plan(m, n, k, scaled, split_workspace(workspace, workspace_bytes)).us;
 }
 
 // Launch of the 8-wave kernel; SCALED selects block scales (scale_a [K/128, M], scale_b [N/128, K/128]) or optional

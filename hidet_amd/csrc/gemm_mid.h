@@ -414,9 +414,10 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 
 // What a launch costs in microseconds: the workgroups of a CU one after the other, each with its fixed part, its rounds of
 // the groups and, where K is cut, the exchange of `parts` partial tiles. The coefficients are fits to the times of every tile height and
-// number of pieces (430 to 1010 each) on 100 to 260 shapes of 24 to 1024 rows, K and N of 1024 to 11008 (FP8 8192), of which they leave 3 to 6 %.
-// With the prefill kernels' estimates beside them the choices they make cost over the best one, in the mean of 110 other random shapes: int8 0.3 %
-// (2.7 with the coefficients of a slower exchange that were here), int4 0.3 (1.3), FP8 0.2 (2.9), block-scaled 0.2 (0.5).
+// number of pieces (430 to 1700 each) on 100 to 430 shapes of 17 to 1100 rows, K and N of 1024 to 11008 (FP8 8192), of which they leave 3 to 8 %;
+// not those of K-contiguous int8 and of int4 in groups of odd multiples of 32, which are older and stand for a slower exchange (the former 17 % too high).
+// The choices they make cost over the best tile and split, from the last-level cache and from memory: int8 0.4 and 1.6 % in the mean of 333 shapes, int4 0.3 and 0.3 of
+// 202, FP8 0.6 and 0.4 of 427, block-scaled 0.5 and 0.7 of 424.
 // `full_round` (0: not known) is the least a round takes with every CU at work: the weights of a round then come at the
 // rate of the memory. `exchange_piece` (0: in the others): what every piece of the launch adds to an exchange, all of them meeting at the same time.
 struct MidCost {

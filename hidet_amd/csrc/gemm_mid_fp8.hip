@@ -162,9 +162,13 @@ struct MidF8 {
 template <bool SCALED>
 bool launch_f8(const void *a, const void *b, const MidF8Args &args, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
                double limit_us, const Workspace &ws, hipStream_t stream) {
-    // (fits to the mean of what a split takes on weights from memory and from the last-level cache: more workgroups pay where the weights come from memory)
-    const MidCost low = SCALED ? MidCost{3.01, 0.798, 1.78, 0.0955, 0.0, 0.0066} : MidCost{3.43, 0.578, 1.81, 0.0854, 0.0, 0.0053};
-    const MidCost high = SCALED ? MidCost{3.81, 1.057, 1.59, 0.295, 0.0, 0.0109} : MidCost{4.69, 0.722, 1.34, 0.25, 0.0, 0.0091};
+    // Fits (7 to 8 %) to the mean of a split's time on weights from memory and from the last-level cache, 427 shapes (block-scaled 424) of 17 to 1100 rows. A workgroup that walks all of K
+    // for 32 rows is the fastest from the cache and 10 to 30 % behind two or three pieces from memory, where each round waits for it: us, cache and memory, in one
+    // piece -> now: 337 x 5760 x 1824 14.2 and 19.0 -> 15.5 and 16.8, block-scaled 146 x 3584 x 3456 13.4 and 17.9 -> 12.8 and 14.1. Rows of the weight that do not begin on a cache line:
+    // a round's 128 bytes of each lie on two (308 x 3024 x 1856 12.4 and 16.3 -> 12.5 and 13.4, 277 x 3680 x 1856 13.7 and 18.5 -> 12.8 and 13.9).
+    const double apart = ldb % 128 != 0 ? 0.266 : 0.0;
+    const MidCost low = SCALED ? MidCost{3.55, 0.845, 1.67, 0.108, 0.0, 0.004} : MidCost{3.84, 0.576 + apart, 1.72, 0.095, 0.0, 0.0031};
+    const MidCost high = SCALED ? MidCost{4.55, 1.071, 1.19, 0.304, 0.0, 0.0092} : MidCost{5.24, 0.699 + apart, 1.01, 0.221, 0.0, 0.0085};
     const MidChoice c2 = mid_choose<MidF8<SCALED, 2>, 2, 3>(low, ws, m, n, k), c4 = mid_choose<MidF8<SCALED, 4>, 4, 3>(high, ws, m, n, k);
     if (std::min(c2.us, c4.us) > limit_us) return false;
     if (c2.us < c4.us) mid_launch<MidF8<SCALED, 2>, 2, 3>(c2, a, b, lda, ldb, args, m, n, k, ws, stream);

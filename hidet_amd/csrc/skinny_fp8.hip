@@ -370,9 +370,9 @@ void skinny_fp8_launch(const void *a, const void *b, void *c, int64_t m, int64_t
 }
 
 // Row blocks and column groups per workgroup of the smallest estimated time: fits (7 %) to 1550 to 1790 launches on 270 to 310 shapes of 17 to 1024 rows, K and N of 512
-// to 8192, in the mean of weights from memory and from the last-level cache. The caller takes this kernel where it is ahead of the other estimates by 15 %: over the
-// fastest kernel that costs 0.8 % in the mean (block-scaled 1.0 to 1.3), at an even chance 0.6 to 1.1 (0.7 to 0.9), but then 39 of 1158 calls would be more than 3 % slower
-// than on the others, now 3.
+// to 8192, in the mean of weights from memory and from the last-level cache. The caller takes this kernel where it is ahead of the other estimates by 15 %: over the fastest of all
+// kernels, splits and variants that costs 1.7 % in the mean of 427 shapes of 17 to 1100 rows, 1.7 on weights from memory (block-scaled, 424 shapes, 1.1 and 2.7). By 5 % it would be 1.1 and
+// 1.2 (0.6 and 1.6), but of 550 other shapes 10 from the cache and 5 from memory would be more than 6 % slower than on what they had before; by 15 % 7 and 2 are.
 SkinnyFp8TallPlan skinny_fp8_tall_plan(bool scaled, int64_t m, int64_t n, int64_t k) {
     SkinnyFp8TallPlan best;
     const double cus = std::max(1, device_cus()), steps = double(cdiv(cdiv(k, 128), kTallWaves));  // steps of a wave

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from hidet_amd.graph.ops.matmul import matmul_f8 as F8
-from gpu_util import announce, dev, host
+from gpu_util import announce, dev, host, last_launch, variant
 from test_gpu_fp8_tiles import operands
 
 pytestmark = pytest.mark.gpu
@@ -60,4 +60,23 @@ def test_narrow_tiles_beside(m, k, n):
     ai, bi, a, b = operands(rng, m, k, n, False)
     one = torch.ones((), device='cuda')
     got = F8.matmul_f8_per_tensor(a, b, one, one, output_dtype=torch.float32)
+    assert np.array_equal(host(got), ai.astype(np.float32) @ bi.T.astype(np.float32))
+
+
+# Shapes that one-piece tiles of 32 rows, K whole, were chosen for: few column tiles then fetch the weight, one stage after the other, and from memory that
+# is 10 to 30 % slower than tiles of 64 rows in two or three pieces, or strips (1 to 10 % from the cache, either way)
+@pytest.mark.parametrize('m,k,n,scaled', [(308, 3024, 1856, False), (369, 3360, 1472, False), (277, 3680, 1856, False), (125, 5456, 7104, False), (337, 5760, 1824, False),
+                                          (307, 2944, 1664, True), (155, 2944, 3456, True), (388, 3584, 1536, True)])
+def test_weights_from_memory_not_in_one_piece(m, k, n, scaled):
+    announce('fp8: not in one piece', m, k, n, scaled)
+    rng = np.random.default_rng(m + k + n)
+    ai, bi, a, b = operands(rng, m, k, n, False)
+    one = torch.ones((), device='cuda')
+    if scaled:
+        got = F8.matmul_f8_scaled(a, b, scale_a=torch.ones((k // 128, m), device='cuda'), scale_b=torch.ones((n // 128, k // 128), device='cuda'), output_dtype='float32')
+    else:
+        got = F8.matmul_f8_per_tensor(a, b, one, one, output_dtype=torch.float32)
+    name, workgroups, _ = last_launch()
+    one_piece = 8 * -(-(-(-m // 32) * -(-n // 128)) // 8)
+    assert not (variant('MidF8', scaled, 2) in name and workgroups == one_piece), name
     assert np.array_equal(host(got), ai.astype(np.float32) @ bi.T.astype(np.float32))
