@@ -14,6 +14,9 @@ namespace qmm {
 namespace {
 
 constexpr int64_t kSmallMostRows = 512, kSmallMostK = 4096, kSmallMostBytes = 6300000, kFewRowsMostK = 2944;  // (kFewRows...: up to 16 rows)
+// Rounds of one workgroup per CU, beyond which the estimate is up to 40 % too low. us, strips -> the other kernels, from the cache and from memory: 504 x 1024 x 7040 28.9 and 31.7 -> 22.0 and
+// 23.9, 150 x 1024 x 11008 18.7 and 21.3 -> 16.9 and 18.7, 330 x 1024 x 7040 21.8 and 23.6 -> 21.4 and 22.7; but 260 x 1024 x 8192 18.9 and 21.8 -> 20.5 and 21.9.
+constexpr double kSmallMostRounds = 2.0;
 constexpr int kWideSteps = 16;  // 128-deep steps of K from which on workgroups have sixteen waves
 template <int WAVES, int RB, int CB>
 constexpr int small_lds_bytes() {
@@ -168,6 +171,7 @@ SkinnyW4SmallPlan skinny_w4a16_small_plan(const void *a, const void *scales, int
         for (int cb = 2; cb <= 4; cb += 2) {
             // (of the XCD with the most column tiles, times eight)
             const double groups = double(tiles_m) * double(8 * cdiv(cdiv(n, 16 * cb), 8)), share = std::max(1.0, groups / cus), rounds = std::ceil(share);
+            if (rounds > kSmallMostRounds) continue;
             const int waves = rb == 1 && cb == 2 && groups <= cus && k >= 128 * kWideSteps ? 16 : 8;
             const double us = (waves == 16 ? 0.95 : 1.0) * (1.915 + 0.0134 * share * rb * cb + rounds * steps * (0.545 + 0.342 * rb + 0.154 * cb + 0.114 * rb * cb));
             if (us < best.us) best = SkinnyW4SmallPlan{us, rb, cb, waves};

@@ -7,7 +7,7 @@ import torch
 
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
-from gpu_util import announce, dev
+from gpu_util import announce, dev, last_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,12 @@ def test_bias_and_strides():
     c = torch.empty((m, n), dtype=torch.bfloat16, device='cuda')
     ffi.call('hidet_symmetric_quant_matmul_w4a16_bias', wide, packed, scales, bias, c, m, k, n, k + 2, group, ffi.DTYPE_CODE[torch.bfloat16], 0, ws, ws.numel(), ffi.current_stream(a.device))
     assert torch.equal(c.cpu(), exact.bfloat16() + bias.cpu())
+
+
+@pytest.mark.parametrize('m,k,n,strips', [(504, 1024, 7040, False), (150, 1024, 11008, False), (64, 1024, 4096, True)])
+def test_strips_of_up_to_two_rounds_of_the_chip(m, k, n, strips):
+    announce('int4 small weight: rounds', m, k, n)
+    a, packed, scales, exact = _case(m, k, n, 128, torch.bfloat16)
+    got = quant.symmetric_quant_matmul_w4a16(a, packed, scales, 128)
+    assert ('skinny_w4a16_small' in last_launch()[0]) == strips
+    assert torch.equal(got.cpu(), exact.bfloat16())
