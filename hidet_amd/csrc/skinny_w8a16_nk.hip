@@ -420,9 +420,16 @@ void skinny_w8a16_nk_launch(const void *a, const void *w, const void *scale, con
                             int64_t n, int64_t lda, int64_t ldw, hipStream_t stream) {
     const bool aligned_a = (lda % 8 == 0) && aligned(a, 16);
     // K off the steps: the kernel below, with conditions in all of its loop, only where the activations are not aligned. us, that one and the tall one: 1 x 4032 x 4096 6.8 and
-    // 6.3, 16 x 4032 x 4096 9.4 and 6.3, 16 x 2112 x 11008 12.5 and 8.2, 16 x 9024 x 4096 17.7 and 10.0.
+    // 6.3, 16 x 4032 x 4096 9.4 and 6.3, 16 x 2112 x 11008 12.5 and 8.2, 16 x 9024 x 4096 17.7 and 10.0; large weights from the cache and from memory, 1 x 5776 x 9792 15.8 and 19.3, 14.7 and
+    // 18.2, 1 x 10320 x 5376 18.1 and 22.1, 14.3 and 19.7, 8 x 10464 x 10240 40.0 and 41.5, 34.2 and 35.7; of 50 shapes of 1 to 16 rows, 1 to 107 MB, none is slower.
     if (k % 128 != 0 && aligned_a) {
-        skinny_w8a16_nk_tall_launch(skinny_w8a16_nk_tall_plan(a, m, n, k, lda), a, w, scale, bias, c, m, k, n, lda, ldw, stream);
+        // (as many rows at a time as a launch has threads for, whatever the plan: 32-column tiles of 64 rows need the fewest, 16-column tiles of 16 rows eight times as many)
+        const int64_t most = (int64_t(1) << 32) / (64 * kTallWaves) - 1, rows = std::max<int64_t>(1, most / (cdiv(cdiv(n, 16), 8) * 8)) * 16;
+        for (int64_t m0 = 0; m0 < m; m0 += rows) {
+            const int64_t mt = std::min(rows, m - m0);
+            const _Float16 *am = static_cast<const _Float16 *>(a) + m0 * lda;
+            skinny_w8a16_nk_tall_launch(skinny_w8a16_nk_tall_plan(am, mt, n, k, lda), am, w, scale, bias, static_cast<_Float16 *>(c) + m0 * n, mt, k, n, lda, ldw, stream);
+        }
         return;
     }
     const dim3 grid(uint32_t(cdiv(n, 16)));
