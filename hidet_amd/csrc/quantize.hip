@@ -386,9 +386,8 @@ __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const v
 // A weight of half of the last-level cache and more of which whole cache lines are read, and read once, passes that cache by, which then keeps what the next kernel reads and
 // writes (4096 x 11008 float32, quantized and dequantized along rows 90.0 -> 74.3 us; int4 groups 40.4 -> 36.1). Smaller weights may lie in it. us, plain and non-temporal, three weights in
 // turn (and weights from memory): along rows bfloat16 902 x 3712 4.5 and 5.3 (4.6 and 5.5), float16 1632 x 10624 14.4 and 17.6 (16.8 and 17.1), float32 1086 x 8640 9.4 and 10.6
-// (10.7 and 10.6), 2032 x 10496 18.2 and 20.1 (19.8 and 20.1), but 1408 x 3648 6.5 and 6.2; in strips bfloat16 1297 x 6720 10.6 and 11.8 (11.9 and 11.3). int4, groups of 64: 3712 x
-// 5760 18.7 and 20.8 (21.6 and 20.9), 896 x 4288 7.9 and 8.7 (8.9 and 8.9), 3840 x 8896 31.8 and 30.1 (32.7 and 30.3). Of a line read in parts the others pay for it
-// (float16 700 x 1600 in strips of 8 columns 7.0 -> 7.8).
+// (10.7 and 10.6), 2032 x 10496 18.2 and 20.1 (19.8 and 20.1), but 1408 x 3648 6.5 and 6.2. int4, groups of 64: 3712 x 5760 18.7 and 20.8 (21.6 and 20.9), 896 x 4288 7.9 and 8.7
+// (8.9 and 8.9), 3840 x 8896 31.8 and 30.1 (32.7 and 30.3).
 constexpr int kNonTemporal = 2;
 constexpr int64_t kReadOnceFrom = int64_t(128) << 20;  // bytes
 
@@ -455,7 +454,7 @@ __device__ __forceinline__ void keep_packed(V (&x)[N]) {
 // lines of the codes, so an XCD has a run of them. The last quad of a row that is no multiple of four is moved back into the row: its lane and
 // the one before store the same codes twice.
 constexpr int kStripThreads = 512;
-template <int DT, int QT, int CL, int NV, int WAVES, bool ONCE>
+template <int DT, int QT, int CL, int NV, int WAVES>
 __global__ __launch_bounds__(kStripThreads, WAVES) void quantize_strip_kernel(const char *__restrict__ w, char *__restrict__ q, void *__restrict__ scale, int R, int inner,
                                                                               int strips, int items, int per_xcd) {
     constexpr int kElement = DT == HIDET_QMM_F32 ? 4 : 2, kCode = QT == HIDET_QMM_I8 ? 1 : 2;
@@ -476,7 +475,7 @@ __global__ __launch_bounds__(kStripThreads, WAVES) void quantize_strip_kernel(co
     };
     V x[NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) x[v] = load_quad<DT, ONCE>(trip(v), offset);
+    for (int v = 0; v < NV; ++v) x[v] = load_quad<DT>(trip(v), offset);
     __builtin_amdgcn_sched_barrier(0);
     float m[4] = {0.f, 0.f, 0.f, 0.f};
     const int trips = (R + kLanes - 1) / kLanes;
@@ -1143,14 +1142,8 @@ bool quantize_in_one_pass(F &&go, const void *w, void *wq, void *scale, int64_t 
     auto strips = [&](auto cl, auto nv, auto waves) {
         constexpr int CL = decltype(cl)::value, NV = decltype(nv)::value, WAVES = decltype(waves)::value;
         const int64_t per_slice = cdiv(inner, 4 * CL), items = outer * per_slice, per_xcd = cdiv(items, 8);
-        auto run = [&](auto once) {
-            constexpr bool ONCE = decltype(once)::value;
-            go(quantize_strip_kernel<DT, HIDET_QMM_I8, CL, NV, WAVES, ONCE>, quantize_strip_kernel<DT, HIDET_QMM_I16, CL, NV, WAVES, ONCE>, dim3(uint32_t(8 * per_xcd)),
-               kStripThreads, 0, from, to, scale, int(reduce), int(inner), int(per_slice), int(items), int(per_xcd));
-        };
-        constexpr bool kLines = CL * 4 * kElement >= 64;
-        if (kLines && outer * reduce * row_bytes >= kReadOnceFrom) run(integral_constant<bool, kLines>());
-        else run(integral_constant<bool, false>());
+        go(quantize_strip_kernel<DT, HIDET_QMM_I8, CL, NV, WAVES>, quantize_strip_kernel<DT, HIDET_QMM_I16, CL, NV, WAVES>, dim3(uint32_t(8 * per_xcd)), kStripThreads, 0,
+           from, to, scale, int(reduce), int(inner), int(per_slice), int(items), int(per_xcd));
         return true;
     };
     auto one_round = [&](int columns) { return outer * cdiv(inner, columns) <= cus; };
