@@ -387,7 +387,9 @@ __global__ __launch_bounds__(64 * kQuantLanes) void quantize_rows_kernel(const v
 // writes (4096 x 11008 float32, quantized and dequantized along rows 90.0 -> 74.3 us; int4 groups 40.4 -> 36.1). Smaller weights may lie in it. us, plain and non-temporal, three weights in
 // turn (and weights from memory): along rows bfloat16 902 x 3712 4.5 and 5.3 (4.6 and 5.5), float16 1632 x 10624 14.4 and 17.6 (16.8 and 17.1), float32 1086 x 8640 9.4 and 10.6
 // (10.7 and 10.6), 2032 x 10496 18.2 and 20.1 (19.8 and 20.1), but 1408 x 3648 6.5 and 6.2. int4, groups of 64: 3712 x 5760 18.7 and 20.8 (21.6 and 20.9), 896 x 4288 7.9 and 8.7
-// (8.9 and 8.9), 3840 x 8896 31.8 and 30.1 (32.7 and 30.3).
+// (8.9 and 8.9), 3840 x 8896 31.8 and 30.1 (32.7 and 30.3). From 128 MiB on the same weight quantized again and again is the one case that plain loads serve better (float32 along rows 4096 x
+// 10496 31.8 and 36.7, int4 34.3 and 38.5 of 4096 x 11008); three in turn 36.4 and 36.5, 40.1 and 37.6, and with the dequantization behind it the one weight too 80.4 and 69.2.
+// quantize_meet_kernel is apart: it reads all that it holds this way (below).
 constexpr int kNonTemporal = 2;
 constexpr int64_t kReadOnceFrom = int64_t(128) << 20;  // bytes
 
@@ -527,6 +529,8 @@ __global__ __launch_bounds__(kStripThreads, WAVES) void quantize_strip_kernel(co
 // memory, count themselves in, and go on when all have. What a workgroup waits for is bounded: one that gives up reads its columns itself,
 // so a launch ends with the right codes whatever else keeps workgroups of it from starting. Counters of a group lie on cache lines of their own (next to each other the atomics of all
 // groups queue up: 2048 x 4096 float32 35 us instead of 16); the last to leave returns them to zero.
+// What a workgroup holds passes the last-level cache by, at every size: against plain loads, 120 weights of 6 to 190 MB, that is 8 % faster from memory (7 with the dequantization behind
+// it) and with three weights in turn the same (2); 2 % slower only where, besides, the codes and values go to the same memory each time.
 constexpr int kMeetCounterWords = 64, kMeetGroups = kExchangeLostWord / (2 * kMeetCounterWords), kMeetSpins = 512;
 template <int DT, int QT, int NV, int NL>
 __global__ __launch_bounds__(kStripThreads, 4) void quantize_meet_kernel(const char *__restrict__ w, char *__restrict__ q, void *__restrict__ scale, float *partials,
