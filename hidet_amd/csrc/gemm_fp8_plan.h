@@ -17,6 +17,7 @@ struct Fp8Plan {
 // least 4 k blocks, and only with a workspace that holds the partial tiles (8 XCDs x their tail tiles x parts) in its scratch part.
 inline GemmTail fp8_most_ranges(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
     GemmTail tail = make_gemm_tail(tiling, kConcurrent8, kConcurrent8, 4);
+    static_assert(tail_counters_fit(kConcurrent8), "one counter per tile that is cut");
     if (ws.scratch == nullptr) tail.parts = 1;
     while (tail.parts > 1 &&
            (k / 128 < 4 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * kM8 * kN8 * 4))

@@ -192,6 +192,10 @@ __device__ __forceinline__ bool gemm_work_item(int tiles_m, int tiles_n, int xm,
     return gemm_work_item_of_block(int(blockIdx.x), tiles_m, tiles_n, xm, xn, concurrent, tail_parts, tail_stride, item, panel_cols);
 }
 
+// One arrival counter per tile that is cut (GemmWorkItem::slot), fewer than `concurrent` of them on each of 8 XCDs, in front of the word that the exchange of the
+// bandwidth-bound kernels uses: what every launch with a tail asserts.
+constexpr bool tail_counters_fit(int concurrent) { return 8 * (concurrent - 1) * kCounterWords <= kExchangeLostWord; }
+
 // Fix-up of a tile computed in K ranges by item.parts workgroups of THREADS threads, each holding R x T float4
 // accumulators per thread. Every part writes its accumulators to the workspace (16 bytes per lane, agent scope),
 // waits for the writes to be acknowledged and counts itself in; the part that arrives last reads all of them back

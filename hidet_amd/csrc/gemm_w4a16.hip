@@ -453,6 +453,7 @@ void launch_cfg16(const void *a, const void *w, const void *scales, void *c, int
     constexpr int kConcurrent = 32 * MIN_BLOCKS;
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, kConcurrent);
     GemmTail tail = make_gemm_tail(tiling, kConcurrent, kConcurrent, 4);
+    static_assert(tail_counters_fit(kConcurrent), "one counter per tile that is cut");
     const Workspace ws = split_workspace(workspace, workspace_bytes);
     while (tail.parts > 1 &&
            (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
@@ -887,6 +888,7 @@ __global__ __launch_bounds__(512, 1) void gemm_w4a16_lds_kernel(
 GemmTail lds_tail_of(const GemmTiling &tiling, int64_t k, const Workspace &ws) {
     using Cfg = GemmW4LdsCfg<4>;
     GemmTail tail = make_gemm_tail_by_rounds(tiling, 32, 4, 0.0007 * 4096.0 / double(k));
+    static_assert(tail_counters_fit(32), "one counter per tile that is cut");
     while (tail.parts > 1 &&
            (k / kBK < 8 * tail.parts || ws.scratch_bytes < int64_t(8) * tail.max_tiles * tail.parts * Cfg::kBM * Cfg::kBN * 4))
         --tail.parts;

@@ -349,7 +349,7 @@ void launch_cfg16(const void *a, const void *w, const void *scale, const void *b
     const GemmTiling tiling = make_gemm_tiling(tiles_m, tiles_n, kConcurrent);
     int split_unit;
     const GemmTail tail = tail_of<Cfg, kConcurrent, RBA>(tiling, k, ws, &split_unit);
-    static_assert(8 * 32 * kCounterWords <= kExchangeLostWord, "one counter per tail tile: fewer than 32 per XCD are cut");
+    static_assert(tail_counters_fit(kConcurrent), "one counter per tile that is cut");
     const int64_t grid = gemm_grid_with_tail(tiling, split_unit, tail);
     QMM_CHECK(grid < (int64_t(1) << 31), "problem too large for one launch");
     allow_dynamic_lds(reinterpret_cast<const void *>(gemm_w8a16_kernel16<RB, WM, WN, MIN_BLOCKS, RBA, W_NK>), Cfg::kLdsBytes);
