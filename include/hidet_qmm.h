@@ -22,12 +22,15 @@
  *     workspace, and nothing else may write to one while a call is in flight.
  *     In bytes: counters = 65536; mailbox = min(16 MiB, (workspace_bytes - 65536) / 4) rounded down to a multiple of 256;
  *     scratch = workspace_bytes - 65536 - mailbox.  What each entry point needs of it:
- *       hidet_symmetric_quantize          scratch >= 4 * outer * inner bytes (an error otherwise);
+ *       hidet_symmetric_quantize          scratch >= 4 * outer * inner bytes (an error otherwise); weights of several
+ *                                         megabytes are read once instead of twice with 1 KiB of scratch per 256 columns
+ *                                         and range of rows, 512 KiB in all at most (optional), and use the counters;
  *       hidet_fp8_quantize_per_tensor     scratch >= 4 bytes (an error otherwise);
  *       hidet_symmetric_quant_matmul_f16_i8[_bias], hidet_symmetric_quant_matmul_w4a16[_bias] with up to 16 rows
  *                                         mailbox >= 1024 * min(m, 16) bytes per workgroup of the K split, at most 256
  *                                         workgroups unless parallel_k_parts asks for more (4 MiB serve every automatic
- *                                         plan); with less the kernels use fewer workgroups, never an error;
+ *                                         plan); with less the kernels use fewer workgroups, never an error; batches
+ *                                         that the tiles serve sooner use counters and scratch as with more rows;
  *       the same with more rows, hidet_matmul_f8, hidet_matmul_f8_scaled, the _nk matmuls
  *                                         scratch: 64 KiB per tile computed in K ranges times the ranges (optional: with
  *                                         less, fewer or no tiles are split; hidet_qmm_min_workspace_bytes() serves
@@ -82,8 +85,11 @@ int64_t hidet_qmm_workspace_bytes_for_scratch(int64_t scratch_bytes);
  * last rows polls the mailbox for the partial tiles of the others.  The poll is bounded; if a partial tile never shows
  * up (a workspace that was not zero-filled, two overlapping calls on one workspace, a device fault) the workgroup
  * writes NaN to its outputs, sets a flag in the workspace and returns, and the mailbox may be left with stale words that
- * would corrupt later calls.  No counterpart in the reference, whose split-K parts are separate outputs summed by a
- * second operator (python/hidet/graph/ops/quant/resolve.py:99).
+ * would corrupt later calls.  The flag is about the mailbox alone.  Tiles computed in K ranges and hidet_symmetric_quantize meet
+ * through the arrival counters, which have to be zero when a call begins: with stale ones they take partial sums or maxima for
+ * whole ones, and no flag says so.  (A workgroup of the quantizer that waits in vain reads its columns itself: right codes, no flag.)
+ * No counterpart in the reference, whose split-K parts are separate outputs summed by a second operator
+ * (python/hidet/graph/ops/quant/resolve.py:99).
  * hidet_qmm_exchange_status waits for `stream`, then returns 1 if any launch on this workspace gave up since the last
  * reset, 0 if none did, -1 on an error (last-error string).  hidet_qmm_exchange_reset enqueues kernels on `stream` that
  * zero the counters, the flag and the mailbox; call it after a status of 1, with no other call on the workspace in
