@@ -1,5 +1,4 @@
-"""FP8 matmuls of 17 and more rows of small weights, which one workgroup per column strip computes over all of K: one to four row blocks and one or two
-column groups per workgroup, several row tiles, waves without a step of K, K that ends inside a step, rows and columns past the end, every output type; and shapes next to them that stay with
+"""FP8 matmuls of 17 and more rows of small weights, which one workgroup per column strip computes over all of K: several row tiles, waves without a step of K, K that ends inside a step, rows and columns past the end, every output type; and shapes next to them that stay with
 the narrow tiles. Integer-valued codes and scales whose sums stay below 2^24: exact in float32, so the results must be equal."""
 import numpy as np
 import pytest

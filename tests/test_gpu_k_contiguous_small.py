@@ -1,12 +1,13 @@
-"""int8 matmuls of 17 to 64 rows on small K-contiguous weights, and of up to 16 where K is no multiple of 128, which one workgroup per column strip computes over all of K: every number of row blocks and column groups, waves
-without a step of K, K that ends inside a step, rows and columns past the end, a bias, strided activations; and shapes that stay with the narrow tiles. Small
-integers whose sums float16 holds: the results must be equal."""
+"""int8 matmuls of 17 to 64 rows on small K-contiguous weights, and of any number where K is no multiple of 128 (above 64, through the entry point alone, of 64), which one workgroup per column strip computes over
+all of K: waves without a step of K, K that ends inside a step, rows and columns past the end, a bias, strided activations; and shapes that stay with the narrow tiles (the
+variants of the kernel by name: test_gpu_strips.py). Small integers whose sums float16 holds: the results must be equal."""
 import numpy as np
 import pytest
 import torch
 
+from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
-from gpu_util import announce, dev
+from gpu_util import announce, dev, last_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +41,7 @@ def test_random_against_float64():
         x, scale = torch.randn((m, k), generator=g, device='cuda').half(), scale.half()
         want = (x.double() @ w.double()) * scale.double()
         got = quant.symmetric_quant_matmul(x, quant.to_decode_layout(w), scale).double()
+        assert 'skinny_w8a16_nk_tall_kernel' in last_launch()[0]
         # float32 sums of k products: at most 2^-24 log2(k) of the sum of their magnitudes each way, and half a unit of float16
         bound = (x.double().abs() @ w.double().abs()) * scale.double() * 2.0 ** -24 * (k / 128 + 12) + want.abs() * 2.0 ** -11 + 2.0 ** -24
         assert ((got - want).abs() <= bound).all()
@@ -53,3 +55,13 @@ def test_strided_activations():
         wide = torch.zeros((40, 1024 + pad), dtype=torch.float16, device='cuda')
         wide[:, :1024] = a
         assert torch.equal(quant.symmetric_quant_matmul(wide[:, :1024], w, one).float().cpu(), exact)
+
+
+@pytest.mark.parametrize('m', [65, 130, 201])
+def test_more_rows_of_k_off_the_stages_through_the_entry_point(m):
+    announce('int8 K-contiguous: more rows', m)
+    a, w, exact = _case(m, 1040, 516)
+    one, c = torch.ones(516, dtype=torch.float16, device='cuda'), torch.empty((m, 516), dtype=torch.float16, device='cuda')
+    ffi.call('hidet_symmetric_quant_matmul_f16_i8_nk', a, w.T.contiguous(), one, c, m, 1040, 516, 1040, 1040, None, 0, ffi.current_stream(a.device))
+    assert torch.equal(c.float().cpu(), exact)
+    assert 'skinny_w8a16_nk_tall_kernel' in last_launch()[0]

@@ -1,5 +1,6 @@
-"""int4 matmuls on small weights, which one workgroup per column strip computes over all of K: one to four row blocks, two and four columns per lane, eight and sixteen waves, several row tiles, waves without a
-step of K, groups of 64, 128 and more, columns past the end, a bias, strides; and sizes next to those that take this kernel. Small integers and scales of powers of
+"""int4 matmuls on small weights, which one workgroup per column strip computes over all of K: several row tiles, waves without a
+step of K, groups of 64, 128 and more, columns past the end, a bias, strides; and sizes next to those that take this kernel
+(its variants by name: test_gpu_strips.py). Small integers and scales of powers of
 two: the results must be equal."""
 import numpy as np
 import pytest

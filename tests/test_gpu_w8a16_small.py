@@ -1,6 +1,6 @@
-"""int8 matmuls on small row-major weights, which one workgroup per column strip computes over all of K: one to four row blocks, two and four columns per lane, several row
+"""int8 matmuls on small row-major weights, which one workgroup per column strip computes over all of K: several row
 tiles, waves without a step of K, K that ends inside a step, columns moved back into a row, rows of the weight at any alignment, a bias, strides; and sizes next to
-those that take this kernel. Small integers whose sums float16 holds: the results must be equal."""
+those that take this kernel (its variants by name: test_gpu_strips.py). Small integers whose sums float16 holds: the results must be equal."""
 import numpy as np
 import pytest
 import torch
