@@ -1,5 +1,5 @@
-"""int8 and int4 matmuls of up to 16 rows on the narrow tiles, where those are estimated to be ahead of the bandwidth-bound kernels: exact on small integers, on both
-sides of the choice, with part of a row block, a bias, strides, K in pieces and whole; the workspace is zero where it has to be; equal to what a captured graph
+"""int8 and int4 matmuls of up to 16 rows: on the narrow tiles, where those are estimated to be ahead of the bandwidth-bound kernels, and on what is ahead of them (strips on
+small weights). Exact on small integers, with part of a row block, a bias, strides, K in pieces and whole; the workspace is zero where it has to be; equal to what a captured graph
 computes; a wanted number of K parts still goes to the bandwidth-bound kernel."""
 import numpy as np
 import pytest
@@ -7,7 +7,7 @@ import torch
 
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
-from gpu_util import announce, dev
+from gpu_util import announce, dev, last_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +47,30 @@ def test_int4(m, k, n, group, dtype):
     assert torch.equal(got.cpu(), exact.to(ty))
 
 
+# sizes that the kernels of strips leave to the narrow tiles
+@pytest.mark.parametrize('m', [9, 15, 16])
+@pytest.mark.parametrize('k,n', [(2624, 132), (2880, 1000), (3002, 2500), (4096, 2048), (9152, 2640)])
+def test_int8_on_the_narrow_tiles(m, k, n):
+    announce('int8 decode batch on the narrow tiles', m, k, n)
+    a, q, exact = _int8(m, k, n, 1)
+    assert torch.equal(quant.symmetric_quant_matmul(a, q, torch.ones(n, dtype=torch.float16, device='cuda')).float().cpu(), exact)
+    assert 'gemm_mid_kernel' in last_launch()[0]
+    assert not ffi.workspace(a.device)[:65536 + (16 << 20)].any()
+
+
+@pytest.mark.parametrize('k,n,group', [(3072, 520, 128), (4096, 4096, 128), (6144, 1024, 64), (3840, 2504, 128)])
+def test_int4_on_the_narrow_tiles(k, n, group):
+    announce('int4 decode batch on the narrow tiles', k, n, group)
+    rng = np.random.default_rng(k + n)
+    a, q = rng.integers(-1, 2, (16, k)).astype(np.float32), rng.integers(-7, 8, (k, n))
+    packed = dev(((q[:, 0::2] & 15) | ((q[:, 1::2] & 15) << 4)).astype(np.uint8))
+    scales = 2.0 ** rng.integers(-2, 1, (k // group, n)).astype(np.float32)
+    exact = torch.from_numpy(a @ (q * np.repeat(scales, group, axis=0)).astype(np.float32))
+    got = quant.symmetric_quant_matmul_w4a16(dev(a).bfloat16(), packed, dev(scales).bfloat16(), group)
+    assert 'gemm_mid_kernel' in last_launch()[0]
+    assert torch.equal(got.cpu(), exact.bfloat16())
+
+
 def test_wanted_parts_and_strides():
     announce('int8 decode batch: parts, strides')
     a, q, exact = _int8(16, 2048, 2048)
@@ -78,4 +102,5 @@ def test_replayed_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got.float().cpu(), exact)
+        assert 'gemm_mid_kernel' in last_launch()[0]
         quant.symmetric_quant_matmul(a, q, one)
