@@ -412,8 +412,10 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
     }
 }
 
-// What a launch costs in microseconds: the workgroups of a CU one after the other, each with its fixed part, its rounds of
-// the groups and, where K is cut, the exchange of `parts` partial tiles. The coefficients are fits to the times of every tile height and
+// What a launch costs in microseconds: the workgroups of a CU one after the other, each with its fixed part and its rounds of
+// the groups, and, where K is cut, once the exchange of `parts` partial tiles: that of the first workgroups of a CU runs beside the next ones (counted with
+// each of them, pieces that take two and three turns were estimated 25 and 50 % too high: 1900 splits of two turns of int8 and int4 take 0.95 to 0.98 of this, 890 of three 0.93 to 0.94. int4
+// 171 x 9600 x 6016, in one and in three pieces, 55.6 and 50.5 us). The coefficients are fits to the times of every tile height and
 // number of pieces (430 to 1700 each) on 100 to 430 shapes of 17 to 1100 rows, K and N of 1024 to 11008 (FP8 8192), of which they leave 3 to 8 %;
 // not those of K-contiguous int8 and of int4 in groups of odd multiples of 32, which are older and stand for a slower exchange (the former 17 % too high).
 // The choices they make cost over the best tile and split, from the last-level cache and from memory: int8 0.4 and 1.6 % in the mean of 333 shapes, int4 0.3 and 0.3 of
@@ -440,13 +442,13 @@ MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_
     MidChoice best;
     for (int64_t p = 1; p <= std::max<int64_t>(1, most); ++p) {
         const int64_t rounds = cdiv(cdiv(stages, p), Cfg::kGroups), share = rounds * Cfg::kGroups, parts = cdiv(stages, share);
-        const double rest = cost.fixed + (parts > 1 ? cost.exchange + double(parts) * (cost.exchange_part + double(tiles) * cost.exchange_piece) : 0.0);
-        const double us = double(cdiv(tiles * parts, cus)) * (rest + double(rounds) * cost.round);
+        const double exchange = parts > 1 ? cost.exchange + double(parts) * (cost.exchange_part + double(tiles) * cost.exchange_piece) : 0.0;
+        const double us = double(cdiv(tiles * parts, cus)) * (cost.fixed + double(rounds) * cost.round) + exchange;
         if (us >= best.us) continue;
         const auto batch = [&](int64_t active) {  // workgroups side by side
-            return active == 0 ? 0.0 : rest + double(rounds) * std::max(cost.round, cost.full_round * double(active) / double(cus));
+            return active == 0 ? 0.0 : cost.fixed + double(rounds) * std::max(cost.round, cost.full_round * double(active) / double(cus));
         };
-        best = MidChoice{parts, share, us, double(tiles * parts / cus) * batch(cus) + batch(tiles * parts % cus)};
+        best = MidChoice{parts, share, us, double(tiles * parts / cus) * batch(cus) + batch(tiles * parts % cus) + exchange};
     }
     return best;
 }

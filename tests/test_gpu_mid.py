@@ -8,7 +8,7 @@ import torch
 from hidet_amd import ffi
 from hidet_amd.graph.ops import quant
 from hidet_amd.graph.ops.matmul import matmul_f8 as f8
-from gpu_util import announce, fastest_ms
+from gpu_util import announce, fastest_ms, last_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -189,3 +189,18 @@ def test_w8a16_few_rows_of_a_wide_ragged_weight(m):
     want = ((a.float() @ w.float()) * s.float()).half()
     assert torch.equal(quant.symmetric_quant_matmul(a, w, s), want)
     assert torch.equal(quant.symmetric_quant_matmul(a, w, s, b), (want.float() + b.float()).half())
+
+
+# Three pieces of K on 64-row tiles, although they take two turns of the chip (4 us less than whole tiles)
+@pytest.mark.parametrize('m,k,n', [(171, 9600, 6016), (433, 9472, 2560)])
+def test_w4a16_pieces_in_two_turns_of_the_chip(m, k, n):
+    announce('int4: pieces in two turns', m, k, n)
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m)
+    packed, scales, w = _int4(g, k, n, 128, torch.bfloat16)
+    x = _ints(g, (m, k), -1, 1).bfloat16()
+    got = quant.symmetric_quant_matmul_w4a16(x, packed, scales, 128)
+    name, workgroups, _ = last_launch()
+    tiles = -(-m // 64) * -(-n // 128)
+    assert 'gemm_mid_kernel' in name and workgroups == 8 * -(-3 * tiles // 8), (name, workgroups)
+    assert torch.equal(got, (x.double() @ w).to(torch.bfloat16))
