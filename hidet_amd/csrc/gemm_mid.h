@@ -421,7 +421,7 @@ __global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(const char *a, co
 // The choices they make cost over the best tile and split, from the last-level cache and from memory: int8 0.4 and 1.6 % in the mean of 333 shapes, int4 0.3 and 0.3 of
 // 202, FP8 0.6 and 0.4 of 427, block-scaled 0.5 and 0.7 of 424.
 // `full_round` (0: not known) is the least a round takes with every CU at work: the weights of a round then come at the
-// rate of the memory. `exchange_piece` (0: in the others): what every piece of the launch adds to an exchange, all of them meeting at the same time.
+// rate of the memory, once for all row tiles of a column tile (up to eight are in step). `exchange_piece` (0: in the others): what every piece of the launch adds to an exchange, all of them meeting at the same time.
 struct MidCost {
     double fixed, round, exchange, exchange_part, full_round, exchange_piece;
 };
@@ -435,7 +435,7 @@ struct MidChoice {
 template <class Op, int RB, int DEPTH>
 MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_t n, int64_t k) {
     using Cfg = MidCfg<Op, RB, DEPTH>;
-    const int64_t tiles = cdiv(m, RB * 16) * cdiv(n, Cfg::kPitch), stages = cdiv(k, Op::kStageK), cus = std::max(1, device_cus());
+    const int64_t row_tiles = cdiv(m, RB * 16), tiles = row_tiles * cdiv(n, Cfg::kPitch), stages = cdiv(k, Op::kStageK), cus = std::max(1, device_cus());
     int64_t most = 8;
     if (ws.counters == nullptr || tiles > cus) most = 1;
     else most = std::min(most, ws.scratch_bytes / (tiles * Cfg::kTileFloats * 4));
@@ -446,7 +446,7 @@ MidChoice mid_choose(const MidCost &cost, const Workspace &ws, int64_t m, int64_
         const double us = double(cdiv(tiles * parts, cus)) * (cost.fixed + double(rounds) * cost.round) + exchange;
         if (us >= best.us) continue;
         const auto batch = [&](int64_t active) {  // workgroups side by side
-            return active == 0 ? 0.0 : cost.fixed + double(rounds) * std::max(cost.round, cost.full_round * double(active) / double(cus));
+            return active == 0 ? 0.0 : cost.fixed + double(rounds) * std::max(cost.round, cost.full_round * double(active) / double(cus * std::min<int64_t>(8, row_tiles)));
         };
         best = MidChoice{parts, share, us, double(tiles * parts / cus) * batch(cus) + batch(tiles * parts % cus) + exchange};
     }
