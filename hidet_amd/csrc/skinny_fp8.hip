@@ -200,7 +200,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_fp8_staged_kernel(const uin
 
 // 17 rows and more, K a multiple of 16 (block-scaled 128), aligned activations: the kernel above for 16 RB rows x 16 CG columns per workgroup. A weight of a few megabytes is
 // read in less time than the narrow tiles (gemm_mid.h) take to fill their rings and to bring the pieces of K together: nothing is shared between waves here before the end, so
-// there is no barrier and no exchange, and a launch costs 2.5 us beside its loads. Those bound it, about 70 KB per us and CU from the L2: every workgroup reads its
+// there is no barrier and no exchange, and a launch costs 2.5 us beside its loads. Those bound it, about 60 KB per us and CU from the L2: every workgroup reads its
 // rows' activations for 16 or 32 columns only, so wide and deep matrices stay with the narrow tiles. Per-tensor scales, narrow tiles -> here, us, weights from
 // the last-level cache: 24 x 1024 x 1024 5.5 -> 2.9, 32 x 2048 x 2048 7.1 -> 3.6, 32 x 4096 x 4096 9.2 -> 5.8, 64 x 4096 x 4096 9.4 -> 7.4, 128 x 4096 x 1024 7.5 -> 5.2, 256 x
 // 2048 x 2048 7.4 -> 6.8; block-scaled 24 x 7168 x 1536 9.5 -> 7.0. One step of a wave in flight: with the next one's loads (two) in front of the multiplication

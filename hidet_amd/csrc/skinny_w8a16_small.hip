@@ -1,7 +1,7 @@
 // W8A16 on small row-major weights: c[m, n] = (sum_k a[m, k] * w[k, n]) * scale[n] (+ bias[n]), a workgroup per 16 RB rows and 16 CB columns (CB = 2 or 4) for all of K.
 //
 // The bandwidth-bound kernel and the narrow tiles (gemm_mid.h) read rows of 256 and 128 columns and therefore cut K between workgroups, whose exchange and rings take 5 us of
-// the 7 that a weight of 2 MB does. Here eight independent waves cut K and meet once, in LDS. What bounds it is what a CU gets from the L2, about 70 KB per us: few
+// the 7 that a weight of 2 MB does. Here eight independent waves cut K and meet once, in LDS. What bounds it is what a CU gets from the L2, about 60 KB per us: few
 // workgroups, each with its strip of the weight and all of its rows' activations.
 //
 // Per step of 128 k a lane (kg, ls) reads CB bytes of rows 32 s + 8 kg + j (s = 0 .. 3, j = 0 .. 7) at columns CB ls and on, whatever their alignment: 16 lanes
