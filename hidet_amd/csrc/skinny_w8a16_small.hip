@@ -143,7 +143,7 @@ bool skinny_w8a16_small_supported(const void *a, int64_t n, int64_t k, int64_t l
 // weights from memory and from the last-level cache. Weights of more than 8.5 MB or 2560 rows stay with the others: there the strips of rows that a workgroup reads of a weight
 // in memory cost more than the exchange that they save (1 x 2048 x 6144 8.2 us and 11.2 here, 16 x 3072 x 1024 7.1 and 8.5, 16 x 3072 x 3072 9.0 and 13.3; 64 x 3072 x 2260 27 % more, 16 x 2772
 // x 2572 18; K of 2601 to 2944 4 to 12 % less time from the cache and the same from memory). K of 1900 to 2600, 64 shapes: 14 to 27 % less time, 7 to 17 % from memory, there six of 64 more than 3 %
-// slower (4 to 7 %, 64 x 2296 x 2476 15).
+// slower (4 to 7 %; of 500 other shapes 71 x 2496 x 2048 9.5 us and 11.6 here, from the cache 9.0 and 6.4).
 // Within K = 2048, where this is ahead of the other kernels' estimates by 8 %, those 456 calls take 36 % less time in the mean (30 on weights from memory), and one of them in the former case and two in the latter take 3 to 4 % more.
 SkinnySmallPlan skinny_w8a16_small_plan(const void *a, int64_t m, int64_t n, int64_t k, int64_t lda) {
     SkinnySmallPlan best;
